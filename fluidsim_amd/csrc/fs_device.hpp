@@ -60,7 +60,7 @@ struct PcgScalars {
     int restarts;
     int mg_failed;      // coarse factorisation failed (the hierarchy must be rebuilt next time)
     int replace;        // check not triggered by the tolerance: refresh r from FP64, restart only on drift
-    int pad;
+    int flush;          // a check refreshed r from p + x: the next direction folds x into p
     double window_rmax; // true residual max-norm that started the current refinement window
     // r.z of the direction used by the iteration that starts at iteration count c, kept in slot c & 1:
     // the direction kernel reads the previous slot and writes the next one while other workgroups of
@@ -281,5 +281,83 @@ __device__ __forceinline__ double finish_max(const double* partials, int n, int 
     __syncthreads();
     return r;
 }
+
+// Block-wide sums of NC values in block_sum's order, one barrier for all; result valid in thread 0 (which
+// every thread may read again only after another barrier).  `lds` holds NC * blockDim/64 doubles.
+template <int NT, int NC> __device__ __forceinline__ void block_sums(double (&v)[NC], double* lds)
+{
+    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+#pragma unroll
+    for (int c = 0; c < NC; ++c) {
+        v[c] = wave_sum(v[c]);
+        if (lane == 0)
+            lds[c * (NT / 64) + wid] = v[c];
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+#pragma unroll
+        for (int c = 0; c < NC; ++c) {
+            double r = 0.0;
+#pragma unroll
+            for (int i = 0; i < NT / 64; ++i)
+                r += lds[c * (NT / 64) + i];
+            v[c] = r;
+        }
+    }
+}
+
+// The NC interleaved components of `n` partials reduced by every workgroup for itself, in finish_sum's order
+// (component c < NSUM summed, the others their maximum).  load() only issues the loads of up to kAhead strides,
+// through clamped indices, so that a kernel's other loads travel with them; finish() adds them up with two barriers
+// for all components, and every thread returns the values.
+template <int NT, int NC, int NSUM = NC> struct Partials {
+    static constexpr int kAhead = 4;
+    double t[kAhead][NC];
+    __device__ __forceinline__ void load(const double* partials, int n)
+    {
+#pragma unroll
+        for (int u = 0; u < kAhead; ++u)
+#pragma unroll
+            for (int c = 0; c < NC; ++c)
+                t[u][c] = load_partial(partials, min((int)threadIdx.x + u * NT, n - 1) * NC + c);
+    }
+    __device__ __forceinline__ void finish(const double* partials, int n, double (&out)[NC], double* lds)
+    {
+        double v[NC] = {};
+        auto add = [&](int c, double x) { v[c] = c < NSUM ? v[c] + x : fmax(v[c], x); };
+#pragma unroll
+        for (int u = 0; u < kAhead; ++u)
+#pragma unroll
+            for (int c = 0; c < NC; ++c)
+                if ((int)threadIdx.x + u * NT < n)
+                    add(c, t[u][c]);
+        for (int i = threadIdx.x + kAhead * NT; i < n; i += NT)
+#pragma unroll
+            for (int c = 0; c < NC; ++c)
+                add(c, load_partial(partials, i * NC + c));
+        const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+#pragma unroll
+        for (int c = 0; c < NC; ++c) {
+            v[c] = c < NSUM ? wave_sum(v[c]) : wave_max(v[c]);
+            if (lane == 0)
+                lds[c * (NT / 64) + wid] = v[c];
+        }
+        __syncthreads();
+#pragma unroll
+        for (int c = 0; c < NC; ++c) {
+            double r = 0.0;
+#pragma unroll
+            for (int k = 0; k < NT / 64; ++k)
+                r = c < NSUM ? r + lds[c * (NT / 64) + k] : fmax(r, lds[c * (NT / 64) + k]);
+            out[c] = r;
+        }
+        __syncthreads();
+    }
+    __device__ __forceinline__ void all(const double* partials, int n, double (&out)[NC], double* lds)
+    {
+        load(partials, n);
+        finish(partials, n, out, lds);
+    }
+};
 
 }  // namespace fsim

@@ -396,7 +396,7 @@ struct fs_context {
 };
 
 constexpr int kPressureBudget = 100000;   // PCG iterations of an unbounded (negative) budget
-constexpr size_t kFoldBlocks = 1536;      // cell blocks (64 x 16) beyond which PCG partials are pre-reduced
+constexpr int kFoldBlocks = 1024;         // workgroups of the PCG kernels beyond which partials are pre-reduced
 // Multigrid levels above this many cells take the grid's chosen smoother (fs_set_pressure_smoother); smaller
 // ones, the single-workgroup tail's levels among them, always run red-black V(4,4).
 constexpr long long kSmootherMinCells = 4096;
@@ -499,7 +499,7 @@ struct fs_grid {
     ViscositySolver* visc = nullptr;       // implicit viscosity workspace (created on first use)
     int vis_sweeps = 0;                    // fs_set_viscosity_smoother (0: the reference's V(2,2))
     DevBuf<double2> st_heights, st_orient, st_raw, st_curv;   // capillary geometry (first use)
-    DevBuf<float> x, r, d, q, zdiag;
+    DevBuf<float> x, r, d, d2, q, zdiag;
     DevBuf<unsigned char> solid;   // solid-mask extension (empty: no mask)
     DevBuf<float> color_px;        // writeColorPixels output, 4 floats per cell (first use)
     DevBuf<EditCell> edit_cells;   // resolved material edits of the last commit (first use)
@@ -570,6 +570,7 @@ struct fs_grid {
     }
 
     size_t N() const { return (size_t)W * H; }
+    size_t cell_tiles() const { return (size_t)((W + 63) / 64) * ((H + 15) / 16); }   // 64 x 16
     size_t NP() const { return (size_t)(W + 2) * (H + 2); }
     size_t NU() const { return (size_t)(W + 1) * H; }
     size_t NV() const { return (size_t)W * (H + 1); }
@@ -622,19 +623,24 @@ struct fs_grid {
         g.x = x.p;
         g.r = r.p;
         g.d = d.p;
+        g.d2 = d2.p;
         g.q = q.p;
         g.zdiag = zdiag.p;
         g.S = S.p;
         g.partials = partials.p;
-        const size_t blocks = (size_t)((W + 63) / 64) * ((H + 15) / 16);
+        const size_t blocks = cell_tiles();
         g.partials_ad = partials.p + 5 * blocks;
-        // every consumer workgroup reading every block's partial costs blocks^2 loads: past this many
-        // blocks (a 1024 x 1536 grid) one extra single-workgroup launch pre-reduces them
-        const bool fold = blocks > kFoldBlocks;
-        g.fold_ad = fold ? partials.p + 6 * blocks : g.partials_ad;
-        g.fold_ad_n = fold ? 1 : (int)blocks;
-        g.fold_rz = fold ? partials.p + 6 * blocks + 8 : partials.p;
-        g.fold_rz_n = fold ? 1 : (int)blocks;
+        g.partials_up = partials.p + 6 * blocks;
+        g.partials_tr = partials.p + 8 * blocks;
+        // every consumer workgroup reading every block's partial costs blocks^2 loads: past kFoldBlocks
+        // (four tiles each: 2048 x 2048) one extra single-workgroup launch pre-reduces them
+        const int loop_blocks = pcg_blocks(W, H);
+        const bool fold = loop_blocks > kFoldBlocks;
+        double* folded = partials.p + 10 * blocks;
+        g.fold_ad = fold ? folded : g.partials_ad;
+        g.fold_up = fold ? folded + 8 : g.partials_up;
+        g.fold_rz = fold ? folded + 16 : partials.p;
+        g.fold_ad_n = g.fold_up_n = g.fold_rz_n = fold ? 1 : loop_blocks;
         g.solid = solid.n ? solid.p : nullptr;
         return g;
     }
@@ -674,14 +680,14 @@ struct fs_grid {
         bytes += x.alloc(NPd);
         bytes += r.alloc(NPd);
         bytes += d.alloc(NPd);
+        bytes += d2.alloc(NPd);
         bytes += q.alloc(NPd);
         bytes += zdiag.alloc(NPd);
         bytes += S.alloc(1);
         bytes += S_aux.alloc(1);
-        const size_t blocks = (size_t)((W + 63) / 64) * ((H + 15) / 16);
-        // region A: up to five partials per cell block; region B (after it): the operator's d.q partials,
-        // read by the update kernel while it writes region A; then 16 slots of pre-reduced sums
-        bytes += partials.alloc(6 * blocks + 64);
+        // up to five partials per cell block, then the operator's d.q, the update's and the check's partials
+        // (read while the next kernel writes its own), then the pre-reduced sums
+        bytes += partials.alloc(10 * cell_tiles() + 64);
         build_hierarchy();
         tune_tiles();
         if (smoother == FS_SMOOTHER_CHEBYSHEV)
@@ -1345,13 +1351,11 @@ struct fs_grid {
     void iteration_kernels()
     {
         GridDev g = dev();
-        launch_pcg_ad(st(), g);
+        launch_pcg_direction_ad(st(), g, z_ptr(), flexible());
         launch_pcg_update(st(), g);
-        launch_flush(st(), g);
-        launch_true_residual(st(), g, 1);
+        launch_pcg_check(st(), g);
         precondition(status_ptr());
         launch_pcg_rz(st(), g, z_ptr(), flexible());
-        launch_pcg_direction(st(), g, z_ptr(), flexible());
     }
 
     void ensure_graph()
@@ -1375,7 +1379,7 @@ struct fs_grid {
     }
 
     // FluidGridCPU::project (FluidGridCPU.cpp:1030-1124), first phase: scalar block, coefficients,
-    // hierarchy, rhs, predicted pressure, its residual and the first direction -- launches only.
+    // hierarchy, rhs, predicted pressure, its residual and the first V-cycle -- launches only.
     void project_begin(double dt, int max_iterations, double tol)
     {
         const double scale = h * h / dt;
@@ -1407,7 +1411,7 @@ struct fs_grid {
         launch_zero_pressure(st(), g);
         launch_predict(st(), g);
         launch_sub_mean_p(st(), g, 0);
-        launch_true_residual(st(), g, 0);
+        launch_true_residual(st(), g);
         if (rebuild) {
             if (late_tail) {
                 HIPC(hipStreamWaitEvent(st(), ctx->join_levels, 0));
@@ -1428,7 +1432,6 @@ struct fs_grid {
             precondition(status_ptr());
         }
         launch_pcg_rz(st(), g, z_ptr(), flexible());
-        launch_pcg_direction(st(), g, z_ptr(), flexible());
     }
 
     // Last phase: fold the correction into the pressure, remove its mean, correct the velocity and
@@ -3371,13 +3374,19 @@ fs_status fs_time_kernel(fs_grid* grid, int kernel, int reps, double* ms_per_lau
             g.bytes += g.calib_src.alloc(kCalibWords);
             g.bytes += g.calib_dst.alloc(kCalibWords);
         }
+        if (kernel == 1 || kernel == 2 || kernel == 8) {
+            // positive r.z and d.q, so that the timed kernels do not find the solve stopped
+            const std::vector<double> ones(g.partials.n, 1.0);
+            HIPC(hipStreamSynchronize(g.st()));
+            device_upload(g.partials.p, ones.data(), ones.size() * sizeof(double));
+        }
         auto launch_once = [&](int i) {
             switch (kernel) {
             case 10: launch_copy_f32(g.st(), g.calib_src.p, g.calib_dst.p, kCalibWords); break;
             case 0:  // the finest post-smoothing launch of a V-cycle (prolongation + four sweeps)
                 g.fine_post_smooth(i & 1);
                 break;
-            case 1: launch_pcg_ad(g.st(), gd); break;
+            case 1: launch_pcg_direction_ad(g.st(), gd, g.levels[0].sol0.p); break;
             case 2: launch_pcg_update(g.st(), gd); break;
             case 3: launch_copy_f32(g.st(), g.r.p, g.q.p, g.NP()); break;
             case 4:  // second level's smoother (or the finest, if the tail starts at level 1)
@@ -3452,6 +3461,7 @@ static void batch_projection(fs_context* ctx, fs_grid* const* grids, const std::
             const int i = batched[(size_t)k];
             fs_grid& g = *grids[i];
             g.project_begin(dts[i], fs_grid::budget(max_iterations[i]), tolerances[i]);
+            launch_pcg_direction(st, g.dev(), g.z_ptr(), g.flexible());
             desc[(size_t)k] = g.batch_instance();
             if (g.precond == FS_PRECOND_MULTIGRID)
                 lds = std::max(lds, g.tail_lds);
@@ -3772,7 +3782,7 @@ fs_status fs_grid_estimate_bytes(int width, int height, int n_liquid, int n_gas,
         const size_t NP = (W + 2) * (H + 2), nl = (size_t)n_liquid, ng = (size_t)n_gas;
         const size_t blocks = ((W + 63) / 64) * ((H + 15) / 16);
         // state, pressure history, PCG vectors and reductions (fs_grid::allocate)
-        size_t b = 8 * (3 * N + NU + NV + 3 * NP) + 4 * 5 * NP + 8 * (6 * blocks + 64) +
+        size_t b = 8 * (3 * N + NU + NV + 3 * NP) + 4 * 6 * NP + 8 * (10 * blocks + 64) +
                    4 * sizeof(PcgScalars) + 8 * (nl + ng) * N;
         // pressure hierarchy (build_hierarchy): FP64 + FP32 conductances, 1/diag, rhs, two solutions,
         // residual, transfer tables; dense coarse factor and inverse; tail tables

@@ -327,14 +327,12 @@ __global__ __launch_bounds__(kNT) void k_sub_mean_p(GridDev g, int final_pass)
             g.p[T.P[k]] = pv[k] - mean;
 }
 
-// True residual r = b - A p in FP64 (FP64 weights), stored as the FP32 working residual.
-// mode 0: initial residual of the predicted pressure.  mode 1: verification of a recurrence that
-// reached the tolerance; accept (converged) or restart from the true residual.
-__global__ __launch_bounds__(kNT) void k_true_residual(GridDev g, int mode)
+// True residual r = b - A p of the predicted pressure in FP64 (FP64 weights), stored as the FP32 working
+// residual.
+__global__ __launch_bounds__(kNT) void k_true_residual(GridDev g)
 {
-    __shared__ double lds[kNT / 64];
-    const int st = g.S->status;
-    if (st != kRunning || (mode == 1 && !g.S->verify))
+    __shared__ double lds[2 * kNT / 64];
+    if (g.S->status != kRunning)
         return;
     const int s = g.s;
     const Tile4 T = tile4(g.W, g.H, s);
@@ -352,8 +350,7 @@ __global__ __launch_bounds__(kNT) void k_true_residual(GridDev g, int mode)
     for (int k = 0; k < 4; ++k) {
         if (T.in[k]) {
             g.r[T.P[k]] = (float)r[k];
-            if (mode == 0)
-                g.x[T.P[k]] = 0.0f;
+            g.x[T.P[k]] = 0.0f;
             sum += r[k];
             m = fmax(m, fabs(r[k]));
         }
@@ -363,28 +360,6 @@ __global__ __launch_bounds__(kNT) void k_true_residual(GridDev g, int mode)
     if (threadIdx.x == 0) {
         g.partials[2 * block_id()] = bs;
         g.partials[2 * block_id() + 1] = bm;
-    }
-}
-
-// Fold the FP32 correction into the FP64 pressure before a true-residual check.
-__global__ __launch_bounds__(kNT) void k_flush(GridDev g)
-{
-    if (g.S->status != kRunning || !g.S->verify)
-        return;
-    const Tile4 T = tile4(g.W, g.H, g.s);
-    double pv[4];
-    float xv[4];
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-        pv[k] = g.p[T.P[k]];
-        xv[k] = g.x[T.P[k]];
-    }
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-        if (T.in[k]) {
-            g.p[T.P[k]] = pv[k] + (double)xv[k];
-            g.x[T.P[k]] = 0.0f;
-        }
     }
 }
 
@@ -637,77 +612,196 @@ __global__ __launch_bounds__(kNT) void k_pad_copy(const double* src, double* dst
 // PCG loop (FluidGridCPU.cpp:1779-1819) with FP32 vectors and FP64 scalars.
 // ------------------------------------------------------------------------------------------
 
-// q = A d (5-point, variable coefficient; walls have zero weight), d.q, then alpha.
-__global__ __launch_bounds__(kNT) void k_pcg_ad(GridDev g)
+// A workgroup of the loop kernels takes G tiles of 64 x 16 cells, one below the other: G = 1 spreads a small
+// grid over the compute units, G = 4 keeps the number of partials that every consumer workgroup reads
+// small on a large one (pcg_groups).
+__device__ __forceinline__ Tile4 tile4_group(int W, int H, int s, int group)
 {
-    __shared__ double lds[kNT / 64];
-    const int s = g.s;
-    const float* d = g.d;
-    const Tile4 T = tile4(g.W, g.H, s);
-    float c[4], q[4];
+    Tile4 t;
+    const int x = blockIdx.x * kTX + (threadIdx.x & 63);
+    const int xc = min(x, W - 1);
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
-        const int i = T.P[k];
-        c[k] = d[i];
-        const float dl = d[i - 1], dr = d[i + 1], du = d[i - s], dd = d[i + s];
-        const float wl = g.right32[i - 1], wr = g.right32[i], wu = g.down32[i - s], wd = g.down32[i];
-        q[k] = (wl * (c[k] - dl) + wr * (c[k] - dr)) + (wu * (c[k] - du) + wd * (c[k] - dd));
+        const int y = group * kTY + (threadIdx.x >> 6) + 4 * k;
+        t.in[k] = x < W && y < H;
+        t.P[k] = pidx(xc, min(y, H - 1), s);
     }
-    if (g.S->status != kRunning)
-        return;
-    double dot = 0.0;
+    return t;
+}
+
+// The direction of iteration c lives in d or d2 by the parity of c: the fused direction and operator kernel
+// reads its neighbours' old values while other workgroups write new ones.
+__device__ __forceinline__ float* direction_of(const GridDev& g, int c) { return c & 1 ? g.d2 : g.d; }
+
+// The next direction from the r.z sums: every workgroup reduces the partials itself (same order, same
+// value): beta = next / previous r.z (zero after a restart), or with FLEX the Polak-Ribiere
+// -alpha (z - mean z).q / previous r.z.  Workgroup 0 records the new r.z in the next slot and stops the solve
+// on a non-positive r.z (the budget stops it at the check).  Returns false when the solve stops.
+template <bool FLEX>
+__device__ __forceinline__ bool next_direction(const GridDev& g, const double (&t)[FLEX ? 5 : 3], bool first,
+    float& mean, double& beta64)
+{
+    const double n = (double)g.W * g.H;
+    const double zmean = t[0] / n;
+    const double next = t[1] - zmean * t[2];
+    const int c = g.S->iterations;
+    double numerator = next;
+    if constexpr (FLEX)
+        numerator = -g.S->alpha * (t[3] - zmean * t[4]);
+    beta64 = g.S->restart ? 0.0 : numerator / g.S->rz_slot[(c + 1) & 1];
+    const bool stop = !isfinite(beta64) || !(c < g.S->max_iterations && next > 0.0 && isfinite(next));
+    if (first && threadIdx.x == 0) {
+        g.S->z_mean = zmean;
+        g.S->beta = beta64;
+        if (isfinite(beta64))
+            g.S->rz_slot[c & 1] = next;
+        if (stop)
+            g.S->status = kStopped;
+    }
+    mean = (float)zmean;
+    return !stop;
+}
+
+// d = (z - mean z) + beta d and q = A d (5-point, variable coefficient; walls have zero weight), d.q.
+// One launch where there were two: it reads z and the old d once more around each tile (66 x 18 cells for 64 x 16,
+// 66 x 66 for four) instead of writing d and reading it back, and a launch of a small grid costs about
+// 4 us whatever it does.  A check that refreshed r left x to be folded into p: done here.
+template <bool FLEX, int G> __global__ __launch_bounds__(kNT) void k_pcg_direction_ad(GridDev g, const float* z)
+{
+    constexpr int LX = kTX + 2, LY = kTY * G + 2;
+    __shared__ double lds[5 * kNT / 64];
+    __shared__ float s_d[LY * LX];
+    const int s = g.s, W = g.W, H = g.H;
+    const int x0 = blockIdx.x * kTX - 1, y0 = blockIdx.y * kTY * G - 1;
+    constexpr int LOADS = (LX * LY + kNT - 1) / kNT;
+    constexpr int NP = FLEX ? 5 : 3;
+    Partials<kNT, NP> sums;
+    sums.load(g.fold_rz, g.fold_rz_n);
+    float zv[LOADS], dv[LOADS];
+    int at[LOADS];
+    // clamped to the zero halo: the values of cells outside the grid meet zero weights only
 #pragma unroll
-    for (int k = 0; k < 4; ++k) {
-        if (T.in[k]) {
-            g.q[T.P[k]] = q[k];
-            dot += (double)c[k] * (double)q[k];
+    for (int it = 0; it < LOADS; ++it) {
+        const int e = min((int)threadIdx.x + it * kNT, LX * LY - 1);
+        const int ly = e / LX, lx = e - ly * LX;
+        at[it] = pidx(min(x0 + lx, W), min(y0 + ly, H), s);
+        zv[it] = z[at[it]];
+    }
+    const int st = g.S->status;
+    const int c = g.S->iterations;
+    const float* d_old = direction_of(g, c + 1);
+    float* d_new = direction_of(g, c);
+#pragma unroll
+    for (int it = 0; it < LOADS; ++it)
+        dv[it] = d_old[at[it]];
+    double t[NP];
+    sums.finish(g.fold_rz, g.fold_rz_n, t, lds);
+    if (st != kRunning)
+        return;
+    float mean;
+    double beta64;
+    if (!next_direction<FLEX>(g, t, block_id() == 0, mean, beta64))
+        return;
+    const float beta = (float)beta64;
+#pragma unroll
+    for (int it = 0; it < LOADS; ++it) {
+        const int e = threadIdx.x + it * kNT;
+        if (e < LX * LY) {
+            const float zz = zv[it] - mean;
+            s_d[e] = beta64 == 0.0 ? zz : zz + beta * dv[it];
         }
     }
-    const double bs = block_sum<kNT>(dot, lds);
-    if (threadIdx.x == 0)
-        g.partials_ad[block_id()] = bs;
-}
-
-// Large grids: one workgroup reduces the per-block partials (stride components) into out[0 .. stride),
-// with the same fixed-order finish_sum every consumer workgroup would otherwise repeat over all blocks.
-__global__ __launch_bounds__(kNT) void k_fold_partials(const double* partials, int nb, int stride, double* out)
-{
-    __shared__ double lds[kNT / 64];
-    for (int c = 0; c < stride; ++c) {
-        const double v = finish_sum<kNT>(partials, nb, stride, c, lds);
-        if (threadIdx.x == 0)
-            out[c] = v;
-    }
-}
-
-// x += alpha d ; r -= alpha q ; residual sum and max-norm; convergence test of the recurrence.
-// Every workgroup first reduces the operator's d.q partials itself (same order, same value) and forms
-// alpha; workgroup 0 records it, clears the restart flag the previous direction consumed, and stops
-// the solve on a non-positive d.q.
-__global__ __launch_bounds__(kNT) void k_pcg_update(GridDev g)
-{
-    __shared__ double lds[kNT / 64];
-    const Tile4 T = tile4(g.W, g.H, g.s);
-    float xv[4], dv[4], rv[4], qv[4];
+    const bool fold = g.S->flush != 0;
+    __syncthreads();
+    double dot[1] = {0.0};
 #pragma unroll
-    for (int k = 0; k < 4; ++k) {
-        const int i = T.P[k];
-        xv[k] = g.x[i];
-        dv[k] = g.d[i];
-        rv[k] = g.r[i];
-        qv[k] = g.q[i];
+    for (int group = 0; group < G; ++group) {
+        const Tile4 T = tile4_group(W, H, s, blockIdx.y * G + group);
+        float dc[4], q[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const int i = T.P[k];
+            const float wl = g.right32[i - 1], wr = g.right32[i], wu = g.down32[i - s], wd = g.down32[i];
+            const int e = (group * kTY + (threadIdx.x >> 6) + 4 * k + 1) * LX + (threadIdx.x & 63) + 1;
+            dc[k] = s_d[e];
+            const float dl = s_d[e - 1], dr = s_d[e + 1], du = s_d[e - LX], dd = s_d[e + LX];
+            q[k] = (wl * (dc[k] - dl) + wr * (dc[k] - dr)) + (wu * (dc[k] - du) + wd * (dc[k] - dd));
+        }
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            if (T.in[k]) {
+                d_new[T.P[k]] = dc[k];
+                g.q[T.P[k]] = q[k];
+                dot[0] += (double)dc[k] * (double)q[k];
+            }
+        }
+        if (fold) {
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                if (T.in[k]) {
+                    g.p[T.P[k]] += (double)g.x[T.P[k]];
+                    g.x[T.P[k]] = 0.0f;
+                }
+            }
+        }
     }
-    if (g.S->status != kRunning)
+    block_sums<kNT, 1>(dot, lds);
+    if (threadIdx.x == 0)
+        g.partials_ad[block_id()] = dot[0];
+}
+
+// Large grids: one workgroup reduces the per-block partials (NC components, the first NSUM summed) into
+// out[0 .. NC), in the order every consumer workgroup would otherwise repeat over all blocks.
+template <int NC, int NSUM>
+__global__ __launch_bounds__(kNT) void k_fold_partials(const double* partials, int nb, double* out)
+{
+    __shared__ double lds[NC * kNT / 64];
+    double t[NC];
+    Partials<kNT, NC, NSUM>().all(partials, nb, t, lds);
+    if (threadIdx.x == 0)
+#pragma unroll
+        for (int c = 0; c < NC; ++c)
+            out[c] = t[c];
+}
+
+// x += alpha d ; r -= alpha q ; residual sum and max-norm.
+// Every workgroup first reduces the operator's d.q partials itself (same order, same value) and forms
+// alpha; workgroup 0 records it, clears the flags the previous direction consumed, and stops
+// the solve on a non-positive d.q.
+template <int G> __global__ __launch_bounds__(kNT) void k_pcg_update(GridDev g)
+{
+    __shared__ double lds[2 * kNT / 64];
+    Partials<kNT, 1> dot;
+    dot.load(g.fold_ad, g.fold_ad_n);
+    const int st = g.S->status;
+    const int c = g.S->iterations;
+    const float* d = direction_of(g, c);
+    Tile4 T = tile4_group(g.W, g.H, g.s, blockIdx.y * G);
+    float xv[4], dv[4], rv[4], qv[4];
+    auto load = [&] {
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const int i = T.P[k];
+            xv[k] = g.x[i];
+            dv[k] = d[i];
+            rv[k] = g.r[i];
+            qv[k] = g.q[i];
+        }
+    };
+    load();
+    const double rz = g.S->rz_slot[c & 1];
+    double dq[1];
+    dot.finish(g.fold_ad, g.fold_ad_n, dq, lds);
+    if (st != kRunning)
         return;
-    const double dq = finish_sum<kNT>(g.fold_ad, g.fold_ad_n, 1, 0, lds);
-    const double rz = g.S->rz_slot[g.S->iterations & 1];
-    bool stop = dq <= 0.0 || !isfinite(dq);
-    const double alpha64 = stop ? 0.0 : rz / dq;
+    bool stop = dq[0] <= 0.0 || !isfinite(dq[0]);
+    const double alpha64 = stop ? 0.0 : rz / dq[0];
     stop = stop || !isfinite(alpha64);
     if (block_id() == 0 && threadIdx.x == 0) {
-        g.S->dq = dq;
+        g.S->dq = dq[0];
         g.S->alpha = alpha64;
         g.S->restart = 0;
+        g.S->flush = 0;
         if (stop)
             g.S->status = kStopped;
     }
@@ -716,21 +810,87 @@ __global__ __launch_bounds__(kNT) void k_pcg_update(GridDev g)
     const float alpha = (float)alpha64;
     double sum = 0.0, m = 0.0;
 #pragma unroll
-    for (int k = 0; k < 4; ++k) {
-        if (T.in[k]) {
-            const int i = T.P[k];
-            g.x[i] = xv[k] + alpha * dv[k];
-            const float r = rv[k] - alpha * qv[k];
-            g.r[i] = r;
-            sum += (double)r;
-            m = fmax(m, (double)fabsf(r));
+    for (int group = 0; group < G; ++group) {
+        if (group) {
+            T = tile4_group(g.W, g.H, g.s, blockIdx.y * G + group);
+            load();
+        }
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            if (T.in[k]) {
+                const int i = T.P[k];
+                g.x[i] = xv[k] + alpha * dv[k];
+                const float r = rv[k] - alpha * qv[k];
+                g.r[i] = r;
+                sum += (double)r;
+                m = fmax(m, (double)fabsf(r));
+            }
         }
     }
     const double bs = block_sum<kNT>(sum, lds);
     const double bm = block_max<kNT>(m, lds);
     if (threadIdx.x == 0) {
-        g.partials[2 * block_id()] = bs;
-        g.partials[2 * block_id() + 1] = bm;
+        g.partials_up[2 * block_id()] = bs;
+        g.partials_up[2 * block_id() + 1] = bm;
+    }
+}
+
+// What the update's residual (sum, max-norm) calls for: a check of the true residual when the recurrence
+// reached the tolerance, or a refresh of r (replace) when it dropped far enough or ran long enough.
+struct Recurrence {
+    double rmax;
+    bool verify, replace;
+};
+__device__ __forceinline__ Recurrence recurrence(const PcgScalars* S, const double (&t)[2])
+{
+    Recurrence c;
+    c.rmax = isfinite(t[0]) ? t[1] : INFINITY;
+    const bool done = c.rmax <= S->tol;
+    c.replace = !done && (c.rmax <= kRefineDrop * S->window_rmax || (S->iterations + 1) % kReplaceEvery == 0);
+    c.verify = done || c.replace;
+    return c;
+}
+
+// The check: every workgroup reduces the update's partials itself and, where they call for it, forms the FP64
+// true residual b - A (p + x) as the new working residual.  p and x stay as they are (the neighbours read them):
+// the next direction folds x into p.  The scalar block is written by the finish launch alone.
+template <int G> __global__ __launch_bounds__(kNT) void k_pcg_check(GridDev g)
+{
+    __shared__ double lds[2 * kNT / 64];
+    const int st = g.S->status;
+    double t[2];
+    Partials<kNT, 2, 1>().all(g.fold_up, g.fold_up_n, t, lds);
+    if (st != kRunning || !recurrence(g.S, t).verify)
+        return;
+    const int s = g.s;
+    double sum = 0.0, m = 0.0;
+#pragma unroll 1
+    for (int group = 0; group < G; ++group) {
+        const Tile4 T = tile4_group(g.W, g.H, s, blockIdx.y * G + group);
+        double r[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const int i = T.P[k];
+            auto at = [&](int j) { return g.p[j] + (double)g.x[j]; };
+            const double c = at(i);
+            const double product = (g.right64[i - 1] * (c - at(i - 1)) + g.right64[i] * (c - at(i + 1))) +
+                                   (g.down64[i - s] * (c - at(i - s)) + g.down64[i] * (c - at(i + s)));
+            r[k] = g.b[i] - product;
+        }
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            if (T.in[k]) {
+                g.r[T.P[k]] = (float)r[k];
+                sum += r[k];
+                m = fmax(m, fabs(r[k]));
+            }
+        }
+    }
+    const double bs = block_sum<kNT>(sum, lds);
+    const double bm = block_max<kNT>(m, lds);
+    if (threadIdx.x == 0) {
+        g.partials_tr[2 * block_id()] = bs;
+        g.partials_tr[2 * block_id() + 1] = bm;
     }
 }
 
@@ -757,48 +917,43 @@ __global__ __launch_bounds__(kNT) void k_precond_diag(GridDev g)
 // FLEX (flexible CG, for a preconditioner that is not exactly linear): also sum z.q and q, from which
 // the direction kernel forms the Polak-Ribiere beta z_new.(r_new - r_old) / r_old.z_old with
 // r_new - r_old = -alpha q (Notay 2000).
-template <bool FLEX> __global__ __launch_bounds__(kNT) void k_pcg_rz(GridDev g, const float* z)
+template <bool FLEX, int G> __global__ __launch_bounds__(kNT) void k_pcg_rz(GridDev g, const float* z)
 {
-    __shared__ double lds[kNT / 64];
     constexpr int NP = FLEX ? 5 : 3;
-    const Tile4 T = tile4(g.W, g.H, g.s);
-    float zv[4], rv[4], qv[4];
+    __shared__ double lds[NP * kNT / 64];
+    const int st = g.S->status;
+    double sums[NP] = {};
 #pragma unroll
-    for (int k = 0; k < 4; ++k) {
-        zv[k] = z[T.P[k]];
-        rv[k] = g.r[T.P[k]];
-        qv[k] = FLEX ? g.q[T.P[k]] : 0.f;
-    }
-    if (g.S->status != kRunning)
-        return;
-    double sz = 0.0, srz = 0.0, sr = 0.0, szq = 0.0, sq = 0.0;
+    for (int group = 0; group < G; ++group) {
+        const Tile4 T = tile4_group(g.W, g.H, g.s, blockIdx.y * G + group);
+        float zv[4], rv[4], qv[4];
 #pragma unroll
-    for (int k = 0; k < 4; ++k) {
-        if (T.in[k]) {
-            const double zz = (double)zv[k], rr = (double)rv[k];
-            sz += zz;
-            srz += rr * zz;
-            sr += rr;
-            if (FLEX) {
-                szq += zz * (double)qv[k];
-                sq += (double)qv[k];
+        for (int k = 0; k < 4; ++k) {
+            zv[k] = z[T.P[k]];
+            rv[k] = g.r[T.P[k]];
+            qv[k] = FLEX ? g.q[T.P[k]] : 0.f;
+        }
+        if (st != kRunning)
+            return;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            if (T.in[k]) {
+                const double zz = (double)zv[k], rr = (double)rv[k];
+                sums[0] += zz;
+                sums[1] += rr * zz;
+                sums[2] += rr;
+                if constexpr (FLEX) {
+                    sums[3] += zz * (double)qv[k];
+                    sums[4] += (double)qv[k];
+                }
             }
         }
     }
-    const double b0 = block_sum<kNT>(sz, lds);
-    const double b1 = block_sum<kNT>(srz, lds);
-    const double b2 = block_sum<kNT>(sr, lds);
-    const double b3 = FLEX ? block_sum<kNT>(szq, lds) : 0.0;
-    const double b4 = FLEX ? block_sum<kNT>(sq, lds) : 0.0;
-    if (threadIdx.x == 0) {
-        g.partials[NP * block_id()] = b0;
-        g.partials[NP * block_id() + 1] = b1;
-        g.partials[NP * block_id() + 2] = b2;
-        if (FLEX) {
-            g.partials[NP * block_id() + 3] = b3;
-            g.partials[NP * block_id() + 4] = b4;
-        }
-    }
+    block_sums<kNT, NP>(sums, lds);
+    if (threadIdx.x == 0)
+#pragma unroll
+        for (int c = 0; c < NP; ++c)
+            g.partials[NP * block_id() + c] = sums[c];
 }
 
 // d = (z - mean z) + beta d.  Every workgroup reduces the r.z partials itself (same order, same
@@ -860,18 +1015,16 @@ template <bool FLEX> __global__ __launch_bounds__(kNT) void k_pcg_direction(Grid
 // boundaries instead of a device-scope fence in every producer block.
 // ------------------------------------------------------------------------------------------
 enum FinishOp : int {
-    kFinRhs = 0, kFinRhsCenter, kFinPredict, kFinTrueRes0, kFinTrueRes1, kFinFinalSum, kFinDiv, kFinAd,
-    kFinUpdate, kFinRz, kFinDivDone
+    kFinRhs = 0, kFinRhsCenter, kFinPredict, kFinTrueRes0, kFinCheck, kFinFinalSum, kFinDiv, kFinDivDone
 };
 
 __global__ __launch_bounds__(kNT) void k_finish(GridDev g, int op, int nb)
 {
-    __shared__ double lds[kNT / 64];
+    __shared__ double lds[2 * kNT / 64];
     PcgScalars* S = g.S;
     const int st = S->status;
     bool run;
     switch (op) {
-    case kFinTrueRes1: run = st == kRunning && S->verify; break;
     case kFinFinalSum: run = st == kConverged || st == kStopped; break;
     case kFinDiv: run = true; break;
     case kFinDivDone: run = st != kRunning; break;
@@ -906,37 +1059,55 @@ __global__ __launch_bounds__(kNT) void k_finish(GridDev g, int op, int nb)
             S->p_mean = t / n;
         break;
     }
-    case kFinTrueRes0:
-    case kFinTrueRes1: {
-        const double total = finish_sum<kNT>(P, nb, 2, 0, lds);
-        double maximum = finish_max<kNT>(P, nb, 2, 1, lds);
+    case kFinTrueRes0: {
+        double t[2];
+        Partials<kNT, 2, 1>().all(P, nb, t, lds);
         if (threadIdx.x == 0) {
-            if (!isfinite(total))
-                maximum = INFINITY;
+            const double maximum = isfinite(t[0]) ? t[1] : INFINITY;
             S->true_rmax = maximum;
-            S->r_sum = total;
-            if (op == kFinTrueRes0) {
-                S->rmax = maximum;
-                S->initial_rmax = maximum;
-                S->window_rmax = maximum;
-                S->r_mean = total / n;
-                if (maximum <= S->tol || S->max_iterations == 0)
-                    S->status = kInitialOk;
-            } else {
+            S->r_sum = t[0];
+            S->rmax = maximum;
+            S->initial_rmax = maximum;
+            S->window_rmax = maximum;
+            S->r_mean = t[0] / n;
+            if (maximum <= S->tol || S->max_iterations == 0)
+                S->status = kInitialOk;
+        }
+        break;
+    }
+    case kFinCheck: {
+        // the update's residual norm; where it called for a check, the true residual's verdict as well
+        double t[2];
+        Partials<kNT, 2, 1>().all(g.fold_up, g.fold_up_n, t, lds);
+        const Recurrence c = recurrence(S, t);
+        double e[2] = {0.0, 0.0};
+        if (c.verify)
+            Partials<kNT, 2, 1>().all(g.partials_tr, nb, e, lds);
+        if (threadIdx.x == 0) {
+            S->iterations += 1;
+            S->rmax = c.rmax;
+            S->r_sum = t[0];
+            S->r_mean = t[0] / n;
+            if (c.verify) {
+                const double maximum = isfinite(e[0]) ? e[1] : INFINITY;
+                S->true_rmax = maximum;
+                S->r_sum = e[0];
+                S->flush = 1;
                 if (maximum <= S->tol) {
                     S->status = kConverged;
                 } else {
-                    S->r_mean = total / n;
-                    if (!S->replace || maximum > kDriftRatio * S->rmax) {
+                    S->r_mean = e[0] / n;
+                    if (!c.replace || maximum > kDriftRatio * c.rmax) {
                         S->restart = 1;
                         S->restarts += 1;
                     }
                     S->rmax = maximum;
                     S->window_rmax = maximum;
                 }
-                S->verify = 0;
-                S->replace = 0;
             }
+            // out of budget: the next direction would never be used
+            if (S->status == kRunning && S->iterations >= S->max_iterations)
+                S->status = kStopped;
         }
         break;
     }
@@ -945,61 +1116,6 @@ __global__ __launch_bounds__(kNT) void k_finish(GridDev g, int op, int nb)
         const double t = finish_max<kNT>(P, nb, 1, 0, lds);
         if (threadIdx.x == 0)
             S->div_max = t;
-        break;
-    }
-    case kFinAd: {
-        const double total = finish_sum<kNT>(P, nb, 1, 0, lds);
-        if (threadIdx.x == 0) {
-            S->dq = total;
-            if (total <= 0.0 || !isfinite(total)) {
-                S->status = kStopped;
-            } else {
-                const double alpha = S->rz / total;
-                if (!isfinite(alpha))
-                    S->status = kStopped;
-                S->alpha = alpha;
-            }
-        }
-        break;
-    }
-    case kFinUpdate: {
-        const double total = finish_sum<kNT>(P, nb, 2, 0, lds);
-        double maximum = finish_max<kNT>(P, nb, 2, 1, lds);
-        if (threadIdx.x == 0) {
-            if (!isfinite(total))
-                maximum = INFINITY;
-            S->iterations += 1;
-            S->rmax = maximum;
-            S->r_sum = total;
-            S->r_mean = total / n;
-            if (maximum <= S->tol) {
-                S->verify = 1;
-            } else if (maximum <= kRefineDrop * S->window_rmax || S->iterations % kReplaceEvery == 0) {
-                S->verify = 1;
-                S->replace = 1;
-            }
-        }
-        break;
-    }
-    case kFinRz: {
-        const double tz = finish_sum<kNT>(P, nb, 3, 0, lds);
-        const double trz = finish_sum<kNT>(P, nb, 3, 1, lds);
-        const double tr = finish_sum<kNT>(P, nb, 3, 2, lds);
-        if (threadIdx.x == 0) {
-            const double mean = tz / n;
-            const double next = trz - mean * tr;
-            S->z_mean = mean;
-            const double beta = S->restart ? 0.0 : next / S->rz;
-            S->beta = beta;
-            S->restart = 0;
-            if (!isfinite(beta)) {
-                S->status = kStopped;
-            } else {
-                S->rz = next;
-                if (!(S->iterations < S->max_iterations && next > 0.0 && isfinite(next)))
-                    S->status = kStopped;
-            }
-        }
         break;
     }
     default:
@@ -1133,16 +1249,10 @@ void launch_sub_mean_p(hipStream_t st, const GridDev& g, int final_pass)
     hipLaunchKernelGGL(k_sub_mean_p, cell_grid(g.W, g.H), dim3(kNT), 0, st, g, final_pass);
 }
 
-void launch_true_residual(hipStream_t st, const GridDev& g, int mode)
+void launch_true_residual(hipStream_t st, const GridDev& g)
 {
-    hipLaunchKernelGGL(k_true_residual, cell_grid(g.W, g.H), dim3(kNT), 0, st, g, mode);
-    hipLaunchKernelGGL(k_finish, dim3(1), dim3(kNT), 0, st, g, mode == 0 ? (int)kFinTrueRes0 : (int)kFinTrueRes1,
-        (int)cell_blocks(g.W, g.H));
-}
-
-void launch_flush(hipStream_t st, const GridDev& g)
-{
-    hipLaunchKernelGGL(k_flush, cell_grid(g.W, g.H), dim3(kNT), 0, st, g);
+    hipLaunchKernelGGL(k_true_residual, cell_grid(g.W, g.H), dim3(kNT), 0, st, g);
+    hipLaunchKernelGGL(k_finish, dim3(1), dim3(kNT), 0, st, g, (int)kFinTrueRes0, (int)cell_blocks(g.W, g.H));
 }
 
 void launch_final_flush_sum(hipStream_t st, const GridDev& g)
@@ -1205,29 +1315,84 @@ void launch_pad_copy(hipStream_t st, const double* src, double* dst, int W, int 
     hipLaunchKernelGGL(k_pad_copy, cell_grid(W, H), dim3(kNT), 0, st, src, dst, W, H, to_padded);
 }
 
-void launch_pcg_ad(hipStream_t st, const GridDev& g)
+// Tiles per workgroup of the loop kernels: a consumer workgroup reads every producer workgroup's partial, blocks^2
+// loads in all, which shows past about a thousand workgroups; four tiles each keep a 2048 x 2048 grid at 1024.
+// k_fold_partials takes over beyond kFoldBlocks of those.
+int pcg_groups(int W, int H) { return cell_blocks(W, H) > 1024 ? 4 : 1; }
+int pcg_blocks(int W, int H)
 {
-    hipLaunchKernelGGL(k_pcg_ad, cell_grid(g.W, g.H), dim3(kNT), 0, st, g);
+    return ((W + kTX - 1) / kTX) * (((H + kTY - 1) / kTY + pcg_groups(W, H) - 1) / pcg_groups(W, H));
+}
+
+static dim3 loop_grid(const GridDev& g)
+{
+    const int G = pcg_groups(g.W, g.H);
+    return dim3((g.W + kTX - 1) / kTX, ((g.H + kTY - 1) / kTY + G - 1) / G);
+}
+
+void launch_pcg_direction_ad(hipStream_t st, const GridDev& g, const float* z, int flexible)
+{
+    const dim3 grid = loop_grid(g);
+    if (pcg_groups(g.W, g.H) == 1) {
+        if (flexible)
+            hipLaunchKernelGGL((k_pcg_direction_ad<true, 1>), grid, dim3(kNT), 0, st, g, z);
+        else
+            hipLaunchKernelGGL((k_pcg_direction_ad<false, 1>), grid, dim3(kNT), 0, st, g, z);
+    } else {
+        if (flexible)
+            hipLaunchKernelGGL((k_pcg_direction_ad<true, 4>), grid, dim3(kNT), 0, st, g, z);
+        else
+            hipLaunchKernelGGL((k_pcg_direction_ad<false, 4>), grid, dim3(kNT), 0, st, g, z);
+    }
     if (g.fold_ad_n == 1)
-        hipLaunchKernelGGL(k_fold_partials, dim3(1), dim3(kNT), 0, st, (const double*)g.partials_ad,
-            (int)cell_blocks(g.W, g.H), 1, g.fold_ad);
+        hipLaunchKernelGGL((k_fold_partials<1, 1>), dim3(1), dim3(kNT), 0, st, (const double*)g.partials_ad,
+            (int)(grid.x * grid.y), g.fold_ad);
 }
 
 void launch_pcg_update(hipStream_t st, const GridDev& g)
 {
-    hipLaunchKernelGGL(k_pcg_update, cell_grid(g.W, g.H), dim3(kNT), 0, st, g);
-    hipLaunchKernelGGL(k_finish, dim3(1), dim3(kNT), 0, st, g, (int)kFinUpdate, (int)cell_blocks(g.W, g.H));
+    const dim3 grid = loop_grid(g);
+    if (pcg_groups(g.W, g.H) == 1)
+        hipLaunchKernelGGL(k_pcg_update<1>, grid, dim3(kNT), 0, st, g);
+    else
+        hipLaunchKernelGGL(k_pcg_update<4>, grid, dim3(kNT), 0, st, g);
+    if (g.fold_up_n == 1)
+        hipLaunchKernelGGL((k_fold_partials<2, 1>), dim3(1), dim3(kNT), 0, st, (const double*)g.partials_up,
+            (int)(grid.x * grid.y), g.fold_up);
+}
+
+void launch_pcg_check(hipStream_t st, const GridDev& g)
+{
+    const dim3 grid = loop_grid(g);
+    if (pcg_groups(g.W, g.H) == 1)
+        hipLaunchKernelGGL(k_pcg_check<1>, grid, dim3(kNT), 0, st, g);
+    else
+        hipLaunchKernelGGL(k_pcg_check<4>, grid, dim3(kNT), 0, st, g);
+    hipLaunchKernelGGL(k_finish, dim3(1), dim3(kNT), 0, st, g, (int)kFinCheck, (int)(grid.x * grid.y));
 }
 
 void launch_pcg_rz(hipStream_t st, const GridDev& g, const float* z, int flexible)
 {
-    if (flexible)
-        hipLaunchKernelGGL(k_pcg_rz<true>, cell_grid(g.W, g.H), dim3(kNT), 0, st, g, z);
-    else
-        hipLaunchKernelGGL(k_pcg_rz<false>, cell_grid(g.W, g.H), dim3(kNT), 0, st, g, z);
-    if (g.fold_rz_n == 1)
-        hipLaunchKernelGGL(k_fold_partials, dim3(1), dim3(kNT), 0, st, (const double*)g.partials,
-            (int)cell_blocks(g.W, g.H), flexible ? 5 : 3, g.fold_rz);
+    const dim3 grid = loop_grid(g);
+    if (pcg_groups(g.W, g.H) == 1) {
+        if (flexible)
+            hipLaunchKernelGGL((k_pcg_rz<true, 1>), grid, dim3(kNT), 0, st, g, z);
+        else
+            hipLaunchKernelGGL((k_pcg_rz<false, 1>), grid, dim3(kNT), 0, st, g, z);
+    } else {
+        if (flexible)
+            hipLaunchKernelGGL((k_pcg_rz<true, 4>), grid, dim3(kNT), 0, st, g, z);
+        else
+            hipLaunchKernelGGL((k_pcg_rz<false, 4>), grid, dim3(kNT), 0, st, g, z);
+    }
+    if (g.fold_rz_n == 1) {
+        if (flexible)
+            hipLaunchKernelGGL((k_fold_partials<5, 5>), dim3(1), dim3(kNT), 0, st, (const double*)g.partials,
+                (int)(grid.x * grid.y), g.fold_rz);
+        else
+            hipLaunchKernelGGL((k_fold_partials<3, 3>), dim3(1), dim3(kNT), 0, st, (const double*)g.partials,
+                (int)(grid.x * grid.y), g.fold_rz);
+    }
 }
 
 void launch_pcg_direction(hipStream_t st, const GridDev& g, const float* z, int flexible)

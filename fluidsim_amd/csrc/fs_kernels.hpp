@@ -25,18 +25,23 @@ struct GridDev {
     float* invd32;            // padded 1/diagonal (FP32), level 0 and the diagonal preconditioner
     float* x;                 // padded FP32 correction accumulated since the last flush
     float* r;                 // padded FP32 residual
-    float* d;                 // padded FP32 direction
+    float* d;                 // padded FP32 direction (of the even iterations; the batched solve's only one)
+    float* d2;                // padded FP32 direction of the odd iterations
     float* q;                 // padded FP32 A d
     float* zdiag;             // padded FP32 diagonal-preconditioned residual
     PcgScalars* S;            // device scalar block
-    double* partials;         // reduction partials (>= 4 * max blocks)
+    double* partials;         // reduction partials (up to five per block)
     double* partials_ad;      // d.q partials of the operator kernel (one per block)
-    // Where the update and direction kernels read the d.q and r.z partials, and how many blocks' worth:
+    double* partials_up;      // residual sum and max-norm of the update kernel (two per block)
+    double* partials_tr;      // the same of the true-residual check
+    // Where the consumers of the d.q, update and r.z partials read them, and how many blocks' worth:
     // the producers' own per-block partials (every consumer workgroup reduces them: cheap while the
     // grid has few blocks), or, on large grids, one pre-reduced entry written by k_fold_partials (the
     // same fixed-order sum, so the result is identical).
     double* fold_ad;
     int fold_ad_n;
+    double* fold_up;
+    int fold_up_n;
     double* fold_rz;
     int fold_rz_n;
     const unsigned char* solid;   // W * H, nonzero = solid cell (solid-mask extension); null: no mask
@@ -134,8 +139,7 @@ void launch_rhs_center(hipStream_t st, const GridDev& g);
 void launch_zero_pressure(hipStream_t st, const GridDev& g);
 void launch_predict(hipStream_t st, const GridDev& g);
 void launch_sub_mean_p(hipStream_t st, const GridDev& g, int only_if_loop);
-void launch_true_residual(hipStream_t st, const GridDev& g, int mode);  // 0 initial, 1 verify
-void launch_flush(hipStream_t st, const GridDev& g);                     // only when S->verify
+void launch_true_residual(hipStream_t st, const GridDev& g);   // of the predicted pressure
 void launch_final_flush_sum(hipStream_t st, const GridDev& g);
 void launch_correct_velocity(hipStream_t st, const GridDev& g, double dt);
 // when_stopped: measure only once the grid's solve has stopped (otherwise a no-op).
@@ -179,11 +183,18 @@ struct EditCell {
 void launch_commit_edits(hipStream_t st, const GridDev& g, const EditCell* cells, int n);
 
 // ---- PCG loop (FP32 vectors, FP64 reductions) ----
-void launch_pcg_ad(hipStream_t st, const GridDev& g);
+// Tiles per workgroup of these kernels and the number of their workgroups (partials per component).
+int pcg_groups(int W, int H);
+int pcg_blocks(int W, int H);
+// The next direction from z and the r.z partials, and the operator on it with d.q.
+void launch_pcg_direction_ad(hipStream_t st, const GridDev& g, const float* z, int flexible = 0);
 void launch_pcg_update(hipStream_t st, const GridDev& g);
+// The true residual where the update's residual norm calls for it, and the iteration's bookkeeping.
+void launch_pcg_check(hipStream_t st, const GridDev& g);
 // flexible: Polak-Ribiere beta from z.q (for a V-cycle with bfloat16 vectors, not exactly linear); the
 // two kernels of one iteration must agree on it (it changes the partials' layout).
 void launch_pcg_rz(hipStream_t st, const GridDev& g, const float* z, int flexible = 0);
+// The direction alone, into d (the first one of a batched solve).
 void launch_pcg_direction(hipStream_t st, const GridDev& g, const float* z, int flexible = 0);
 void launch_precond_diag(hipStream_t st, const GridDev& g);
 
