@@ -36,18 +36,16 @@ METRIC = "MGPCG solves/s to 1e-6 rel. residual (1024², mixed batch); p50/p99 st
 # (c = 4 bytes per FP32 level value): bilinear prolongation 2.25c (read the coarse correction, read and
 # write the fine solution) plus nu sweeps of 5c each (read solution, rhs and the two face conductances,
 # write solution; a red-black sweep or a Jacobi sweep alike) = 22.25c = 89 B at nu = 4.  The kernels fuse
-# all passes through LDS, so their HBM traffic (measured with rocprofv3 counters) is far lower than this.
+# all passes in registers, so their HBM traffic (measured with rocprofv3 counters) is far lower than this.
 def smooth_bytes_per_cell(nu=4):
     return (2.25 + 5.0 * nu) * 4.0
 
 
 SMOOTH_BYTES_PER_CELL = smooth_bytes_per_cell(4)
-# Tile variants (tx, ty, threads) of the fused smoothers, as fs_mg_level_tiles numbers them.
-RB_VARIANTS = {0: (64, 32, 256), 1: (32, 32, 256), 2: (32, 16, 256), 3: (16, 16, 256), 4: (64, 32, 512),
-               5: (32, 32, 512), 6: (32, 32, 384), 7: (64, 32, 640), 8: (32, 64, 640), 9: (64, 32, 960),
-               10: (32, 64, 960)}
-JACOBI_VARIANTS = {0: (64, 32, 512), 1: (32, 32, 256), 2: (32, 16, 256), 3: (16, 16, 256), 4: (32, 32, 512),
-                   5: (64, 64, 1024), 6: (64, 32, 1024), 7: (32, 64, 1024)}
+# Tiles of the post-smoothing kernel k_rows as fs_mg_level_tiles numbers them: lanes per row, wavefronts and rows per lane
+# group (a tile of 2 lanes x (64 wavefronts / lanes x rows) cells, halo included).
+POST_TILES = [(64, 8, 8), (64, 16, 4), (32, 8, 4), (32, 16, 2), (32, 4, 4), (32, 8, 2), (16, 4, 2), (16, 4, 4), (64, 8, 4),
+              (64, 16, 8), (16, 8, 2)]
 HBM_PEAK_GBS = 8000.0
 PROFILES = os.path.join(HERE, "profiles")
 TRACE_PROFILE = os.path.join(HERE, "profiles", "bench_1024_kernel_trace.md")
@@ -837,15 +835,12 @@ def main():
     # Dominant kernel: the finest-level post-smoothing launch, timed with HIP events on the grid's stream.
     post_variant = grid.multigridTiles(0)[1]
     chebyshev = kind == FS_SMOOTHER_CHEBYSHEV
+    fine_kernel = "k_rows<{},1,{},{},{}>".format(int(chebyshev), *POST_TILES[post_variant])
     if chebyshev:
-        tx, ty, nt = JACOBI_VARIANTS[post_variant]
-        fine_kernel = f"k_jacobi_multi<{tx},{ty},1,{nt}>"
         smoother = (f"Chebyshev-weighted damped Jacobi, {nu} sweeps per side, on the levels above 4096 cells "
                     f"(red-black Gauss-Seidel, {coarse} sweeps per side, below)")
         fine_what = f"finest-level prolongation + {nu} Chebyshev-weighted Jacobi sweeps, autotuned tile"
     else:
-        tx, ty, nt = RB_VARIANTS[post_variant]
-        fine_kernel = f"k_rb_multi<{tx},{ty},4,{1 if post_variant in (0, 4) else 0},1,{nt},float,float,float>"
         smoother = f"red-black Gauss-Seidel, {nu} sweeps per side on the levels above 4096 cells ({coarse} below)"
         fine_what = f"finest-level prolongation + {nu} red-black Gauss-Seidel sweeps, autotuned tile"
     sweep_ms = grid.timeKernel(0, args.kernel_reps)

@@ -269,12 +269,10 @@ struct Level {
     // solutions of levels 1 .. tail start
     DevBuf<unsigned short> right16, down16, rhs16, sol16a, sol16b;
 
-    int smooth_variant = 0;     // tile of k_rb_multi pre-smoothing on this level (autotuned)
-    int post_variant = 0;       // tile of k_rb_multi prolongation + post-smoothing (autotuned)
-    int restrict_variant = 0;   // tile of k_res_restrict from this level (autotuned)
-    int jacobi_pre = 0;         // tiles of k_jacobi_multi pre- and post-smoothing (autotuned on first use)
-    int jacobi_post = 0;
-    int jacobi_fused = -1;      // k_jacobi_res_restrict tile for pre-smoothing + restriction; -1: two launches
+    // launch choices of the level's smoothers (autotuned; Chebyshev's on first use), as fs_mg_level_tiles numbers them
+    int smooth_variant = 0, post_variant = 0;   // red-black
+    int jacobi_pre = 0, jacobi_post = 0;        // Chebyshev
+    int restrict_variant = 0;                   // of the separate restriction launch
 
     size_t padded() const { return (size_t)s * (h + 2); }
 };
@@ -410,6 +408,21 @@ float chebyshev_weight(int i, int sweeps)
 {
     const double pi = 3.14159265358979323846;
     return (float)(1.0 / (1.1 + 0.9 * std::cos(pi * (i + 0.5) / sweeps)));
+}
+
+// Launch choices of a level's smoothers, as fs_mg_level_tiles numbers them: the tile of the post-smoothing, and the
+// pre-smoothing apart from the restriction (a tile of its own) or fused with it.
+constexpr int kRedBlackChoices = 11, kChebyshevChoices = 11, kChebyshevTiles = 8;
+struct PreChoice {
+    bool fused;
+    int tile;
+};
+PreChoice pre_choice(bool chebyshev, int id)
+{
+    constexpr int apart[5] = {0, 1, 2, 4, 6}, together[3] = {0, 2, 5};
+    if (chebyshev)
+        return id < kChebyshevTiles ? PreChoice{false, id} : PreChoice{true, together[id - kChebyshevTiles]};
+    return id < 5 ? PreChoice{false, apart[id]} : PreChoice{true, id - 5};
 }
 constexpr size_t kBatchSpreadLds = 84 * 1024;   // LDS of a batched-solve workgroup: one per compute unit
 
@@ -689,7 +702,7 @@ struct fs_grid {
         // (read while the next kernel writes its own), then the pre-reduced sums
         bytes += partials.alloc(10 * cell_tiles() + 64);
         build_hierarchy();
-        tune_tiles();
+        tune_for_precision();
         if (smoother == FS_SMOOTHER_CHEBYSHEV)
             tune_jacobi();
     }
@@ -1024,151 +1037,16 @@ struct fs_grid {
         return CoarseLinkT<VC>{csol, Cl.s, F.d_pxf.p, F.d_pxs.p, F.d_pxw.p, F.d_pyf.p, F.d_pys.p, F.d_pyw.p};
     }
 
-    // Pre-smoothing (from_zero) or prolongation + post-smoothing of tiled level l with 16-bit storage;
-    // VL is the vector type of levels >= 1.
-    template <class C, class VL> void smooth16(int l, int cur, int first_color, int from_zero, const int* status,
-        int variant)
+    // Tiled level l in the storage of the current mode: C conductances (16-bit modes) or the FP32 level.
+    template <class C, class V> LevelViewT<C, V> level_of(int l)
     {
-        const CoarseLinkT<VL> link = from_zero ? CoarseLinkT<VL>{} : link_t<VL>(l);
-        if (l == 0)
-            launch_rb_multi_t<C, float, VL>(st(), view_t<C, float>(0), cur, r.p, rmean_ptr(), first_color, from_zero,
-                link, status, variant, sweeps_on(l));
-        else {
-            const LevelViewT<C, VL> L = view_t<C, VL>(l);
-            launch_rb_multi_t<C, VL, VL>(st(), L, cur, L.rhs, nullptr, first_color, from_zero, link, status, variant,
-                sweeps_on(l));
-        }
-    }
-
-    template <class C, class VL> void restrict16(int l, int cur, const int* status, int variant)
-    {
-        const Level& F = levels[l];
-        const AxisRestrict rx{F.d_rxc.p, F.d_rxi.p, F.d_rxw.p};
-        const AxisRestrict ry{F.d_ryc.p, F.d_ryi.p, F.d_ryw.p};
-        if (l == 0)
-            launch_res_restrict_t<C, float, VL>(st(), view_t<C, float>(0), cur, r.p, rmean_ptr(), view_t<C, VL>(1), rx,
-                ry, status, variant);
-        else {
-            const LevelViewT<C, VL> L = view_t<C, VL>(l);
-            launch_res_restrict_t<C, VL, VL>(st(), L, cur, L.rhs, nullptr, view_t<C, VL>(l + 1), rx, ry, status,
-                variant);
-        }
-    }
-
-    template <class C, class VL> void vcycle16(const int* status)
-    {
-        const int T = tail_start;
-        for (int l = 0; l < T; ++l) {
-            smooth16<C, VL>(l, 0, 0, 1, status, levels[l].smooth_variant);
-            restrict16<C, VL>(l, 1, status, levels[l].restrict_variant);
-        }
-        join_before_tail();
-        launch_mg_tail(st(), tail, tail_lds, nullptr, status, std::is_same<VL, bf16>::value);
-        for (int l = T - 1; l >= 0; --l)
-            smooth16<C, VL>(l, 1, 1, 0, status, levels[l].post_variant);
-    }
-
-    template <class C, class VL> void tune_tiles16()
-    {
-        auto time = [&](auto&& launch) {
-            launch();
-            HIPC(hipEventRecord(ctx->ev0, st()));
-            for (int k = 0; k < 3; ++k)
-                launch();
-            HIPC(hipEventRecord(ctx->ev1, st()));
-            HIPC(hipEventSynchronize(ctx->ev1));
-            float ms = 0.f;
-            HIPC(hipEventElapsedTime(&ms, ctx->ev0, ctx->ev1));
-            return ms;
-        };
-        for (int l = 0; l < tail_start; ++l) {
-            Level& F = levels[l];
-            auto pick = [&](int count, auto&& launch) {
-                float best = std::numeric_limits<float>::infinity();
-                int choice = 0;
-                for (int v = 0; v < count; ++v) {
-                    const float ms = time([&] { launch(v); });
-                    if (ms < best) {
-                        best = ms;
-                        choice = v;
-                    }
-                }
-                return choice;
-            };
-            F.smooth_variant = pick(kSmoothVariants, [&](int v) { smooth16<C, VL>(l, 0, 0, 1, nullptr, v); });
-            F.post_variant = pick(kSmoothVariants, [&](int v) { smooth16<C, VL>(l, 1, 1, 0, nullptr, v); });
-            F.restrict_variant = pick(kRestrictVariants, [&](int v) { restrict16<C, VL>(l, 0, nullptr, v); });
-        }
-        drop_graph();
-    }
-
-    void tune_for_precision()
-    {
-        if (!active16())
-            tune_tiles();
-        else if (mg_prec == FS_MG_FP16)
-            tune_tiles16<half16, float>();
-        else if (mg_prec == FS_MG_BF16)
-            tune_tiles16<bf16, float>();
+        if constexpr (std::is_same<C, float>::value)
+            return view(l);
         else
-            tune_tiles16<bf16, bf16>();
+            return view_t<C, V>(l);
     }
 
-    // The finest post-smoothing launch of a V-cycle in the grid's storage mode (kernel timing).
-    void fine_post_smooth(int cur)
-    {
-        if (mg_prec == FS_MG_FP16 && active16())
-            smooth16<half16, float>(0, cur, 1, 0, nullptr, levels[0].post_variant);
-        else if (mg_prec == FS_MG_BF16 && active16())
-            smooth16<bf16, float>(0, cur, 1, 0, nullptr, levels[0].post_variant);
-        else if (active16())
-            smooth16<bf16, bf16>(0, cur, 1, 0, nullptr, levels[0].post_variant);
-        else if (tail_start > 0)
-            smooth_level(0, cur, r.p, rmean_ptr(), false, link_t<float>(0), nullptr, -1);
-        else
-            launch_rb_multi(st(), view(0), cur, r.p, rmean_ptr(), 1, 0, CoarseLink{}, nullptr, 1, levels[0].post_variant);
-    }
-
-    // One V(4,4) cycle on the residual r (minus its mean) into levels[0].sol0.
-    void vcycle(const int* status)
-    {
-        if (active16()) {
-            if (mg_prec == FS_MG_FP16)
-                vcycle16<half16, float>(status);
-            else if (mg_prec == FS_MG_BF16)
-                vcycle16<bf16, float>(status);
-            else
-                vcycle16<bf16, bf16>(status);
-            return;
-        }
-        const int T = tail_start;
-        const CoarseLink none{};
-        for (int l = 0; l < T; ++l) {
-            LevelView L = view(l);
-            const float* rhs = l == 0 ? r.p : L.rhs;
-            const double* shift = l == 0 ? rmean_ptr() : nullptr;
-            const Level& F = levels[l];
-            AxisRestrict rx{F.d_rxc.p, F.d_rxi.p, F.d_rxw.p};
-            AxisRestrict ry{F.d_ryc.p, F.d_ryi.p, F.d_ryw.p};
-            if (chebyshev_on(l) && F.jacobi_fused >= 0) {
-                launch_jacobi_res_restrict(st(), L, 0, rhs, shift, chebyshev_weights(true), smooth_sweeps, view(l + 1),
-                    rx, ry, status, F.jacobi_fused);
-                continue;
-            }
-            smooth_level(l, 0, rhs, shift, true, none, status, -1);
-            launch_res_restrict(st(), L, 1, rhs, shift, view(l + 1), rx, ry, status, F.restrict_variant);
-        }
-        join_before_tail();
-        launch_mg_tail(st(), tail, tail_lds, T == 0 ? rmean_ptr() : nullptr, status);
-        for (int l = T - 1; l >= 0; --l) {
-            LevelView L = view(l);
-            const float* rhs = l == 0 ? r.p : L.rhs;
-            const double* shift = l == 0 ? rmean_ptr() : nullptr;
-            smooth_level(l, 1, rhs, shift, false, link_t<float>(l), status, -1);
-        }
-    }
-
-    // Smoother of tiled level l: the chosen one above kSmootherMinCells cells, red-black V(4,4) below.
+    // Smoother of tiled level l: the chosen one above kSmootherMinCells cells, red-black with the coarse sweeps below.
     bool chebyshev_on(int l) const
     {
         return smoother == FS_SMOOTHER_CHEBYSHEV && (long long)levels[l].w * levels[l].h > kSmootherMinCells;
@@ -1185,23 +1063,68 @@ struct fs_grid {
             wt.w[pre ? k : smooth_sweeps - 1 - k] = chebyshev_weight(k, smooth_sweeps);
         return wt;
     }
-    // Pre-smoothing (from zero: reads nothing, writes sol[cur ^ 1]) or prolongation + post-smoothing of
-    // tiled level l in FP32 storage; variant -1 takes the level's tuned tile.
-    void smooth_level(int l, int cur, const float* rhs, const double* shift, bool pre, const CoarseLink& link,
-        const int* status, int variant)
+
+    // Pre-smoothing of tiled level l from zero into sol[1], its residual and the restriction to level l + 1; VL is the
+    // vector type of levels >= 1 (level 0's rhs and solution are the FP32 residual and z in every mode).
+    template <class C, class V, class VC>
+    void descend_level(int l, const V* rhs, const double* shift, const int* status, bool chebyshev, int nu, int id,
+        int restrict_id)
     {
         const Level& F = levels[l];
-        if (chebyshev_on(l)) {
-            launch_jacobi_multi(st(), view(l), cur, rhs, shift, pre ? 1 : 0, chebyshev_weights(pre), smooth_sweeps,
-                link, status, variant >= 0 ? variant : pre ? F.jacobi_pre : F.jacobi_post);
+        const LevelViewT<C, V> L = level_of<C, V>(l);
+        const LevelViewT<C, VC> Cl = level_of<C, VC>(l + 1);
+        const AxisRestrict rx{F.d_rxc.p, F.d_rxi.p, F.d_rxw.p};
+        const AxisRestrict ry{F.d_ryc.p, F.d_ryi.p, F.d_ryw.p};
+        const SmoothWeights wt = chebyshev ? chebyshev_weights(true) : SmoothWeights{};
+        const PreChoice pre = pre_choice(chebyshev, id);
+        if (pre.fused) {
+            launch_smooth_restrict(st(), chebyshev, L, 0, rhs, shift, wt, nu, Cl, rx, ry, status, pre.tile);
         } else {
-            launch_rb_multi(st(), view(l), cur, rhs, shift, pre ? 0 : 1, pre ? 1 : 0, link, status, l == 0,
-                variant >= 0 ? variant : pre ? F.smooth_variant : F.post_variant, sweeps_on(l));
+            launch_smooth(st(), chebyshev, L, 0, rhs, shift, 1, wt, nu, CoarseLinkT<VC>{}, status, pre.tile);
+            launch_res_restrict(st(), L, 1, rhs, shift, Cl, rx, ry, status, restrict_id);
+        }
+    }
+    template <class C, class VL>
+    void descend(int l, const int* status, bool chebyshev, int nu, int id, int restrict_id)
+    {
+        if (l == 0)
+            descend_level<C, float, VL>(l, r.p, rmean_ptr(), status, chebyshev, nu, id, restrict_id);
+        else
+            descend_level<C, VL, VL>(l, level_of<C, VL>(l).rhs, nullptr, status, chebyshev, nu, id, restrict_id);
+    }
+    // Prolongation of level l + 1's solution and post-smoothing of tiled level l, from sol[cur] into sol[cur ^ 1].
+    template <class C, class VL> void ascend(int l, int cur, const int* status, bool chebyshev, int nu, int id)
+    {
+        const SmoothWeights wt = chebyshev ? chebyshev_weights(false) : SmoothWeights{};
+        if (l == 0)
+            launch_smooth(st(), chebyshev, level_of<C, float>(0), cur, (const float*)r.p, rmean_ptr(), 0, wt, nu,
+                link_t<VL>(0), status, id);
+        else {
+            const LevelViewT<C, VL> L = level_of<C, VL>(l);
+            launch_smooth(st(), chebyshev, L, cur, (const VL*)L.rhs, nullptr, 0, wt, nu, link_t<VL>(l), status, id);
         }
     }
 
-    // Autotuner of the Chebyshev smoother's tiles (first use): every variant on each level's buffers.
-    void tune_jacobi()
+    template <class C, class VL> void vcycle_t(const int* status)
+    {
+        const int T = tail_start;
+        for (int l = 0; l < T; ++l) {
+            const Level& F = levels[l];
+            const bool chebyshev = chebyshev_on(l);
+            descend<C, VL>(l, status, chebyshev, sweeps_on(l), chebyshev ? F.jacobi_pre : F.smooth_variant,
+                F.restrict_variant);
+        }
+        join_before_tail();
+        launch_mg_tail(st(), tail, tail_lds, T == 0 ? rmean_ptr() : nullptr, status, std::is_same<VL, bf16>::value);
+        for (int l = T - 1; l >= 0; --l) {
+            const bool chebyshev = chebyshev_on(l);
+            ascend<C, VL>(l, 1, status, chebyshev, sweeps_on(l), chebyshev ? levels[l].jacobi_post : levels[l].post_variant);
+        }
+    }
+
+    // Autotuner: times every launch choice of a level's smoother on the level's own buffers and keeps the fastest.
+    // All of them compute the same values, so the choice affects time only.
+    template <class C, class VL> void tune_levels(bool chebyshev)
     {
         auto time = [&](auto&& launch) {
             launch();
@@ -1214,109 +1137,86 @@ struct fs_grid {
             HIPC(hipEventElapsedTime(&ms, ctx->ev0, ctx->ev1));
             return ms;
         };
-        const CoarseLink none{};
-        const SmoothWeights pre = chebyshev_weights(true), post = chebyshev_weights(false);
+        auto pick = [&](int count, auto&& launch) {
+            float best = std::numeric_limits<float>::infinity();
+            int choice = 0;
+            for (int v = 0; v < count; ++v) {
+                const float ms = time([&] { launch(v); });
+                if (ms < best) {
+                    best = ms;
+                    choice = v;
+                }
+            }
+            return choice;
+        };
         for (int l = 0; l < tail_start; ++l) {
             Level& F = levels[l];
-            if ((long long)F.w * F.h <= kSmootherMinCells)
+            if (chebyshev && (long long)F.w * F.h <= kSmootherMinCells)
                 continue;
-            const LevelView L = view(l);
-            const float* rhs = l == 0 ? r.p : L.rhs;
-            const CoarseLink link = link_t<float>(l);
-            float best = std::numeric_limits<float>::infinity();
-            for (int v = 0; v < kJacobiVariants; ++v) {
-                const float ms = time([&] { launch_jacobi_multi(st(), L, 0, rhs, nullptr, 1, pre, smooth_sweeps, none, nullptr, v); });
-                if (ms < best) {
-                    best = ms;
-                    F.jacobi_pre = v;
-                }
-            }
-            best = std::numeric_limits<float>::infinity();
-            for (int v = 0; v < kJacobiVariants; ++v) {
-                const float ms = time([&] { launch_jacobi_multi(st(), L, 1, rhs, nullptr, 0, post, smooth_sweeps, link, nullptr, v); });
-                if (ms < best) {
-                    best = ms;
-                    F.jacobi_post = v;
-                }
-            }
-            // pre-smoothing + residual + restriction: the two launches against the fused one
-            F.jacobi_fused = -1;
-            const Level& Cn = levels[l + 1];
-            if (2 * (long long)Cn.w >= F.w && 2 * (long long)Cn.h >= F.h) {
-                const LevelView C = view(l + 1);
+            const int nu = chebyshev ? smooth_sweeps : smoother == FS_SMOOTHER_RED_BLACK ? sweeps_on(l) : 4;
+            if (!chebyshev) {
                 const AxisRestrict rx{F.d_rxc.p, F.d_rxi.p, F.d_rxw.p};
                 const AxisRestrict ry{F.d_ryc.p, F.d_ryi.p, F.d_ryw.p};
-                best = time([&] {
-                    launch_jacobi_multi(st(), L, 0, rhs, nullptr, 1, pre, smooth_sweeps, none, nullptr, F.jacobi_pre);
-                    launch_res_restrict(st(), L, 1, rhs, nullptr, C, rx, ry, nullptr, F.restrict_variant);
+                F.restrict_variant = pick(kRestrictVariants, [&](int v) {
+                    if (l == 0)
+                        launch_res_restrict(st(), level_of<C, float>(0), 0, (const float*)r.p, nullptr,
+                            level_of<C, VL>(1), rx, ry, nullptr, v);
+                    else
+                        launch_res_restrict(st(), level_of<C, VL>(l), 0, (const VL*)level_of<C, VL>(l).rhs, nullptr,
+                            level_of<C, VL>(l + 1), rx, ry, nullptr, v);
                 });
-                for (int v = 0; v < kJacobiRestrictVariants; ++v) {
-                    const float ms = time([&] {
-                        launch_jacobi_res_restrict(st(), L, 0, rhs, nullptr, pre, smooth_sweeps, C, rx, ry, nullptr, v);
-                    });
-                    if (ms < best) {
-                        best = ms;
-                        F.jacobi_fused = v;
-                    }
-                }
             }
-        }
-        jacobi_tuned = true;
-        drop_graph();
-    }
-
-    // Autotuner: times every tile variant of the level smoother (plain sweeps) and of the residual +
-    // restriction on each level's own buffers and keeps the fastest.  The fused kernels compute the same
-    // values with any tile, so the choice affects time only.
-    void tune_tiles()
-    {
-        const CoarseLink none{};
-        auto time = [&](auto&& launch) {
-            launch();
-            HIPC(hipEventRecord(ctx->ev0, st()));
-            for (int k = 0; k < 3; ++k)
-                launch();
-            HIPC(hipEventRecord(ctx->ev1, st()));
-            HIPC(hipEventSynchronize(ctx->ev1));
-            float ms = 0.f;
-            HIPC(hipEventElapsedTime(&ms, ctx->ev0, ctx->ev1));
-            return ms;
-        };
-        for (int l = 0; l < tail_start; ++l) {
-            Level& F = levels[l];
-            const LevelView L = view(l);
-            const float* rhs = l == 0 ? r.p : L.rhs;
-            const Level& Cl = levels[l + 1];
-            const CoarseLink link{Cl.sol0.p, Cl.s, F.d_pxf.p, F.d_pxs.p, F.d_pxw.p, F.d_pyf.p, F.d_pys.p, F.d_pyw.p};
-            float best = std::numeric_limits<float>::infinity();
-            for (int v = 0; v < kSmoothVariants; ++v) {
-                const float ms = time([&] { launch_rb_multi(st(), L, 0, rhs, nullptr, 0, 1, none, nullptr, l == 0, v); });
-                if (ms < best) {
-                    best = ms;
-                    F.smooth_variant = v;
-                }
-            }
-            best = std::numeric_limits<float>::infinity();
-            for (int v = 0; v < kSmoothVariants; ++v) {
-                const float ms = time([&] { launch_rb_multi(st(), L, 1, rhs, nullptr, 1, 0, link, nullptr, l == 0, v); });
-                if (ms < best) {
-                    best = ms;
-                    F.post_variant = v;
-                }
-            }
-            const AxisRestrict rx{F.d_rxc.p, F.d_rxi.p, F.d_rxw.p};
-            const AxisRestrict ry{F.d_ryc.p, F.d_ryi.p, F.d_ryw.p};
-            const LevelView C = view(l + 1);
-            best = std::numeric_limits<float>::infinity();
-            for (int v = 0; v < kRestrictVariants; ++v) {
-                const float ms = time([&] { launch_res_restrict(st(), L, 0, rhs, nullptr, C, rx, ry, nullptr, v); });
-                if (ms < best) {
-                    best = ms;
-                    F.restrict_variant = v;
-                }
-            }
+            (chebyshev ? F.jacobi_pre : F.smooth_variant) =
+                pick(chebyshev ? kChebyshevChoices : kRedBlackChoices, [&](int v) {
+                    descend<C, VL>(l, nullptr, chebyshev, nu, v, F.restrict_variant);
+                });
+            (chebyshev ? F.jacobi_post : F.post_variant) = pick(chebyshev ? kChebyshevTiles : kSmoothTiles,
+                [&](int v) { ascend<C, VL>(l, 1, nullptr, chebyshev, nu, v); });
         }
         drop_graph();   // launches captured before the choice keep the old tiles
+    }
+
+    // Calls f with the storage types of the current mode: conductances and level vectors.
+    template <class F> void in_storage(F&& f)
+    {
+        if (!active16())
+            f(float{}, float{});
+        else if (mg_prec == FS_MG_FP16)
+            f(half16{}, float{});
+        else if (mg_prec == FS_MG_BF16)
+            f(bf16{}, float{});
+        else
+            f(bf16{}, bf16{});
+    }
+    void tune_for_precision()
+    {
+        in_storage([&](auto c, auto v) { tune_levels<decltype(c), decltype(v)>(false); });
+    }
+    void tune_jacobi()
+    {
+        tune_levels<float, float>(true);
+        jacobi_tuned = true;
+    }
+
+    // The finest post-smoothing launch of a V-cycle in the grid's storage mode (kernel timing); a grid without
+    // tiled levels times the smoother alone.
+    void fine_post_smooth(int cur)
+    {
+        if (tail_start == 0) {
+            launch_smooth(st(), 0, view(0), cur, (const float*)r.p, rmean_ptr(), 1, SmoothWeights{}, 4, CoarseLink{}, nullptr, 2);
+            return;
+        }
+        const bool chebyshev = chebyshev_on(0);
+        in_storage([&](auto c, auto v) {
+            ascend<decltype(c), decltype(v)>(0, cur, nullptr, chebyshev, sweeps_on(0),
+                chebyshev ? levels[0].jacobi_post : levels[0].post_variant);
+        });
+    }
+
+    // One V-cycle on the residual r (minus its mean) into levels[0].sol0.
+    void vcycle(const int* status)
+    {
+        in_storage([&](auto c, auto v) { vcycle_t<decltype(c), decltype(v)>(status); });
     }
 
     const float* z_ptr() const { return precond == FS_PRECOND_MULTIGRID ? levels[0].sol0.p : zdiag.p; }
@@ -3233,9 +3133,7 @@ fs_status fs_mg_level_tiles(fs_grid* grid, int level, int* pre, int* post, int* 
         const bool fused = level < grid->tail_start;
         const bool jacobi = fused && grid->chebyshev_on(level);
         if (pre)
-            *pre = fused ? (jacobi ? (L.jacobi_fused >= 0 ? kJacobiVariants + L.jacobi_fused : L.jacobi_pre)
-                                   : L.smooth_variant)
-                         : -1;
+            *pre = fused ? (jacobi ? L.jacobi_pre : L.smooth_variant) : -1;
         if (post)
             *post = fused ? (jacobi ? L.jacobi_post : L.post_variant) : -1;
         if (restriction)
@@ -3249,21 +3147,12 @@ fs_status fs_mg_set_level_tiles(fs_grid* grid, int level, int pre, int post, int
         need(grid != nullptr, FS_E_INVALID_ARGUMENT, "null grid");
         need(level >= 0 && level < grid->tail_start, FS_E_INVALID_ARGUMENT, "no tiled level with this index");
         const bool jacobi = grid->chebyshev_on(level);
-        const int smooth_variants = jacobi ? kJacobiVariants : kSmoothVariants;
         Level& L = grid->levels[(size_t)level];
-        const Level& Cn = grid->levels[(size_t)level + 1];
-        const bool can_fuse = jacobi && 2 * (long long)Cn.w >= L.w && 2 * (long long)Cn.h >= L.h;
-        const int pre_variants = smooth_variants + (can_fuse ? kJacobiRestrictVariants : 0);
-        need(pre >= -1 && pre < pre_variants && post >= -1 && post < smooth_variants && restriction >= -1 &&
-                 restriction < kRestrictVariants,
+        need(pre >= -1 && pre < (jacobi ? kChebyshevChoices : kRedBlackChoices) && post >= -1 &&
+                 post < (jacobi ? kChebyshevTiles : kSmoothTiles) && restriction >= -1 && restriction < kRestrictVariants,
             FS_E_INVALID_ARGUMENT, "unknown tile variant");
-        if (pre >= kJacobiVariants && jacobi)
-            L.jacobi_fused = pre - kJacobiVariants;   // the fused pre-smoothing + restriction launch
-        else if (pre >= 0 && jacobi) {
-            L.jacobi_fused = -1;   // the separate launches with this Jacobi tile
-            L.jacobi_pre = pre;
-        } else if (pre >= 0)
-            L.smooth_variant = pre;
+        if (pre >= 0)
+            (jacobi ? L.jacobi_pre : L.smooth_variant) = pre;
         if (post >= 0)
             (jacobi ? L.jacobi_post : L.post_variant) = post;
         if (restriction >= 0)
@@ -3390,9 +3279,8 @@ fs_status fs_time_kernel(fs_grid* grid, int kernel, int reps, double* ms_per_lau
             case 2: launch_pcg_update(g.st(), gd); break;
             case 3: launch_copy_f32(g.st(), g.r.p, g.q.p, g.NP()); break;
             case 4:  // second level's smoother (or the finest, if the tail starts at level 1)
-                launch_rb_multi(g.st(), g.view(l1), i & 1, l1 == 0 ? g.r.p : g.view(l1).rhs,
-                    l1 == 0 ? g.rmean_ptr() : nullptr, 0, 0, CoarseLink{}, nullptr, l1 == 0,
-                    g.levels[l1].smooth_variant);
+                launch_smooth(g.st(), 0, g.view(l1), i & 1, (const float*)(l1 == 0 ? g.r.p : g.view(l1).rhs),
+                    l1 == 0 ? g.rmean_ptr() : nullptr, 1, SmoothWeights{}, 4, CoarseLink{}, nullptr, 2);
                 break;
             case 5: {
                 if (g.tail_start == 0 || nlev < 2)
@@ -3400,7 +3288,7 @@ fs_status fs_time_kernel(fs_grid* grid, int kernel, int reps, double* ms_per_lau
                 const Level& F = g.levels[0];
                 AxisRestrict rx{F.d_rxc.p, F.d_rxi.p, F.d_rxw.p};
                 AxisRestrict ry{F.d_ryc.p, F.d_ryi.p, F.d_ryw.p};
-                launch_res_restrict(g.st(), L0, 1, g.r.p, g.rmean_ptr(), g.view(1), rx, ry, nullptr,
+                launch_res_restrict(g.st(), L0, 1, (const float*)g.r.p, g.rmean_ptr(), g.view(1), rx, ry, nullptr,
                     F.restrict_variant);
                 break;
             }

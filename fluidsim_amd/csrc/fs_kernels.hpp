@@ -199,42 +199,38 @@ void launch_pcg_direction(hipStream_t st, const GridDev& g, const float* z, int 
 void launch_precond_diag(hipStream_t st, const GridDev& g);
 
 // ---- multigrid V-cycle pieces (FP32) ----
-// nu (1..4, default 4) red-black sweeps in one launch (reads sol[cur], writes sol[cur ^ 1]); with link.csol
-// set the coarse correction is prolonged and added first.  fine selects the finest-level symbol.
-// variant: interior tile and threads 0 = 64 x 32 / 256, 1 = 32 x 32 / 256, 2 = 32 x 16 / 256,
-// 3 = 16 x 16 / 256, 4 = 64 x 32 / 512, 5 = 32 x 32 / 512, 6 = 32 x 32 / 384, 7 = 64 x 32 / 640,
-// 8 = 32 x 64 / 640, 9 = 64 x 32 / 960, 10 = 32 x 64 / 960 (same results, different speed).
-constexpr int kSmoothVariants = 11;
-void launch_rb_multi(hipStream_t st, const LevelView& L, int cur, const float* rhs, const double* shift,
-    int first_color, int from_zero, const CoarseLink& link, const int* status, int fine, int variant, int nu = 4);
-// Chebyshev-weighted damped Jacobi (the reference WebGPU multigrid's polynomial smoother,
-// PressureMultigridGPU.cpp:24-28, 619-631; PressureSmoothingKernels.h:91-176): nu (1..kJacobiMaxSweeps)
-// sweeps x <- x + w_k (b - A x) / diag in one launch on an LDS tile with an nu-cell halo, reading sol[cur]
-// (from_zero: x = 0) and writing sol[cur ^ 1]; with link.csol set the coarse correction is prolonged and
-// added first.  A cell without conductance is set to zero.  weights.w[k] is sweep k's weight (the caller
-// reverses them for post-smoothing).  variant: 0 = 64 x 32 / 512, 1 = 32 x 32 / 256, 2 = 32 x 16 / 256,
-// 3 = 16 x 16 / 256, 4 = 32 x 32 / 512, 5 = 64 x 64 / 1024, 6 = 64 x 32 / 1024, 7 = 32 x 64 / 1024 (same
-// results, different speed).
+// The level smoothers on tiles held in registers: nu (1..4) red-black sweeps or, jacobi != 0 (FP32 levels only), nu
+// (1..kJacobiMaxSweeps) sweeps x <- x + w_k (b - A x) / diag of Chebyshev-weighted damped Jacobi (the reference WebGPU
+// multigrid's polynomial smoother, PressureMultigridGPU.cpp:24-28, 619-631; PressureSmoothingKernels.h:91-176),
+// weights.w[k] being sweep k's weight (the caller reverses them for post-smoothing); a cell without conductance is
+// set to zero.  pre: from zero into sol[cur ^ 1]; else post-smoothing (red-black in reversed order): the prolonged
+// coarse correction added to sol[cur] first, into sol[cur ^ 1].
+// C: conductance storage, V: this level's vectors, VC: the coarse ones.  tile: 0 .. kSmoothTiles - 1, columns x rows
+// (threads): 128x64 (512), 128x64 (1024), 64x64 (512), 64x64 (1024), 64x32 (256), 64x32 (512), 32x32 (256),
+// 32x64 (256), 128x32 (512), 128x128 (1024), 32x64 (512); the same values, different speed.
+constexpr int kSmoothTiles = 11;
 constexpr int kJacobiMaxSweeps = 8;
-constexpr int kJacobiShortHalo = 5;   // tile halo of the kernels used for up to this many sweeps
-constexpr int kJacobiVariants = 8;
 struct SmoothWeights {
     float w[kJacobiMaxSweeps];
 };
-void launch_jacobi_multi(hipStream_t st, const LevelView& L, int cur, const float* rhs, const double* shift,
-    int from_zero, const SmoothWeights& weights, int nu, const CoarseLink& link, const int* status, int variant);
-// Pre-smoothing from zero (launch_jacobi_multi with from_zero) and the residual + restriction into C
-// (launch_res_restrict) in one launch, same values; tile variants 0 = 16x8 coarse cells on 512 threads,
-// 1 = 16x16/512, 2 = 32x16/1024.  C must cover the fine level (2 C.w >= L.w, 2 C.h >= L.h).
-constexpr int kJacobiRestrictVariants = 3;
-void launch_jacobi_res_restrict(hipStream_t st, const LevelView& L, int cur, const float* rhs, const double* shift,
-    const SmoothWeights& weights, int nu, const LevelView& C, AxisRestrict rx, AxisRestrict ry, const int* status,
-    int variant);
+template <class C, class V, class VC>
+void launch_smooth(hipStream_t st, int jacobi, const LevelViewT<C, V>& L, int cur, const V* rhs,
+    const double* shift, int pre, const SmoothWeights& wt, int nu, const CoarseLinkT<VC>& link, const int* status,
+    int tile);
+// Pre-smoothing, residual and its restriction into Cl.rhs in one launch; the values of launch_smooth and
+// launch_res_restrict.  tile: 0 .. kRestrictTiles - 1: 128x128 (1024), 128x64 (1024), 64x64 (512), 64x64 (1024),
+// 32x64 (512), 32x32 (256).
+constexpr int kRestrictTiles = 6;
+template <class C, class V, class VC>
+void launch_smooth_restrict(hipStream_t st, int jacobi, const LevelViewT<C, V>& L, int cur, const V* rhs,
+    const double* shift, const SmoothWeights& wt, int nu, const LevelViewT<C, VC>& Cl, AxisRestrict rx, AxisRestrict ry,
+    const int* status, int tile);
 // Residual of sol[cur] and its restriction into C.rhs in one launch; variant: coarse tile 0 = 32 x 16,
 // 1 = 16 x 16, 2 = 16 x 8, 3 = 8 x 8.
 constexpr int kRestrictVariants = 4;
-void launch_res_restrict(hipStream_t st, const LevelView& F, int cur, const float* rhs, const double* shift,
-    const LevelView& C, AxisRestrict rx, AxisRestrict ry, const int* status, int variant);
+template <class C, class V, class VC>
+void launch_res_restrict(hipStream_t st, const LevelViewT<C, V>& F, int cur, const V* rhs, const double* shift,
+    const LevelViewT<C, VC>& Cl, AxisRestrict rx, AxisRestrict ry, const int* status, int variant);
 // bf16_top: the first tail level's rhs and solution are stored as bfloat16 (else FP32).
 void launch_mg_tail(hipStream_t st, const TailDesc& desc, size_t lds_bytes, const double* shift, const int* status,
     int bf16_top = 0);
@@ -243,16 +239,8 @@ void launch_mg_tail(hipStream_t st, const TailDesc& desc, size_t lds_bytes, cons
 // Conductances of one level rounded (FP64 -> FP32 -> C, each to nearest even) into 16-bit copies.
 template <class C> void launch_level_pack(hipStream_t st, int w, int h, const double* right64, const double* down64,
     C* right, C* down);
-// The fused smoother and residual-restriction kernels of launch_rb_multi / launch_res_restrict with
-// C conductances, V vectors on this level (its rhs argument included) and VC vectors on the next
-// coarser level; MODE 0 and 1 only.  Instantiated for (half16, float, float), (bf16, float, float),
-// (bf16, float, bf16) and (bf16, bf16, bf16).
-template <class C, class V, class VC>
-void launch_rb_multi_t(hipStream_t st, const LevelViewT<C, V>& L, int cur, const V* rhs, const double* shift,
-    int first_color, int from_zero, const CoarseLinkT<VC>& link, const int* status, int variant, int nu = 4);
-template <class C, class V, class VC>
-void launch_res_restrict_t(hipStream_t st, const LevelViewT<C, V>& F, int cur, const V* rhs, const double* shift,
-    const LevelViewT<C, VC>& Cl, AxisRestrict rx, AxisRestrict ry, const int* status, int variant);
+// The smoothers and the residual restriction are instantiated for (C, V, VC) = (float, float, float),
+// (half16, float, float), (bf16, float, float), (bf16, float, bf16) and (bf16, bf16, bf16).
 
 // ---- batched PCG: one 1024-thread workgroup runs the whole iteration loop of one instance ----
 constexpr int kMaxBatchLevels = 16;   // tiled levels above an instance's tail

@@ -1,10 +1,8 @@
 // fs_multigrid.hip -- the multigrid preconditioner of PressureMultigrid.cpp on gfx950.
 //
-// One V(4,4) cycle per level is three launches:
-//   k_rb_multi      four red-black Gauss-Seidel sweeps on a (64+16) x (32+16) LDS tile (halo 8: each
-//                   half-sweep shrinks the valid region by one cell), from zero on the way down;
-//   k_res_restrict  residual of the smoothed solution and its transpose-of-bilinear restriction;
-//   k_rb_multi      prolongation of the coarse correction fused into the load, then four reversed sweeps.
+// A cycle's level smoothers are in fs_rows.hip: on the way down the sweeps, the residual and its
+// transpose-of-bilinear restriction in one launch (or the restriction apart, k_res_restrict), on the way up
+// the prolongation and the reversed sweeps in one.
 // The deepest levels (up to 64 x 64, as LDS allows) and the coarse solve run in k_mg_tail, one
 // 1024-thread workgroup with every array in LDS.  The pinned coarse system (PressureMultigrid.cpp:
 // 300-384) is factored bit-exactly by k_coarse_factor, which also forms its inverse so the per-cycle
@@ -13,6 +11,7 @@
 // Smoothers divide by the sum of the four face conductances formed in FP32 (one rcp); pre- and
 // post-smoothing use the same diagonal, so the V-cycle stays symmetric.
 #include "fs_kernels.hpp"
+#include "fs_mg_device.hpp"
 
 #include <math.h>
 
@@ -24,358 +23,6 @@ namespace fsim {
 namespace {
 
 constexpr int kNT = 256;
-
-__device__ __forceinline__ float inv_or_zero(float d) { return d > 0.f ? __builtin_amdgcn_rcpf(d) : 0.f; }
-
-// Loads and stores of multigrid storage formats; arithmetic is FP32.  Stores round to nearest even.
-__device__ __forceinline__ float ldv(float v) { return v; }
-__device__ __forceinline__ float ldv(half16 v) { return (float)__builtin_bit_cast(_Float16, v.bits); }
-__device__ __forceinline__ float ldv(bf16 v) { return __uint_as_float((unsigned)v.bits << 16); }
-template <class T> __device__ __forceinline__ T stv(float f);
-template <> __device__ __forceinline__ float stv<float>(float f) { return f; }
-template <> __device__ __forceinline__ half16 stv<half16>(float f)
-{
-    return half16{__builtin_bit_cast(unsigned short, (_Float16)f)};
-}
-template <> __device__ __forceinline__ bf16 stv<bf16>(float f)
-{
-    // round to nearest even on the 16 bits dropped (finite inputs: the levels hold no NaN)
-    const unsigned u = __float_as_uint(f);
-    return bf16{(unsigned short)((u + 0x7fffu + ((u >> 16) & 1u)) >> 16)};
-}
-
-// XCD-aware tile order.  Workgroups of a launch are dealt to the 8 XCDs round-robin (workgroup b runs
-// on XCD b % 8), each XCD with its own L2.  Mapping the workgroups an XCD receives onto a contiguous
-// run of row-major tiles keeps neighbouring tiles, whose 8-cell halos overlap, on the same L2.  The
-// launch is one-dimensional with exactly gx * gy workgroups; the map is a bijection onto the tiles.
-constexpr int kXcds = 8;
-__device__ __forceinline__ void xcd_tile(int gx, int gy, int& bx, int& by)
-{
-    const int n = gx * gy;
-    const int b = blockIdx.x;
-    const int per = n / kXcds, rem = n % kXcds;
-    const int xcd = b % kXcds, q = b / kXcds;
-    const int t = xcd * per + min(xcd, rem) + q;
-    by = t / gx;
-    bx = t - by * gx;
-}
-
-// ---------------------------------------------------------------------------------------------
-// Four-sweep red-black Gauss-Seidel with optional fused prolongation.
-// ---------------------------------------------------------------------------------------------
-// Layout: the tile's solution lives in two colour arrays (red, black), each LX/2 wide, so a wavefront
-// updating 64 same-colour cells of a row touches 64 consecutive LDS words (no bank conflicts).  Each
-// thread owns fixed (row, pair) slots; the four conductances, rhs and 1/diagonal of its cells stay in
-// registers for all eight half-sweeps, so an update reads four neighbours from LDS and writes one value.
-// MODE 0: pre-smoothing from a zero guess (no solution read); 1: post-smoothing, the prolonged coarse
-// correction added to the solution first; 2: plain sweeps of the stored solution.
-// Post-smoothing tiles are held to the registers that keep their workgroups per CU: 128 VGPRs for 512
-// threads (four waves per SIMD, two workgroups) and 960 (one), 170 for 384 (two) and 640 threads (one).
-template <int MODE, int NT> constexpr int rb_waves_per_eu()
-{
-    return MODE != 1 ? 1 : (NT == 512 || NT == 960) ? 4 : (NT == 384 || NT == 640) ? 3 : 1;
-}
-
-// C: conductance storage, V: this level's vectors (rhs, solution), VC: the coarse solution (MODE 1).
-template <int TX, int TY, int NS, int FINE, int MODE, int NT, class C = float, class V = float, class VC = float>
-__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(rb_waves_per_eu<MODE, NT>())))
-void k_rb_multi(LevelViewT<C, V> L, int cur, const V* rhs, const double* shift, int c0, int nu, CoarseLinkT<VC> link,
-    const int* status)
-{
-    constexpr bool from_zero = MODE == 0;
-    constexpr int HALO = 2 * NS;
-    constexpr int LX = TX + 2 * HALO, LY = TY + 2 * HALO;
-    constexpr int HX = LX / 2;                       // colour-array row width
-    constexpr int NE = LX * LY;
-    constexpr int SLOTS = HX * (LY - 2);             // rows 1 .. LY-2, every pair
-    constexpr int ROUNDS = (SLOTS + NT - 1) / NT;
-    static_assert(LX % 2 == 0 && (TX % 2) == 0 && (HALO % 2) == 0, "tile must keep colour parity");
-    __shared__ float s_col[2][LY * HX];
-    const int w = L.w, h = L.h, s = L.s;
-    int bx, by;
-    xcd_tile((w + TX - 1) / TX, (h + TY - 1) / TY, bx, by);
-    const int x0 = bx * TX - HALO, y0 = by * TY - HALO;  // x0 + y0 is even
-    const V* sol_in = L.sol[cur];
-    // Every global load below goes through a clamped (valid) interior index and is masked afterwards,
-    // so a thread issues all its loads before its first wait.
-    float cl[2][ROUNDS], cr[2][ROUNDS], cu[2][ROUNDS], cd[2][ROUNDS], cb[2][ROUNDS];
-    int cly[ROUNDS], cj[ROUNDS];
-    bool cin[2][ROUNDS];
-#pragma unroll
-    for (int r = 0; r < ROUNDS; ++r) {
-        const int t = threadIdx.x + r * NT;
-        const int ly = 1 + t / HX, jj = t - (t / HX) * HX;
-        cly[r] = t < SLOTS ? ly : -1;
-        cj[r] = jj;
-#pragma unroll
-        for (int c = 0; c < 2; ++c) {
-            const int lx = 2 * jj + ((c + ly) & 1);
-            const int x = x0 + lx, y = y0 + ly;
-            cin[c][r] = t < SLOTS && x >= 0 && x < w && y >= 0 && y < h;
-            const int P = (min(max(y, 0), h - 1) + 1) * s + (min(max(x, 0), w - 1) + 1);
-            cl[c][r] = ldv(L.right[P - 1]);
-            cr[c][r] = ldv(L.right[P]);
-            cu[c][r] = ldv(L.down[P - s]);
-            cd[c][r] = ldv(L.down[P]);
-            cb[c][r] = ldv(rhs[P]);
-        }
-    }
-    constexpr int LOADS = (NE + NT - 1) / NT;
-    float vs[LOADS];
-    bool vin[LOADS];
-    int ix[LOADS], iy[LOADS];
-#pragma unroll
-    for (int it = 0; it < LOADS; ++it) {
-        const int e = threadIdx.x + it * NT;
-        const int ly = e / LX, lx = e - ly * LX;
-        const int x = x0 + lx, y = y0 + ly;
-        vin[it] = e < NE && x >= 0 && x < w && y >= 0 && y < h;
-        ix[it] = min(max(x, 0), w - 1);
-        iy[it] = min(max(y, 0), h - 1);
-        vs[it] = MODE == 0 ? 0.f : ldv(sol_in[(iy[it] + 1) * s + (ix[it] + 1)]);
-    }
-    if (MODE == 1) {
-        // per chunk of PC cells, two batched phases: transfer tables, then the four coarse values (chunks
-        // bound the registers this prologue adds to the kernel)
-        constexpr int PC = NT >= 384 ? 1 : 4;   // large tiles keep to 128 VGPRs without spilling
-#pragma unroll
-        for (int c0 = 0; c0 < LOADS; c0 += PC) {
-            int a0[PC], a1[PC], b0[PC], b1[PC];
-            float wx[PC], wy[PC];
-#pragma unroll
-            for (int k = 0; k < PC; ++k) {
-                const int it = min(c0 + k, LOADS - 1);
-                wx[k] = link.pxw[ix[it]];
-                wy[k] = link.pyw[iy[it]];
-                a0[k] = link.pxf[ix[it]];
-                a1[k] = link.pxs[ix[it]];
-                b0[k] = link.pyf[iy[it]];
-                b1[k] = link.pys[iy[it]];
-            }
-#pragma unroll
-            for (int k = 0; k < PC; ++k) {
-                if (c0 + k >= LOADS)
-                    break;
-                const VC* top = link.csol + (b0[k] + 1) * link.cs + 1;
-                const VC* bot = link.csol + (b1[k] + 1) * link.cs + 1;
-                const float t0 = ldv(top[a0[k]]), t1 = ldv(top[a1[k]]), u0 = ldv(bot[a0[k]]), u1 = ldv(bot[a1[k]]);
-                const float a = (1.f - wx[k]) * t0 + wx[k] * t1;
-                const float b = (1.f - wx[k]) * u0 + wx[k] * u1;
-                vs[c0 + k] += (1.f - wy[k]) * a + wy[k] * b;
-            }
-        }
-    }
-    if (status && *status != kRunning)
-        return;
-    const double sh = shift ? *shift : 0.0;
-#pragma unroll
-    for (int r = 0; r < ROUNDS; ++r) {
-#pragma unroll
-        for (int c = 0; c < 2; ++c) {
-            if (!cin[c][r]) {
-                cl[c][r] = cr[c][r] = cu[c][r] = cd[c][r] = cb[c][r] = 0.f;
-            } else if (shift) {
-                cb[c][r] = (float)((double)cb[c][r] - sh);
-            }
-        }
-    }
-#pragma unroll
-    for (int it = 0; it < LOADS; ++it) {
-        const int e = threadIdx.x + it * NT;
-        if (e < NE) {
-            const int ly = e / LX, lx = e - ly * LX;
-            s_col[(lx + ly) & 1][ly * HX + (lx >> 1)] = vin[it] ? vs[it] : 0.f;
-        }
-    }
-    __syncthreads();
-    // Per-slot invariants of the eight half-sweeps, computed once: the slot's LDS index, the index of
-    // its left neighbour for each colour, 1/diagonal of each colour's cell, and (one byte per colour)
-    // the cell's distance to the tile edge plus one -- zero for a slot outside the grid -- so the
-    // half-sweep at depth k (region shrunk by k + 1 cells) updates the cell iff its byte exceeds k + 1.
-    int sdst[ROUNDS], sleft[2][ROUNDS], sreach[ROUNDS];
-    float sinv[2][ROUNDS];
-#pragma unroll
-    for (int r = 0; r < ROUNDS; ++r) {
-        const int ly = max(cly[r], 1);        // unused slots address a valid row and stay inactive
-        const int jj = cj[r];
-        sdst[r] = ly * HX + jj;
-        int reach = 0;
-#pragma unroll
-        for (int c = 0; c < 2; ++c) {
-            const int p = (c + ly) & 1;
-            sleft[c][r] = sdst[r] + p - 1;    // rows 1 .. LY-2: every neighbour index stays inside the array
-            const int lx = 2 * jj + p;
-            const int dist = min(min(ly, LY - 1 - ly), min(lx, LX - 1 - lx));
-            if (cin[c][r])
-                reach |= (dist + 1) << (8 * c);
-            sinv[c][r] = inv_or_zero((cl[c][r] + cr[c][r]) + (cu[c][r] + cd[c][r]));
-        }
-        sreach[r] = reach;
-    }
-    // ---- 2 nu half-sweeps (nu <= NS), each region one cell smaller than the last; with nu < NS the
-    // outer 2 (NS - nu) rings of the halo are loaded but never updated ----
-    const int skip = 2 * (NS - nu);
-    // A half-sweep reads only the other colour, so all neighbour values are gathered first and the
-    // updates written afterwards: one LDS latency per half-sweep instead of one per round.  The colour
-    // is a compile-time constant inside a half-sweep, so per-colour registers are addressed directly.
-    auto half = [&](auto color_tag, int k) {
-        constexpr int color = decltype(color_tag)::value;
-        const int lo = k + 1 + skip;
-        const bool neighbours = !(from_zero && k == 0);
-        float* mine = s_col[color];
-        const float* other = s_col[color ^ 1];
-        float n0[ROUNDS], n1[ROUNDS], n2[ROUNDS], n3[ROUNDS];
-#pragma unroll
-        for (int r = 0; r < ROUNDS; ++r) {
-            n0[r] = other[sleft[color][r]];
-            n1[r] = other[sleft[color][r] + 1];
-            n2[r] = other[sdst[r] - HX];
-            n3[r] = other[sdst[r] + HX];
-        }
-#pragma unroll
-        for (int r = 0; r < ROUNDS; ++r) {
-            const float a = cl[color][r], b = cr[color][r], u = cu[color][r], d = cd[color][r];
-            float v = cb[color][r];
-            if (neighbours)
-                v += (a * n0[r] + b * n1[r]) + (u * n2[r] + d * n3[r]);
-            if (((sreach[r] >> (8 * color)) & 0xff) > lo)
-                mine[sdst[r]] = v * sinv[color][r];
-        }
-        __syncthreads();
-    };
-#pragma unroll 1
-    for (int k = 0; k < 2 * nu; k += 2) {
-        if (c0 == 0) {
-            half(std::integral_constant<int, 0>{}, k);
-            half(std::integral_constant<int, 1>{}, k + 1);
-        } else {
-            half(std::integral_constant<int, 1>{}, k);
-            half(std::integral_constant<int, 0>{}, k + 1);
-        }
-    }
-    V* sol_out = L.sol[cur ^ 1];
-    for (int e = threadIdx.x; e < TX * TY; e += NT) {
-        const int ly = HALO + e / TX, lx = HALO + e % TX;
-        const int x = x0 + lx, y = y0 + ly;
-        if (x < w && y < h)
-            sol_out[(y + 1) * s + (x + 1)] = stv<V>(s_col[(lx + ly) & 1][ly * HX + (lx >> 1)]);
-    }
-}
-
-// ---------------------------------------------------------------------------------------------
-// Chebyshev-weighted damped Jacobi with optional fused prolongation (the reference WebGPU multigrid's
-// polynomial smoother, PressureMultigridGPU.cpp:24-28, 619-631; PressureSmoothingKernels.h:91-176).
-// ---------------------------------------------------------------------------------------------
-// The tile and a HALO-cell ring live in two LDS buffers (sweep k reads buffer k & 1 and writes the other).
-// Each thread owns fixed cells; their four conductances, rhs and 1/diagonal stay in registers for all
-// sweeps.  Sweep k updates the cells at least k + 1 + (HALO - nu) cells from the tile edge, so after nu
-// sweeps the interior holds exactly what nu global sweeps compute.  Cells outside the grid hold zero in both
-// buffers and are never updated.  MODE 0: from zero (the first sweep is w b / diag); 1: post-smoothing,
-// the prolonged coarse correction added to the solution first.
-template <int TX, int TY, int MODE, int NT, int HALO>
-__global__ __launch_bounds__(NT) void k_jacobi_multi(LevelView L, int cur, const float* rhs, const double* shift,
-    SmoothWeights wt, int nu, CoarseLink link, const int* status)
-{
-    constexpr int LX = TX + 2 * HALO, LY = TY + 2 * HALO;
-    constexpr int NE = LX * LY;
-    constexpr int ROUNDS = (NE + NT - 1) / NT;
-    __shared__ float s_x[2][NE];
-    const int w = L.w, h = L.h, s = L.s;
-    int bx, by;
-    xcd_tile((w + TX - 1) / TX, (h + TY - 1) / TY, bx, by);
-    const int x0 = bx * TX - HALO, y0 = by * TY - HALO;
-    const float* sol_in = L.sol[cur];
-    // every global load goes through a clamped (valid) interior index and is masked afterwards
-    float cl[ROUNDS], cr[ROUNDS], cu[ROUNDS], cd[ROUNDS], cb[ROUNDS], xv[ROUNDS];
-    int ix[ROUNDS], iy[ROUNDS];
-    bool cin[ROUNDS];
-#pragma unroll
-    for (int r = 0; r < ROUNDS; ++r) {
-        const int e = threadIdx.x + r * NT;
-        const int ly = e / LX, lx = e - ly * LX;
-        const int x = x0 + lx, y = y0 + ly;
-        cin[r] = e < NE && x >= 0 && x < w && y >= 0 && y < h;
-        ix[r] = min(max(x, 0), w - 1);
-        iy[r] = min(max(y, 0), h - 1);
-        const int P = (iy[r] + 1) * s + (ix[r] + 1);
-        cl[r] = L.right[P - 1];
-        cr[r] = L.right[P];
-        cu[r] = L.down[P - s];
-        cd[r] = L.down[P];
-        cb[r] = rhs[P];
-        xv[r] = MODE == 0 ? 0.f : sol_in[P];
-    }
-    if (MODE == 1) {
-#pragma unroll
-        for (int r = 0; r < ROUNDS; ++r) {
-            const float wx = link.pxw[ix[r]], wy = link.pyw[iy[r]];
-            const float* top = link.csol + (link.pyf[iy[r]] + 1) * link.cs + 1;
-            const float* bot = link.csol + (link.pys[iy[r]] + 1) * link.cs + 1;
-            const int a0 = link.pxf[ix[r]], a1 = link.pxs[ix[r]];
-            const float a = (1.f - wx) * top[a0] + wx * top[a1];
-            const float b = (1.f - wx) * bot[a0] + wx * bot[a1];
-            xv[r] += (1.f - wy) * a + wy * b;
-        }
-    }
-    if (status && *status != kRunning)
-        return;
-    const double sh = shift ? *shift : 0.0;
-    float inv[ROUNDS];
-    int reach[ROUNDS];   // distance to the tile edge + 1; 0 for a cell outside the grid
-#pragma unroll
-    for (int r = 0; r < ROUNDS; ++r) {
-        const int e = threadIdx.x + r * NT;
-        const int ly = e / LX, lx = e - ly * LX;
-        if (!cin[r]) {
-            cl[r] = cr[r] = cu[r] = cd[r] = cb[r] = xv[r] = 0.f;
-        } else if (shift) {
-            cb[r] = (float)((double)cb[r] - sh);
-        }
-        inv[r] = inv_or_zero((cl[r] + cr[r]) + (cu[r] + cd[r]));
-        reach[r] = cin[r] ? min(min(ly, LY - 1 - ly), min(lx, LX - 1 - lx)) + 1 : 0;
-        if (e < NE) {
-            s_x[0][e] = xv[r];
-            s_x[1][e] = xv[r];
-        }
-    }
-    __syncthreads();
-    const int skip = HALO - nu;
-#pragma unroll 1
-    for (int k = 0; k < nu; ++k) {
-        float wk = wt.w[0];   // uniform select: no dynamic indexing of the argument block
-#pragma unroll
-        for (int j = 1; j < kJacobiMaxSweeps; ++j)
-            wk = k == j ? wt.w[j] : wk;
-        const float* src = s_x[k & 1];
-        float* dst = s_x[(k & 1) ^ 1];
-        const bool neighbours = !(MODE == 0 && k == 0);
-#pragma unroll
-        for (int r = 0; r < ROUNDS; ++r) {
-            if (reach[r] > k + 1 + skip) {
-                const int e = threadIdx.x + r * NT;
-                float v;
-                if (neighbours) {
-                    const float c = src[e];
-                    const float product = (cl[r] * (c - src[e - 1]) + cr[r] * (c - src[e + 1])) +
-                                          (cu[r] * (c - src[e - LX]) + cd[r] * (c - src[e + LX]));
-                    v = c + wk * (cb[r] - product) * inv[r];
-                } else {
-                    v = wk * cb[r] * inv[r];
-                }
-                dst[e] = inv[r] > 0.f ? v : 0.f;
-            }
-        }
-        __syncthreads();
-    }
-    const float* fin = s_x[nu & 1];
-    float* sol_out = L.sol[cur ^ 1];
-    for (int e = threadIdx.x; e < TX * TY; e += NT) {
-        const int ly = HALO + e / TX, lx = HALO + e % TX;
-        const int x = x0 + lx, y = y0 + ly;
-        if (x < w && y < h)
-            sol_out[(y + 1) * s + (x + 1)] = fin[ly * LX + lx];
-    }
-}
 
 // ---------------------------------------------------------------------------------------------
 // Residual + restriction (restrictResidual, PressureMultigrid.cpp:233-276).  A coarse tile of
@@ -507,193 +154,6 @@ __global__ __launch_bounds__(kNT) void k_res_restrict(LevelViewT<C, V> F, int cu
             value += s_ryw[ly * 4 + iy] * horizontal;
         }
         Cl.rhs[(y + 1) * Cl.s + x + 1] = stv<VC>(value);
-    }
-}
-
-// ---------------------------------------------------------------------------------------------
-// Pre-smoothing from zero with the Chebyshev-weighted Jacobi sweeps, fused with the residual and the
-// restriction that follow it, for one coarse tile of CTX x CTY cells.  The smoothing tile is the coarse
-// tile's fine image widened by the restriction's reach and the residual's ring (RING = 3: taps in
-// [2c - 2, 2c + 3], one more cell for the operator) and by HALO (>= nu) cells of smoothing halo; with
-// k_jacobi_multi's update rule its cells at least that halo from the edge hold exactly what nu global
-// sweeps compute.  The fine image's cells are written as the pre-smoothed solution, the residual of the
-// restriction window is formed from LDS with k_res_restrict's expression and restricted with its sums in
-// the same order (a missing tap points at the same cell) -- the values of the two separate launches, in
-// one.  It pays on the levels where launches, not bytes, set the time; the autotuner decides per level.
-// ---------------------------------------------------------------------------------------------
-template <int CTX, int CTY, int NT, int HALO>
-__global__ __launch_bounds__(NT) void k_jacobi_res_restrict(LevelView L, int cur, const float* rhs,
-    const double* shift, SmoothWeights wt, int nu, LevelView Cl, AxisRestrict rx, AxisRestrict ry,
-    const int* status)
-{
-    constexpr int RING = 3;
-    constexpr int EDGE = RING + HALO;
-    constexpr int LX = 2 * CTX + 2 * EDGE, LY = 2 * CTY + 2 * EDGE;
-    constexpr int NE = LX * LY;
-    constexpr int ROUNDS = (NE + NT - 1) / NT;
-    static_assert(CTX + CTY <= NT, "one thread per restriction table row");
-    __shared__ float s_x[2][NE];
-    __shared__ int s_rxi[CTX * 4], s_ryi[CTY * 4];
-    __shared__ float s_rxw[CTX * 4], s_ryw[CTY * 4];
-    const int w = L.w, h = L.h, s = L.s;
-    int bx, by;
-    xcd_tile((Cl.w + CTX - 1) / CTX, (Cl.h + CTY - 1) / CTY, bx, by);
-    const int cx0 = bx * CTX, cy0 = by * CTY;
-    const int x0 = 2 * cx0 - EDGE, y0 = 2 * cy0 - EDGE;
-    // every global load goes through a clamped (valid) interior index and is masked afterwards
-    float cl[ROUNDS], cr[ROUNDS], cu[ROUNDS], cd[ROUNDS], cb[ROUNDS];
-    bool cin[ROUNDS];
-#pragma unroll
-    for (int r = 0; r < ROUNDS; ++r) {
-        const int e = threadIdx.x + r * NT;
-        const int ly = e / LX, lx = e - ly * LX;
-        const int x = x0 + lx, y = y0 + ly;
-        cin[r] = e < NE && x >= 0 && x < w && y >= 0 && y < h;
-        const int P = (min(max(y, 0), h - 1) + 1) * s + (min(max(x, 0), w - 1) + 1);
-        cl[r] = L.right[P - 1];
-        cr[r] = L.right[P];
-        cu[r] = L.down[P - s];
-        cd[r] = L.down[P];
-        cb[r] = rhs[P];
-    }
-    // restriction tables of this coarse tile, as k_res_restrict stages them (indices relative to x0, y0;
-    // a missing tap: weight 0 at the cell k_res_restrict's missing taps read)
-    int tc[2], ti[2][4];
-    float tw[2][4];
-#pragma unroll
-    for (int a = 0; a < 2; ++a) {
-        const int e = threadIdx.x - a * CTX;  // threads [0, CTX) take x, [CTX, CTX + CTY) take y
-        const bool isx = a == 0;
-        const int n_axis = isx ? CTX : CTY;
-        const int c = (isx ? cx0 : cy0) + min(max(e, 0), n_axis - 1);
-        const int limit = isx ? Cl.w : Cl.h;
-        const AxisRestrict& R = isx ? rx : ry;
-        const int cc = min(c, limit - 1);
-        const int n = R.count[cc];
-        tc[a] = c < limit ? n : 0;
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            ti[a][k] = R.index[cc * 4 + k];
-            tw[a][k] = R.weight[cc * 4 + k];
-        }
-    }
-    if (status && *status != kRunning)
-        return;
-    const double sh = shift ? *shift : 0.0;
-    float inv[ROUNDS];
-    int reach[ROUNDS];   // distance to the tile edge + 1; 0 for a cell outside the grid
-#pragma unroll
-    for (int r = 0; r < ROUNDS; ++r) {
-        const int e = threadIdx.x + r * NT;
-        const int ly = e / LX, lx = e - ly * LX;
-        if (!cin[r]) {
-            cl[r] = cr[r] = cu[r] = cd[r] = cb[r] = 0.f;
-        } else if (shift) {
-            cb[r] = (float)((double)cb[r] - sh);
-        }
-        inv[r] = inv_or_zero((cl[r] + cr[r]) + (cu[r] + cd[r]));
-        reach[r] = cin[r] ? min(min(ly, LY - 1 - ly), min(lx, LX - 1 - lx)) + 1 : 0;
-        if (e < NE) {
-            s_x[0][e] = 0.f;
-            s_x[1][e] = 0.f;
-        }
-    }
-    constexpr int MISS = EDGE - 2;   // k_res_restrict's missing-tap cell, 2c0 - 2 on each axis
-    if (threadIdx.x < CTX) {
-        const int e = threadIdx.x;
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            const bool on = k < tc[0];
-            s_rxi[e * 4 + k] = on ? ti[0][k] - x0 : MISS;
-            s_rxw[e * 4 + k] = on ? tw[0][k] : 0.f;
-        }
-    } else if (threadIdx.x < CTX + CTY) {
-        const int e = threadIdx.x - CTX;
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            const bool on = k < tc[1];
-            s_ryi[e * 4 + k] = on ? ti[1][k] - y0 : MISS;
-            s_ryw[e * 4 + k] = on ? tw[1][k] : 0.f;
-        }
-    }
-    __syncthreads();
-    const int skip = HALO - nu;
-#pragma unroll 1
-    for (int k = 0; k < nu; ++k) {
-        float wk = wt.w[0];   // uniform select: no dynamic indexing of the argument block
-#pragma unroll
-        for (int j = 1; j < kJacobiMaxSweeps; ++j)
-            wk = k == j ? wt.w[j] : wk;
-        const float* src = s_x[k & 1];
-        float* dst = s_x[(k & 1) ^ 1];
-        const bool neighbours = k != 0;
-#pragma unroll
-        for (int r = 0; r < ROUNDS; ++r) {
-            if (reach[r] > k + 1 + skip) {
-                const int e = threadIdx.x + r * NT;
-                float v;
-                if (neighbours) {
-                    const float c = src[e];
-                    const float product = (cl[r] * (c - src[e - 1]) + cr[r] * (c - src[e + 1])) +
-                                          (cu[r] * (c - src[e - LX]) + cd[r] * (c - src[e + LX]));
-                    v = c + wk * (cb[r] - product) * inv[r];
-                } else {
-                    v = wk * cb[r] * inv[r];
-                }
-                dst[e] = inv[r] > 0.f ? v : 0.f;
-            }
-        }
-        __syncthreads();
-    }
-    const float* fin = s_x[nu & 1];
-    float* res = s_x[(nu & 1) ^ 1];
-    float* sol_out = L.sol[cur ^ 1];
-    // the pre-smoothed solution of the coarse tile's fine image, and the residual of the restriction
-    // window ([2 c0 - 2, 2 c1 + 2) on each axis; zero outside the grid and at cells without conductance)
-#pragma unroll
-    for (int r = 0; r < ROUNDS; ++r) {
-        const int e = threadIdx.x + r * NT;
-        const int ly = e / LX, lx = e - ly * LX;
-        if (e >= NE)
-            continue;
-        if (cin[r] && lx >= EDGE && lx < EDGE + 2 * CTX && ly >= EDGE && ly < EDGE + 2 * CTY)
-            sol_out[(y0 + ly + 1) * s + (x0 + lx + 1)] = fin[e];
-        if (lx >= EDGE - 2 && lx < EDGE + 2 * CTX + 2 && ly >= EDGE - 2 && ly < EDGE + 2 * CTY + 2) {
-            float v = 0.f;
-            if (cin[r]) {
-                const float c = fin[e];
-                const float product = (cl[r] * (c - fin[e - 1]) + cr[r] * (c - fin[e + 1])) +
-                                      (cu[r] * (c - fin[e - LX]) + cd[r] * (c - fin[e + LX]));
-                const bool active = (cl[r] + cr[r]) + (cu[r] + cd[r]) > 0.f;
-                v = active ? cb[r] - product : 0.f;
-            }
-            res[e] = v;
-        }
-    }
-    __syncthreads();
-    for (int e = threadIdx.x; e < CTX * CTY; e += NT) {
-        const int ly = e / CTX, lx = e - ly * CTX;
-        const int x = cx0 + lx, y = cy0 + ly;
-        if (x >= Cl.w || y >= Cl.h)
-            continue;
-        float tap[4][4];
-#pragma unroll
-        for (int iy = 0; iy < 4; ++iy) {
-            const float* row = res + s_ryi[ly * 4 + iy] * LX;
-#pragma unroll
-            for (int ix = 0; ix < 4; ++ix)
-                tap[iy][ix] = row[s_rxi[lx * 4 + ix]];
-        }
-        float value = 0.f;
-#pragma unroll
-        for (int iy = 0; iy < 4; ++iy) {
-            float horizontal = 0.f;
-#pragma unroll
-            for (int ix = 0; ix < 4; ++ix)
-                horizontal += s_rxw[lx * 4 + ix] * tap[iy][ix];
-            value += s_ryw[ly * 4 + iy] * horizontal;
-        }
-        Cl.rhs[(y + 1) * Cl.s + x + 1] = value;
     }
 }
 
@@ -1398,8 +858,6 @@ __global__ __launch_bounds__(kTailThreads) void k_mg_tail(const TailDesc D, cons
     tail_run<TV>(D, shift, status, lds);
 }
 
-constexpr int kMultiNS = 4;
-
 // ---------------------------------------------------------------------------------------------
 // Batched PCG: one 1024-thread workgroup per instance runs the instance's whole iteration loop (the
 // kernels of one captured PCG iteration become phases separated by workgroup barriers), so a batch of
@@ -1445,7 +903,7 @@ __device__ __forceinline__ double wg_max(double v, double* slot)
     return r;
 }
 
-// 2 * sweeps red-black half-sweeps of one level in place on `sol` (k_rb_multi's update): colours from
+// 2 * sweeps red-black half-sweeps of one level in place on `sol` (the level smoothers' update): colours from
 // `first`, alternating; the first half-sweep of a pre-smoothing ignores the (zero) neighbours.
 __device__ void wg_sweeps(const LevelView& L, float* sol, const float* rhs, const double* shift, int first,
     bool from_zero, int sweeps)
@@ -1560,7 +1018,7 @@ __device__ void wg_res_restrict(const LevelView& F, const float* rhs, const doub
     __syncthreads();
 }
 
-// sol[0] = sol[1] + bilinear prolongation of the coarse correction (k_rb_multi MODE 1's load).
+// sol[0] = sol[1] + bilinear prolongation of the coarse correction (the post-smoothing's load).
 __device__ void wg_prolong(const LevelView& L, const CoarseLink& link)
 {
     const int w = L.w, h = L.h, s = L.s;
@@ -1861,132 +1319,6 @@ bool tail_allow_lds(size_t bytes)
                (int)bytes) == hipSuccess;
 }
 
-// Tile variants (interior cells per workgroup).  The fused sweeps compute every interior cell exactly as
-// global sweeps would, whatever the tile, so the choice changes time only; small levels use small
-// tiles to spread over more compute units.  Variants 6-8 size the workgroup to the tile's red-black
-// slots (32 x 32: 1104 slots on 384 threads; 64 x 32 and 32 x 64: 1840 and 1872 on 640), three
-// rounds each with at most 4% of the lanes idle, against 28% for 32 x 32 on 512 threads; 9 runs the
-// 64 x 32 and 32 x 64 slots in two rounds of 960 threads.
-void launch_rb_multi(hipStream_t st, const LevelView& L, int cur, const float* rhs, const double* shift,
-    int first_color, int from_zero, const CoarseLink& link, const int* status, int fine, int variant, int nu)
-{
-    const int mode = from_zero ? 0 : (link.csol ? 1 : 2);
-    nu = std::min(std::max(nu, 1), kMultiNS);
-#define FS_RB(TX, TY, F, M, NT)                                                                               \
-    hipLaunchKernelGGL((k_rb_multi<TX, TY, kMultiNS, F, M, NT>), dim3(((L.w + TX - 1) / TX) * ((L.h + TY - 1) / TY)), \
-        dim3(NT), 0, st, L, cur, rhs, shift, first_color, nu, link, status)
-#define FS_RB_MODES(TX, TY, F, NT)      \
-    do {                                \
-        if (mode == 0)                  \
-            FS_RB(TX, TY, F, 0, NT);    \
-        else if (mode == 1)             \
-            FS_RB(TX, TY, F, 1, NT);    \
-        else                            \
-            FS_RB(TX, TY, F, 2, NT);    \
-    } while (0)
-    switch (variant) {
-    case 1: FS_RB_MODES(32, 32, 0, 256); break;
-    case 2: FS_RB_MODES(32, 16, 0, 256); break;
-    case 3: FS_RB_MODES(16, 16, 0, 256); break;
-    case 4:
-        if (fine)
-            FS_RB_MODES(64, 32, 1, 512);
-        else
-            FS_RB_MODES(64, 32, 0, 512);
-        break;
-    case 5: FS_RB_MODES(32, 32, 0, 512); break;
-    case 6: FS_RB_MODES(32, 32, 0, 384); break;
-    case 7: FS_RB_MODES(64, 32, 0, 640); break;
-    case 8: FS_RB_MODES(32, 64, 0, 640); break;
-    case 9: FS_RB_MODES(64, 32, 0, 960); break;
-    case 10: FS_RB_MODES(32, 64, 0, 960); break;
-    default:
-        if (fine)
-            FS_RB_MODES(64, 32, 1, 256);
-        else
-            FS_RB_MODES(64, 32, 0, 256);
-        break;
-    }
-#undef FS_RB_MODES
-#undef FS_RB
-}
-
-void launch_jacobi_multi(hipStream_t st, const LevelView& L, int cur, const float* rhs, const double* shift,
-    int from_zero, const SmoothWeights& weights, int nu, const CoarseLink& link, const int* status, int variant)
-{
-    nu = std::min(std::max(nu, 1), kJacobiMaxSweeps);
-    // the halo the sweeps need: 5 cells up to 5 sweeps (the common case), 8 beyond
-#define FS_JM(TX, TY, M, NT, HALO)                                                                            \
-    hipLaunchKernelGGL((k_jacobi_multi<TX, TY, M, NT, HALO>),                                                  \
-        dim3(((L.w + TX - 1) / TX) * ((L.h + TY - 1) / TY)), dim3(NT), 0, st, L, cur, rhs, shift, weights, nu,  \
-        link, status)
-#define FS_JM_MODES(TX, TY, NT)                  \
-    do {                                         \
-        if (nu <= kJacobiShortHalo) {            \
-            if (from_zero)                       \
-                FS_JM(TX, TY, 0, NT, kJacobiShortHalo); \
-            else                                 \
-                FS_JM(TX, TY, 1, NT, kJacobiShortHalo); \
-        } else if (from_zero) {                  \
-            FS_JM(TX, TY, 0, NT, kJacobiMaxSweeps); \
-        } else {                                 \
-            FS_JM(TX, TY, 1, NT, kJacobiMaxSweeps); \
-        }                                        \
-    } while (0)
-    switch (variant) {
-    case 1: FS_JM_MODES(32, 32, 256); break;
-    case 2: FS_JM_MODES(32, 16, 256); break;
-    case 3: FS_JM_MODES(16, 16, 256); break;
-    case 4: FS_JM_MODES(32, 32, 512); break;
-    case 5: FS_JM_MODES(64, 64, 1024); break;
-    case 6: FS_JM_MODES(64, 32, 1024); break;
-    case 7: FS_JM_MODES(32, 64, 1024); break;
-    default: FS_JM_MODES(64, 32, 512); break;
-    }
-#undef FS_JM_MODES
-#undef FS_JM
-}
-
-void launch_jacobi_res_restrict(hipStream_t st, const LevelView& L, int cur, const float* rhs, const double* shift,
-    const SmoothWeights& weights, int nu, const LevelView& C, AxisRestrict rx, AxisRestrict ry, const int* status,
-    int variant)
-{
-    nu = std::min(std::max(nu, 1), kJacobiMaxSweeps);
-#define FS_JRR_H(CX, CY, NT, HALO)                                                                            \
-    hipLaunchKernelGGL((k_jacobi_res_restrict<CX, CY, NT, HALO>),                                              \
-        dim3(((C.w + CX - 1) / CX) * ((C.h + CY - 1) / CY)), dim3(NT), 0, st, L, cur, rhs, shift, weights, nu, C, \
-        rx, ry, status)
-#define FS_JRR(CX, CY, NT)                      \
-    do {                                        \
-        if (nu <= kJacobiShortHalo)             \
-            FS_JRR_H(CX, CY, NT, kJacobiShortHalo); \
-        else                                    \
-            FS_JRR_H(CX, CY, NT, kJacobiMaxSweeps); \
-    } while (0)
-    switch (variant) {
-    case 1: FS_JRR(16, 16, 512); break;
-    case 2: FS_JRR(32, 16, 1024); break;
-    default: FS_JRR(16, 8, 512); break;
-    }
-#undef FS_JRR
-#undef FS_JRR_H
-}
-
-void launch_res_restrict(hipStream_t st, const LevelView& F, int cur, const float* rhs, const double* shift,
-    const LevelView& C, AxisRestrict rx, AxisRestrict ry, const int* status, int variant)
-{
-#define FS_RR(CX, CY)                                                                                         \
-    hipLaunchKernelGGL((k_res_restrict<CX, CY>), dim3(((C.w + CX - 1) / CX) * ((C.h + CY - 1) / CY)), dim3(kNT), 0, \
-        st, F, cur, rhs, shift, C, rx, ry, status)
-    switch (variant) {
-    case 1: FS_RR(16, 16); break;
-    case 2: FS_RR(16, 8); break;
-    case 3: FS_RR(8, 8); break;
-    default: FS_RR(32, 16); break;
-    }
-#undef FS_RR
-}
-
 void launch_coarse_factor(hipStream_t st, int w, int h, const double* right64, const double* down64,
     double* factor, float* ginv, int n, PcgScalars* S, int pin)
 {
@@ -2047,40 +1379,7 @@ template void launch_level_pack<half16>(hipStream_t, int, int, const double*, co
 template void launch_level_pack<bf16>(hipStream_t, int, int, const double*, const double*, bf16*, bf16*);
 
 template <class C, class V, class VC>
-void launch_rb_multi_t(hipStream_t st, const LevelViewT<C, V>& L, int cur, const V* rhs, const double* shift,
-    int first_color, int from_zero, const CoarseLinkT<VC>& link, const int* status, int variant, int nu)
-{
-    nu = std::min(std::max(nu, 1), kMultiNS);
-#define FS_RBT(TX, TY, M, NT)                                                                                 \
-    hipLaunchKernelGGL((k_rb_multi<TX, TY, kMultiNS, 0, M, NT, C, V, VC>),                                   \
-        dim3(((L.w + TX - 1) / TX) * ((L.h + TY - 1) / TY)), dim3(NT), 0, st, L, cur, rhs, shift, first_color, nu, \
-        link, status)
-#define FS_RBT_MODES(TX, TY, NT)      \
-    do {                              \
-        if (from_zero)                \
-            FS_RBT(TX, TY, 0, NT);    \
-        else                          \
-            FS_RBT(TX, TY, 1, NT);    \
-    } while (0)
-    switch (variant) {
-    case 1: FS_RBT_MODES(32, 32, 256); break;
-    case 2: FS_RBT_MODES(32, 16, 256); break;
-    case 3: FS_RBT_MODES(16, 16, 256); break;
-    case 4: FS_RBT_MODES(64, 32, 512); break;
-    case 5: FS_RBT_MODES(32, 32, 512); break;
-    case 6: FS_RBT_MODES(32, 32, 384); break;
-    case 7: FS_RBT_MODES(64, 32, 640); break;
-    case 8: FS_RBT_MODES(32, 64, 640); break;
-    case 9: FS_RBT_MODES(64, 32, 960); break;
-    case 10: FS_RBT_MODES(32, 64, 960); break;
-    default: FS_RBT_MODES(64, 32, 256); break;
-    }
-#undef FS_RBT_MODES
-#undef FS_RBT
-}
-
-template <class C, class V, class VC>
-void launch_res_restrict_t(hipStream_t st, const LevelViewT<C, V>& F, int cur, const V* rhs, const double* shift,
+void launch_res_restrict(hipStream_t st, const LevelViewT<C, V>& F, int cur, const V* rhs, const double* shift,
     const LevelViewT<C, VC>& Cl, AxisRestrict rx, AxisRestrict ry, const int* status, int variant)
 {
 #define FS_RRT(CX, CY)                                                                                        \
@@ -2095,16 +1394,15 @@ void launch_res_restrict_t(hipStream_t st, const LevelViewT<C, V>& F, int cur, c
 #undef FS_RRT
 }
 
-#define FS_MG16(C, V, VC)                                                                                      \
-    template void launch_rb_multi_t<C, V, VC>(hipStream_t, const LevelViewT<C, V>&, int, const V*, const double*, \
-        int, int, const CoarseLinkT<VC>&, const int*, int, int);                                               \
-    template void launch_res_restrict_t<C, V, VC>(hipStream_t, const LevelViewT<C, V>&, int, const V*,          \
-        const double*, const LevelViewT<C, VC>&, AxisRestrict, AxisRestrict, const int*, int);
-FS_MG16(half16, float, float)
-FS_MG16(bf16, float, float)
-FS_MG16(bf16, float, bf16)
-FS_MG16(bf16, bf16, bf16)
-#undef FS_MG16
+#define FS_RESTRICT(C, V, VC)                                                                                  \
+    template void launch_res_restrict<C, V, VC>(hipStream_t, const LevelViewT<C, V>&, int, const V*, const double*, \
+        const LevelViewT<C, VC>&, AxisRestrict, AxisRestrict, const int*, int);
+FS_RESTRICT(float, float, float)
+FS_RESTRICT(half16, float, float)
+FS_RESTRICT(bf16, float, float)
+FS_RESTRICT(bf16, float, bf16)
+FS_RESTRICT(bf16, bf16, bf16)
+#undef FS_RESTRICT
 
 bool batch_allow_lds(size_t bytes)
 {

@@ -341,21 +341,17 @@ fs_status fs_mg_level_weights(fs_grid* grid, int level, double* right, double* d
 fs_status fs_mg_level_prolong(fs_grid* grid, int level, int axis, int* first, int* second, double* weight);
 /* Restriction stencils of the next coarser level: count[n], index[4n], weight[4n]. */
 fs_status fs_mg_level_restrict(fs_grid* grid, int level, int axis, int* count, int* index, double* weight);
-/* Autotuned kernel tiles of a level (build's own): pre- and post-smoothing variants of the fused
- * four-sweep kernel (0 = 64x32/256 threads, 1 = 32x32/256, 2 = 32x16/256, 3 = 16x16/256, 4 = 64x32/512,
- * 5 = 32x32/512, 6 = 32x32/384, 7 = 64x32/640, 8 = 32x64/640, 9 = 64x32/960, 10 = 32x64/960) and the
- * residual-restriction variant (0 = 32x16, 1 = 16x16, 2 = 16x8, 3 = 8x8 coarse
- * cells); -1 for levels solved inside the single-workgroup tail.  On a level that runs the Chebyshev smoother,
- * pre and post are tiles of the Jacobi kernel instead (0 = 64x32/512, 1 = 32x32/256, 2 = 32x16/256,
- * 3 = 16x16/256, 4 = 32x32/512, 5 = 64x64/1024, 6 = 64x32/1024, 7 = 32x64/1024), and pre 8, 9, 10 mean
- * that the pre-smoothing runs fused with the residual and restriction (16x8/512, 16x16/512, 32x16/1024
- * coarse cells per workgroup; same values). */
+/* Autotuned launch choices of a level's smoothers (build's own).  A tile is columns x rows (threads), its smoothing
+ * halo included.  post: 0 = 128x64 (512), 1 = 128x64 (1024), 2 = 64x64 (512), 3 = 64x64 (1024), 4 = 64x32 (256),
+ * 5 = 64x32 (512), 6 = 32x32 (256), 7 = 32x64 (256), 8 = 128x32 (512), 9 = 128x128 (1024), 10 = 32x64 (512); a
+ * level that runs the Chebyshev smoother has 0..7 of them.  pre: on a red-black level 0..4 run the pre-smoothing apart
+ * from the residual and restriction, on the tiles 0, 1, 2, 4, 6 above, and 5..10 all three in one launch: 128x128 (1024),
+ * 128x64 (1024), 64x64 (512), 64x64 (1024), 32x64 (512), 32x32 (256); on a Chebyshev level 0..7 run it apart and
+ * 8..10 fused: 128x128 (1024), 64x64 (512), 32x32 (256).  restriction (of the separate launch): 0 = 32x16, 1 = 16x16,
+ * 2 = 16x8, 3 = 8x8 coarse cells.  -1 for levels solved inside the single-workgroup tail. */
 fs_status fs_mg_level_tiles(fs_grid* grid, int level, int* pre, int* post, int* restriction);
-/* Overrides the autotuned variants of a tiled level (-1 keeps one): every variant computes the same
- * values, so this changes time only -- for profiling one fixed configuration and for testing that claim.
- * The autotuner may run a Chebyshev level's pre-smoothing fused with its residual and restriction (one
- * launch, the same values): pre 0..7 selects the separate launches with that Jacobi tile, 8..10 the fused
- * launch with the tiles fs_mg_level_tiles lists. */
+/* Overrides the autotuned choices of a tiled level (-1 keeps one): all of them compute the same values, so this
+ * changes time only -- for profiling one fixed configuration and for testing that claim. */
 fs_status fs_mg_set_level_tiles(fs_grid* grid, int level, int pre, int post, int restriction);
 /* Coarsest dense Cholesky factor, n*n row-major (lower triangle); *n receives the unknown count. */
 fs_status fs_mg_coarse_factor(fs_grid* grid, double* factor, int* n);
@@ -369,7 +365,7 @@ fs_status fs_face_weights(fs_grid* grid, double* inv_density_u, double* inv_dens
 /* Times `reps` back-to-back launches of one hot kernel on the grid's stream with HIP events and
  * returns the mean milliseconds per launch.  kernel: 0 = finest-level post-smoothing (prolongation +
  * the grid's smoother sweeps, as in the V-cycle),
- * 1 = operator + dot (A d), 2 = PCG update, 3 = FP32 copy of one padded vector (reference kernel),
+ * 1 = direction + operator + dot (A d), 2 = PCG update, 3 = FP32 copy of one padded vector (reference kernel),
  * 4 = second level's smoother, 5 = finest residual + restriction, 6 = coarse tail, 7 = coarse
  * inverse (sweep operator), 8 = direction update, 9 = r.z reduction, 10 = FP32 copy of a 64 MiB buffer
  * into another (HBM copy-bandwidth reference; 128 MiB moved per launch). */
