@@ -155,20 +155,56 @@ __device__ __forceinline__ void level_diag_values(double rl, double rr, double d
     down32 = (float)dd;
 }
 
+// The two values that meet when lanes K apart (32, 16) are combined: (lower, upper) in both lanes of a pair.
+template <int K> __device__ __forceinline__ void lane_halves(double v, double& lower, double& upper)
+{
+    const unsigned lo = (unsigned)__double2loint(v), hi = (unsigned)__double2hiint(v);
+    if constexpr (K == 32) {
+        const auto l = __builtin_amdgcn_permlane32_swap(lo, lo, false, false);
+        const auto h = __builtin_amdgcn_permlane32_swap(hi, hi, false, false);
+        lower = __hiloint2double((int)h[0], (int)l[0]);
+        upper = __hiloint2double((int)h[1], (int)l[1]);
+    } else {
+        const auto l = __builtin_amdgcn_permlane16_swap(lo, lo, false, false);
+        const auto h = __builtin_amdgcn_permlane16_swap(hi, hi, false, false);
+        lower = __hiloint2double((int)h[0], (int)l[0]);
+        upper = __hiloint2double((int)h[1], (int)l[1]);
+    }
+}
+
+// v rotated by N lanes within each row of 16.
+template <int N> __device__ __forceinline__ double row_rotate(double v)
+{
+    const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), 0x120 + N, 0xf, 0xf, true);
+    const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), 0x120 + N, 0xf, 0xf, true);
+    return __hiloint2double(hi, lo);
+}
+
+// Combines the wavefront's values as the butterfly over lanes 32, 16, 8, 4, 2, 1 apart does (after lanes 8 apart are
+// combined a row repeats every 8 lanes, so a rotation by 4 is the exchange with the lane 4 apart, and so on), with
+// register lane exchanges alone: a shuffle through the LDS hardware costs about 60 ns a step, and every reduction
+// of the solver takes twelve of them.
+template <class Op> __device__ __forceinline__ double wave_combine(double v, Op op)
+{
+    double a, b;
+    lane_halves<32>(v, a, b);
+    v = op(a, b);
+    lane_halves<16>(v, a, b);
+    v = op(a, b);
+    v = op(v, row_rotate<8>(v));
+    v = op(v, row_rotate<4>(v));
+    v = op(v, row_rotate<2>(v));
+    return op(v, row_rotate<1>(v));
+}
+
 __device__ __forceinline__ double wave_sum(double v)
 {
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1)
-        v += __shfl_xor(v, off, 64);
-    return v;
+    return wave_combine(v, [](double a, double b) { return a + b; });
 }
 
 __device__ __forceinline__ double wave_max(double v)
 {
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1)
-        v = fmax(v, __shfl_xor(v, off, 64));
-    return v;
+    return wave_combine(v, [](double a, double b) { return fmax(a, b); });
 }
 
 // Block-wide sum in a fixed order; result valid in thread 0.  `lds` holds blockDim/64 doubles.
