@@ -529,6 +529,7 @@ struct fs_grid {
     TailDesc tail{};
     DevBuf<TailDesc> tail_dev;
     DevBuf<unsigned> tail_tables;
+    DevBuf<float4> tail_pairs;
 
     hipGraphExec_t iter_exec = nullptr;
     hipGraph_t iter_graph = nullptr;
@@ -776,6 +777,61 @@ struct fs_grid {
         tail.tables = tail_tables.p;
     }
 
+    // The held tail's transfer entries (TailDesc::pair_tables).
+    void build_pair_tables()
+    {
+        tail_hold(tail);
+        if (!tail.held_rows)
+            return;
+        std::vector<float4> entries;
+        auto bits = [](int v) {
+            float f;
+            std::memcpy(&f, &v, 4);
+            return f;
+        };
+        auto axis = [&](int fine, int coarse, const std::vector<int>& first, const std::vector<int>& second,
+                        const std::vector<double>& weight, const std::vector<int>& count, const std::vector<int>& index,
+                        const std::vector<double>& rweight) {
+            for (int c = 0; c < coarse; ++c) {
+                float w[2] = {0.f, 0.f}, r[4] = {0.f, 0.f, 0.f, 0.f};
+                int code = 0;
+                for (int j = 0; j < 2; ++j) {
+                    const int f = 2 * c + j;
+                    if (f >= fine)
+                        continue;
+                    w[j] = (float)weight[f];
+                    if (first[f] < c - 1 || first[f] > c || second[f] < c - 1 || second[f] > c + 1)
+                        fail(FS_E_RUNTIME, "multigrid prolongation reaches past the neighbouring cells");
+                    code |= ((first[f] == c ? 1 : 0) | (second[f] == c ? 2 : second[f] == c + 1 ? 4 : 0)) << (4 * j);
+                }
+                for (int k = 0; k < count[c]; ++k) {
+                    const int at = index[(size_t)c * 4 + k] - (2 * c - 1);
+                    if (at < 0 || at > 3)
+                        fail(FS_E_RUNTIME, "multigrid restriction reaches past the neighbouring cells");
+                    r[at] = (float)rweight[(size_t)c * 4 + k];
+                }
+                entries.push_back(make_float4(w[0], w[1], bits(code), 0.f));
+                entries.push_back(make_float4(r[0], r[1], r[2], r[3]));
+            }
+        };
+        for (int i = 0; i + 1 < tail.levels; ++i) {
+            const Level& L = levels[tail_start + i];
+            const Level& Cn = levels[tail_start + i + 1];
+            axis(L.w, Cn.w, L.pxf, L.pxs, L.pxw, L.rxc, L.rxi, L.rxw);
+            axis(L.h, Cn.h, L.pyf, L.pys, L.pyw, L.ryc, L.ryi, L.ryw);
+        }
+        upload_vec(tail_pairs, entries, bytes);
+        tail.pair_tables = tail_pairs.p;
+        tail.pair_table_n = (int)entries.size();
+    }
+    void launch_tail(const double* shift, const int* status, bool bf16_top)
+    {
+        if (tail.held_rows)
+            launch_held_tail(st(), tail, shift, status, bf16_top);
+        else
+            launch_mg_tail(st(), tail, tail_lds, shift, status, bf16_top);
+    }
+
     // PressureMultigrid constructor (PressureMultigrid.cpp:38-62): halve until w*h <= 64.
     void build_hierarchy()
     {
@@ -869,6 +925,7 @@ struct fs_grid {
                 break;
             limit = 65536 - 4096;  // the device refused a larger dynamic LDS request
         }
+        build_pair_tables();
         bytes += tail_dev.alloc(1);
         device_upload(tail_dev.p, &tail, sizeof(TailDesc));
     }
@@ -1115,7 +1172,7 @@ struct fs_grid {
                 F.restrict_variant);
         }
         join_before_tail();
-        launch_mg_tail(st(), tail, tail_lds, T == 0 ? rmean_ptr() : nullptr, status, std::is_same<VL, bf16>::value);
+        launch_tail(T == 0 ? rmean_ptr() : nullptr, status, std::is_same<VL, bf16>::value);
         for (int l = T - 1; l >= 0; --l) {
             const bool chebyshev = chebyshev_on(l);
             ascend<C, VL>(l, 1, status, chebyshev, sweeps_on(l), chebyshev ? levels[l].jacobi_post : levels[l].post_variant);
@@ -3292,8 +3349,7 @@ fs_status fs_time_kernel(fs_grid* grid, int kernel, int reps, double* ms_per_lau
                     F.restrict_variant);
                 break;
             }
-            case 6: launch_mg_tail(g.st(), g.tail, g.tail_lds, g.tail_start == 0 ? g.rmean_ptr() : nullptr,
-                        nullptr); break;
+            case 6: g.launch_tail(g.tail_start == 0 ? g.rmean_ptr() : nullptr, nullptr, false); break;
             case 7: {
                 const Level& last = g.levels.back();
                 launch_coarse_inverse(g.st(), last.w, last.h, last.right64.p, last.down64.p, g.ginv.p, g.coarse_n,

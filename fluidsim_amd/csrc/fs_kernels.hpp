@@ -72,6 +72,7 @@ struct TailLevel {
     const int* ryc; const int* ryi; const float* ryw;
     int lds_arrays;      // word offset of right, down, rhs, sol, res (each s * (h + 2))
     int lds_tables;      // word offset of this level's transfer tables (3w + 3h + 9cw + 9ch words)
+    int lanes, table;    // held levels (fs_tail.hip): log2 of a row's lanes, first entry of the pair tables
 };
 
 constexpr int kMaxTailLevels = 8;
@@ -89,6 +90,13 @@ struct TailDesc {
     int lds_tables_base;       // word offset of the table block in LDS
     int lds_words;             // total LDS words
     int sweeps;                // red-black sweeps per side on every tail level (4: the reference's V(4,4))
+    // Held levels (fs_tail.hip): rows per thread of the first level, 0 when the levels' shapes do not fit; and per level
+    // its column pairs' then its row pairs' transfer entries, two of four words each: the prolongation's two weights
+    // and coarse neighbours (four bits per fine cell: 1 first = own, 2 second = own, 4 second = next, else
+    // previous), and the restriction's weights of fine cells 2 c - 1 .. 2 c + 2.
+    int held_rows;
+    int pair_table_n;
+    const float4* pair_tables;
     TailLevel lev[kMaxTailLevels];
 };
 
@@ -97,6 +105,8 @@ size_t tail_layout(TailDesc& t);
 // Raises the dynamic-LDS limit of the tail kernel; false if the device refuses.
 bool tail_allow_lds(size_t bytes);
 
+// Sets held_rows and the levels' lanes and table offsets.
+void tail_hold(TailDesc& t);
 // rel_tol > 0 replaces tol by rel_tol * max|b| once the rhs b is formed (a relative residual).
 void launch_init_scalars(hipStream_t st, PcgScalars* S, double tol, int max_iterations, double rel_tol = 0.0);
 // Copies a coarse-factorisation failure flagged in `from` into the solve's scalar block.
@@ -234,6 +244,9 @@ void launch_res_restrict(hipStream_t st, const LevelViewT<C, V>& F, int cur, con
 // bf16_top: the first tail level's rhs and solution are stored as bfloat16 (else FP32).
 void launch_mg_tail(hipStream_t st, const TailDesc& desc, size_t lds_bytes, const double* shift, const int* status,
     int bf16_top = 0);
+
+// The same with the levels held in registers, same values; needs desc.held_rows.
+void launch_held_tail(hipStream_t st, const TailDesc& desc, const double* shift, const int* status, int bf16_top = 0);
 
 // ---- 16-bit multigrid levels: conductances as C (half16 or bf16), vectors as V ----
 // Conductances of one level rounded (FP64 -> FP32 -> C, each to nearest even) into 16-bit copies.

@@ -102,3 +102,26 @@ def test_every_choice_is_the_same_16_bit_vcycle(W, H, mode):
     # rounding the conductances moves the V-cycle by their relative error, 2^-11 or 2^-8, vectors by 2^-8 a store
     assert np.linalg.norm(reference - full) < (2e-3 if mode == FS_MG_FP16 else 3e-2) * np.linalg.norm(full)
     g.destroy()
+
+
+@pytest.mark.parametrize("coarse", [1, 4])
+@pytest.mark.parametrize("W,H", [(64, 64), (63, 65), (65, 33), (70, 58), (66, 62), (128, 32), (129, 31), (200, 20), (2, 700),
+                                 (9, 9), (12, 7), (31, 130), (33, 17)])
+def test_coarse_levels_match_the_oracle(O, W, H, coarse):
+    """Grids whose levels all run in the single-workgroup tail: two, four and eight rows per thread, one to four levels
+    above the coarsest, and shapes its register layout does not take (more than 128 columns)."""
+    wl, _ = tank(W, H, False)
+    g = grid(wl, None)
+    g.setPressureSmoother(FS_SMOOTHER_RED_BLACK, 4, coarse)
+    O.set_smoother(FS_SMOOTHER_RED_BLACK, 4, coarse)
+    o = O.OracleGrid(W, H, wl.cell_size)
+    o.configure(wl.liquid_density, wl.gas_density)
+    o.upload(wl.fraction, wl.u, wl.v, None, wl.liquid_mass, wl.gas_mass)
+    o.project(wl.dt, 0, 1.0)
+    g.project(wl.dt, 0, 1.0)
+    i = np.arange(W * H)
+    a = np.sin(i * 0.31) + np.cos(i * 0.073)
+    a -= a.mean()
+    expected, out = o.multigrid().apply(a, 0.0), g.multigridApply(a)
+    assert np.linalg.norm(out - expected) < 1e-5 * np.linalg.norm(expected)
+    g.destroy()
