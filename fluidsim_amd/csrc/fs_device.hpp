@@ -60,12 +60,13 @@ struct PcgScalars {
     int restarts;
     int mg_failed;      // coarse factorisation failed (the hierarchy must be rebuilt next time)
     int replace;        // check not triggered by the tolerance: refresh r from FP64, restart only on drift
-    int flush;          // a check refreshed r from p + x: the next direction folds x into p
+    int flush;          // r was formed from (p - p_shift) + x: the next direction folds that into p
     double window_rmax; // true residual max-norm that started the current refinement window
     // r.z of the direction used by the iteration that starts at iteration count c, kept in slot c & 1:
     // the direction kernel reads the previous slot and writes the next one while other workgroups of
     // the same launch still read the previous value.
     double rz_slot[2];
+    double p_shift;     // mean of the predicted pressure, still in p until it is folded
     // > 0: the tolerance is relative, tol = rel_tol * bmax once the rhs is formed (max-norm relative residual)
     double rel_tol;
 };
@@ -105,43 +106,40 @@ struct AxisRestrict {
 __device__ __forceinline__ int pidx(int x, int y, int s) { return (y + 1) * s + (x + 1); }
 
 // PressureMultigrid::coarsen (PressureMultigrid.cpp:142-202) for coarse cell (x, y): parallel paths add,
-// series resistances combine across the two or three fine faces between coarse centres.  Writes the
-// coarse right face (x + 1 < cw) and down face (y + 1 < ch) of the cell.
-__device__ __forceinline__ void coarsen_cell(int x, int y, int fw, int fh, const double* fcx, const double* fcy,
-    const double* fright, const double* fdown, int cw, int ch, const double* ccx, const double* ccy,
-    double* cright, double* cdown)
+// series resistances combine across the two or three fine faces between coarse centres.  Returns the
+// cell's coarse right face (zero for the last column) and down face (zero for the last row).
+__device__ __forceinline__ double2 coarsen_cell(int x, int y, int fw, int fh, const double* fcx, const double* fcy,
+    const double* fright, const double* fdown, int cw, int ch, const double* ccx, const double* ccy)
 {
-    const int fs = fw + 2, cs = cw + 2;
+    const int fs = fw + 2;
+    double2 c = make_double2(0.0, 0.0);
     if (x + 1 < cw) {
         const int edge = 2 * x + 2;
         const double left = (fcx[edge - 1] - ccx[x]) / (fcx[edge - 1] - fcx[edge - 2]);
         const double right = edge + 1 < fw ? (ccx[x + 1] - fcx[edge]) / (fcx[edge + 1] - fcx[edge]) : 0.0;
-        double conductance = 0.0;
         const int fy_end = min(2 * y + 2, fh);
         for (int fy = 2 * y; fy < fy_end; ++fy) {
             const int i = (fy + 1) * fs + edge;
             double resistance = left / fright[i - 1] + 1.0 / fright[i];
             if (right != 0.0)
                 resistance += right / fright[i + 1];
-            conductance += 1.0 / resistance;
+            c.x += 1.0 / resistance;
         }
-        cright[(y + 1) * cs + x + 1] = conductance;
     }
     if (y + 1 < ch) {
         const int edge = 2 * y + 2;
         const double up = (fcy[edge - 1] - ccy[y]) / (fcy[edge - 1] - fcy[edge - 2]);
         const double down = edge + 1 < fh ? (ccy[y + 1] - fcy[edge]) / (fcy[edge + 1] - fcy[edge]) : 0.0;
-        double conductance = 0.0;
         const int fx_end = min(2 * x + 2, fw);
         for (int fx = 2 * x; fx < fx_end; ++fx) {
             const int i = edge * fs + fx + 1;
             double resistance = up / fdown[i - fs] + 1.0 / fdown[i];
             if (down != 0.0)
                 resistance += down / fdown[i + fs];
-            conductance += 1.0 / resistance;
+            c.y += 1.0 / resistance;
         }
-        cdown[(y + 1) * cs + x + 1] = conductance;
     }
+    return c;
 }
 
 // Level::rebuildDiagonal (PressureMultigrid.cpp:104-117) of one cell from its four FP64 face

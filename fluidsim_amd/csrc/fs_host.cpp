@@ -399,7 +399,7 @@ constexpr int kFoldBlocks = 1024;         // workgroups of the PCG kernels beyon
 // ones, the single-workgroup tail's levels among them, always run red-black V(4,4).
 constexpr long long kSmootherMinCells = 4096;
 // Levels of at most this many cells are coarsened by the hierarchy rebuild's single-workgroup launch.
-constexpr long long kChainCells = 4096;
+constexpr long long kChainCells = 1024;
 
 // Weight i of `sweeps` Chebyshev-weighted Jacobi sweeps: PressureMultigridGPU's constructor
 // (PressureMultigridGPU.cpp:24-28), 1 / (1.1 + 0.9 cos(pi (i + 1/2) / sweeps)) -- the reciprocals of the
@@ -502,7 +502,7 @@ struct fs_grid {
 
     DevBuf<double> fraction, u, v, lmass, gmass, density, p, p_prev, b, tmp64;
     DevBuf<double> snap_fraction, snap_u, snap_v, snap_p, snap_p_prev, snap_lmass, snap_gmass;
-    DevBuf<double> sl_u, sl_v, sl_cells;
+    DevBuf<double> sl_u, sl_v, sl_fraction, sl_lmass, sl_gmass;   // semi-Lagrangian transport's outputs (swapped in)
     // reference transport: second fraction/mass buffers, transported velocities (ping-pong), momenta,
     // per-pass face transfers, frozen corrections
     DevBuf<double> tr_fraction, tr_lmass, tr_gmass, tr_nu[2], tr_nv[2], tr_mom_u, tr_mom_v, tr_lt, tr_mt;
@@ -640,6 +640,7 @@ struct fs_grid {
         g.d2 = d2.p;
         g.q = q.p;
         g.zdiag = zdiag.p;
+        g.z = z_ptr();
         g.S = S.p;
         g.partials = partials.p;
         const size_t blocks = cell_tiles();
@@ -934,17 +935,23 @@ struct fs_grid {
     void rebuild_coefficients()
     {
         GridDev g = dev();
-        launch_density(st(), g);
-        launch_face_weights(st(), g);
-        Level& L0 = levels[0];
-        launch_level_diag(st(), W, H, L0.right64.p, L0.down64.p, L0.right32.p, L0.down32.p, L0.invd32.p);
+        launch_coefficients(st(), g);
         coeff_valid = true;
         mg_valid = false;
     }
 
+    // Level l as the hierarchy rebuild sees it.
+    ChainLevel chain_level(size_t l)
+    {
+        const Level& F = levels[l - 1];
+        Level& Cl = levels[l];
+        return ChainLevel{F.w, F.h, Cl.w, Cl.h, F.d_cx.p, F.d_cy.p, F.right64.p, F.down64.p, Cl.d_cx.p, Cl.d_cy.p,
+            Cl.right64.p, Cl.down64.p, Cl.right32.p, Cl.down32.p, Cl.invd32.p};
+    }
+
     // PressureMultigrid::rebuild (PressureMultigrid.cpp:119-140) on the device, FP64, on `stream`; a
     // failed coarse factorisation is flagged in `flag`.
-    // The levels of more than kChainCells cells are built one launch pair each; the smaller ones (at most
+    // The levels of more than kChainCells cells are built one launch each; the smaller ones (at most
     // kMaxTailLevels of them) and the coarse inverse in one single-workgroup launch, whose phases are
     // too small to fill the device -- the same values either way.
     // `levels_done` (optional) is recorded on `stream` once the levels the tiled V-cycle kernels read are
@@ -958,12 +965,7 @@ struct fs_grid {
                (long long)levels[chain_from - 1].w * levels[chain_from - 1].h <= kChainCells)
             --chain_from;
         for (size_t l = 0; l + 1 < chain_from; ++l) {
-            Level& F = levels[l];
-            Level& Cl = levels[l + 1];
-            launch_coarsen(stream, F.w, F.h, F.d_cx.p, F.d_cy.p, F.right64.p, F.down64.p, Cl.w, Cl.h, Cl.d_cx.p,
-                Cl.d_cy.p, Cl.right64.p, Cl.down64.p);
-            launch_level_diag(stream, Cl.w, Cl.h, Cl.right64.p, Cl.down64.p, Cl.right32.p, Cl.down32.p,
-                Cl.invd32.p);
+            launch_coarsen(stream, chain_level(l + 1));
         }
         const Level& last = levels.back();
         // the chain builds tail levels only: pack the tiled levels and let the V-cycle start
@@ -975,11 +977,7 @@ struct fs_grid {
         if (chain_from < nlev) {
             ChainDesc chain{};
             for (size_t l = chain_from; l < nlev; ++l) {
-                const Level& F = levels[l - 1];
-                Level& Cl = levels[l];
-                chain.lev[chain.levels++] = ChainLevel{F.w, F.h, Cl.w, Cl.h, F.d_cx.p, F.d_cy.p, F.right64.p,
-                    F.down64.p, Cl.d_cx.p, Cl.d_cy.p, Cl.right64.p, Cl.down64.p, Cl.right32.p, Cl.down32.p,
-                    Cl.invd32.p};
+                chain.lev[chain.levels++] = chain_level(l);
             }
             launch_coarse_chain(stream, chain, ginv.p, coarse_n, flag, solid.n > 0);
         } else {
@@ -1308,11 +1306,11 @@ struct fs_grid {
     void iteration_kernels()
     {
         GridDev g = dev();
-        launch_pcg_direction_ad(st(), g, z_ptr(), flexible());
+        launch_pcg_direction_ad(st(), g, flexible());
         launch_pcg_update(st(), g);
         launch_pcg_check(st(), g);
         precondition(status_ptr());
-        launch_pcg_rz(st(), g, z_ptr(), flexible());
+        launch_pcg_rz(st(), g, flexible());
     }
 
     void ensure_graph()
@@ -1347,6 +1345,7 @@ struct fs_grid {
         if (!coeff_valid)
             rebuild_coefficients();
         GridDev g = dev();
+        g.dt = dt;
         // The hierarchy depends only on the face weights: rebuild it on the second stream while the main
         // stream forms the rhs, the predicted pressure and its residual; join before the first V-cycle.
         const bool rebuild = precond == FS_PRECOND_MULTIGRID && !mg_valid;
@@ -1363,12 +1362,7 @@ struct fs_grid {
             if (ctx->aux)
                 HIPC(hipEventRecord(ctx->join, side));
         }
-        launch_rhs(st(), g, scale);
-        launch_rhs_center(st(), g);
-        launch_zero_pressure(st(), g);
-        launch_predict(st(), g);
-        launch_sub_mean_p(st(), g, 0);
-        launch_true_residual(st(), g);
+        launch_project_setup(st(), g);
         if (rebuild) {
             if (late_tail) {
                 HIPC(hipStreamWaitEvent(st(), ctx->join_levels, 0));
@@ -1388,7 +1382,7 @@ struct fs_grid {
             } clear{tail_join};
             precondition(status_ptr());
         }
-        launch_pcg_rz(st(), g, z_ptr(), flexible());
+        launch_pcg_rz(st(), g, flexible());
     }
 
     // Last phase: fold the correction into the pressure, remove its mean, correct the velocity and
@@ -1398,10 +1392,8 @@ struct fs_grid {
     void project_end(double dt)
     {
         GridDev g = dev();
-        launch_final_flush_sum(st(), g);
-        launch_sub_mean_p(st(), g, 1);
-        launch_correct_velocity(st(), g, dt);
-        launch_max_divergence(st(), g, true);
+        g.dt = dt;
+        launch_project_end(st(), g);
     }
 
     // `tol` is the caller's divergence tolerance; in the relative mode the accepted divergence is the
@@ -2418,24 +2410,22 @@ fs_status fs_max_divergence(fs_grid* grid, double* out)
 
 static void advect_sl(fs_grid& g, double dt)
 {
-    const size_t N = g.N();
-    const size_t fields = 1 + g.rho_l.size() + g.rho_g.size();
-    if (g.sl_u.n != g.NU())
-        g.bytes += g.sl_u.alloc(g.NU());
-    if (g.sl_v.n != g.NV())
-        g.bytes += g.sl_v.alloc(g.NV());
-    if (g.sl_cells.n != fields * N)
-        g.bytes += g.sl_cells.alloc(fields * N);
-    launch_semi_lagrangian(g.st(), g.dev(), g.ox, g.oy, dt, g.sl_u.p, g.sl_v.p, g.sl_cells.p);
-    HIPC(hipMemcpyAsync(g.u.p, g.sl_u.p, g.NU() * sizeof(double), hipMemcpyDeviceToDevice, g.st()));
-    HIPC(hipMemcpyAsync(g.v.p, g.sl_v.p, g.NV() * sizeof(double), hipMemcpyDeviceToDevice, g.st()));
-    HIPC(hipMemcpyAsync(g.fraction.p, g.sl_cells.p, N * sizeof(double), hipMemcpyDeviceToDevice, g.st()));
-    if (g.rho_l.size())
-        HIPC(hipMemcpyAsync(g.lmass.p, g.sl_cells.p + N, g.rho_l.size() * N * sizeof(double),
-            hipMemcpyDeviceToDevice, g.st()));
-    if (g.rho_g.size())
-        HIPC(hipMemcpyAsync(g.gmass.p, g.sl_cells.p + (1 + g.rho_l.size()) * N, g.rho_g.size() * N * sizeof(double),
-            hipMemcpyDeviceToDevice, g.st()));
+    auto ensure = [&](DevBuf<double>& b, size_t n) {
+        if (b.n != n)
+            g.bytes += b.alloc(n);
+    };
+    ensure(g.sl_u, g.NU());
+    ensure(g.sl_v, g.NV());
+    ensure(g.sl_fraction, g.N());
+    ensure(g.sl_lmass, g.rho_l.size() * g.N());
+    ensure(g.sl_gmass, g.rho_g.size() * g.N());
+    launch_semi_lagrangian(g.st(), g.dev(), g.ox, g.oy, dt, g.sl_u.p, g.sl_v.p, g.sl_fraction.p, g.sl_lmass.p,
+        g.sl_gmass.p);
+    g.u.swap(g.sl_u);
+    g.v.swap(g.sl_v);
+    g.fraction.swap(g.sl_fraction);
+    g.lmass.swap(g.sl_lmass);
+    g.gmass.swap(g.sl_gmass);
     g.coeff_valid = false;
     g.mg_valid = false;
 }
@@ -3314,6 +3304,7 @@ fs_status fs_time_kernel(fs_grid* grid, int kernel, int reps, double* ms_per_lau
             g.rebuild_hierarchy();
         LevelView L0 = g.view(0);
         GridDev gd = g.dev();
+        gd.z = g.levels[0].sol0.p;
         const int nlev = (int)g.levels.size();
         const int l1 = std::min(1, g.tail_start);
         if (kernel == 10 && g.calib_src.n != kCalibWords) {
@@ -3332,7 +3323,7 @@ fs_status fs_time_kernel(fs_grid* grid, int kernel, int reps, double* ms_per_lau
             case 0:  // the finest post-smoothing launch of a V-cycle (prolongation + four sweeps)
                 g.fine_post_smooth(i & 1);
                 break;
-            case 1: launch_pcg_direction_ad(g.st(), gd, g.levels[0].sol0.p); break;
+            case 1: launch_pcg_direction_ad(g.st(), gd); break;
             case 2: launch_pcg_update(g.st(), gd); break;
             case 3: launch_copy_f32(g.st(), g.r.p, g.q.p, g.NP()); break;
             case 4:  // second level's smoother (or the finest, if the tail starts at level 1)
@@ -3356,8 +3347,8 @@ fs_status fs_time_kernel(fs_grid* grid, int kernel, int reps, double* ms_per_lau
                     nullptr, g.solid.n > 0);
                 break;
             }
-            case 8: launch_pcg_direction(g.st(), gd, g.levels[0].sol0.p); break;
-            default: launch_pcg_rz(g.st(), gd, g.levels[0].sol0.p); break;
+            case 8: launch_pcg_direction(g.st(), gd); break;
+            default: launch_pcg_rz(g.st(), gd); break;
             }
         };
         launch_once(0);
@@ -3405,7 +3396,7 @@ static void batch_projection(fs_context* ctx, fs_grid* const* grids, const std::
             const int i = batched[(size_t)k];
             fs_grid& g = *grids[i];
             g.project_begin(dts[i], fs_grid::budget(max_iterations[i]), tolerances[i]);
-            launch_pcg_direction(st, g.dev(), g.z_ptr(), g.flexible());
+            launch_pcg_direction(st, g.dev(), g.flexible());
             desc[(size_t)k] = g.batch_instance();
             if (g.precond == FS_PRECOND_MULTIGRID)
                 lds = std::max(lds, g.tail_lds);

@@ -8,6 +8,7 @@ namespace fsim {
 struct GridDev {
     int W, H, s;              // cells, padded stride (W + 2)
     double h;                 // cell size
+    double dt;                // projection: time step
     int nl, ng;               // liquid / gas component counts
     double* fraction;         // N   (reference layout)
     double* u;                // (W+1) * H
@@ -29,6 +30,7 @@ struct GridDev {
     float* d2;                // padded FP32 direction of the odd iterations
     float* q;                 // padded FP32 A d
     float* zdiag;             // padded FP32 diagonal-preconditioned residual
+    const float* z;           // padded FP32 preconditioned residual (level 0's solution, or zdiag)
     PcgScalars* S;            // device scalar block
     double* partials;         // reduction partials (up to five per block)
     double* partials_ad;      // d.q partials of the operator kernel (one per block)
@@ -114,12 +116,8 @@ void launch_merge_failure(hipStream_t st, const PcgScalars* from, PcgScalars* S)
 
 // ---- fields, coefficients, hierarchy (FP64) ----
 void launch_density(hipStream_t st, const GridDev& g);
-void launch_face_weights(hipStream_t st, const GridDev& g);
-void launch_level_diag(hipStream_t st, int w, int h, const double* right64, const double* down64,
-    float* right32, float* down32, float* invd32);
-void launch_coarsen(hipStream_t st, int fw, int fh, const double* fcx, const double* fcy,
-    const double* fright, const double* fdown, int cw, int ch, const double* ccx, const double* ccy,
-    double* cright, double* cdown);
+// Density, face weights and the finest level's FP32 copies and 1/diagonal.
+void launch_coefficients(hipStream_t st, const GridDev& g);
 // Bit-exact Cholesky of the pinned coarse matrix (factorCoarsest), plus its FP32 inverse when ginv is set.
 // pin != 0 (grids with a solid mask): a vanishing pivot pins its unknown at zero instead of failing.
 void launch_coarse_factor(hipStream_t st, int w, int h, const double* right64, const double* down64,
@@ -128,7 +126,7 @@ void launch_coarse_factor(hipStream_t st, int w, int h, const double* right64, c
 void launch_coarse_inverse(hipStream_t st, int w, int h, const double* right64, const double* down64, float* ginv,
     int n, PcgScalars* S, int pin);
 // The coarse end of the hierarchy rebuild in one single-workgroup launch: for each listed level, the
-// coarsening from its finer level and its diagonal (the values of launch_coarsen + launch_level_diag),
+// coarsening from its finer level and its diagonal (the values of launch_coarsen),
 // then the inverse of the last level's pinned matrix (the values of launch_coarse_inverse).
 struct ChainLevel {
     int fw, fh, cw, ch;
@@ -141,24 +139,23 @@ struct ChainDesc {
     int levels;
     ChainLevel lev[kMaxTailLevels];
 };
+// One level coarsened from its finer one, with its FP32 copies and 1/diagonal.
+void launch_coarsen(hipStream_t st, const ChainLevel& level);
 void launch_coarse_chain(hipStream_t st, const ChainDesc& chain, float* ginv, int n, PcgScalars* S, int pin);
 
 // ---- projection set-up and finish (FP64) ----
-void launch_rhs(hipStream_t st, const GridDev& g, double scale);
-void launch_rhs_center(hipStream_t st, const GridDev& g);
-void launch_zero_pressure(hipStream_t st, const GridDev& g);
-void launch_predict(hipStream_t st, const GridDev& g);
-void launch_sub_mean_p(hipStream_t st, const GridDev& g, int only_if_loop);
-void launch_true_residual(hipStream_t st, const GridDev& g);   // of the predicted pressure
-void launch_final_flush_sum(hipStream_t st, const GridDev& g);
-void launch_correct_velocity(hipStream_t st, const GridDev& g, double dt);
-// when_stopped: measure only once the grid's solve has stopped (otherwise a no-op).
-void launch_max_divergence(hipStream_t st, const GridDev& g, bool when_stopped = false);
+// Wall faces zeroed, rhs = -div h^2 / dt; then its mean removed and the pressure predicted; then the residual of the
+// prediction.  The prediction's mean stays in p (S->p_shift) until the first direction folds it.
+void launch_project_setup(hipStream_t st, const GridDev& g);
+// Once the solve has stopped (a no-op before): the velocity correction, the pressure with the correction folded in and
+// its mean removed, and the largest divergence.
+void launch_project_end(hipStream_t st, const GridDev& g);
+void launch_max_divergence(hipStream_t st, const GridDev& g);
 void launch_gravity(hipStream_t st, const GridDev& g, double gy, double dt);
 void launch_add_vortex(hipStream_t st, const GridDev& g, double ox, double oy, double cx, double cy, double radius,
     double strength);
 void launch_semi_lagrangian(hipStream_t st, const GridDev& g, double ox, double oy, double dt, double* new_u,
-    double* new_v, double* scratch_cells);
+    double* new_v, double* new_fraction, double* new_lmass, double* new_gmass);
 // Up to eight FP64 device-to-device copies in one launch.
 struct CopyList {
     struct Item {
@@ -197,15 +194,15 @@ void launch_commit_edits(hipStream_t st, const GridDev& g, const EditCell* cells
 int pcg_groups(int W, int H);
 int pcg_blocks(int W, int H);
 // The next direction from z and the r.z partials, and the operator on it with d.q.
-void launch_pcg_direction_ad(hipStream_t st, const GridDev& g, const float* z, int flexible = 0);
+void launch_pcg_direction_ad(hipStream_t st, const GridDev& g, int flexible = 0);
 void launch_pcg_update(hipStream_t st, const GridDev& g);
 // The true residual where the update's residual norm calls for it, and the iteration's bookkeeping.
 void launch_pcg_check(hipStream_t st, const GridDev& g);
 // flexible: Polak-Ribiere beta from z.q (for a V-cycle with bfloat16 vectors, not exactly linear); the
 // two kernels of one iteration must agree on it (it changes the partials' layout).
-void launch_pcg_rz(hipStream_t st, const GridDev& g, const float* z, int flexible = 0);
-// The direction alone, into d (the first one of a batched solve).
-void launch_pcg_direction(hipStream_t st, const GridDev& g, const float* z, int flexible = 0);
+void launch_pcg_rz(hipStream_t st, const GridDev& g, int flexible = 0);
+// The direction alone, into d, the pressure folded (the first one of a batched solve).
+void launch_pcg_direction(hipStream_t st, const GridDev& g, int flexible = 0);
 void launch_precond_diag(hipStream_t st, const GridDev& g);
 
 // ---- multigrid V-cycle pieces (FP32) ----

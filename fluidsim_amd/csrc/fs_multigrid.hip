@@ -323,6 +323,7 @@ __device__ void coarse_inverse(int w, int h, const double* right, const double* 
     PcgScalars* S, int pin)
 {
     __shared__ double rowbuf[2][64];
+    __shared__ double pivot[2];
     __shared__ double assembled[64];   // diagonal before elimination (pinning bound)
     const int s = w + 2;
     const int lane = threadIdx.x & 63;
@@ -360,10 +361,17 @@ __device__ void coarse_inverse(int w, int h, const double* right, const double* 
             if (k >= n || failed)
                 break;
             double* row = rowbuf[k & 1];
-            if (wv == kb)
-                row[lane] = a[r0];
+            if (wv == kb) {
+                // the row's wavefront alone divides and publishes the scaled row; lane k's own entry becomes 1 / d
+                const double d = lane_value(a[r0], k);
+                const double inv_d = 1.0 / d;
+                row[lane] = lane == k ? inv_d : a[r0] * inv_d;
+                if (lane == k)
+                    pivot[k & 1] = d;
+            }
             __syncthreads();   // also orders the assembled[] writes before the first read
-            const double d = row[k];
+            const double t = row[lane];
+            const double d = pivot[k & 1];
             if (pin && isfinite(d) && fabs(d) <= kPinRatio * assembled[k]) {
                 pinned |= 1ull << k;
                 continue;
@@ -372,8 +380,6 @@ __device__ void coarse_inverse(int w, int h, const double* right, const double* 
                 failed = true;   // d is the same in every thread: the whole block leaves together
                 break;
             }
-            const double inv_d = 1.0 / d;
-            const double t = lane == k ? inv_d : row[lane] * inv_d;
 #pragma unroll
             for (int r = 0; r < kSweepRows; ++r) {
                 const int i = wv * kSweepRows + r;
@@ -416,8 +422,10 @@ __global__ __launch_bounds__(64 * kSweepWaves) void k_coarse_chain(const ChainDe
         const int cells = L.cw * L.ch;
         for (int t = threadIdx.x; t < cells; t += 64 * kSweepWaves) {
             const int y = t / L.cw, x = t - y * L.cw;
-            coarsen_cell(x, y, L.fw, L.fh, L.fcx, L.fcy, L.fright, L.fdown, L.cw, L.ch, L.ccx, L.ccy, L.cright,
-                L.cdown);
+            const double2 c = coarsen_cell(x, y, L.fw, L.fh, L.fcx, L.fcy, L.fright, L.fdown, L.cw, L.ch, L.ccx, L.ccy);
+            const int i = (y + 1) * (L.cw + 2) + x + 1;
+            L.cright[i] = c.x;
+            L.cdown[i] = c.y;
         }
         __syncthreads();
         const int s = L.cw + 2;
@@ -1067,6 +1075,8 @@ __global__ __launch_bounds__(kBT) void k_batch_pcg(const BatchInstance* batch)
         S = *g.S;
         S.rz = S.rz_slot[S.iterations & 1];   // r.z of the first direction (written by its kernel)
         S.restart = 0;                         // consumed by that direction
+        S.flush = 0;
+        S.p_shift = 0.0;
     }
     __syncthreads();
     const float* z = I.multigrid ? (I.levels > 0 ? I.lev[0].L.sol[0] : (const float*)I.tail->top_sol) : g.zdiag;
