@@ -261,7 +261,7 @@ def serving_leg(count, rates, steps, lanes, seed=5, max_size=2048, repeats=3, ba
     (which large grids step side by side depends on arrival and thread timing), so the serial pass and each
     rate run `repeats` times and the median run is reported, with every run's rate listed.  With
     `compare_batch_cells`, one more run at the last rate batches the requests of at most that many cells
-    (fs_batch_step: one workgroup per instance in the persistent solves).  `smoother` (kind, sweeps, coarse
+    (fs_batch_step).  `smoother` (kind, sweeps, coarse
     sweeps) is the pressure smoother of the served FP32-level requests (one more run at the last rate then
     serves them with the reference's cycle and bfloat16 conductances); the serial pass keeps the
     reference's V(4,4) cycle.  `precision` (an fs_mg_precision) overrides the served requests' multigrid storage.
@@ -568,11 +568,11 @@ def batch_leg(count, seed=4, splits=(0,)):
     drop, vortex velocity, obstacles over 0-25% of the cells), each projected once to 1e-6 of its own initial
     max divergence.  Timed twice
     from the same device-resident inputs: one fs_project per grid in turn (the plain GPU MGPCG), then one
-    fs_batch_project over all of them (one persistent launch for all PCG iterations).  Each instance's
+    fs_batch_project over all of them (each phase one launch over all their tiles).  Each instance's
     implicit viscosity solve (nu log-uniform 1e-3..1) is timed the same two ways: fs_apply_viscosity one
     grid after another, then fs_batch_apply_viscosity over all of them.  `splits` are the
-    fs_context_set_batch_split values timed for the projections (instances above the split run the
-    multi-kernel solve beside the persistent launch); the first one is the headline batched number."""
+    fs_context_set_batch_split values timed (viscous instances above the split run the multi-kernel solve beside
+    the persistent launch; the projections have no split); the first one is the headline batched number."""
     from fluidsim_amd import (FluidGridHIP, FluidMixture, MixtureComponent, batch_apply_viscosity, batch_project,
                               tune_batch_smoother, FS_TRANSPORT_NONE)
     from fluidsim_amd import workloads as WL

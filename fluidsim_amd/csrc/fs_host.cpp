@@ -382,7 +382,9 @@ struct fs_context {
     PcgScalars* pinned = nullptr;   // host-pinned mirror of a grid's scalar block
     double* pinned_value = nullptr; // host-pinned landing slot of single device reductions
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
-    DevBuf<BatchInstance> batch_desc;       // descriptors of the last batched solve
+    DevBuf<BatchItem> batch_desc;           // descriptors of the last batched projection
+    DevBuf<int> batch_maps;                 // its workgroup maps and lists
+    DevBuf<PcgScalars> batch_scalars;       // its scalar blocks, gathered
     DevBuf<unsigned char> vis_batch_desc;   // descriptors of the last batched viscosity solve
     PcgScalars* batch_pinned = nullptr;     // host-pinned landing slots of a batch's scalar blocks
     size_t batch_pinned_n = 0;
@@ -426,7 +428,7 @@ PreChoice pre_choice(bool chebyshev, int id)
 }
 constexpr size_t kBatchSpreadLds = 84 * 1024;   // LDS of a batched-solve workgroup: one per compute unit
 
-// A batched solve split by fs_context_set_batch_split: grids above the split take their single-grid solve
+// A batched viscosity step split by fs_context_set_batch_split: grids above the split take their single-grid solve
 // on the context's stream while the persistent launch runs on a stream of its own.
 bool batch_solo(const fs_context* ctx, int W, int H)
 {
@@ -940,6 +942,24 @@ struct fs_grid {
         mg_valid = false;
     }
 
+    // First level built by the chain launch of a hierarchy rebuild (the number of levels: none).
+    size_t chain_from() const
+    {
+        const size_t nlev = levels.size();
+        size_t from = nlev;
+        while (from > 1 && nlev - (from - 1) <= (size_t)kMaxTailLevels &&
+               (long long)levels[from - 1].w * levels[from - 1].h <= kChainCells)
+            --from;
+        return from;
+    }
+    ChainDesc chain_desc(size_t from)
+    {
+        ChainDesc chain{};
+        for (size_t l = from; l < levels.size(); ++l)
+            chain.lev[chain.levels++] = chain_level(l);
+        return chain;
+    }
+
     // Level l as the hierarchy rebuild sees it.
     ChainLevel chain_level(size_t l)
     {
@@ -960,10 +980,7 @@ struct fs_grid {
     bool rebuild_hierarchy(hipStream_t stream, PcgScalars* flag, hipEvent_t levels_done = nullptr)
     {
         const size_t nlev = levels.size();
-        size_t chain_from = nlev;   // first level built by the chain launch
-        while (chain_from > 1 && nlev - (chain_from - 1) <= (size_t)kMaxTailLevels &&
-               (long long)levels[chain_from - 1].w * levels[chain_from - 1].h <= kChainCells)
-            --chain_from;
+        const size_t chain_from = this->chain_from();
         for (size_t l = 0; l + 1 < chain_from; ++l) {
             launch_coarsen(stream, chain_level(l + 1));
         }
@@ -975,11 +992,7 @@ struct fs_grid {
             HIPC(hipEventRecord(levels_done, stream));
         }
         if (chain_from < nlev) {
-            ChainDesc chain{};
-            for (size_t l = chain_from; l < nlev; ++l) {
-                chain.lev[chain.levels++] = chain_level(l);
-            }
-            launch_coarse_chain(stream, chain, ginv.p, coarse_n, flag, solid.n > 0);
+            launch_coarse_chain(stream, chain_desc(chain_from), ginv.p, coarse_n, flag, solid.n > 0);
         } else {
             launch_coarse_inverse(stream, last.w, last.h, last.right64.p, last.down64.p, ginv.p, coarse_n, flag,
                 solid.n > 0);
@@ -1453,16 +1466,31 @@ struct fs_grid {
         return project_result(s, tol, dt);
     }
 
-    // This grid's entry of a batched solve (the iteration body of iteration_kernels()).
-    BatchInstance batch_instance()
+    // Whether this grid's projection can be part of a batched one: decided by its shape and settings alone.
+    bool batchable() const
     {
-        if (tail_start > kMaxBatchLevels)
-            fail(FS_E_UNSUPPORTED, "grid has more multigrid levels than a batched solve supports");
-        BatchInstance b{};
+        return batch_cell_blocks(W, H) <= kBatchTiles && tail_start <= kMaxBatchLevels && levels.size() >= 2 &&
+               (int)chain_from() <= kMaxBatchLevels + 2 && !flexible();
+    }
+
+    // This grid's entry of a batched projection.
+    BatchItem batch_item(double dt, int budget, double tol)
+    {
+        BatchItem b{};
         b.g = dev();
-        b.multigrid = precond == FS_PRECOND_MULTIGRID;
+        b.g.dt = dt;
+        b.tol = relative_tol ? 0.0 : tol * (h * h / dt);
+        b.rel_tol = relative_tol ? tol : 0.0;
+        b.max_iterations = budget;
+        b.pin = solid.n > 0;
+        b.coarse_n = coarse_n;
+        b.ginv = ginv.p;
         b.levels = tail_start;
-        b.tail = tail_dev.p;
+        const size_t from = chain_from();
+        for (size_t l = 1; l < from; ++l)
+            b.coarsen[l - 1] = chain_level(l);
+        b.chain = chain_desc(from);
+        b.tail = tail;
         for (int l = 0; l < tail_start; ++l) {
             const Level& F = levels[l];
             const Level& Cl = levels[l + 1];
@@ -1515,6 +1543,50 @@ void need(bool cond, fs_status code, const char* message)
 }
 
 void set_device(fs_context* ctx) { HIPC(hipSetDevice(ctx->device)); }
+
+// Workgroup maps and item lists of the batched launches, built on the host and uploaded together.
+struct BatchMaps {
+    struct Part {
+        size_t item = 0, first = 0;
+        int blocks = 0;
+    };
+    struct List {
+        size_t at = 0;
+        int n = 0;
+    };
+    std::vector<int> words;
+    const int* base = nullptr;   // the uploaded words
+    int items = 0;
+
+    // The items among `of` that `blocks` gives workgroups.
+    template <class F> Part part(const std::vector<int>& of, F&& blocks)
+    {
+        Part p;
+        p.first = words.size();
+        words.resize(words.size() + (size_t)items, 0);
+        p.item = words.size();
+        for (int i : of) {
+            const int n = blocks(i);
+            words[p.first + (size_t)i] = p.blocks;
+            words.insert(words.end(), (size_t)n, i);
+            p.blocks += n;
+        }
+        return p;
+    }
+    template <class F> List list(const std::vector<int>& of, F&& take)
+    {
+        List l;
+        l.at = words.size();
+        for (int i : of)
+            if (take(i)) {
+                words.push_back(i);
+                ++l.n;
+            }
+        return l;
+    }
+    BatchPart operator()(const Part& p) const { return BatchPart{base + p.item, base + p.first, p.blocks}; }
+    const int* operator()(const List& l) const { return base + l.at; }
+};
 
 // ---- resident-instance checkpoint (FluidGridGPU.cpp:566-695 save, 697-880 load) ----
 //
@@ -3323,7 +3395,8 @@ fs_status fs_time_kernel(fs_grid* grid, int kernel, int reps, double* ms_per_lau
             case 0:  // the finest post-smoothing launch of a V-cycle (prolongation + four sweeps)
                 g.fine_post_smooth(i & 1);
                 break;
-            case 1: launch_pcg_direction_ad(g.st(), gd); break;
+            case 1:
+            case 8: launch_pcg_direction_ad(g.st(), gd); break;
             case 2: launch_pcg_update(g.st(), gd); break;
             case 3: launch_copy_f32(g.st(), g.r.p, g.q.p, g.NP()); break;
             case 4:  // second level's smoother (or the finest, if the tail starts at level 1)
@@ -3347,7 +3420,6 @@ fs_status fs_time_kernel(fs_grid* grid, int kernel, int reps, double* ms_per_lau
                     nullptr, g.solid.n > 0);
                 break;
             }
-            case 8: launch_pcg_direction(g.st(), gd); break;
             default: launch_pcg_rz(g.st(), gd); break;
             }
         };
@@ -3371,84 +3443,179 @@ fs_status fs_grid_device_bytes(const fs_grid* grid, size_t* bytes)
     });
 }
 
-// The batched projection of the grids listed in `which`, each with its own dt, budget and tolerance: their
-// set-up on the context's stream, one persistent launch for those at or under the context's split (the others
-// run fs_project's multi-kernel solve beside it), then every velocity correction.  A solo grid's failure
-// lands in errors[i].  Returns with the context's stream drained.
+// The batched projection of the grids listed in `which`, each with its own dt, budget and tolerance.  Every phase of a
+// projection is one launch over the tiles (or one workgroup per item) of all of them, so an iteration of the batch
+// costs about what an iteration of one grid of their total size costs, and every value is the single-grid solve's
+// bit for bit, alone or in any batch.  Grids too large to gain from company (more than kBatchTiles tiles), a grid on its
+// own and the flexible CG take the single-grid solve.  A solo grid's failure lands in errors[i].  Returns with
+// the context's stream drained.
 static void batch_projection(fs_context* ctx, fs_grid* const* grids, const std::vector<int>& which, const double* dts,
     const int* max_iterations, const double* tolerances, fs_projection_result* results, std::vector<std::string>& errors)
 {
     hipStream_t st = ctx->stream;
     const SyncOnExit drain{st};   // the staged descriptors and host results stay valid until then
-    // Instances above the split run fs_project's multi-kernel solve on the context's stream while the
-    // persistent launch runs the others on a stream of its own; the route depends on the instance's
-    // size only, so each result is the same alone and in any batch.
     std::vector<int> batched, solo;
     for (int i : which)
         if (dts[i] > 0.0)
-            (batch_solo(ctx, grids[i]->W, grids[i]->H) ? solo : batched).push_back(i);
-    const int nb = (int)batched.size();
-    const bool split = nb > 0 && !solo.empty();
-    if (nb > 0) {
-        std::vector<BatchInstance> desc((size_t)nb);
+            (grids[i]->batchable() ? batched : solo).push_back(i);
+    if (batched.size() == 1) {
+        solo.push_back(batched[0]);
+        batched.clear();
+    }
+    const int n = (int)batched.size();
+    if (n > 0) {
+        std::vector<fs_grid*> g((size_t)n);
+        std::vector<BatchItem> desc((size_t)n);
+        std::vector<int> all((size_t)n), depth((size_t)n);
+        std::vector<char> coefficients((size_t)n), hierarchy((size_t)n), multigrid((size_t)n);
+        int levels = 0, built = 0, predicted = 1;
         size_t lds = 0;
-        for (int k = 0; k < nb; ++k) {
+        for (int k = 0; k < n; ++k) {
             const int i = batched[(size_t)k];
-            fs_grid& g = *grids[i];
-            g.project_begin(dts[i], fs_grid::budget(max_iterations[i]), tolerances[i]);
-            launch_pcg_direction(st, g.dev(), g.flexible());
-            desc[(size_t)k] = g.batch_instance();
-            if (g.precond == FS_PRECOND_MULTIGRID)
-                lds = std::max(lds, g.tail_lds);
+            g[(size_t)k] = grids[i];
+            fs_grid& G = *grids[i];
+            desc[(size_t)k] = G.batch_item(dts[i], fs_grid::budget(max_iterations[i]), tolerances[i]);
+            all[(size_t)k] = k;
+            multigrid[(size_t)k] = G.precond == FS_PRECOND_MULTIGRID;
+            coefficients[(size_t)k] = !G.coeff_valid;
+            hierarchy[(size_t)k] = multigrid[(size_t)k] && (!G.coeff_valid || !G.mg_valid);
+            if (multigrid[(size_t)k]) {
+                levels = std::max(levels, G.tail_start);
+                if (!G.tail.batch_rows)
+                    lds = std::max(lds, G.tail_lds);
+            }
+            if (hierarchy[(size_t)k])
+                built = std::max(built, (int)G.chain_from() - 1);
+            predicted = std::max(predicted, G.predicted);
         }
-        if (ctx->batch_desc.n < (size_t)nb)
-            ctx->batch_desc.alloc((size_t)nb);
-        // the descriptors go through pinned staging: `desc` dies at the end of this block, before the
-        // stream is synchronised
-        stage_upload(ctx, ctx->batch_desc.p, desc.data(), desc.size() * sizeof(BatchInstance));
-        // One workgroup is one instance's whole solve: while the instances fit on the compute units one
-        // each, reserve more than half a unit's 160 KB of LDS so that no two of them share a unit.
-        if (nb <= ctx->compute_units && ctx->lds_per_block >= kBatchSpreadLds)
-            lds = std::max(lds, kBatchSpreadLds);
         if (lds > 65536)
             need(batch_allow_lds(lds), FS_E_DEVICE, "the device refused the batched solve's LDS request");
-        const hipStream_t bs = split ? batch_side_stream(ctx) : st;
-        launch_batch_pcg(bs, ctx->batch_desc.p, nb, lds);
-        HIPC(hipGetLastError());
-        if (split)
-            HIPC(hipEventRecord(ctx->batch_out, bs));
-    }
-    // the solo instances; a failure is kept for its grid while the batched instances are finished
-    for (int i : solo) {
-        try {
-            results[i] = grids[i]->project(dts[i], max_iterations[i], tolerances[i]);
-        } catch (const std::exception& e) {
-            errors[(size_t)i] = e.what();
-        }
-    }
-    if (nb > 0) {
-        if (split)
-            HIPC(hipStreamWaitEvent(st, ctx->batch_out, 0));
-        for (int i : batched)
-            grids[i]->project_end(dts[i]);
-        if (ctx->batch_pinned_n < (size_t)nb) {
+        if (ctx->batch_desc.n < (size_t)n)
+            ctx->batch_desc.alloc((size_t)n);
+        if (ctx->batch_scalars.n < (size_t)n)
+            ctx->batch_scalars.alloc((size_t)n);
+        if (ctx->batch_pinned_n < (size_t)n) {
             std::lock_guard<std::mutex> lock(device_setup_mutex());
             if (ctx->batch_pinned)
                 (void)hipHostFree(ctx->batch_pinned);
             ctx->batch_pinned = nullptr;
             ctx->batch_pinned_n = 0;
-            HIPC(hipHostMalloc((void**)&ctx->batch_pinned, (size_t)nb * sizeof(PcgScalars), hipHostMallocDefault));
-            ctx->batch_pinned_n = (size_t)nb;
+            HIPC(hipHostMalloc((void**)&ctx->batch_pinned, (size_t)n * sizeof(PcgScalars), hipHostMallocDefault));
+            ctx->batch_pinned_n = (size_t)n;
         }
-        for (int k = 0; k < nb; ++k)
-            HIPC(hipMemcpyAsync(ctx->batch_pinned + k, grids[batched[(size_t)k]]->S.p, sizeof(PcgScalars),
-                hipMemcpyDeviceToHost, st));
+        // the descriptors go through pinned staging, as the maps do: the vectors may die before the copy runs
+        stage_upload(ctx, ctx->batch_desc.p, desc.data(), desc.size() * sizeof(BatchItem));
         HIPC(hipStreamSynchronize(st));
-        for (int k = 0; k < nb; ++k) {
+        const BatchItem* items = ctx->batch_desc.p;
+
+        // The maps of an iteration over the items of `run`.
+        struct Loop {
+            BatchMaps::Part cells, diagonal;
+            BatchMaps::List every, held, other;
+            std::vector<BatchMaps::Part> down, up;
+        } loop;
+        BatchMaps maps;
+        auto plan = [&](const std::vector<int>& run) {
+            const auto cells = [&](int k) { return batch_cell_blocks(g[(size_t)k]->W, g[(size_t)k]->H); };
+            maps = BatchMaps{};
+            maps.items = n;
+            loop.cells = maps.part(run, cells);
+            loop.diagonal = maps.part(run, [&](int k) { return multigrid[(size_t)k] ? 0 : cells(k); });
+            loop.every = maps.list(run, [](int) { return true; });
+            loop.held = maps.list(run, [&](int k) { return multigrid[(size_t)k] && desc[(size_t)k].tail.batch_rows > 0; });
+            loop.other = maps.list(run, [&](int k) { return multigrid[(size_t)k] && desc[(size_t)k].tail.batch_rows == 0; });
+            loop.down.clear();
+            loop.up.clear();
+            for (int l = 0; l < levels; ++l)
+                for (const bool post : {false, true})
+                    (post ? loop.up : loop.down).push_back(maps.part(run, [&](int k) {
+                        const BatchItem& I = desc[(size_t)k];
+                        return multigrid[(size_t)k] && l < I.levels ? batch_level_blocks(I.lev[l], post) : 0;
+                    }));
+        };
+        auto upload = [&] {
+            if (ctx->batch_maps.n < maps.words.size())
+                ctx->batch_maps.alloc(maps.words.size());
+            stage_upload(ctx, ctx->batch_maps.p, maps.words.data(), maps.words.size() * sizeof(int));
+            maps.base = ctx->batch_maps.p;
+        };
+        auto vcycle = [&] {
+            launch_batch_precond_diag(st, items, maps(loop.diagonal));
+            for (int l = 0; l < levels; ++l)
+                launch_batch_smooth(st, items, maps(loop.down[(size_t)l]), l, false);
+            launch_batch_tail(st, items, maps(loop.held), loop.held.n);
+            launch_batch_lds_tail(st, items, maps(loop.other), loop.other.n, lds);
+            for (int l = levels - 1; l >= 0; --l)
+                launch_batch_smooth(st, items, maps(loop.up[(size_t)l]), l, true);
+            launch_batch_rz(st, items, maps(loop.cells));
+        };
+        auto read = [&](const BatchMaps::List& of) {
+            launch_batch_scalars(st, items, maps(of), of.n, ctx->batch_scalars.p);
+            HIPC(hipMemcpyAsync(ctx->batch_pinned, ctx->batch_scalars.p, (size_t)of.n * sizeof(PcgScalars),
+                hipMemcpyDeviceToHost, st));
+            HIPC(hipStreamSynchronize(st));
+        };
+
+        // set-up: coefficients and hierarchies where they are stale, rhs, predicted pressure, residual, first V-cycle
+        std::vector<int> run = all;
+        plan(run);
+        const BatchMaps::Part stale = maps.part(all, [&](int k) {
+            return coefficients[(size_t)k] ? batch_cell_blocks(g[(size_t)k]->W, g[(size_t)k]->H) : 0;
+        });
+        std::vector<BatchMaps::Part> coarsen;
+        for (int l = 0; l < built; ++l)
+            coarsen.push_back(maps.part(all, [&](int k) {
+                return hierarchy[(size_t)k] && l < (int)g[(size_t)k]->chain_from() - 1
+                           ? batch_coarsen_blocks(desc[(size_t)k].coarsen[l]) : 0;
+            }));
+        const BatchMaps::List chains = maps.list(all, [&](int k) { return hierarchy[(size_t)k] != 0; });
+        upload();
+        launch_batch_init(st, items, maps(loop.every), loop.every.n);
+        launch_batch_coefficients(st, items, maps(stale));
+        for (int l = 0; l < built; ++l)
+            launch_batch_coarsen(st, items, maps(coarsen[(size_t)l]), l);
+        launch_batch_chain(st, items, maps(chains), chains.n);
+        for (int k = 0; k < n; ++k) {
+            g[(size_t)k]->mg_valid = multigrid[(size_t)k] || (g[(size_t)k]->mg_valid && !coefficients[(size_t)k]);
+            g[(size_t)k]->coeff_valid = true;
+        }
+        launch_batch_setup(st, items, maps(loop.cells), maps(loop.every), loop.every.n);
+        vcycle();
+        HIPC(hipGetLastError());
+
+        // iterations, as many as the longest of the previous solves first, with the stopped items dropped in between
+        for (int chunk = std::min(predicted, 64); !run.empty(); chunk = 8) {
+            for (int c = 0; c < chunk; ++c) {
+                launch_batch_step(st, items, maps(loop.cells), maps(loop.every), loop.every.n);
+                vcycle();
+            }
+            HIPC(hipGetLastError());
+            read(loop.every);
+            std::vector<int> left;
+            for (size_t k = 0; k < run.size(); ++k)
+                if (ctx->batch_pinned[k].status == kRunning)
+                    left.push_back(run[k]);
+            if (left.size() != run.size()) {
+                run.swap(left);
+                plan(run.empty() ? all : run);
+                upload();
+            }
+        }
+        launch_batch_end(st, items, maps(loop.cells), maps(loop.every), loop.every.n);
+        HIPC(hipGetLastError());
+        read(loop.every);
+        for (int k = 0; k < n; ++k) {
             const int i = batched[(size_t)k];
             const PcgScalars sc = ctx->batch_pinned[k];
             results[i] = grids[i]->project_result(sc, tolerances[i], dts[i]);
             grids[i]->predicted = sc.iterations;
+        }
+    }
+    for (int i : solo) {
+        try {
+            results[i] = grids[i]->project(dts[i], max_iterations[i], tolerances[i]);
+        } catch (const std::exception& e) {
+            errors[(size_t)i] = e.what();
         }
     }
 }

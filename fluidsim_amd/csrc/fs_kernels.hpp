@@ -97,6 +97,7 @@ struct TailDesc {
     // and coarse neighbours (four bits per fine cell: 1 first = own, 2 second = own, 4 second = next, else
     // previous), and the restriction's weights of fine cells 2 c - 1 .. 2 c + 2.
     int held_rows;
+    int batch_rows;            // the same for the batched launch's smaller workgroup
     int pair_table_n;
     const float4* pair_tables;
     TailLevel lev[kMaxTailLevels];
@@ -107,7 +108,7 @@ size_t tail_layout(TailDesc& t);
 // Raises the dynamic-LDS limit of the tail kernel; false if the device refuses.
 bool tail_allow_lds(size_t bytes);
 
-// Sets held_rows and the levels' lanes and table offsets.
+// Sets held_rows, batch_rows and the levels' lanes and table offsets.
 void tail_hold(TailDesc& t);
 // rel_tol > 0 replaces tol by rel_tol * max|b| once the rhs b is formed (a relative residual).
 void launch_init_scalars(hipStream_t st, PcgScalars* S, double tol, int max_iterations, double rel_tol = 0.0);
@@ -201,8 +202,6 @@ void launch_pcg_check(hipStream_t st, const GridDev& g);
 // flexible: Polak-Ribiere beta from z.q (for a V-cycle with bfloat16 vectors, not exactly linear); the
 // two kernels of one iteration must agree on it (it changes the partials' layout).
 void launch_pcg_rz(hipStream_t st, const GridDev& g, int flexible = 0);
-// The direction alone, into d, the pressure folded (the first one of a batched solve).
-void launch_pcg_direction(hipStream_t st, const GridDev& g, int flexible = 0);
 void launch_precond_diag(hipStream_t st, const GridDev& g);
 
 // ---- multigrid V-cycle pieces (FP32) ----
@@ -252,8 +251,9 @@ template <class C> void launch_level_pack(hipStream_t st, int w, int h, const do
 // The smoothers and the residual restriction are instantiated for (C, V, VC) = (float, float, float),
 // (half16, float, float), (bf16, float, float), (bf16, float, bf16) and (bf16, bf16, bf16).
 
-// ---- batched PCG: one 1024-thread workgroup runs the whole iteration loop of one instance ----
-constexpr int kMaxBatchLevels = 16;   // tiled levels above an instance's tail
+// ---- batched projections: every phase of many grids' projections in one launch over all their tiles ----
+constexpr int kMaxBatchLevels = 8;   // tiled levels above an instance's tail
+constexpr int kBatchTiles = 1024;    // 64 x 16 tiles of the largest grid that is batched (pcg_groups(W, H) == 1)
 struct BatchLevel {
     LevelView L;        // tiled level l (rhs: r on level 0)
     LevelView C;        // level l + 1 (its rhs receives the restriction, its sol[0] the coarse correction)
@@ -261,17 +261,47 @@ struct BatchLevel {
     CoarseLink link;    // prolongation l + 1 -> l
     int sweeps;         // red-black sweeps per side on this level (1..4)
 };
-struct BatchInstance {
+struct BatchItem {
     GridDev g;
-    int multigrid;      // 0: diagonal preconditioner
-    int levels;         // tiled levels (the tail starts at this level)
-    const TailDesc* tail;   // device copy of the instance's tail descriptor
+    double tol, rel_tol;    // launch_init_scalars' arguments
+    int max_iterations;
+    int levels;             // tiled levels (the tail starts at this level)
+    int pin;                // launch_coarse_chain's arguments
+    int coarse_n;
+    float* ginv;
+    ChainDesc chain;
+    ChainLevel coarsen[kMaxBatchLevels + 2];   // levels built before the chain
     BatchLevel lev[kMaxBatchLevels];
+    TailDesc tail;
 };
-// Runs every instance's PCG iterations (the captured iteration body, looped on the device until the
-// instance's scalar block leaves kRunning) in one launch of `count` workgroups.
-void launch_batch_pcg(hipStream_t st, const BatchInstance* batch, int count, size_t lds_bytes);
+// Workgroups of a launch over several items: workgroup b works on item[b], of which first[item[b]] is the first.
+struct BatchPart {
+    const int* item;
+    const int* first;
+    int blocks;
+};
+// Workgroups an item takes in the launches over cells, over the coarse cells of a built level, and over a tiled level.
+int batch_cell_blocks(int W, int H);
+int batch_coarsen_blocks(const ChainLevel& level);
+int batch_level_blocks(const BatchLevel& level, bool post);
+// The phases of fs_grid::project_begin, iteration_kernels and project_end on the items of a part, or on the n items of a
+// list (one workgroup each); the values of the single-grid launches bit for bit.
+void launch_batch_init(hipStream_t st, const BatchItem* items, const int* list, int n);
+void launch_batch_coefficients(hipStream_t st, const BatchItem* items, const BatchPart& part);
+void launch_batch_coarsen(hipStream_t st, const BatchItem* items, const BatchPart& part, int level);
+void launch_batch_chain(hipStream_t st, const BatchItem* items, const int* list, int n);
+void launch_batch_setup(hipStream_t st, const BatchItem* items, const BatchPart& part, const int* list, int n);
+void launch_batch_step(hipStream_t st, const BatchItem* items, const BatchPart& part, const int* list, int n);
+void launch_batch_precond_diag(hipStream_t st, const BatchItem* items, const BatchPart& part);
+void launch_batch_rz(hipStream_t st, const BatchItem* items, const BatchPart& part);
+void launch_batch_end(hipStream_t st, const BatchItem* items, const BatchPart& part, const int* list, int n);
+void launch_batch_smooth(hipStream_t st, const BatchItem* items, const BatchPart& part, int level, bool post);
+// The tails: items whose tail.batch_rows is set, and the others (levels in LDS).
+void launch_batch_tail(hipStream_t st, const BatchItem* items, const int* list, int n);
+void launch_batch_lds_tail(hipStream_t st, const BatchItem* items, const int* list, int n, size_t lds_bytes);
 bool batch_allow_lds(size_t bytes);
+// The items' scalar blocks into out[0 .. n).
+void launch_batch_scalars(hipStream_t st, const BatchItem* items, const int* list, int n, PcgScalars* out);
 
 // ---- reference PLIC/VOF transport (FP64, reference layouts, bit-exact) ----
 // One directional pass reads the frozen flow (u, v), the fractions and masses of the pass start and the

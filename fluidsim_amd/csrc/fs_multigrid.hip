@@ -414,8 +414,7 @@ __global__ __launch_bounds__(64 * kSweepWaves) void k_coarse_inverse(int w, int 
 // Coarse end of the hierarchy rebuild: each level's cells coarsened, then its diagonal and FP32 copies,
 // each phase workgroup-strided and closed by a barrier (which also makes this workgroup's global
 // writes visible to its next phase); then the coarse inverse.
-__global__ __launch_bounds__(64 * kSweepWaves) void k_coarse_chain(const ChainDesc C, float* ginv, int n,
-    PcgScalars* S, int pin)
+__device__ __forceinline__ void coarse_chain(const ChainDesc& C, float* ginv, int n, PcgScalars* S, int pin)
 {
     for (int l = 0; l < C.levels; ++l) {
         const ChainLevel& L = C.lev[l];
@@ -441,6 +440,12 @@ __global__ __launch_bounds__(64 * kSweepWaves) void k_coarse_chain(const ChainDe
         const ChainLevel& L = C.lev[C.levels - 1];
         coarse_inverse(L.cw, L.ch, L.cright, L.cdown, ginv, n, S, pin);
     }
+}
+
+__global__ __launch_bounds__(64 * kSweepWaves) void k_coarse_chain(const ChainDesc C, float* ginv, int n,
+    PcgScalars* S, int pin)
+{
+    coarse_chain(C, ginv, n, S, pin);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -866,434 +871,20 @@ __global__ __launch_bounds__(kTailThreads) void k_mg_tail(const TailDesc D, cons
     tail_run<TV>(D, shift, status, lds);
 }
 
-// ---------------------------------------------------------------------------------------------
-// Batched PCG: one 1024-thread workgroup per instance runs the instance's whole iteration loop (the
-// kernels of one captured PCG iteration become phases separated by workgroup barriers), so a batch of
-// small grids is one launch instead of a dozen launches per iteration per grid.  Vectors stay in the
-// instance's own HBM buffers; the scalar block is kept in LDS and written back at the end.  Every value
-// is computed with the expression of the corresponding single-instance kernel; only the FP64
-// reductions run in another order (thread-strided sums, then the 16 wavefronts in order).
-// ---------------------------------------------------------------------------------------------
-constexpr int kBT = kTailThreads;
-constexpr int kBU = 4;   // items per thread whose loads are issued together in the workgroup-strided loops
-
-// t / d in the workgroup-strided loops: the float-reciprocal quotient (tail_div) below 2^22 items, else
-// an integer division; `fast` is uniform across the workgroup.
-__device__ __forceinline__ int bdiv(int t, int d, float inv_d, bool fast) { return fast ? tail_div(t, inv_d) : t / d; }
-constexpr int kBW = kBT / 64;
-
-// Workgroup sum / max, valid in every thread.
-__device__ __forceinline__ double wg_sum(double v, double* slot)
-{
-    v = wave_sum(v);
-    if ((threadIdx.x & 63) == 0)
-        slot[threadIdx.x >> 6] = v;
-    __syncthreads();
-    double r = 0.0;
-#pragma unroll
-    for (int i = 0; i < kBW; ++i)
-        r += slot[i];
-    __syncthreads();
-    return r;
-}
-
-__device__ __forceinline__ double wg_max(double v, double* slot)
-{
-    v = wave_max(v);
-    if ((threadIdx.x & 63) == 0)
-        slot[threadIdx.x >> 6] = v;
-    __syncthreads();
-    double r = 0.0;
-#pragma unroll
-    for (int i = 0; i < kBW; ++i)
-        r = fmax(r, slot[i]);
-    __syncthreads();
-    return r;
-}
-
-// 2 * sweeps red-black half-sweeps of one level in place on `sol` (the level smoothers' update): colours from
-// `first`, alternating; the first half-sweep of a pre-smoothing ignores the (zero) neighbours.
-__device__ void wg_sweeps(const LevelView& L, float* sol, const float* rhs, const double* shift, int first,
-    bool from_zero, int sweeps)
-{
-    const int w = L.w, h = L.h, s = L.s;
-    const int pairs = (w + 1) >> 1;
-    const int items = pairs * h;
-    const double sh = shift ? *shift : 0.0;
-    const float inv_pairs = 1.0f / (float)pairs;
-    const bool fast = items < (1 << 22);
-    for (int k = 0; k < 2 * sweeps; ++k) {
-        const int color = first ^ (k & 1);
-        const bool neighbours = !(from_zero && k == 0);
-        // kBU items per thread at a time: every load of the group issues before the first store (the
-        // items of one colour never read each other), through clamped valid indices
-        for (int t0 = threadIdx.x; t0 < items; t0 += kBU * kBT) {
-            int idx[kBU];
-            bool on[kBU];
-            float a[kBU], b[kBU], u[kBU], d[kBU], rv[kBU], n0[kBU], n1[kBU], n2[kBU], n3[kBU];
-#pragma unroll
-            for (int q = 0; q < kBU; ++q) {
-                const int t = t0 + q * kBT;
-                const int tt = min(t, items - 1);
-                const int y = bdiv(tt, pairs, inv_pairs, fast);
-                const int x = 2 * (tt - y * pairs) + ((color + y) & 1);
-                on[q] = t < items && x < w;
-                const int i = (y + 1) * s + min(x, w - 1) + 1;
-                idx[q] = i;
-                a[q] = L.right[i - 1];
-                b[q] = L.right[i];
-                u[q] = L.down[i - s];
-                d[q] = L.down[i];
-                rv[q] = rhs[i];
-                n0[q] = sol[i - 1];
-                n1[q] = sol[i + 1];
-                n2[q] = sol[i - s];
-                n3[q] = sol[i + s];
-            }
-#pragma unroll
-            for (int q = 0; q < kBU; ++q) {
-                float v = shift ? (float)((double)rv[q] - sh) : rv[q];
-                if (neighbours)
-                    v += (a[q] * n0[q] + b[q] * n1[q]) + (u[q] * n2[q] + d[q] * n3[q]);
-                if (on[q])
-                    sol[idx[q]] = v * inv_or_zero((a[q] + b[q]) + (u[q] + d[q]));
-            }
-        }
-        __syncthreads();
-    }
-}
-
-// Residual of level F's sol[1] into F.res, then its transpose-of-bilinear restriction into C.rhs
-// (k_res_restrict's arithmetic; missing taps have weight 0 and index -1, the zero halo).
-__device__ void wg_res_restrict(const LevelView& F, const float* rhs, const double* shift, const LevelView& C,
-    const AxisRestrict& rx, const AxisRestrict& ry)
-{
-    const int w = F.w, h = F.h, s = F.s;
-    const float* sol = F.sol[1];
-    const double sh = shift ? *shift : 0.0;
-    const int cells = w * h;
-    const float inv_w = 1.0f / (float)w;
-    const bool fast = cells < (1 << 22);
-    for (int e0 = threadIdx.x; e0 < cells; e0 += kBU * kBT) {
-        int idx[kBU];
-        float val[kBU];
-#pragma unroll
-        for (int q = 0; q < kBU; ++q) {
-            const int e = min(e0 + q * kBT, cells - 1);
-            const int y = bdiv(e, w, inv_w, fast), x = e - y * w;
-            const int i = (y + 1) * s + x + 1;
-            idx[q] = i;
-            const float c = sol[i];
-            const float product = (F.right[i - 1] * (c - sol[i - 1]) + F.right[i] * (c - sol[i + 1])) +
-                                  (F.down[i - s] * (c - sol[i - s]) + F.down[i] * (c - sol[i + s]));
-            const float b = shift ? (float)((double)rhs[i] - sh) : rhs[i];
-            const bool active = (F.right[i - 1] + F.right[i]) + (F.down[i - s] + F.down[i]) > 0.f;
-            val[q] = active ? b - product : 0.f;   // cells without conductance are not restricted
-        }
-#pragma unroll
-        for (int q = 0; q < kBU; ++q)
-            if (e0 + q * kBT < cells)
-                F.res[idx[q]] = val[q];
-    }
-    __syncthreads();
-    const int ccells = C.w * C.h;
-    const float inv_cw = 1.0f / (float)C.w;
-    for (int e0 = threadIdx.x; e0 < ccells; e0 += kBU * kBT) {
-        int dst[kBU];
-        float val[kBU];
-#pragma unroll
-        for (int q = 0; q < kBU; ++q) {
-            const int e = min(e0 + q * kBT, ccells - 1);
-            const int y = bdiv(e, C.w, inv_cw, fast), x = e - y * C.w;
-            float value = 0.f;
-#pragma unroll
-            for (int iy = 0; iy < 4; ++iy) {
-                const float* row = F.res + (ry.index[y * 4 + iy] + 1) * s + 1;
-                float horizontal = 0.f;
-#pragma unroll
-                for (int ix = 0; ix < 4; ++ix)
-                    horizontal += rx.weight[x * 4 + ix] * row[rx.index[x * 4 + ix]];
-                value += ry.weight[y * 4 + iy] * horizontal;
-            }
-            val[q] = value;
-            dst[q] = (y + 1) * C.s + x + 1;
-        }
-#pragma unroll
-        for (int q = 0; q < kBU; ++q)
-            if (e0 + q * kBT < ccells)
-                C.rhs[dst[q]] = val[q];
-    }
-    __syncthreads();
-}
-
-// sol[0] = sol[1] + bilinear prolongation of the coarse correction (the post-smoothing's load).
-__device__ void wg_prolong(const LevelView& L, const CoarseLink& link)
-{
-    const int w = L.w, h = L.h, s = L.s;
-    const int cells = w * h;
-    const float inv_w = 1.0f / (float)w;
-    const bool fast = cells < (1 << 22);
-    for (int e0 = threadIdx.x; e0 < cells; e0 += kBU * kBT) {
-        int idx[kBU];
-        float val[kBU];
-#pragma unroll
-        for (int q = 0; q < kBU; ++q) {
-            const int e = min(e0 + q * kBT, cells - 1);
-            const int y = bdiv(e, w, inv_w, fast), x = e - y * w;
-            const int i = (y + 1) * s + x + 1;
-            idx[q] = i;
-            const float wx = link.pxw[x], wy = link.pyw[y];
-            const float* top = link.csol + (link.pyf[y] + 1) * link.cs + 1;
-            const float* bot = link.csol + (link.pys[y] + 1) * link.cs + 1;
-            const int a0 = link.pxf[x], a1 = link.pxs[x];
-            const float a = (1.f - wx) * top[a0] + wx * top[a1];
-            const float b = (1.f - wx) * bot[a0] + wx * bot[a1];
-            float v = L.sol[1][i];
-            v += (1.f - wy) * a + wy * b;
-            val[q] = v;
-        }
-#pragma unroll
-        for (int q = 0; q < kBU; ++q)
-            if (e0 + q * kBT < cells)
-                L.sol[0][idx[q]] = val[q];
-    }
-    __syncthreads();
-}
-
-__global__ __launch_bounds__(kBT) void k_batch_pcg(const BatchInstance* batch)
+// Tails of many grids that fs_tail.hip's register layout does not take, one workgroup each.
+__global__ __launch_bounds__(kTailThreads) void k_lds_tail_batch(const BatchItem* __restrict__ items,
+    const int* __restrict__ list)
 {
     extern __shared__ float lds[];
-    __shared__ PcgScalars S;
-    __shared__ double slot[3][kBW];
-    const BatchInstance& I = batch[blockIdx.x];
-    const GridDev& g = I.g;
-    const int W = g.W, H = g.H, s = g.s, N = W * H;
-    const double n = (double)N;
-    const float inv_W = 1.0f / (float)W;
-    const bool fast = N < (1 << 22);
-    if (threadIdx.x == 0) {
-        S = *g.S;
-        S.rz = S.rz_slot[S.iterations & 1];   // r.z of the first direction (written by its kernel)
-        S.restart = 0;                         // consumed by that direction
-        S.flush = 0;
-        S.p_shift = 0.0;
-    }
-    __syncthreads();
-    const float* z = I.multigrid ? (I.levels > 0 ? I.lev[0].L.sol[0] : (const float*)I.tail->top_sol) : g.zdiag;
-    while (S.status == kRunning) {
-        // q = A d and d.q (k_pcg_ad), alpha (kFinAd)
-        double dot = 0.0;
-        for (int e0 = threadIdx.x; e0 < N; e0 += kBU * kBT) {
-            int idx[kBU];
-            float cv[kBU], qv[kBU];
-#pragma unroll
-            for (int u = 0; u < kBU; ++u) {
-                const int e = min(e0 + u * kBT, N - 1);
-                const int y = bdiv(e, W, inv_W, fast), i = (y + 1) * s + (e - y * W) + 1;
-                idx[u] = i;
-                const float c = g.d[i];
-                const float dl = g.d[i - 1], dr = g.d[i + 1], du = g.d[i - s], dd = g.d[i + s];
-                const float wl = g.right32[i - 1], wr = g.right32[i], wu = g.down32[i - s], wd = g.down32[i];
-                cv[u] = c;
-                qv[u] = (wl * (c - dl) + wr * (c - dr)) + (wu * (c - du) + wd * (c - dd));
-            }
-#pragma unroll
-            for (int u = 0; u < kBU; ++u) {
-                if (e0 + u * kBT < N) {
-                    g.q[idx[u]] = qv[u];
-                    dot += (double)cv[u] * (double)qv[u];
-                }
-            }
-        }
-        dot = wg_sum(dot, slot[0]);
-        if (threadIdx.x == 0) {
-            S.dq = dot;
-            if (dot <= 0.0 || !isfinite(dot)) {
-                S.status = kStopped;
-            } else {
-                const double alpha = S.rz / dot;
-                if (!isfinite(alpha))
-                    S.status = kStopped;
-                S.alpha = alpha;
-            }
-        }
-        __syncthreads();
-        if (S.status != kRunning)
-            break;
-        // x += alpha d, r -= alpha q (k_pcg_update); recurrence checks (kFinUpdate)
-        const float alpha = (float)S.alpha;
-        double sum = 0.0, m = 0.0;
-        for (int e0 = threadIdx.x; e0 < N; e0 += kBU * kBT) {
-            int idx[kBU];
-            float xv[kBU], rv[kBU];
-#pragma unroll
-            for (int u = 0; u < kBU; ++u) {
-                const int e = min(e0 + u * kBT, N - 1);
-                const int y = bdiv(e, W, inv_W, fast), i = (y + 1) * s + (e - y * W) + 1;
-                idx[u] = i;
-                xv[u] = g.x[i] + alpha * g.d[i];
-                rv[u] = g.r[i] - alpha * g.q[i];
-            }
-#pragma unroll
-            for (int u = 0; u < kBU; ++u) {
-                if (e0 + u * kBT < N) {
-                    g.x[idx[u]] = xv[u];
-                    g.r[idx[u]] = rv[u];
-                    sum += (double)rv[u];
-                    m = fmax(m, (double)fabsf(rv[u]));
-                }
-            }
-        }
-        sum = wg_sum(sum, slot[0]);
-        m = wg_max(m, slot[1]);
-        if (threadIdx.x == 0) {
-            if (!isfinite(sum))
-                m = INFINITY;
-            S.iterations += 1;
-            S.rmax = m;
-            S.r_sum = sum;
-            S.r_mean = sum / n;
-            if (m <= S.tol) {
-                S.verify = 1;
-            } else if (m <= kRefineDrop * S.window_rmax || S.iterations % kReplaceEvery == 0) {
-                S.verify = 1;
-                S.replace = 1;
-            }
-        }
-        __syncthreads();
-        // flush and FP64 true residual (k_flush, k_true_residual mode 1, kFinTrueRes1)
-        if (S.verify) {
-            double tsum = 0.0, tmax = 0.0;
-            for (int e = threadIdx.x; e < N; e += kBT) {
-                const int y = bdiv(e, W, inv_W, fast), i = (y + 1) * s + (e - y * W) + 1;
-                g.p[i] = g.p[i] + (double)g.x[i];
-                g.x[i] = 0.0f;
-            }
-            __syncthreads();
-            for (int e = threadIdx.x; e < N; e += kBT) {
-                const int y = bdiv(e, W, inv_W, fast), i = (y + 1) * s + (e - y * W) + 1;
-                const double c = g.p[i];
-                const double product = (g.right64[i - 1] * (c - g.p[i - 1]) + g.right64[i] * (c - g.p[i + 1])) +
-                                       (g.down64[i - s] * (c - g.p[i - s]) + g.down64[i] * (c - g.p[i + s]));
-                const double r = g.b[i] - product;
-                g.r[i] = (float)r;
-                tsum += r;
-                tmax = fmax(tmax, fabs(r));
-            }
-            tsum = wg_sum(tsum, slot[0]);
-            tmax = wg_max(tmax, slot[1]);
-            if (threadIdx.x == 0) {
-                if (!isfinite(tsum))
-                    tmax = INFINITY;
-                S.true_rmax = tmax;
-                S.r_sum = tsum;
-                if (tmax <= S.tol) {
-                    S.status = kConverged;
-                } else {
-                    S.r_mean = tsum / n;
-                    if (!S.replace || tmax > kDriftRatio * S.rmax) {
-                        S.restart = 1;
-                        S.restarts += 1;
-                    }
-                    S.rmax = tmax;
-                    S.window_rmax = tmax;
-                }
-                S.verify = 0;
-                S.replace = 0;
-            }
-            __syncthreads();
-            if (S.status != kRunning)
-                break;
-        }
-        // preconditioner: V(4,4) cycle of r - mean (vcycle) or the diagonal (k_precond_diag)
-        if (I.multigrid) {
-            for (int l = 0; l < I.levels; ++l) {
-                const BatchLevel& B = I.lev[l];
-                const double* shift = l == 0 ? &S.r_mean : nullptr;
-                wg_sweeps(B.L, B.L.sol[1], B.L.rhs, shift, 0, true, B.sweeps);
-                wg_res_restrict(B.L, B.L.rhs, shift, B.C, B.rx, B.ry);
-            }
-            tail_run<float>(*I.tail, I.levels == 0 ? &S.r_mean : nullptr, nullptr, lds);
-            __syncthreads();
-            for (int l = I.levels - 1; l >= 0; --l) {
-                const BatchLevel& B = I.lev[l];
-                wg_prolong(B.L, B.link);
-                wg_sweeps(B.L, B.L.sol[0], B.L.rhs, l == 0 ? &S.r_mean : nullptr, 1, false, B.sweeps);
-            }
-        } else {
-            const double mean = S.r_mean;
-            for (int e = threadIdx.x; e < N; e += kBT) {
-                const int y = bdiv(e, W, inv_W, fast), i = (y + 1) * s + (e - y * W) + 1;
-                g.zdiag[i] = (float)(((double)g.r[i] - mean) * (double)g.invd32[i]);
-            }
-            __syncthreads();
-        }
-        // sum z, r.z, sum r (k_pcg_rz), beta (kFinRz)
-        double sz = 0.0, srz = 0.0, sr = 0.0;
-        for (int e0 = threadIdx.x; e0 < N; e0 += kBU * kBT) {
-            float zv[kBU], rv[kBU];
-#pragma unroll
-            for (int u = 0; u < kBU; ++u) {
-                const int e = min(e0 + u * kBT, N - 1);
-                const int y = bdiv(e, W, inv_W, fast), i = (y + 1) * s + (e - y * W) + 1;
-                zv[u] = z[i];
-                rv[u] = g.r[i];
-            }
-#pragma unroll
-            for (int u = 0; u < kBU; ++u) {
-                if (e0 + u * kBT < N) {
-                    const double zz = (double)zv[u], rr = (double)rv[u];
-                    sz += zz;
-                    srz += rr * zz;
-                    sr += rr;
-                }
-            }
-        }
-        sz = wg_sum(sz, slot[0]);
-        srz = wg_sum(srz, slot[1]);
-        sr = wg_sum(sr, slot[2]);
-        if (threadIdx.x == 0) {
-            const double mean = sz / n;
-            const double next = srz - mean * sr;
-            S.z_mean = mean;
-            const double beta = S.restart ? 0.0 : next / S.rz;
-            S.beta = beta;
-            S.restart = 0;
-            if (!isfinite(beta)) {
-                S.status = kStopped;
-            } else {
-                S.rz = next;
-                if (!(S.iterations < S.max_iterations && next > 0.0 && isfinite(next)))
-                    S.status = kStopped;
-            }
-        }
-        __syncthreads();
-        if (S.status != kRunning)
-            break;
-        // d = (z - mean z) + beta d (k_pcg_direction)
-        const float zmean = (float)S.z_mean;
-        const double beta64 = S.beta;
-        const float beta = (float)beta64;
-        for (int e0 = threadIdx.x; e0 < N; e0 += kBU * kBT) {
-            int idx[kBU];
-            float dv[kBU];
-#pragma unroll
-            for (int u = 0; u < kBU; ++u) {
-                const int e = min(e0 + u * kBT, N - 1);
-                const int y = bdiv(e, W, inv_W, fast), i = (y + 1) * s + (e - y * W) + 1;
-                idx[u] = i;
-                const float zz = z[i] - zmean;
-                dv[u] = beta64 == 0.0 ? zz : zz + beta * g.d[i];
-            }
-#pragma unroll
-            for (int u = 0; u < kBU; ++u)
-                if (e0 + u * kBT < N)
-                    g.d[idx[u]] = dv[u];
-        }
-        __syncthreads();
-    }
-    if (threadIdx.x == 0)
-        *g.S = S;
+    const BatchItem& I = items[list[blockIdx.x]];
+    tail_run<float>(I.tail, I.levels == 0 ? &I.g.S->r_mean : nullptr, &I.g.S->status, lds);
+}
+
+__global__ __launch_bounds__(64 * kSweepWaves) void k_chain_batch(const BatchItem* __restrict__ items,
+    const int* __restrict__ list)
+{
+    const BatchItem& I = items[list[blockIdx.x]];
+    coarse_chain(I.chain, I.ginv, I.coarse_n, I.g.S, I.pin);
 }
 
 }  // namespace
@@ -1416,14 +1007,20 @@ FS_RESTRICT(bf16, bf16, bf16)
 
 bool batch_allow_lds(size_t bytes)
 {
-    return hipFuncSetAttribute((const void*)k_batch_pcg, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes) ==
+    return hipFuncSetAttribute((const void*)k_lds_tail_batch, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes) ==
            hipSuccess;
 }
 
-void launch_batch_pcg(hipStream_t st, const BatchInstance* batch, int count, size_t lds_bytes)
+void launch_batch_lds_tail(hipStream_t st, const BatchItem* items, const int* list, int n, size_t lds_bytes)
 {
-    if (count > 0)
-        hipLaunchKernelGGL(k_batch_pcg, dim3(count), dim3(kBT), lds_bytes, st, batch);
+    if (n > 0)
+        hipLaunchKernelGGL(k_lds_tail_batch, dim3(n), dim3(kTailThreads), lds_bytes, st, items, list);
+}
+
+void launch_batch_chain(hipStream_t st, const BatchItem* items, const int* list, int n)
+{
+    if (n > 0)
+        hipLaunchKernelGGL(k_chain_batch, dim3(n), dim3(64 * kSweepWaves), 0, st, items, list);
 }
 
 }  // namespace fsim

@@ -61,17 +61,21 @@ __device__ __forceinline__ Tile4 tile4(const GridDev& g, int column, int row)
 // ------------------------------------------------------------------------------------------
 // Scalar block (kernels, so they are safe inside captured graphs).
 // ------------------------------------------------------------------------------------------
+__device__ __forceinline__ void init_scalars(PcgScalars* S, double tol, int max_iterations, double rel_tol)
+{
+    PcgScalars z{};
+    z.tol = tol;
+    z.rel_tol = rel_tol;
+    z.max_iterations = max_iterations;
+    z.status = kRunning;
+    z.restart = 1;
+    *S = z;
+}
+
 __global__ void k_init_scalars(PcgScalars* S, double tol, int max_iterations, double rel_tol)
 {
-    if (threadIdx.x == 0 && blockIdx.x == 0) {
-        PcgScalars z{};
-        z.tol = tol;
-        z.rel_tol = rel_tol;
-        z.max_iterations = max_iterations;
-        z.status = kRunning;
-        z.restart = 1;
-        *S = z;
-    }
+    if (threadIdx.x == 0 && blockIdx.x == 0)
+        init_scalars(S, tol, max_iterations, rel_tol);
 }
 
 __global__ void k_merge_failure(const PcgScalars* from, PcgScalars* S)
@@ -150,12 +154,12 @@ struct Coefficients {
 // thread forms one cell's (taller tiles with several cells per thread took 17 us on 256^2 against 5).
 constexpr int kCoarsenY = 4;
 constexpr int kCoarsenThreads = 384;
-__global__ __launch_bounds__(kCoarsenThreads) void k_coarsen(ChainLevel L)
+__device__ __forceinline__ void coarsen_tile(const ChainLevel& L, int column, int row)
 {
     constexpr int LX = kTX + 1, LY = kCoarsenY + 1;
     static_assert(LX * LY <= kCoarsenThreads, "one cell per thread");
     __shared__ double s_right[LY * LX], s_down[LY * LX];
-    const int x0 = blockIdx.x * kTX - 1, y0 = blockIdx.y * kCoarsenY - 1;
+    const int x0 = column * kTX - 1, y0 = row * kCoarsenY - 1;
     const int e = threadIdx.x;
     const int ly = e / LX, lx = e - ly * LX;
     const int x = x0 + lx, y = y0 + ly;
@@ -176,6 +180,8 @@ __global__ __launch_bounds__(kCoarsenThreads) void k_coarsen(ChainLevel L)
             L.down32[i]);
     }
 }
+
+__global__ __launch_bounds__(kCoarsenThreads) void k_coarsen(ChainLevel L) { coarsen_tile(L, blockIdx.x, blockIdx.y); }
 
 // ------------------------------------------------------------------------------------------
 // Projection set-up (FluidGridCPU.cpp:1050-1090, :1728-1756), FP64.
@@ -695,41 +701,6 @@ struct PrecondDiag {
     }
 };
 
-// The first direction of a batched solve: d alone, and the pressure folded.
-template <bool FLEX> struct Direction {
-    template <int G> __device__ __forceinline__ void run(const GridDev& g, Block B) const
-    {
-        constexpr int NP = FLEX ? 5 : 3;
-        __shared__ double lds[NP * kNT / 64];
-        double t[NP];
-        Partials<kNT, NP>().all(g.fold_rz, g.fold_rz_n, t, lds);
-        if (g.S->status != kRunning)
-            return;
-        float mean;
-        double beta64;
-        if (!next_direction<FLEX>(g, t, B.id() == 0, mean, beta64))
-            return;
-        const float beta = (float)beta64;
-        const bool fold = g.S->flush != 0;
-        const double shift = g.S->p_shift;
-#pragma unroll 1
-        for (int group = 0; group < G; ++group) {
-            const Tile4 T = tile4(g, B.x, B.y * G + group);
-#pragma unroll
-            for (int k = 0; k < 4; ++k) {
-                if (T.in[k]) {
-                    const float zz = g.z[T.P[k]] - mean;
-                    g.d[T.P[k]] = beta64 == 0.0 ? zz : zz + beta * g.d[T.P[k]];
-                    if (fold) {
-                        g.p[T.P[k]] = (g.p[T.P[k]] - shift) + (double)g.x[T.P[k]];
-                        g.x[T.P[k]] = 0.0f;
-                    }
-                }
-            }
-        }
-    }
-};
-
 // ------------------------------------------------------------------------------------------
 // Closing phase, once the solve has stopped (a no-op while it runs: it may be queued behind iterations that do not
 // finish the solve).  The pressure's final value is formed from p and x where it is needed and stored last, since the
@@ -985,6 +956,68 @@ __global__ __launch_bounds__(kNT) void k_fold_partials(const double* partials, i
             out[c] = t[c];
 }
 
+// ------------------------------------------------------------------------------------------
+// launches: many grids.  A small grid's kernel leaves most of the chip idle and costs its launch; one launch over
+// the tiles of all of them costs little more than one grid's.
+// ------------------------------------------------------------------------------------------
+template <class Op> __global__ __launch_bounds__(kNT) void k_cells_batch(const BatchItem* __restrict__ items,
+    const int* __restrict__ item, const int* __restrict__ first)
+{
+    const int i = item[blockIdx.x];
+    const int local = (int)blockIdx.x - first[i];
+    const GridDev g = items[i].g;
+    const int columns = (g.W + kTX - 1) / kTX;
+    const int row = local / columns;
+    Op().template run<1>(g, Block{local - row * columns, row, columns});
+}
+
+template <class Op> __global__ __launch_bounds__(kNT) void k_finish_batch(const BatchItem* __restrict__ items,
+    const int* __restrict__ list)
+{
+    __shared__ double lds[2 * kNT / 64];
+    const GridDev g = items[list[blockIdx.x]].g;
+    Op().run(g, g.fold_up_n, lds);
+}
+
+__global__ __launch_bounds__(kCoarsenThreads) void k_coarsen_batch(const BatchItem* __restrict__ items,
+    const int* __restrict__ item, const int* __restrict__ first, int level)
+{
+    const int i = item[blockIdx.x];
+    const int local = (int)blockIdx.x - first[i];
+    const ChainLevel L = items[i].coarsen[level];
+    const int columns = (L.cw + kTX - 1) / kTX;
+    const int row = local / columns;
+    coarsen_tile(L, local - row * columns, row);
+}
+
+__global__ void k_init_batch(const BatchItem* __restrict__ items, const int* __restrict__ list, int n)
+{
+    const int k = blockIdx.x * blockDim.x + threadIdx.x;
+    if (k < n) {
+        const BatchItem& I = items[list[k]];
+        init_scalars(I.g.S, I.tol, I.max_iterations, I.rel_tol);
+    }
+}
+
+__global__ void k_scalars_batch(const BatchItem* __restrict__ items, const int* __restrict__ list, int n, PcgScalars* out)
+{
+    const int k = blockIdx.x * blockDim.x + threadIdx.x;
+    if (k < n)
+        out[k] = *items[list[k]].g.S;
+}
+
+template <class Op> void launch_cells_batch(hipStream_t st, const BatchItem* items, const BatchPart& part)
+{
+    if (part.blocks > 0)
+        hipLaunchKernelGGL(k_cells_batch<Op>, dim3(part.blocks), dim3(kNT), 0, st, items, part.item, part.first);
+}
+
+template <class Op> void launch_finish_batch(hipStream_t st, const BatchItem* items, const int* list, int n)
+{
+    if (n > 0)
+        hipLaunchKernelGGL(k_finish_batch<Op>, dim3(n), dim3(kNT), 0, st, items, list);
+}
+
 template <class Op> void launch_cells(hipStream_t st, const GridDev& g)
 {
     const int G = pcg_groups(g.W, g.H);
@@ -1091,14 +1124,70 @@ void launch_pcg_rz(hipStream_t st, const GridDev& g, int flexible)
     }
 }
 
-void launch_pcg_direction(hipStream_t st, const GridDev& g, int flexible)
+void launch_precond_diag(hipStream_t st, const GridDev& g) { launch_cells<PrecondDiag>(st, g); }
+
+int batch_cell_blocks(int W, int H) { return ((W + kTX - 1) / kTX) * ((H + kTY - 1) / kTY); }
+int batch_coarsen_blocks(const ChainLevel& level)
 {
-    if (flexible)
-        launch_cells<Direction<true>>(st, g);
-    else
-        launch_cells<Direction<false>>(st, g);
+    return ((level.cw + kTX - 1) / kTX) * ((level.ch + kCoarsenY - 1) / kCoarsenY);
 }
 
-void launch_precond_diag(hipStream_t st, const GridDev& g) { launch_cells<PrecondDiag>(st, g); }
+void launch_batch_init(hipStream_t st, const BatchItem* items, const int* list, int n)
+{
+    if (n > 0)
+        hipLaunchKernelGGL(k_init_batch, dim3((n + 63) / 64), dim3(64), 0, st, items, list, n);
+}
+
+void launch_batch_coefficients(hipStream_t st, const BatchItem* items, const BatchPart& part)
+{
+    launch_cells_batch<Coefficients>(st, items, part);
+}
+
+void launch_batch_coarsen(hipStream_t st, const BatchItem* items, const BatchPart& part, int level)
+{
+    if (part.blocks > 0)
+        hipLaunchKernelGGL(k_coarsen_batch, dim3(part.blocks), dim3(kCoarsenThreads), 0, st, items, part.item, part.first,
+            level);
+}
+
+void launch_batch_setup(hipStream_t st, const BatchItem* items, const BatchPart& part, const int* list, int n)
+{
+    launch_cells_batch<Rhs>(st, items, part);
+    launch_cells_batch<Predict>(st, items, part);
+    launch_cells_batch<InitialResidual>(st, items, part);
+    launch_finish_batch<FinishSetup>(st, items, list, n);
+}
+
+void launch_batch_step(hipStream_t st, const BatchItem* items, const BatchPart& part, const int* list, int n)
+{
+    launch_cells_batch<DirectionAd<false>>(st, items, part);
+    launch_cells_batch<Update>(st, items, part);
+    launch_cells_batch<Check>(st, items, part);
+    launch_finish_batch<FinishCheck>(st, items, list, n);
+}
+
+void launch_batch_precond_diag(hipStream_t st, const BatchItem* items, const BatchPart& part)
+{
+    launch_cells_batch<PrecondDiag>(st, items, part);
+}
+
+void launch_batch_rz(hipStream_t st, const BatchItem* items, const BatchPart& part)
+{
+    launch_cells_batch<Rz<false>>(st, items, part);
+}
+
+void launch_batch_end(hipStream_t st, const BatchItem* items, const BatchPart& part, const int* list, int n)
+{
+    launch_cells_batch<FinalSum>(st, items, part);
+    launch_cells_batch<CorrectVelocity>(st, items, part);
+    launch_cells_batch<MaxDivergence<true>>(st, items, part);
+    launch_finish_batch<FinishDivergence<true>>(st, items, list, n);
+}
+
+void launch_batch_scalars(hipStream_t st, const BatchItem* items, const int* list, int n, PcgScalars* out)
+{
+    if (n > 0)
+        hipLaunchKernelGGL(k_scalars_batch, dim3((n + 63) / 64), dim3(64), 0, st, items, list, n, out);
+}
 
 }  // namespace fsim

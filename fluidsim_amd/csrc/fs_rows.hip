@@ -56,9 +56,9 @@ __host__ __device__ constexpr int rows_edge(int mode, int jacobi, int nu)
 }
 
 template <int JACOBI, int MODE, int G, int NW, int M, class C, class V, class VC>
-__global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(4)))
-void k_rows(LevelViewT<C, V> L, int cur, const V* rhs, const double* shift, SmoothWeights wt, int nu,
-    CoarseLinkT<VC> link, LevelViewT<C, VC> Cl, AxisRestrict rx, AxisRestrict ry, const int* status)
+__device__ __forceinline__ void rows_tile(const LevelViewT<C, V>& L, int cur, const V* rhs, const double* shift,
+    const SmoothWeights& wt, int nu, const CoarseLinkT<VC>& link, const LevelViewT<C, VC>& Cl, const AxisRestrict& rx,
+    const AxisRestrict& ry, const int* status, int bx, int by)
 {
     constexpr int NG = NW * 64 / G;   // lane groups, one above the other
     constexpr int LX = 2 * G, LY = NG * M;
@@ -74,8 +74,6 @@ void k_rows(LevelViewT<C, V> L, int cur, const V* rhs, const double* shift, Smoo
     const int w = L.w, h = L.h, s = L.s;
     const int edge = rows_edge(MODE, JACOBI, nu);
     const int TX = LX - 2 * edge, TY = LY - 2 * edge;
-    int bx, by;
-    xcd_tile((w + TX - 1) / TX, (h + TY - 1) / TY, bx, by);
     const int lane = threadIdx.x & (G - 1);
     const int group = G == 64 ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : (int)threadIdx.x / G;
     const int x0 = bx * TX - edge, y0 = by * TY - edge;
@@ -397,6 +395,37 @@ void k_rows(LevelViewT<C, V> L, int cur, const V* rhs, const double* shift, Smoo
     }
 }
 
+template <int JACOBI, int MODE, int G, int NW, int M, class C, class V, class VC>
+__global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(4)))
+void k_rows(LevelViewT<C, V> L, int cur, const V* rhs, const double* shift, SmoothWeights wt, int nu,
+    CoarseLinkT<VC> link, LevelViewT<C, VC> Cl, AxisRestrict rx, AxisRestrict ry, const int* status)
+{
+    constexpr int LX = 2 * G, LY = NW * 64 / G * M;
+    const int edge = rows_edge(MODE, JACOBI, nu);
+    const int TX = LX - 2 * edge, TY = LY - 2 * edge;
+    int bx, by;
+    xcd_tile((L.w + TX - 1) / TX, (L.h + TY - 1) / TY, bx, by);
+    rows_tile<JACOBI, MODE, G, NW, M, C, V, VC>(L, cur, rhs, shift, wt, nu, link, Cl, rx, ry, status, bx, by);
+}
+
+// A tiled level of many grids in one launch: red-black on FP32 levels, 64 x 64 tiles on 512 threads.
+constexpr int kBatchG = 32, kBatchNW = 8, kBatchM = 4;
+template <int MODE>
+__global__ __launch_bounds__(64 * kBatchNW) __attribute__((amdgpu_waves_per_eu(4)))
+void k_rows_batch(const BatchItem* __restrict__ items, const int* __restrict__ item, const int* __restrict__ first, int level)
+{
+    const int i = item[blockIdx.x];
+    const int local = (int)blockIdx.x - first[i];
+    const BatchLevel B = items[i].lev[level];
+    const PcgScalars* S = items[i].g.S;
+    const int TX = 2 * kBatchG - 2 * rows_edge(MODE, 0, B.sweeps);
+    const int columns = (B.L.w + TX - 1) / TX;
+    const int row = local / columns;
+    rows_tile<0, MODE, kBatchG, kBatchNW, kBatchM, float, float, float>(B.L, MODE == kRowsPost ? 1 : 0, B.L.rhs,
+        level == 0 ? &S->r_mean : nullptr, SmoothWeights{}, B.sweeps, B.link, B.C, B.rx, B.ry, &S->status,
+        local - row * columns, row);
+}
+
 // Elements of a level from which byte offsets of FP32 fields pass 32 bits.
 constexpr size_t kRowsWide = (size_t)1 << 30;
 
@@ -443,6 +472,25 @@ void launch_rows_mode(hipStream_t st, const LevelViewT<C, V>& L, int cur, const 
 }
 
 }  // namespace
+
+int batch_level_blocks(const BatchLevel& level, bool post)
+{
+    const int edge = rows_edge(post ? kRowsPost : kRowsPreRestrict, 0, level.sweeps);
+    const int TX = 2 * kBatchG - 2 * edge, TY = kBatchNW * 64 / kBatchG * kBatchM - 2 * edge;
+    return ((level.L.w + TX - 1) / TX) * ((level.L.h + TY - 1) / TY);
+}
+
+void launch_batch_smooth(hipStream_t st, const BatchItem* items, const BatchPart& part, int level, bool post)
+{
+    if (part.blocks <= 0)
+        return;
+    if (post)
+        hipLaunchKernelGGL(k_rows_batch<kRowsPost>, dim3(part.blocks), dim3(64 * kBatchNW), 0, st, items, part.item,
+            part.first, level);
+    else
+        hipLaunchKernelGGL(k_rows_batch<kRowsPreRestrict>, dim3(part.blocks), dim3(64 * kBatchNW), 0, st, items, part.item,
+            part.first, level);
+}
 
 template <class C, class V, class VC>
 void launch_smooth(hipStream_t st, int jacobi, const LevelViewT<C, V>& L, int cur, const V* rhs,

@@ -37,13 +37,15 @@ template <int M> struct Held {
 
 constexpr int kTailMax = 1024;   // threads of the largest workgroup
 
+constexpr int kTables = 512;     // entries of the levels' transfer tables
+
 // LDS of the kernel.
 struct TailShared {
     float edge[2][2][kTailMax];     // [colour][top, bottom][thread]
     float reach[2][kTailMax];       // the restriction's row sums: [top, bottom][thread]
     float field[kTailMax + 256];    // a coarse level's rhs (down) or solution (up), rows of width kernel-wide cells
     float inverse[64 * 64];         // the coarse inverse, column j at 64 j
-    float4 table[4 * 256];          // transfer tables of the levels
+    float4 table[kTables];          // transfer tables of the levels
 };
 
 struct Place {
@@ -302,7 +304,8 @@ __device__ __forceinline__ void coarse_solve(const TailLevel& T, int n, TailShar
         S.field[0] = (float)(-gauge);
 }
 
-template <int K, int NL> struct Cycle {
+// NL levels above the coarsest; ANY: up to NL, as many as D has.
+template <int K, int NL, bool ANY> struct Cycle {
     // Level K's cycle; its rhs is in S.field for K > 0, its solution left in the registers.
     template <int M, class Deeper>
     static __device__ __forceinline__ void run(const TailDesc& D, Held<M>& v, Deeper& deeper, TailShared& S)
@@ -325,32 +328,35 @@ template <int K, int NL> struct Cycle {
         if constexpr (K > 0)
             __syncthreads();   // S.field has been read
         restrict_level<M>(T, v, p, S);
+        bool last = true;
         if constexpr (K + 1 < NL) {
-            Cycle<K + 1, NL>::run(D, deeper[K], deeper, S);
-            const TailLevel& C = D.lev[K + 1];
-            const Place q = place<2>(C);
-            __syncthreads();
+            last = ANY && K + 2 >= D.levels;
+            if (!last) {
+                Cycle<K + 1, NL, ANY>::run(D, deeper[K], deeper, S);
+                const TailLevel& C = D.lev[K + 1];
+                const Place q = place<2>(C);
+                __syncthreads();
 #pragma unroll
-            for (int r = 0; r < 2; ++r)
+                for (int r = 0; r < 2; ++r)
 #pragma unroll
-                for (int j = 0; j < 2; ++j) {
-                    const int x = 2 * q.lane + j, y = q.group * 2 + r;
-                    if (x < C.w && y < C.h)
-                        S.field[y * C.w + x] = deeper[K].x[r][j];
-                }
-        } else if (threadIdx.x < 64) {
-            coarse_solve(D.lev[K + 1], D.coarse_n, S);
+                    for (int j = 0; j < 2; ++j) {
+                        const int x = 2 * q.lane + j, y = q.group * 2 + r;
+                        if (x < C.w && y < C.h)
+                            S.field[y * C.w + x] = deeper[K].x[r][j];
+                    }
+            }
         }
+        if (last && threadIdx.x < 64)
+            coarse_solve(D.lev[K + 1], D.coarse_n, S);
         __syncthreads();
         prolong_level<M>(T, v, p, S);
         smooth<M, true>(v, p, D.sweeps, S);
     }
 };
 
-template <int M, int NT, int NL, class TV>
-__global__ __launch_bounds__(NT) void k_tail(const TailDesc D, const double* shift, const int* status)
+template <int M, int NT, int NL, bool ANY, class TV>
+__device__ __forceinline__ void tail_cycle(const TailDesc& D, const double* shift, const int* status, TailShared& S)
 {
-    __shared__ TailShared S;
     const TailLevel& T = D.lev[0];
     const Place p = place<M>(T);
     Held<M> top;
@@ -361,8 +367,8 @@ __global__ __launch_bounds__(NT) void k_tail(const TailDesc D, const double* shi
         load_two((const TV*)D.top_rhs, pair_index<M>(T, p, r), top.cb[r]);
 #pragma unroll
     for (int k = 0; k + 1 < NL; ++k)
-        load_level<2>(D.lev[k + 1], deeper[k]);
-    constexpr int TG = (63 * 63 + NT - 1) / NT, TT = (1024 + NT - 1) / NT;
+        load_level<2>(D.lev[ANY ? min(k + 1, D.levels - 1) : k + 1], deeper[k]);
+    constexpr int TG = (63 * 63 + NT - 1) / NT, TT = (kTables + NT - 1) / NT;
     const int n = D.coarse_n, nn = n * n;
     float gv[TG];
     float4 tv[TT];
@@ -409,7 +415,7 @@ __global__ __launch_bounds__(NT) void k_tail(const TailDesc D, const double* shi
                 top.cb[r][j] = (float)((double)top.cb[r][j] - sh);
     }
     __syncthreads();
-    Cycle<0, NL>::run(D, top, deeper, S);
+    Cycle<0, NL, ANY>::run(D, top, deeper, S);
     TV* out = (TV*)D.top_sol;
 #pragma unroll
     for (int r = 0; r < M; ++r) {
@@ -422,6 +428,24 @@ __global__ __launch_bounds__(NT) void k_tail(const TailDesc D, const double* shi
                 *q = stv<TV>(top.x[r][0]);
         }
     }
+}
+
+template <int M, int NT, int NL, class TV>
+__global__ __launch_bounds__(NT) void k_tail(const TailDesc D, const double* shift, const int* status)
+{
+    __shared__ TailShared S;
+    tail_cycle<M, NT, NL, false, TV>(D, shift, status, S);
+}
+
+// The tails of many grids, one workgroup each: 512 threads, eight rows per thread, whatever the shapes.
+constexpr int kBatchThreads = 512;
+__global__ __launch_bounds__(kBatchThreads) void k_tail_batch(const BatchItem* __restrict__ items,
+    const int* __restrict__ list)
+{
+    __shared__ TailShared S;
+    const BatchItem& I = items[list[blockIdx.x]];
+    const double* shift = I.levels == 0 ? &I.g.S->r_mean : nullptr;
+    tail_cycle<8, kBatchThreads, 4, true, float>(I.tail, shift, &I.g.S->status, S);
 }
 
 template <int M, int NT, class TV>
@@ -457,27 +481,33 @@ void tail_hold(TailDesc& t)
         return b;
     };
     const auto threads = [&](const TailLevel& T, int rows) { return ((T.h + rows - 1) / rows) << lanes(T); };
-    t.held_rows = 0;
+    t.held_rows = t.batch_rows = 0;
     if (t.levels < 2 || t.levels > 5)
         return;
-    constexpr int rows[3] = {2, 4, 8}, limit[3] = {1024, 768, 512};
-    for (int k = 0; k < 3 && !t.held_rows; ++k) {
-        bool fits = t.lev[0].w <= 128 && threads(t.lev[0], rows[k]) <= limit[k];
+    const auto fits = [&](int rows, int limit) {
+        bool ok = t.lev[0].w <= 128 && threads(t.lev[0], rows) <= limit;
         int table = 0;
         for (int l = 0; l + 1 < t.levels; ++l) {
-            fits = fits && (l == 0 || threads(t.lev[l], 2) <= limit[k]);
-            fits = fits && t.lev[l + 1].w * t.lev[l + 1].h <= kTailMax + 256;
+            ok = ok && (l == 0 || threads(t.lev[l], 2) <= limit);
+            ok = ok && t.lev[l + 1].w * t.lev[l + 1].h <= kTailMax + 256;
             table += 2 * ((t.lev[l].w + 1) / 2 + (t.lev[l].h + 1) / 2);
         }
-        if (fits && table <= 1024)
-            t.held_rows = rows[k];
-    }
+        return ok && table <= kTables;
+    };
+    t.held_rows = fits(2, 1024) ? 2 : fits(4, 768) ? 4 : fits(8, 512) ? 8 : 0;
+    t.batch_rows = fits(8, kBatchThreads) ? 8 : 0;
     int at = 0;
     for (int l = 0; l < t.levels; ++l) {
         t.lev[l].lanes = lanes(t.lev[l]);
         t.lev[l].table = at;
         at += 2 * ((t.lev[l].w + 1) / 2 + (t.lev[l].h + 1) / 2);
     }
+}
+
+void launch_batch_tail(hipStream_t st, const BatchItem* items, const int* list, int n)
+{
+    if (n > 0)
+        hipLaunchKernelGGL(k_tail_batch, dim3(n), dim3(kBatchThreads), 0, st, items, list);
 }
 
 void launch_held_tail(hipStream_t st, const TailDesc& desc, const double* shift, const int* status, int bf16_top)

@@ -204,7 +204,7 @@ class Context:
         call("fs_context_synchronize", self._h)
 
     def set_batch_split(self, solo_cells: int):
-        """fs_context_set_batch_split: batch_project sends grids of more than `solo_cells` cells through
+        """fs_context_set_batch_split: batch_apply_viscosity sends grids of more than `solo_cells` cells through
         the multi-kernel solve, concurrently with the persistent launch of the rest (0: batch all)."""
         call("fs_context_set_batch_split", self._h, int(solo_cells))
 
@@ -256,8 +256,8 @@ def viscosity_solve(width: int, height: int, cell_size: float, material, u, v, d
 
 
 def batch_project(grids, dt: float, max_iterations: int = 200, divergence_tolerance=1e-6):
-    """fs_batch_project: project every grid (all on one context) with one persistent launch running all
-    their PCG iterations.  `divergence_tolerance` is one value or one per grid.  Returns one
+    """fs_batch_project: project every grid (all on one context), each phase one launch over the tiles of all of
+    them.  `divergence_tolerance` is one value or one per grid.  Returns one
     ProjectionResult per grid, with fs_project's contract."""
     grids = list(grids)
     n = len(grids)

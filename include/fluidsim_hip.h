@@ -367,7 +367,7 @@ fs_status fs_face_weights(fs_grid* grid, double* inv_density_u, double* inv_dens
  * the grid's smoother sweeps, as in the V-cycle),
  * 1 = direction + operator + dot (A d), 2 = PCG update, 3 = FP32 copy of one padded vector (reference kernel),
  * 4 = second level's smoother, 5 = finest residual + restriction, 6 = coarse tail, 7 = coarse
- * inverse (sweep operator), 8 = direction update, 9 = r.z reduction, 10 = FP32 copy of a 64 MiB buffer
+ * inverse (sweep operator), 8 = as 1 (one launch), 9 = r.z reduction, 10 = FP32 copy of a 64 MiB buffer
  * into another (HBM copy-bandwidth reference; 128 MiB moved per launch). */
 fs_status fs_time_kernel(fs_grid* grid, int kernel, int reps, double* ms_per_launch);
 /* Cumulative device bytes allocated by this grid. */
@@ -384,13 +384,11 @@ fs_status fs_batch_apply_viscosity(int count, fs_grid* const* grids, double dt, 
 
 /* ---- batched projection (no reference counterpart: the reference projects one grid per call,
  * FluidGridCPU.cpp:1030-1124) ----
- * fs_project on `count` grids of one context at once: every grid's setup (coefficients, hierarchy, rhs,
- * predicted pressure, first direction) is launched on the context's stream, then ONE persistent launch
- * runs all grids' PCG iterations -- one 1024-thread workgroup per grid, looping on the device until that
- * grid converges or stops -- and then every grid's velocity correction.  Each grid's result follows
- * fs_project's contract (same stopping rule, same result fields) and does not depend on the other
- * grids; the FP64 reductions run in another order than fs_project's, so values agree with it to
- * rounding, not bit for bit.  tolerances[i] is grid i's divergence tolerance. */
+ * fs_project on `count` grids of one context at once: each phase of the projections -- coefficients, hierarchy, rhs,
+ * every step of an iteration, every multigrid level, the velocity corrections -- is one launch over the tiles of all
+ * the grids.  Each grid's result is fs_project's bit for bit, alone or in any batch.  Grids of more than 1024 tiles of
+ * 64 x 16 cells, and grids with the flexible CG, project on their own after the others.  tolerances[i] is grid i's
+ * divergence tolerance. */
 fs_status fs_batch_project(int count, fs_grid* const* grids, double dt, int max_iterations,
     const double* divergence_tolerances, fs_projection_result* results);
 /* Autotuner of the batched solves' red-black sweep counts (no reference counterpart): runs fs_batch_project
@@ -401,20 +399,20 @@ fs_status fs_batch_project(int count, fs_grid* const* grids, double dt, int max_
  * the choice and its time per batch.  FS_E_UNSUPPORTED for grids with 16-bit multigrid levels. */
 fs_status fs_tune_batch_smoother(int count, fs_grid* const* grids, double dt, int max_iterations,
     const double* divergence_tolerances, int* sweeps, int* coarse_sweeps, double* ms);
-/* Split of fs_batch_project and fs_batch_apply_viscosity (no reference counterpart): grids of more than
- * `solo_cells` cells are solved by fs_project's / fs_apply_viscosity's own multi-kernel solve, one after
- * another on the context's stream, while the persistent launch runs the smaller ones on a second stream
- * -- one workgroup is slow on a large grid, and the batch lasts as long as its slowest instance.  The
- * route depends on a grid's size only, so a grid's result is the same alone and in any batch.  0 (the
- * default) batches every grid; contexts created with FS_CONTEXT_SINGLE_STREAM always do. */
+/* Split of fs_batch_apply_viscosity (no reference counterpart): grids of more than `solo_cells` cells are solved
+ * by fs_apply_viscosity's own multi-kernel solve, one after another on the context's stream, while the persistent
+ * launch runs the smaller ones on a second stream -- one workgroup is slow on a large grid, and the batch lasts
+ * as long as its slowest instance.  The route depends on a grid's size only, so a grid's result is the same
+ * alone and in any batch.  0 (the default) batches every grid; contexts created with FS_CONTEXT_SINGLE_STREAM
+ * always do.  fs_batch_project spreads a grid of any size over the device and has no use for a split. */
 fs_status fs_context_set_batch_split(fs_context* ctx, long long solo_cells);
 
 /* Batched timestep (no reference counterpart: each instance is FluidGridCPU::step, FluidGridCPU.cpp:300-360,
  * as fs_step runs it): fs_step on `count` grids of one context at once, each with its own dts[i],
  * max_iterations[i] and divergence_tolerances[i].  Per capillary substep, every grid's transport, gravity and
  * surface tension are launched one grid after another on the context's stream, while the implicit viscosity
- * solves and the projections run batched (fs_batch_apply_viscosity's and fs_batch_project's persistent
- * launches, with the context's split; grids with 16-bit multigrid levels project one by one).  results[i]
+ * solves and the projections run batched (fs_batch_apply_viscosity's persistent launch, with the context's
+ * split, and fs_batch_project's shared launches; grids with 16-bit multigrid levels project one by one).  results[i]
  * follows fs_step's contract: a grid stops after its first substep whose projection does not converge, and
  * dts[i] <= 0 leaves it untouched with physical_steps = 0.  Values agree with fs_step to rounding (the batched
  * solves reduce in another order), and a grid's result does not depend on the other grids of the batch.  A
@@ -518,7 +516,7 @@ fs_status fs_advance_frame(fs_grid* grid, const fs_frame_settings* settings, fs_
  * Each step is fs_step(dt, max_iterations, divergence_tolerance) on the instance's own grid, so a
  * request's results do not depend on what else is resident.  With batch_cells > 0, the instances of at
  * most batch_cells cells take each round's step together instead: one fs_batch_step over the lane's small
- * instances (batched viscosity and projection in persistent launches), then fs_step for each larger one.
+ * instances (batched viscosity and projection), then fs_step for each larger one.
  * The route depends only on the request's own size, and a batched step's result does not depend on the
  * other instances, so the results still do not depend on what else is resident; they agree with fs_step's
  * to rounding.  Small instances are placed on the lane with the fewest resident small instances, larger ones

@@ -1,0 +1,72 @@
+"""Batched projections over shapes at the edges of the shared launches: one tile, one row or column, one level, levels
+that only the LDS tail takes, more tiles than are batched (solved on their own), with masks, both preconditioners,
+several sweep counts, absolute and relative tolerances and spent budgets.  Every grid's result is fs_project's on the
+same state bit for bit (the same kernels' arithmetic, the reductions per grid in the same order)."""
+import numpy as np
+import pytest
+
+from fluidsim_amd import FS_PRECOND_DIAGONAL, FS_SMOOTHER_RED_BLACK, FluidGridHIP, batch_project
+from fluidsim_amd import workloads as WL
+
+pytestmark = pytest.mark.gpu
+
+SHAPES = [(1, 1), (8, 8), (2, 1), (1, 130), (64, 16), (65, 17), (9, 9), (200, 20), (129, 65), (61, 47), (300, 111), (70, 58),
+          (1000, 1100), (257, 90)]
+
+
+def grids():
+    out = []
+    for k, (W, H) in enumerate(SHAPES):
+        wl = WL.sloped_pool(W, H, 4.0)
+        g = FluidGridHIP(W, H, 4.0)
+        WL.load_into(g, wl)
+        if k % 3 == 0 and W > 8 and H > 8:
+            solid = np.zeros((H, W), np.uint8)
+            solid[H // 3:H // 3 + 3, W // 4:W // 4 + 5] = 1
+            g.setSolidMask(solid)
+        if k % 4 == 1:
+            g.setPressurePreconditioner(FS_PRECOND_DIAGONAL)
+        if k % 2:
+            g.setPressureSmoother(FS_SMOOTHER_RED_BLACK, 1 + k % 4, 1 + k % 3)
+        if k % 5 == 2:
+            g.setRelativeTolerance(True)
+        g.snapshotSave()
+        out.append(g)
+    return out
+
+
+def state(g):
+    s = g.download()
+    return s.u, s.v, s.pressure
+
+
+@pytest.mark.parametrize("budget", [3, 400])
+def test_batched_projections_are_the_single_ones(budget):
+    many, dt = grids(), 1.0 / 120.0
+    expected = []
+    for rounds in (1, 2):   # the second from the first one's pressure, its hierarchy still valid
+        for g in many:
+            if rounds == 1:
+                g.snapshotRestore()
+            else:
+                g.addVortex((4.0, 4.0), 20.0, 0.1)
+            r = g.project(dt, budget, 1e-5)
+            expected.append((r, state(g)))
+    at = 0
+    for rounds in (1, 2):
+        for g in many:
+            if rounds == 1:
+                g.snapshotRestore()
+            else:
+                g.addVortex((4.0, 4.0), 20.0, 0.1)
+        results = batch_project(many, dt, budget, 1e-5)
+        for g, r in zip(many, results):
+            ref, fields = expected[at]
+            at += 1
+            key = (rounds, g.width, g.height)
+            assert (r.iterations, r.converged, r.restarts) == (ref.iterations, ref.converged, ref.restarts), key
+            assert r.max_divergence == ref.max_divergence and r.final_residual == ref.final_residual, key
+            for a, b in zip(state(g), fields):
+                assert np.array_equal(a, b), key
+    for g in many:
+        g.destroy()
