@@ -9,13 +9,15 @@
 //
 // Layout and numerics: every level stores (w+1) x (h+1) slots of float2 (u face left of
 // cell p, v face on top of cell p) and float4 coefficients (cell mu, vertex mu, u mass, v mass); reads
-// clamp to the slot field like the reference's accessors.  The iterate x starts at v0 in FP32 (the
+// clamp to the slot field like the reference's accessors (fs_viscosity_rows.hpp: the kernels of a solve keep
+// their slots in registers).  The iterate x starts at v0 in FP32 (the
 // reference's formulation: iterating on v - v0 instead loses three digits to cancellation when dt K
 // dominates M) and dot products are FP64.  A solve that needs no iteration leaves u, v untouched.  Kernels read a device scalar block and
 // exit at once when the solve has stopped, so a batch of four iterations is launched without host
 // round trips; the host reads the block once per batch, as the reference does.
 #include "fs_internal.hpp"
 #include "fs_kernels.hpp"
+#include "fs_mg_device.hpp"
 
 #include <math.h>
 
@@ -48,11 +50,11 @@ struct VisScalars {
     float dt;         // time step of this solve: the iteration kernels read it here, so one captured
                       // batch of iterations serves every dt
     int status;       // batched solve: result code (see viscosity_solve)
-    int iterations;   // iterations run (batched solve; single solve: counted by k_vis_decide)
+    int iterations;   // iterations run
     int done;         // single solve, set on the device: 0 running, 1 converged (4 once unpacked),
                       // 2 breakdown, 3 budget spent, 5 no iteration needed, 6 non-finite input
-    int restart;      // single solve: restart from the recomputed residual before the next batch
-    int pad;
+    int restart;      // single solve: the next batch starts from the recomputed residual
+    int pending;      // single solve: the step of length alpha is not yet in the iterate and the residual
 };
 
 struct VLev {
@@ -149,6 +151,16 @@ __device__ __forceinline__ float2 diagonal(const float4* c, int w, int h, int x,
 
 __device__ __forceinline__ unsigned vblock() { return blockIdx.y * gridDim.x + blockIdx.x; }
 
+}  // namespace
+
+}  // namespace fsim
+
+#include "fs_viscosity_rows.hpp"
+
+namespace fsim {
+
+namespace {
+
 // ---- material and coefficients ----
 
 // FluidGridGPU's blend + pack (FluidGridGPU.cpp:173-218): rho = sum(m) / h^2,
@@ -175,19 +187,9 @@ __global__ __launch_bounds__(kVT) void k_vis_blend(int N, double area, int nl, i
     }
 }
 
-__global__ __launch_bounds__(kVT) void k_vis_material(int N, const double* material, float2* mat)
+// "viscosity coarse material" (ViscosityKernels.h:115-135): cell (x, y) of the level below F.
+__device__ __forceinline__ float2 coarse_material(const VLev& F, int x, int y)
 {
-    for (int i = blockIdx.x * kVT + threadIdx.x; i < N; i += gridDim.x * kVT)
-        mat[i] = make_float2((float)material[2 * i], (float)material[2 * i + 1]);
-}
-
-// "viscosity coarse material" (ViscosityKernels.h:115-135)
-__global__ __launch_bounds__(kVT) void k_vis_coarsen(VLev F, VLev C)
-{
-    const int x = blockIdx.x * kVX + (threadIdx.x & 63);
-    const int y = blockIdx.y * kVY + (threadIdx.x >> 6);
-    if (x >= C.w || y >= C.h)
-        return;
     float2 v = make_float2(0.0f, 0.0f);
     float n = 0.0f;
     for (int dy = 0; dy < 2; ++dy)
@@ -200,89 +202,52 @@ __global__ __launch_bounds__(kVT) void k_vis_coarsen(VLev F, VLev C)
                 n += 1.0f;
             }
         }
-    C.mat[y * C.w + x] = make_float2(v.x / n, v.y / n);
+    return make_float2(v.x / n, v.y / n);
 }
 
-// "viscosity coefficients" (ViscosityKernels.h:137-152)
-__global__ __launch_bounds__(kVT) void k_vis_coef(VLev L, float spacing)
+// "viscosity coefficients" (ViscosityKernels.h:137-152) of slot (x, y), from the materials m(cell) of its cells.
+template <class Material>
+__device__ __forceinline__ float4 slot_coefficients(const VLev& L, int x, int y, float spacing, Material m)
+{
+    auto at = [&](int cx, int cy) { return m(min(max(cx, 0), L.w - 1), min(max(cy, 0), L.h - 1)); };
+    const float2 c = at(x, y), left = at(x - 1, y), up = at(x, y - 1);
+    float vertex = 0.0f;
+    if (x > 0 && y > 0 && x < L.w && y < L.h)
+        vertex = 0.25f * (c.y + left.y + up.y + at(x - 1, y - 1).y);
+    const float half_area = 0.5f * spacing * spacing;
+    return make_float4(c.y, vertex, half_area * (c.x + left.x), half_area * (c.x + up.x));
+}
+
+// Materials and coefficients of the finest level (from the FP64 material) ...
+__global__ __launch_bounds__(kVT) void k_vis_finest(VLev L, const double* material, float spacing)
 {
     VIS_SLOT(L)
     if (!inside)
         return;
-    auto m = [&](int cx, int cy) { return L.mat[min(max(cy, 0), L.h - 1) * L.w + min(max(cx, 0), L.w - 1)]; };
-    const float2 c = m(x, y);
-    float vertex = 0.0f;
-    if (x > 0 && y > 0 && x < L.w && y < L.h)
-        vertex = 0.25f * (c.y + m(x - 1, y).y + m(x, y - 1).y + m(x - 1, y - 1).y);
-    const float half_area = 0.5f * spacing * spacing;
-    L.coef[p] = make_float4(c.y, vertex, half_area * (c.x + m(x - 1, y).x), half_area * (c.x + m(x, y - 1).x));
+    auto m = [&](int cx, int cy) {
+        const size_t i = 2 * ((size_t)cy * L.w + cx);
+        return make_float2((float)material[i], (float)material[i + 1]);
+    };
+    L.coef[p] = slot_coefficients(L, x, y, spacing, m);
+    if (x < L.w && y < L.h)
+        L.mat[y * L.w + x] = m(x, y);
+}
+
+// ... of a level from the one above it, the few materials a slot needs computed where they are used: one launch per
+// level instead of two ...
+__global__ __launch_bounds__(kVT) void k_vis_coarser(VLev F, VLev L, float spacing)
+{
+    VIS_SLOT(L)
+    if (!inside)
+        return;
+    L.coef[p] = slot_coefficients(L, x, y, spacing, [&](int cx, int cy) { return coarse_material(F, cx, cy); });
+    if (x < L.w && y < L.h)
+        L.mat[y * L.w + x] = coarse_material(F, x, y);
 }
 
 // ---- set-up of the correction system ----
 
-// "viscosity initial velocity and RHS" (ViscosityKernels.h:154-163): v0 on valid faces (FP32).
-__global__ __launch_bounds__(kVT) void k_vis_pack(VLev L, const double* u, const double* v, float2* v0)
-{
-    VIS_SLOT(L)
-    if (!inside)
-        return;
-    const int W = L.w, H = L.h;
-    const double su = u[min(y, H - 1) * (W + 1) + x];
-    const double sv = v[y * W + min(x, W - 1)];
-    v0[p] = make_float2(valid_u(W, H, x, y) ? (float)su : 0.0f, valid_v(W, H, x, y) ? (float)sv : 0.0f);
-}
-
-// r0 = M v0 - A v0 = -dt K v0 (the rhs of the correction system) and the mode-0 reduction:
-// r0 M^-1 r0, v0 M v0, sum of masses, non-finite flag (ViscosityKernels.h:395-470).
-__global__ __launch_bounds__(kVT) void k_vis_initial(VLev L, const float2* v0, float2* r0, float dt, double* partials)
-{
-    __shared__ double lds[kVT / 64];
-    VIS_SLOT(L)
-    double a = 0.0, b = 0.0, m = 0.0, bad = 0.0;
-    if (inside) {
-        const float4 c = L.coef[p];
-        const float2 q = product(L.coef, v0, L.w, L.h, x, y, dt);
-        const float2 s = v0[p];
-        float2 r;
-        r.x = valid_u(L.w, L.h, x, y) ? c.z * s.x - q.x : 0.0f;
-        r.y = valid_v(L.w, L.h, x, y) ? c.w * s.y - q.y : 0.0f;
-        r0[p] = r;
-        a = (double)r.x / c.z * r.x + (double)r.y / c.w * r.y;
-        b = (double)c.z * s.x * s.x + (double)c.w * s.y * s.y;
-        m = (double)c.z + (double)c.w;
-        if (!isfinite(a) || !isfinite(b) || !isfinite(m)) {
-            a = b = m = 0.0;
-            bad = 1.0;
-        }
-    }
-    const unsigned nb = gridDim.x * gridDim.y;
-    const double sa = block_sum<kVT>(a, lds);
-    const double sb = block_sum<kVT>(b, lds);
-    const double sm = block_sum<kVT>(m, lds);
-    const double sf = block_max<kVT>(bad, lds);
-    if (threadIdx.x == 0) {
-        partials[vblock()] = sa;
-        partials[nb + vblock()] = sb;
-        partials[2 * nb + vblock()] = sm;
-        partials[3 * nb + vblock()] = sf;
-    }
-}
-
-// ---- V-cycle ----
-
-// "viscosity true residual" on a level (ViscosityKernels.h:187-195)
-__global__ __launch_bounds__(kVT) void k_vis_residual(VLev L, const float2* b, const VisScalars* S)
-{
-    if (stopped(S))
-        return;
-    const float dt = S->dt;
-    VIS_SLOT(L)
-    if (!inside)
-        return;
-    const float2 q = product(L.coef, L.x, L.w, L.h, x, y, dt);
-    const float2 rhs = b[p];
-    L.r[p] = make_float2(valid_u(L.w, L.h, x, y) ? rhs.x - q.x : 0.0f, valid_v(L.w, L.h, x, y) ? rhs.y - q.y : 0.0f);
-}
+// ---- transfers of the batched solve ----
 
 // Face-location bilinear transfer (ViscosityKernels.h:286-316).
 __device__ __forceinline__ void transfer_location(int fx, int fy, int comp, int& bx, int& by, float& tx, float& ty)
@@ -318,432 +283,159 @@ __device__ float transfer_weight(int fx, int fy, int cx, int cy, int comp, int c
     return result;
 }
 
-// "viscosity transpose restriction" (ViscosityKernels.h:318-357): C.b = P^T F.r
-__global__ __launch_bounds__(kVT) void k_vis_restrict(VLev F, VLev C, const VisScalars* S)
-{
-    if (stopped(S))
-        return;
-    VIS_SLOT(C)
-    if (!inside)
-        return;
-    float val[2] = {0.0f, 0.0f};
-    for (int comp = 0; comp < 2; ++comp) {
-        if ((comp == 0 && (x == 0 || x == C.w || y == C.h)) || (comp == 1 && (y == 0 || y == C.h || x == C.w)))
-            continue;
-        const int ex = comp == 1 ? 2 : 1, ey = comp == 1 ? 1 : 2;
-        for (int dy = -1; dy <= ey; ++dy)
-            for (int dx = -1; dx <= ex; ++dx) {
-                const int qx = 2 * x + dx, qy = 2 * y + dy;
-                if (qx < 0 || qy < 0 || qx > F.w || qy > F.h)
-                    continue;
-                const float2 r = F.r[qy * (F.w + 1) + qx];
-                val[comp] += transfer_weight(qx, qy, x, y, comp, C.w, C.h) * (comp == 0 ? r.x : r.y);
-            }
-    }
-    C.b[p] = make_float2(val[0], val[1]);
-}
-
-// NS sweeps of the "viscosity symmetric smoother" (ViscosityKernels.h:214-236: damped Jacobi, weight 1/2 in
-// the reference's two sweeps per side; the weights of VisSmooth otherwise) fused on an LDS tile:
-// pre-smoothing from zero (result in L.x), or (POST) the "viscosity prolongation" F.x + P C.x on valid
-// faces (ViscosityKernels.h:359-391) followed by the sweeps (result in L.xn).  The tile holds an NS-slot
-// halo of coefficients, rhs and the starting solution, each slot loaded from its clamped position; sweep k
-// covers the tile less k + 1 rings, the last one the interior, and every stencil read maps through the same
-// clamp to the tile, so each sweep reads exactly the values a per-sweep kernel would read from the slot
-// field (results identical to one launch per sweep).
-constexpr int kSX = 32, kSY = 16;   // interior slots per workgroup
-
-template <bool POST, int NS>
-__global__ __launch_bounds__(kVT) void k_vis_smooth(VLev L, VLev C, const float2* b, const VisScalars* S,
-    const VisSmooth M)
-{
-    constexpr int LX = kSX + 2 * NS, LY = kSY + 2 * NS, LN = LX * LY;   // NS 2: 36 x 20, NS 6: 44 x 28
-    __shared__ float4 sc[LN];
-    __shared__ float2 sb[LN];
-    __shared__ float2 s0[LN];   // starting solution of the first sweep (POST: prolonged); even sweeps' input
-    __shared__ float2 s1[LN];   // odd sweeps' input
-    if (stopped(S))
-        return;
-    const float dt = S->dt;
-    const int w = L.w, h = L.h;
-    const int x0 = blockIdx.x * kSX - NS, y0 = blockIdx.y * kSY - NS;
-    const auto at = [=](int x, int y) { return (min(max(y, 0), h) - y0) * LX + (min(max(x, 0), w) - x0); };
-    for (int e = threadIdx.x; e < LN; e += kVT) {
-        const int gx = x0 + e % LX, gy = y0 + e / LX;
-        const int g = sidx(w, h, gx, gy);
-        sc[e] = L.coef[g];
-        sb[e] = b[g];
-        if (POST)
-            s0[e] = L.x[g];
-    }
-    __syncthreads();
-    if (POST) {
-        // prolongation on every in-field slot of the tile (interior and every halo ring)
-        for (int e = threadIdx.x; e < LN; e += kVT) {
-            const int x = x0 + e % LX, y = y0 + e / LX;
-            if (x < 0 || y < 0 || x > w || y > h)
-                continue;
-            const float2 sv = s0[e];
-            float val[2] = {sv.x, sv.y};
-            for (int comp = 0; comp < 2; ++comp) {
-                int bx, by;
-                float tx, ty;
-                transfer_location(x, y, comp, bx, by, tx, ty);
-                for (int dy = 0; dy < 2; ++dy)
-                    for (int dx = 0; dx < 2; ++dx) {
-                        int px, py;
-                        coarse_point(bx + dx, by + dy, comp, C.w, C.h, px, py);
-                        const float2 c = C.x[py * (C.w + 1) + px];
-                        val[comp] +=
-                            (dx == 1 ? tx : 1.0f - tx) * (dy == 1 ? ty : 1.0f - ty) * (comp == 0 ? c.x : c.y);
-                    }
-            }
-            s0[e] = make_float2(valid_u(w, h, x, y) ? val[0] : 0.0f, valid_v(w, h, x, y) ? val[1] : 0.0f);
-        }
-        __syncthreads();
-    }
-    // sweeps 0..NS-2 on the tile less k + 1 rings
-#pragma unroll
-    for (int k = 0; k + 1 < NS; ++k) {
-        const float wk = M.w[POST ? NS - 1 - k : k];
-        const float2* src = (k & 1) ? s1 : s0;
-        float2* dst = (k & 1) ? s0 : s1;
-        const int RX = LX - 2 * (k + 1), RY = LY - 2 * (k + 1);
-        for (int e = threadIdx.x; e < RX * RY; e += kVT) {
-            const int x = x0 + k + 1 + e % RX, y = y0 + k + 1 + e / RX;
-            if (x < 0 || y < 0 || x > w || y > h)
-                continue;
-            const int i = at(x, y);
-            const float2 d = diagonal_at(sc, at, x, y, dt);
-            const float2 rhs = sb[i];
-            float2 v;
-            if (!POST && k == 0) {
-                v.x = wk * rhs.x / d.x;
-                v.y = wk * rhs.y / d.y;
-            } else {
-                const float2 q = product_at(sc, src, at, w, h, x, y, dt);
-                const float2 sv = src[i];
-                v.x = sv.x + wk * (rhs.x - q.x) / d.x;
-                v.y = sv.y + wk * (rhs.y - q.y) / d.y;
-            }
-            dst[i] = make_float2(valid_u(w, h, x, y) ? v.x : 0.0f, valid_v(w, h, x, y) ? v.y : 0.0f);
-        }
-        __syncthreads();
-    }
-    // the last sweep on the interior, written out
-    const float wl = M.w[POST ? 0 : NS - 1];
-    const float2* src = ((NS - 1) & 1) ? s1 : s0;
-    float2* out = POST ? L.xn : L.x;
-    for (int e = threadIdx.x; e < kSX * kSY; e += kVT) {
-        const int x = x0 + NS + e % kSX, y = y0 + NS + e / kSX;
-        if (x > w || y > h)
-            continue;
-        const int i = at(x, y);
-        const float2 d = diagonal_at(sc, at, x, y, dt);
-        const float2 rhs = sb[i];
-        const float2 q = product_at(sc, src, at, w, h, x, y, dt);
-        const float2 sv = src[i];
-        float2 v;
-        v.x = sv.x + wl * (rhs.x - q.x) / d.x;
-        v.y = sv.y + wl * (rhs.y - q.y) / d.y;
-        out[y * (w + 1) + x] = make_float2(valid_u(w, h, x, y) ? v.x : 0.0f, valid_v(w, h, x, y) ? v.y : 0.0f);
-    }
-}
-
-// "viscosity shared coarse solve" (ViscosityKernels.h:242-282): 16 Jacobi sweeps from zero in LDS.
 constexpr int kCoarseSlots = 256;
-__global__ __launch_bounds__(kCoarseSlots) void k_vis_coarse(VLev L, const float2* b, const VisScalars* S)
-{
-    __shared__ float2 vel[kCoarseSlots];
-    __shared__ float4 cof[kCoarseSlots];
-    if (stopped(S))
-        return;
-    const float dt = S->dt;
-    const int lane = threadIdx.x;
-    const int stride = L.w + 1;
-    const int n = stride * (L.h + 1);
-    const int x = lane % stride, y = lane / stride;
-    const int src = lane < n ? lane : n - 1;
-    vel[lane] = make_float2(0.0f, 0.0f);
-    cof[lane] = L.coef[src];
-    const float2 rhs = b[src];
-    __syncthreads();
-    for (int sweep = 0; sweep < 16; ++sweep) {
-        float2 v = make_float2(0.0f, 0.0f);
-        if (lane < n) {
-            const float2 d = diagonal(cof, L.w, L.h, x, y, dt);
-            const float2 q = product(cof, vel, L.w, L.h, x, y, dt);
-            const float2 s = vel[lane];
-            v.x = valid_u(L.w, L.h, x, y) ? s.x + 0.5f * (rhs.x - q.x) / d.x : 0.0f;
-            v.y = valid_v(L.w, L.h, x, y) ? s.y + 0.5f * (rhs.y - q.y) / d.y : 0.0f;
-        }
-        __syncthreads();
-        vel[lane] = v;
-        __syncthreads();
-    }
-    if (lane < n)
-        L.x[lane] = vel[lane];
-}
-
-// ---- CG ----
-
-// mode-1 reduction: r . z, r M^-1 r (ViscosityKernels.h:395-470)
-__global__ __launch_bounds__(kVT) void k_vis_rz(VLev L, const float2* r, const float2* z, const VisScalars* S,
-    double* partials)
-{
-    __shared__ double lds[kVT / 64];
-    if (stopped(S))
-        return;
-    VIS_SLOT(L)
-    double a = 0.0, b = 0.0, bad = 0.0;
-    if (inside) {
-        const float4 c = L.coef[p];
-        const float2 rr = r[p], zz = z[p];
-        a = (double)rr.x * zz.x + (double)rr.y * zz.y;
-        b = (double)rr.x / c.z * rr.x + (double)rr.y / c.w * rr.y;
-        if (!isfinite(a) || !isfinite(b)) {
-            a = b = 0.0;
-            bad = 1.0;
-        }
-    }
-    const unsigned nb = gridDim.x * gridDim.y;
-    const double sa = block_sum<kVT>(a, lds);
-    const double sb = block_sum<kVT>(b, lds);
-    const double sf = block_max<kVT>(bad, lds);
-    if (threadIdx.x == 0) {
-        partials[vblock()] = sa;
-        partials[nb + vblock()] = sb;
-        partials[3 * nb + vblock()] = sf;
-    }
-}
-
-__global__ __launch_bounds__(kVT) void k_vis_direction(VLev L, const float2* z, float2* d, const VisScalars* S)
-{
-    if (stopped(S))
-        return;
-    VIS_SLOT(L)
-    if (!inside)
-        return;
-    const float2 zz = z[p];
-    if (S->steps > 0) {
-        const float beta = (float)S->beta;
-        const float2 dd = d[p];
-        d[p] = make_float2(zz.x + beta * dd.x, zz.y + beta * dd.y);
-    } else {
-        d[p] = zz;
-    }
-}
-
-// q = A d and the mode-2 reduction d . q
-__global__ __launch_bounds__(kVT) void k_vis_apply(VLev L, const float2* d, float2* q, const VisScalars* S,
-    double* partials)
-{
-    __shared__ double lds[kVT / 64];
-    if (stopped(S))
-        return;
-    const float dt = S->dt;
-    VIS_SLOT(L)
-    double a = 0.0, bad = 0.0;
-    if (inside) {
-        const float2 v = product(L.coef, d, L.w, L.h, x, y, dt);
-        q[p] = v;
-        const float2 dd = d[p];
-        a = (double)dd.x * v.x + (double)dd.y * v.y;
-        if (!isfinite(a)) {
-            a = 0.0;
-            bad = 1.0;
-        }
-    }
-    const unsigned nb = gridDim.x * gridDim.y;
-    const double sa = block_sum<kVT>(a, lds);
-    const double sf = block_max<kVT>(bad, lds);
-    if (threadIdx.x == 0) {
-        partials[vblock()] = sa;
-        partials[3 * nb + vblock()] = sf;
-    }
-}
-
-__global__ __launch_bounds__(kVT) void k_vis_update(VLev L, float2* xs, float2* r, const float2* d, const float2* q,
-    const VisScalars* S)
-{
-    if (stopped(S))
-        return;
-    VIS_SLOT(L)
-    if (!inside)
-        return;
-    const float alpha = (float)S->alpha;
-    const float2 dd = d[p], qq = q[p], xx = xs[p], rr = r[p];
-    xs[p] = make_float2(xx.x + alpha * dd.x, xx.y + alpha * dd.y);
-    r[p] = make_float2(rr.x - alpha * qq.x, rr.y - alpha * qq.y);
-}
-
-// recomputed residual t = M v0 - A x and t M^-1 t (mode 3)
-__global__ __launch_bounds__(kVT) void k_vis_truth(VLev L, const float2* v0, const float2* xs, float2* t, float dt,
-    double* partials, const VisScalars* S)
-{
-    __shared__ double lds[kVT / 64];
-    if (S && S->done != 0)
-        return;
-    VIS_SLOT(L)
-    double a = 0.0, bad = 0.0;
-    if (inside) {
-        const float4 c = L.coef[p];
-        const float2 q = product(L.coef, xs, L.w, L.h, x, y, dt);
-        const float2 s0 = v0[p];
-        float2 v;
-        v.x = valid_u(L.w, L.h, x, y) ? c.z * s0.x - q.x : 0.0f;
-        v.y = valid_v(L.w, L.h, x, y) ? c.w * s0.y - q.y : 0.0f;
-        t[p] = v;
-        a = (double)v.x / c.z * v.x + (double)v.y / c.w * v.y;
-        if (!isfinite(a)) {
-            a = 0.0;
-            bad = 1.0;
-        }
-    }
-    const unsigned nb = gridDim.x * gridDim.y;
-    const double sa = block_sum<kVT>(a, lds);
-    const double sf = block_max<kVT>(bad, lds);
-    if (threadIdx.x == 0) {
-        partials[vblock()] = sa;
-        partials[3 * nb + vblock()] = sf;
-    }
-}
+constexpr int kFinishThreads = 256;
 
 enum VisFinish : int { kVisInitial = 0, kVisRz, kVisDq, kVisTruth };
 
-// One workgroup reduces the partials in block order and updates the scalar block
-// (the reference's "viscosity CG scalars", ViscosityKernels.h:490-535).
-__global__ __launch_bounds__(kVT) void k_vis_finish(VisScalars* S, const double* partials, int nb, int op, double tol2,
-    float dt)
+// One workgroup reduces the partials in block order and updates the scalar block (the reference's "viscosity CG
+// scalars", ViscosityKernels.h:490-535).  After the recomputed residual of a batch of `batch` iterations (kVisTruth)
+// it also takes the decision (ViscositySolverGPU.cpp:264-294, on the device so that batches queue without a
+// read-back): breakdown, convergence of the recomputed residual, a restart when only the recurrence claims
+// convergence, and the iteration budget (`maximum` < 0: none).  A batch queued after the solve ended changes
+// nothing (its kernels exit at once); the first such batch marks the converged result as unpacked.
+template <int OP>
+__global__ __launch_bounds__(kFinishThreads) void k_vis_finish(VisScalars* S, const double* partials, int nb,
+    double tol2, float dt, int batch, int maximum)
 {
-    __shared__ double lds[kVT / 64];
-    if ((op == kVisRz || op == kVisDq) && stopped(S))
+    constexpr int NC = OP == kVisInitial ? 4 : OP == kVisRz ? 3 : 2;
+    __shared__ double lds[NC * (kFinishThreads / 64)];
+    double v[NC];
+    Partials<kFinishThreads, NC> sums;
+    sums.load(partials, nb);
+    const double target = S->target, rz = S->rz;
+    const double rnorm = S->rnorm;
+    const int bad = S->bad, done = S->done, steps = S->steps;
+    int iterations = S->iterations;
+    if ((OP == kVisRz || OP == kVisDq) && (bad != 0 || rnorm <= target || done != 0))
         return;
-    if (op == kVisTruth && S->done != 0)
+    if (OP == kVisTruth && done != 0) {
+        if (threadIdx.x == 0 && done == 1)
+            S->done = 4;
         return;
-    const double a = finish_sum<kVT>(partials, nb, 1, 0, lds);
-    const double b = (op == kVisInitial || op == kVisRz) ? finish_sum<kVT>(partials + nb, nb, 1, 0, lds) : 0.0;
-    const double m = op == kVisInitial ? finish_sum<kVT>(partials + 2 * nb, nb, 1, 0, lds) : 0.0;
-    const double f = finish_max<kVT>(partials + 3 * nb, nb, 1, 0, lds);
+    }
+    sums.finish(partials, nb, v, lds);
     if (threadIdx.x != 0)
         return;
-    VisScalars s = *S;
-    const bool bad = f != 0.0;
-    switch (op) {
-    case kVisInitial:
-        s = VisScalars{};
-        s.dt = dt;
-        s.energy = b;
-        s.mass_sum = m;
-        s.target = tol2 * b + 1e-12 * m;
-        s.rnorm = a;
-        s.truth = a;
-        s.bad = bad ? 1 : 0;
-        s.done = s.bad ? 6 : (s.rnorm <= s.target ? 5 : 0);
-        break;
-    case kVisRz:
-        s.bad |= bad ? 1 : 0;
-        s.rnorm = b;
-        if (s.rnorm > s.target && !s.bad) {
-            if (a <= 0.0 || !isfinite(a)) {
-                s.bad = 1;
-            } else {
-                s.beta = s.steps > 0 ? a / s.rz : 0.0;
-                s.rz = a;
-            }
+    const double a = v[0];
+    const bool flagged = v[NC - 1] != 0.0;
+    if constexpr (OP == kVisInitial) {
+        const double limit = tol2 * v[1] + 1e-12 * v[2];
+        *S = VisScalars{};
+        S->dt = dt;
+        S->energy = v[1];
+        S->mass_sum = v[2];
+        S->target = limit;
+        S->rnorm = a;
+        S->truth = a;
+        S->bad = flagged ? 1 : 0;
+        S->done = flagged ? 6 : (a <= limit ? 5 : 0);
+    } else if constexpr (OP == kVisRz) {
+        // the descent has taken the pending step, or the restart's residual
+        S->pending = 0;
+        S->restart = 0;
+        S->rnorm = v[1];
+        if (flagged || (v[1] > target && (a <= 0.0 || !isfinite(a)))) {
+            S->bad = 1;
+        } else if (v[1] > target) {
+            S->beta = steps > 0 ? a / rz : 0.0;
+            S->rz = a;
         }
-        break;
-    case kVisDq:
-        if (bad || a <= 0.0 || !isfinite(a)) {
-            s.bad = 1;
+    } else if constexpr (OP == kVisDq) {
+        if (flagged || a <= 0.0 || !isfinite(a)) {
+            S->bad = 1;
         } else {
-            s.alpha = s.rz / a;
-            s.steps += 1;
+            S->alpha = rz / a;
+            S->steps = steps + 1;
+            S->pending = 1;
         }
-        break;
-    default:  // kVisTruth
-        s.truth = bad ? INFINITY : a;
-        if (bad)
-            s.bad = 1;
-        break;
-    }
-    *S = s;
-}
-
-// Restart from the recomputed residual ("viscosity refresh residual", ViscosityKernels.h:607-620), when
-// k_vis_decide asked for it.
-__global__ void k_vis_refresh(VisScalars* S)
-{
-    if (threadIdx.x == 0 && blockIdx.x == 0) {
-        VisScalars s = *S;
-        if (!s.restart)
-            return;
-        s.rnorm = s.truth;
-        s.rz = s.alpha = s.beta = 0.0;
-        s.steps = 0;
-        s.restart = 0;
-        *S = s;
-    }
-}
-
-// The decision after a batch of `batch` iterations and the recomputed residual (ViscositySolverGPU.cpp:
-// 264-294, taken on the device so that batches queue without a read-back): breakdown, convergence of the
-// recomputed residual, a restart when only the recurrence claims convergence, and the iteration budget
-// (`maximum` < 0: none).  A batch queued after the solve ended changes nothing (its kernels exit at once);
-// the first such batch marks the converged result as unpacked.
-__global__ void k_vis_decide(VisScalars* S, int batch, int maximum)
-{
-    if (threadIdx.x != 0 || blockIdx.x != 0)
-        return;
-    VisScalars s = *S;
-    if (s.done != 0) {
-        if (s.done == 1) {
-            s.done = 4;
-            *S = s;
-        }
-        return;
-    }
-    s.iterations += batch;
-    if (s.bad) {
-        s.done = 2;
-    } else if (s.truth <= s.target) {
-        s.done = 1;
     } else {
-        if (s.rnorm <= s.target)
-            s.restart = 1;
-        if (maximum >= 0 && s.iterations >= maximum)
-            s.done = 3;
+        const double truth = flagged ? INFINITY : a;
+        S->truth = truth;
+        iterations += batch;
+        S->iterations = iterations;
+        if (flagged || bad) {
+            S->bad = 1;
+            S->done = 2;
+        } else if (truth <= target) {
+            S->done = 1;
+        } else {
+            if (rnorm <= target) {
+                // "viscosity refresh residual" (ViscosityKernels.h:607-620)
+                S->restart = 1;
+                S->rnorm = truth;
+                S->rz = S->beta = 0.0;
+                S->steps = 0;
+            }
+            if (maximum >= 0 && iterations >= maximum)
+                S->done = 3;
+        }
     }
-    *S = s;
 }
 
-// r = the recomputed residual t, when k_vis_decide asked for a restart.
-__global__ __launch_bounds__(kVT) void k_vis_restart_copy(const VisScalars* S, float2* r, const float2* t, size_t n)
+// After the decision on a batch.  Converged: "viscosity staggered result" (ViscosityKernels.h:165-185), every face
+// of u and v takes the solution x + alpha d (walls 0), once.  The output is the FP32 iterate, as in the reference:
+// writing u0 + (x - v0) instead would keep the FP32 rounding noise of u0, which the stiff operator dt K amplifies in
+// the residual.  Restart: r becomes the recomputed residual t and x takes its pending step.
+__global__ __launch_bounds__(kVT) void k_vis_land(VLev L, float2* xs, const float2* d, float2* r, const float2* t,
+    double* u, double* v, const VisScalars* S)
 {
-    if (!S->restart)
+    const bool converged = S->done == 1, restart = S->restart != 0 && S->done == 0;
+    if (!converged && !restart)
         return;
-    for (size_t i = (size_t)blockIdx.x * kVT + threadIdx.x; i < n; i += (size_t)gridDim.x * kVT)
-        r[i] = t[i];
+    VIS_SLOT(L)
+    if (!inside)
+        return;
+    float2 c = xs[p];
+    if (S->pending) {
+        const float alpha = (float)S->alpha;
+        const float2 dd = d[p];
+        c = make_float2(c.x + alpha * dd.x, c.y + alpha * dd.y);
+    }
+    if (restart) {
+        xs[p] = c;
+        r[p] = t[p];
+        return;
+    }
+    if (y < L.h)
+        u[y * (L.w + 1) + x] = valid_u(L.w, L.h, x, y) ? (double)c.x : 0.0;
+    if (x < L.w)
+        v[y * L.w + x] = valid_v(L.w, L.h, x, y) ? (double)c.y : 0.0;
 }
 
-// "viscosity staggered result" (ViscosityKernels.h:165-185): every face of u and v takes the solution
-// (walls 0).  The output is the FP32 iterate, as in the reference: writing u0 + (x - v0) instead would
-// keep the FP32 rounding noise of u0, which the stiff operator dt K amplifies in the residual.
-// S (single solve): only once k_vis_decide has found the solve converged, and only the first time.
-__global__ __launch_bounds__(kVT) void k_vis_unpack(int W, int H, const float2* xs, double* u, double* v,
-    const VisScalars* S)
+// A grid of one level (at most 64 cells): the pending step and the sums that k_vis_down and k_vis_up take with them.
+__global__ __launch_bounds__(kVT) void k_vis_step(VLev L, VisStep io, const VisScalars* S)
 {
-    if (S && S->done != 1)
+    if (stopped(S))
         return;
-    const int x = blockIdx.x * kVX + (threadIdx.x & 63);
-    const int y = blockIdx.y * kVY + (threadIdx.x >> 6);
-    if (x <= W && y < H) {
-        const int i = y * (W + 1) + x;
-        u[i] = valid_u(W, H, x, y) ? (double)xs[i].x : 0.0;
+    VIS_SLOT(L)
+    if (!inside)
+        return;
+    float2 r = io.r[p];
+    if (step_pending(S)) {
+        const float alpha = (float)S->alpha;
+        const float2 dd = io.d[p], qq = io.q[p], xx = io.x[p];
+        io.x[p] = make_float2(xx.x + alpha * dd.x, xx.y + alpha * dd.y);
+        r = make_float2(r.x - alpha * qq.x, r.y - alpha * qq.y);
     }
-    if (x < W && y <= H) {
-        v[y * W + x] = valid_v(W, H, x, y) ? (double)xs[y * (W + 1) + x].y : 0.0;
+    io.r_new[p] = r;
+}
+
+__global__ __launch_bounds__(kVT) void k_vis_rz(VLev L, const float2* r, const VisScalars* S, double* partials)
+{
+    __shared__ double lds[3 * (kVT / 64)];
+    if (stopped(S))
+        return;
+    VIS_SLOT(L)
+    double v[3] = {0.0, 0.0, 0.0};
+    if (inside) {
+        const float4 c = L.coef[p];
+        add_rz(c.z, c.w, r[p], L.x[p], v);
     }
+    block_sums<kVT, 3>(v, lds);
+    if (threadIdx.x == 0)
+        for (int i = 0; i < 3; ++i)
+            partials[3 * vblock() + i] = v[i];
 }
 
 inline dim3 slot_grid(int w, int h) { return dim3((w + 1 + kVX - 1) / kVX, (h + 1 + kVY - 1) / kVY); }
@@ -942,7 +634,7 @@ __device__ void bv_prolong(const VLev& F, const VLev& C)
     __syncthreads();
 }
 
-// 16 Jacobi sweeps from zero on the coarsest level (k_vis_coarse), slots in LDS.
+// 16 Jacobi sweeps from zero on the coarsest level (ViscosityKernels.h:242-282), slots in LDS.
 __device__ void bv_coarse(const VLev& L, const float2* b, float dt, float2* vel, float4* cof)
 {
     const int lane = threadIdx.x;
@@ -990,41 +682,6 @@ __device__ void bv_cycle(const BatchVisDesc& D, float dt, float2* vel, float4* c
         const float2* b = l == 0 ? (const float2*)D.r : D.lev[l].b;
         bv_prolong(D.lev[l], D.lev[l + 1]);
         bv_post(D.lev[l], b, dt, D.M);
-    }
-}
-
-// The coarse end of a V-cycle in one workgroup: levels whose sweeps are too small to fill the device cost
-// more in launches than in work, so cycle() hands every level from the first with at most kVisTailSlots
-// slots down to the coarsest to this kernel (1024: one level of 1196 slots more made a 1417 x 787 solve
-// slower, one of 4590 slots 20% slower) (the same sweeps, restriction, Jacobi coarse solve and
-// prolongation as the per-level kernels, each a workgroup-strided loop).  b0 is the first level's rhs;
-// the result lands in lev[0].x.
-constexpr int kVisTailSlots = 1024;
-
-struct VisTail {
-    int levels;
-    VLev lev[kMaxVisLevels];
-    VisSmooth M;
-};
-
-__global__ __launch_bounds__(kBVT) void k_vis_tail(const VisTail T, const float2* b0, const VisScalars* S)
-{
-    __shared__ float2 vel[kCoarseSlots];
-    __shared__ float4 cof[kCoarseSlots];
-    if (stopped(S))
-        return;
-    const float dt = S->dt;
-    const int nl = T.levels;
-    for (int l = 0; l + 1 < nl; ++l) {
-        const float2* b = l == 0 ? b0 : T.lev[l].b;
-        bv_pre(T.lev[l], b, dt, T.M);
-        bv_residual_restrict(T.lev[l], b, T.lev[l + 1], dt);
-    }
-    bv_coarse(T.lev[nl - 1], nl == 1 ? b0 : T.lev[nl - 1].b, dt, vel, cof);
-    for (int l = nl - 2; l >= 0; --l) {
-        const float2* b = l == 0 ? b0 : T.lev[l].b;
-        bv_prolong(T.lev[l], T.lev[l + 1]);
-        bv_post(T.lev[l], b, dt, T.M);
     }
 }
 
@@ -1163,7 +820,7 @@ __global__ __launch_bounds__(kBVT) void k_batch_vis(const BatchVisDesc* descs)
             }
             if (truth <= target) {
                 status = 0;
-                // the staggered result (k_vis_unpack)
+                // the staggered result (k_vis_land)
                 for (int e = threadIdx.x; e < n0; e += kBVT) {
                     int x, y;
                     slot_xy(e, W, x, y);
@@ -1263,7 +920,8 @@ struct ViscositySolver {
             place(L->b, ns);
             place(L->x, ns);
             place(L->xn, ns);
-            place(L->r, ns);
+            if (!arena || levels.count == 1)   // residuals of the batched solve; the finest level's is a direction buffer
+                place(L->r, ns);
             if (w * h <= 64)
                 break;
             w = (w + 1) / 2;
@@ -1278,7 +936,10 @@ struct ViscositySolver {
         place(t, ns);
         if (!arena)
             place(material, 2 * (size_t)W * H);
-        place(partials, 4 * (size_t)std::max(slot_blocks(W, H), 1u));
+        // four components a tile of k_vis_apply, three a tile of k_vis_up (60 x 12 slots or 52 x 20 at the least) or,
+        // with one level, a block of k_vis_rz
+        place(partials, std::max(4 * (size_t)apply_tiles_x() * apply_tiles_y(),
+            3 * (levels.count > 1 ? (size_t)tiles(W, 52) * tiles(H, 12) : (size_t)slot_blocks(W, H))));
         place(S, 1);
         if (!arena)
             pinned = (VisScalars*)pinned_alloc(sizeof(VisScalars));
@@ -1296,8 +957,6 @@ struct ViscositySolver {
         return VLev{L.w, L.h, L.coef.p, L.mat.p, L.b.p, L.x.p, L.xn.p, L.r.p};
     }
 
-    void swap_x(int l) { std::swap(levels[l]->x.p, levels[l]->xn.p); }
-
     VisScalars read(hipStream_t st)
     {
         VisScalars* slot = pinned ? pinned : &landing;
@@ -1306,23 +965,27 @@ struct ViscositySolver {
         return *slot;
     }
 
-    void finish(hipStream_t st, int nb, int op, double tol2, float dt = 0.0f)
+    template <int OP> void finish(hipStream_t st, int nb, double tol2 = 0.0, float dt = 0.0f, int batch = 0,
+        int maximum = 0)
     {
-        hipLaunchKernelGGL(k_vis_finish, dim3(1), dim3(kVT), 0, st, S.p, partials.p, nb, op, tol2, dt);
+        hipLaunchKernelGGL(k_vis_finish<OP>, dim3(1), dim3(kFinishThreads), 0, st, S.p, partials.p, nb, tol2, dt,
+            batch, maximum);
     }
 
-    // cycle (ViscositySolverGPU.cpp:134-167); the result is levels[l]->x.  Every level swaps its x / xn
-    // pair once per cycle, so four cycles leave the pointers where they started.
-    // First level of the one-workgroup tail (k_vis_tail): the first level below the finest with at most
-    // kVisTailSlots slots, when at least one level lies between it and the coarsest; else none (-1).
+    // First level of the one-workgroup tail: the first level below the finest with at most kVisTailSlots slots
+    // (a thread each) and at most kVisTailLevels levels from there on; a grid of one level is its own tail.
     int tail_level() const
     {
         const int nl = (int)levels.size();
-        for (int l = 1; l + 1 < nl; ++l)
-            if ((size_t)(levels[l]->w + 1) * (levels[l]->h + 1) <= (size_t)kVisTailSlots)
-                return nl - l <= kMaxVisLevels ? l : -1;
-        return -1;
+        int l = nl > 1 ? 1 : 0;
+        while (l + 1 < nl && (slots(l) > (size_t)kVisTailSlots || nl - l > kVisTailLevels))
+            ++l;
+        return l;
     }
+    size_t slots(int l) const { return (size_t)(levels[l]->w + 1) * (levels[l]->h + 1); }
+
+    // Where a level's solution lies after its way up.
+    float2* solution(int l) { return l >= tail_level() ? levels[l]->x.p : levels[l]->xn.p; }
 
     // Smoothing weights of every level (fs_set_viscosity_smoother): the reference's two sweeps of weight 1/2,
     // or 2, 4 or 6 Chebyshev-weighted sweeps, 1 / (2.125 + 1.875 cos(pi (k + 1/2) / n)) rounded to float --
@@ -1348,80 +1011,149 @@ struct ViscositySolver {
         drop_batch_graph();   // the captured launches carry the weights
     }
 
-    template <bool POST> void launch_smooth(hipStream_t st, dim3 g2, const VLev& L, const VLev& C, const float2* b)
+    // Eight wavefronts of 2, 4 or 6 rows.  Fewer rows are more tiles and a shorter chain in each, more rows less halo:
+    // with two sweeps 2 rows are best on small levels (641 x 363 solve 71.1 us per iteration against 78.7 with 4
+    // below its finest level), 4 on large ones (2048^2 267 against 288); with four sweeps, whose halo leaves 2 rows nothing to own, 4
+    // throughout; with six 6 on large ones (2048^2 505 against 530, 641 x 363 137 against 133).  16 wavefronts of 4
+    // rows leave a compute unit one tile, which nothing overlaps: 304 us at 2048^2 with two sweeps.
+    int tile_rows(int l) const
+    {
+        if (smooth.sweeps == 2)
+            return slots(l) < ((size_t)1 << 19) ? 2 : 4;
+        return smooth.sweeps == 6 && slots(l) >= ((size_t)1 << 20) ? 6 : 4;
+    }
+
+    // Tiles of OX x OY slots over the slots whose coarse images exist (the way down writes every coarse slot).
+    static int tiles(int n, int o) { return (2 * ((n + 1) / 2) + 1 + o - 1) / o; }
+
+    template <int NS, int NW, int R, bool TOP> void launch_down(hipStream_t st, int l, const VisStep& io)
+    {
+        const VLev L = view(l);
+        const int gx = tiles(L.w, 64 - 2 * (NS + 2)), gy = tiles(L.h, NW * R - 2 * (NS + 2));
+        hipLaunchKernelGGL((k_vis_down<NS, NW, R, TOP>), dim3(gx * gy), dim3(NW * 64), 0, st, L, view(l + 1), io, S.p,
+            smooth, gx, gy);
+    }
+
+    template <int NS, int NW, int R, bool TOP> int launch_up(hipStream_t st, int l, const float2* b)
+    {
+        const VLev L = view(l);
+        const int gx = tiles(L.w, 64 - 2 * NS), gy = tiles(L.h, NW * R - 2 * NS);
+        hipLaunchKernelGGL((k_vis_up<NS, NW, R, TOP>), dim3(gx * gy), dim3(NW * 64), 0, st, L, view(l + 1),
+            (const float2*)solution(l + 1), b, S.p, smooth, gx, gy, partials.p);
+        return gx * gy;
+    }
+
+    template <int NS, bool TOP> void down_sweeps(hipStream_t st, int l, const VisStep& io)
+    {
+        constexpr int other = NS == 2 ? 2 : NS == 6 ? 6 : 4;
+        if (tile_rows(l) == 4)
+            launch_down<NS, 8, 4, TOP>(st, l, io);
+        else
+            launch_down<NS, 8, other, TOP>(st, l, io);
+    }
+
+    template <int NS, bool TOP> int up_sweeps(hipStream_t st, int l, const float2* b)
+    {
+        constexpr int other = NS == 2 ? 2 : NS == 6 ? 6 : 4;
+        return tile_rows(l) == 4 ? launch_up<NS, 8, 4, TOP>(st, l, b) : launch_up<NS, 8, other, TOP>(st, l, b);
+    }
+
+    template <bool TOP> void down(hipStream_t st, int l, const VisStep& io)
     {
         if (smooth.sweeps == 6)
-            hipLaunchKernelGGL((k_vis_smooth<POST, 6>), g2, dim3(kVT), 0, st, L, C, b, S.p, smooth);
+            down_sweeps<6, TOP>(st, l, io);
         else if (smooth.sweeps == 4)
-            hipLaunchKernelGGL((k_vis_smooth<POST, 4>), g2, dim3(kVT), 0, st, L, C, b, S.p, smooth);
+            down_sweeps<4, TOP>(st, l, io);
         else
-            hipLaunchKernelGGL((k_vis_smooth<POST, 2>), g2, dim3(kVT), 0, st, L, C, b, S.p, smooth);
+            down_sweeps<2, TOP>(st, l, io);
     }
 
-    void cycle(hipStream_t st, int l, const float2* b)
+    template <bool TOP> int up(hipStream_t st, int l, const float2* b)
     {
-        VLev L = view(l);
-        if (l + 1 == (int)levels.size()) {
-            hipLaunchKernelGGL(k_vis_coarse, dim3(1), dim3(kCoarseSlots), 0, st, L, b, S.p);
-            return;
-        }
-        if (l == tail_level()) {
-            // the tail leaves each of its levels' results in x: no swaps there
-            VisTail T{};
-            T.levels = (int)levels.size() - l;
-            for (int k = 0; k < T.levels; ++k)
-                T.lev[k] = view(l + k);
-            T.M = smooth;
-            hipLaunchKernelGGL(k_vis_tail, dim3(1), dim3(kBVT), 0, st, T, b, S.p);
-            return;
-        }
-        const dim3 g = slot_grid(L.w, L.h);
-        const dim3 g2((L.w + 1 + kSX - 1) / kSX, (L.h + 1 + kSY - 1) / kSY);
-        // pre-smoothing: every sweep from zero in one launch (the result lands in L.x, as after an even
-        // number of swaps)
-        launch_smooth<false>(st, g2, L, L, b);
-        hipLaunchKernelGGL(k_vis_residual, g, dim3(kVT), 0, st, L, b, S.p);
-        VLev C = view(l + 1);
-        hipLaunchKernelGGL(k_vis_restrict, slot_grid(C.w, C.h), dim3(kVT), 0, st, L, C, S.p);
-        cycle(st, l + 1, C.b);
-        C = view(l + 1);
-        // prolongation + every sweep in one launch into L.xn: one swap, as after the odd number of the
-        // per-sweep kernels
-        launch_smooth<true>(st, g2, L, C, b);
-        swap_x(l);
+        if (smooth.sweeps == 6)
+            return up_sweeps<6, TOP>(st, l, b);
+        if (smooth.sweeps == 4)
+            return up_sweeps<4, TOP>(st, l, b);
+        return up_sweeps<2, TOP>(st, l, b);
     }
 
-    // One CG iteration (ViscositySolverGPU.cpp:238-262): V-cycle, r.z and beta, direction, A d and alpha,
-    // update of the iterate `delta` and the residual.
-    void iteration(hipStream_t st, float2* delta)
+    void tail(hipStream_t st, int l, const float2* b)
     {
-        const VLev L0 = view(0);
-        const dim3 g0 = slot_grid(W, H);
-        const int nb = (int)slot_blocks(W, H);
-        cycle(st, 0, r.p);
-        const VLev Lc = view(0);
-        hipLaunchKernelGGL(k_vis_rz, g0, dim3(kVT), 0, st, Lc, (const float2*)r.p, (const float2*)Lc.x, S.p,
+        VisTail T{};
+        const int n = (int)levels.size() - l;
+        for (int k = 0; k < n; ++k)
+            T.lev[k] = view(l + k);
+        T.M = smooth;
+        switch (n) {
+        case 1: hipLaunchKernelGGL(k_vis_tail<1>, dim3(1), dim3(kVisTailSlots), 0, st, T, b, S.p); break;
+        case 2: hipLaunchKernelGGL(k_vis_tail<2>, dim3(1), dim3(kVisTailSlots), 0, st, T, b, S.p); break;
+        case 3: hipLaunchKernelGGL(k_vis_tail<3>, dim3(1), dim3(kVisTailSlots), 0, st, T, b, S.p); break;
+        default: hipLaunchKernelGGL(k_vis_tail<4>, dim3(1), dim3(kVisTailSlots), 0, st, T, b, S.p); break;
+        }
+    }
+
+    // Residual and direction of iteration k of a batch lie in buffer k & 1; the iteration writes the other one,
+    // since its tiles still read their neighbours' old values.  The finest level's residual buffer, which only the
+    // batched solve uses, is the second direction.
+    float2* residual(int k) { return k & 1 ? r.p : r0.p; }
+    float2* direction(int k) { return k & 1 ? levels[0]->r.p : d.p; }
+
+    static constexpr int kApplyRows = 4, kApplyTile = kApplyRows * (kVT / 64);
+    int apply_tiles_x() const { return (W + 1 + 61) / 62; }
+    int apply_tiles_y() const { return (H + 1 + kApplyTile - 1) / kApplyTile; }
+
+    template <int MODE> int apply(hipStream_t st, const VisApply& io)
+    {
+        const int gx = apply_tiles_x(), gy = apply_tiles_y();
+        hipLaunchKernelGGL((k_vis_apply<MODE, kApplyRows>), dim3(gx * gy), dim3(kVT), 0, st, view(0), io, S.p, gx, gy,
             partials.p);
-        finish(st, nb, kVisRz, 0.0);
-        hipLaunchKernelGGL(k_vis_direction, g0, dim3(kVT), 0, st, Lc, (const float2*)Lc.x, d.p, S.p);
-        hipLaunchKernelGGL(k_vis_apply, g0, dim3(kVT), 0, st, L0, (const float2*)d.p, q.p, S.p, partials.p);
-        finish(st, nb, kVisDq, 0.0);
-        hipLaunchKernelGGL(k_vis_update, g0, dim3(kVT), 0, st, L0, delta, r.p, (const float2*)d.p,
-            (const float2*)q.p, S.p);
+        return gx * gy;
+    }
+
+    // Iteration k of a batch (ViscositySolverGPU.cpp:238-262): the pending step of the one before, V-cycle, r . z and
+    // beta, direction, A d and alpha.
+    void iteration(hipStream_t st, int k)
+    {
+        const VisStep io{residual(k), residual(k + 1), q.p, direction(k), t.p};
+        const float2* rhs = residual(k + 1);
+        const int tl = tail_level();
+        int nb = 0;
+        if (tl == 0) {
+            const VLev L = view(0);
+            hipLaunchKernelGGL(k_vis_step, slot_grid(W, H), dim3(kVT), 0, st, L, io, S.p);
+            tail(st, 0, rhs);
+            hipLaunchKernelGGL(k_vis_rz, slot_grid(W, H), dim3(kVT), 0, st, L, rhs, S.p, partials.p);
+            nb = (int)slot_blocks(W, H);
+        } else {
+            down<true>(st, 0, io);
+            for (int l = 1; l < tl; ++l)
+                down<false>(st, l, io);
+            tail(st, tl, levels[tl]->b.p);
+            for (int l = tl - 1; l > 0; --l)
+                up<false>(st, l, levels[l]->b.p);
+            nb = up<true>(st, 0, rhs);
+        }
+        finish<kVisRz>(st, nb);
+        VisApply ap{};
+        ap.z = solution(0);
+        ap.d = direction(k);
+        ap.d_new = direction(k + 1);
+        ap.q = q.p;
+        finish<kVisDq>(st, apply<kVisDirection>(st, ap));
     }
 
     // A batch of four iterations captured once into a hipGraph: the kernels take every changing value
-    // (dt, alpha, beta, the stop state) from the scalar block, and the x / xn swaps of four cycles return
-    // to their starting pointers, so one graph replays every full batch of every solve on this solver.
+    // (dt, alpha, beta, the stop state) from the scalar block, and four iterations end on the buffers they start
+    // from, so one graph replays every full batch of every solve on this solver.
     hipGraph_t batch_graph = nullptr;
     hipGraphExec_t batch_exec = nullptr;
     hipStream_t batch_stream = nullptr;
 
-    void run_batch(hipStream_t st, float2* delta)
+    void run_batch(hipStream_t st)
     {
         if (arena) {   // instantiating a graph allocates: the same four iterations, launched one by one
             for (int i = 0; i < 4; ++i)
-                iteration(st, delta);
+                iteration(st, i);
             return;
         }
         if (!batch_exec || batch_stream != st) {
@@ -1429,7 +1161,7 @@ struct ViscositySolver {
             std::lock_guard<std::mutex> lock(device_setup_mutex());
             vhip(hipStreamBeginCapture(st, hipStreamCaptureModeRelaxed), "hipStreamBeginCapture");
             for (int i = 0; i < 4; ++i)
-                iteration(st, delta);
+                iteration(st, i);
             vhip(hipStreamEndCapture(st, &batch_graph), "hipStreamEndCapture");
             vhip(hipGraphInstantiate(&batch_exec, batch_graph, nullptr, nullptr, 0), "hipGraphInstantiate");
             batch_stream = st;
@@ -1451,23 +1183,20 @@ struct ViscositySolver {
     // the initial reduction into the scalar block.
     void prepare(hipStream_t st, double* u, double* v, const double* mat64, float fdt, double spacing, double tol)
     {
-        const int N = W * H;
-        hipLaunchKernelGGL(k_vis_material, dim3(std::min((N + kVT - 1) / kVT, 4096)), dim3(kVT), 0, st, N, mat64,
-            levels[0]->mat.p);
-        for (size_t l = 0; l < levels.size(); ++l) {
-            if (l > 0) {
-                VLev F = view((int)l - 1), C = view((int)l);
-                hipLaunchKernelGGL(k_vis_coarsen, dim3((C.w + kVX - 1) / kVX, (C.h + kVY - 1) / kVY), dim3(kVT), 0,
-                    st, F, C);
-            }
-            VLev L = view((int)l);
-            hipLaunchKernelGGL(k_vis_coef, slot_grid(L.w, L.h), dim3(kVT), 0, st, L, (float)ldexp(spacing, (int)l));
+        hipLaunchKernelGGL(k_vis_finest, slot_grid(W, H), dim3(kVT), 0, st, view(0), mat64, (float)spacing);
+        for (size_t l = 1; l < levels.size(); ++l) {
+            const VLev L = view((int)l);
+            hipLaunchKernelGGL(k_vis_coarser, slot_grid(L.w, L.h), dim3(kVT), 0, st, view((int)l - 1), L,
+                (float)ldexp(spacing, (int)l));
         }
-        VLev L0 = view(0);
-        const dim3 g0 = slot_grid(W, H);
-        hipLaunchKernelGGL(k_vis_pack, g0, dim3(kVT), 0, st, L0, (const double*)u, (const double*)v, v0.p);
-        hipLaunchKernelGGL(k_vis_initial, g0, dim3(kVT), 0, st, L0, (const float2*)v0.p, r0.p, fdt, partials.p);
-        finish(st, (int)slot_blocks(W, H), kVisInitial, tol * tol, fdt);
+        VisApply io{};
+        io.q = r0.p;
+        io.x = t.p;
+        io.v0 = v0.p;
+        io.u64 = u;
+        io.v64 = v;
+        io.dt = fdt;
+        finish<kVisInitial>(st, apply<kVisInitialOf>(st, io), tol * tol, fdt);
     }
 
     // Batched solve (k_batch_vis): set-up, and the descriptor of this solver's instance.
@@ -1479,7 +1208,6 @@ struct ViscositySolver {
         prepare(st, u, v, mat64, (float)dt, spacing, tol);
         const size_t ns = (size_t)(W + 1) * (H + 1);
         vhip(hipMemcpyAsync(r.p, r0.p, ns * sizeof(float2), hipMemcpyDeviceToDevice, st), "copy");
-        vhip(hipMemcpyAsync(t.p, v0.p, ns * sizeof(float2), hipMemcpyDeviceToDevice, st), "copy");
         *desc = BatchVisDesc{};
         desc->levels = (int)levels.size();
         desc->W = W;
@@ -1528,15 +1256,7 @@ struct ViscositySolver {
             return 0;
         const float fdt = (float)dt;
         prepare(st, u, v, mat64, fdt, spacing, tol);
-        VLev L0 = view(0);
-        const dim3 g0 = slot_grid(W, H);
-        const int nb = (int)slot_blocks(W, H);
-        const size_t ns = (size_t)(W + 1) * (H + 1);
-        vhip(hipMemcpyAsync(r.p, r0.p, ns * sizeof(float2), hipMemcpyDeviceToDevice, st), "copy");
-        vhip(hipMemcpyAsync(t.p, v0.p, ns * sizeof(float2), hipMemcpyDeviceToDevice, st), "copy");
-        float2* delta = t.p;   // the iterate x, starting from v0 (the reference's formulation)
-        VBuf<float2>& truth = q;   // q is free between iterations
-        // Batches of four iterations, each followed by the recomputed residual and k_vis_decide, are queued
+        // Batches of four iterations, each followed by the recomputed residual and the decision on it, are queued
         // without a read-back in between: one batch fewer than the previous solve needed (a batch past the
         // solve's end costs its launches, a missing one a read-back), then one at a time.  Every decision
         // is taken on the device, so the iterations and values are those of reading back after each batch.
@@ -1548,26 +1268,25 @@ struct ViscositySolver {
             for (int k = 0; k < rounds && (maximum < 0 || queued < maximum); ++k) {
                 const int batch = maximum < 0 ? 4 : std::min(4, maximum - queued);
                 if (batch == 4) {
-                    run_batch(st, delta);
+                    run_batch(st);
                 } else {
                     for (int i = 0; i < batch; ++i)
-                        iteration(st, delta);
+                        iteration(st, i);
                 }
                 queued += batch;
-                L0 = view(0);
-                hipLaunchKernelGGL(k_vis_truth, g0, dim3(kVT), 0, st, L0, (const float2*)v0.p,
-                    (const float2*)delta, truth.p, fdt, partials.p, (const VisScalars*)S.p);
-                finish(st, nb, kVisTruth, 0.0);
-                hipLaunchKernelGGL(k_vis_decide, dim3(1), dim3(64), 0, st, S.p, batch, maximum);
-                // the recurrence claims convergence the recomputed residual denies: restart from it
-                hipLaunchKernelGGL(k_vis_restart_copy, dim3((unsigned)std::min<size_t>((ns + kVT - 1) / kVT, 2048)),
-                    dim3(kVT), 0, st, (const VisScalars*)S.p, r.p, (const float2*)truth.p, ns);
-                hipLaunchKernelGGL(k_vis_refresh, dim3(1), dim3(64), 0, st, S.p);
-                hipLaunchKernelGGL(k_vis_unpack, g0, dim3(kVT), 0, st, W, H, (const float2*)delta, u, v,
+                // the residual buffer that does not hold the recurrence's receives the recomputed one
+                VisApply io{};
+                io.x = t.p;   // the iterate, starting from v0 (the reference's formulation)
+                io.d = direction(batch);
+                io.v0 = v0.p;
+                io.q = residual(batch + 1);
+                finish<kVisTruth>(st, apply<kVisTruthOf>(st, io), 0.0, 0.0f, batch, maximum);
+                hipLaunchKernelGGL(k_vis_land, slot_grid(W, H), dim3(kVT), 0, st, view(0), t.p,
+                    (const float2*)direction(batch), residual(0), (const float2*)residual(batch + 1), u, v,
                     (const VisScalars*)S.p);
             }
             s = read(st);
-            // (k_vis_decide ends the solve once the budget is spent: nothing left to queue means done)
+            // (k_vis_finish ends the solve once the budget is spent: nothing left to queue means done)
             if (s.done != 0 || maximum == 0 || (rounds > 0 && queued == queued_before))
                 break;
             rounds = 1;
