@@ -381,6 +381,7 @@ struct fs_context {
     hipEvent_t join_levels = nullptr;   // the rebuild's tiled levels are done (the coarse chain may still run)
     PcgScalars* pinned = nullptr;   // host-pinned mirror of a grid's scalar block
     double* pinned_value = nullptr; // host-pinned landing slot of single device reductions
+    hipEvent_t value_ready = nullptr; // recorded behind the kernel that writes it
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     DevBuf<BatchItem> batch_desc;           // descriptors of the last batched projection
     DevBuf<int> batch_maps;                 // its workgroup maps and lists
@@ -507,7 +508,7 @@ struct fs_grid {
     DevBuf<double> sl_u, sl_v, sl_fraction, sl_lmass, sl_gmass;   // semi-Lagrangian transport's outputs (swapped in)
     // reference transport: second fraction/mass buffers, transported velocities (ping-pong), momenta,
     // per-pass face transfers, frozen corrections
-    DevBuf<double> tr_fraction, tr_lmass, tr_gmass, tr_nu[2], tr_nv[2], tr_mom_u, tr_mom_v, tr_lt, tr_mt;
+    DevBuf<double> tr_fraction, tr_lmass, tr_gmass, tr_nu[2], tr_nv[2], tr_mom_u, tr_mom_v, tr_mt;
     DevBuf<double> tr_lcw, tr_gcw, tr_mcw, tr_out;
     DevBuf<unsigned char> tr_split;
     DevBuf<float> calib_src, calib_dst;   // 64 MiB copy-bandwidth reference (allocated on first use)
@@ -1833,6 +1834,7 @@ fs_status fs_context_create_ex(int device, int flags, fs_context** out)
         }
         HIPC(hipHostMalloc((void**)&ctx->pinned, sizeof(PcgScalars), hipHostMallocDefault));
         HIPC(hipHostMalloc((void**)&ctx->pinned_value, sizeof(double), hipHostMallocDefault));
+        HIPC(hipEventCreateWithFlags(&ctx->value_ready, hipEventDisableTiming));
         viscosity_scratch_setup(device);   // this device's copy of the allocation-free solve's scratch
         HIPC(hipEventCreate(&ctx->ev0));
         HIPC(hipEventCreate(&ctx->ev1));
@@ -1858,6 +1860,8 @@ fs_status fs_context_destroy(fs_context* ctx)
                 (void)hipHostFree(ctx->pinned);
             if (ctx->pinned_value)
                 (void)hipHostFree(ctx->pinned_value);
+            if (ctx->value_ready)
+                (void)hipEventDestroy(ctx->value_ready);
             if (ctx->batch_pinned)
                 (void)hipHostFree(ctx->batch_pinned);
             if (ctx->staging)
@@ -2524,7 +2528,6 @@ static int advect_reference(fs_grid& g, double dt)
     }
     ensure(g.tr_mom_u, NU);
     ensure(g.tr_mom_v, NV);
-    ensure(g.tr_lt, std::max(NU, NV));
     ensure(g.tr_mt, std::max(NU, NV));
     ensure(g.tr_lcw, nl * N);
     ensure(g.tr_gcw, ng * N);
@@ -2555,7 +2558,6 @@ static int advect_reference(fs_grid& g, double dt)
         t.nv_out = g.tr_nv[cur ^ 1].p;
         t.mom_u = g.tr_mom_u.p;
         t.mom_v = g.tr_mom_v.p;
-        t.lt = g.tr_lt.p;
         t.mt = g.tr_mt.p;
         t.lcw = g.tr_lcw.p;
         t.gcw = g.tr_gcw.p;
@@ -2572,29 +2574,36 @@ static int advect_reference(fs_grid& g, double dt)
         cur ^= 1;
     };
 
-    // rebuildMomentum into tr_nu[0] / tr_nv[0], then the CFL limit
-    launch_density(g.st(), g.dev());
+    // rebuildMomentum into tr_nu[0] / tr_nv[0], then the CFL limit.  The first substep is queued behind it with the
+    // scale left on the device, so that the device works while the host waits for the limit.
+    auto substep = [&](const double* device_scale, double scale) {
+        TransportDev t = view();
+        t.scale = device_scale;
+        launch_transport_pass(g.st(), t, 1, scale);
+        swap_state();
+        t = view();
+        t.scale = device_scale;
+        launch_transport_pass(g.st(), t, 0, scale);
+        swap_state();
+    };
     cur = 1;
-    launch_transport_begin(g.st(), view());
+    launch_transport_begin(g.st(), view(), g.h, dt, kMaxTransportSubsteps, g.ctx->pinned_value);
     cur = 0;
-    HIPC(hipMemcpyAsync(g.ctx->pinned_value, g.tr_out.p, sizeof(double), hipMemcpyDeviceToHost, g.st()));
-    HIPC(hipStreamSynchronize(g.st()));
+    HIPC(hipEventRecord(g.ctx->value_ready, g.st()));
+    substep(g.tr_out.p, 0.0);
+    HIPC(hipEventSynchronize(g.ctx->value_ready));
     const double max_outflow = *g.ctx->pinned_value;
     // no cell exports more than half its volume per substep (FluidGridCPU.cpp:388-389)
     const double max_step = max_outflow > 0.0 ? 0.5 * g.h / max_outflow : dt;
-    if (!(max_step > 0.0) || dt / max_step > kMaxTransportSubsteps)
+    if (!(max_step > 0.0) || dt / max_step > kMaxTransportSubsteps) {
+        // the queued substep saw the same and wrote nothing: its two passes' swaps have undone each other
         fail(FS_E_RUNTIME, "Transport would need more than 1e6 CFL substeps (non-finite or extreme velocity)");
-
-    double remaining = dt;
-    int substeps = 0;
+    }
+    double remaining = dt - std::min(dt, max_step);
+    int substeps = 1;
     while (remaining > 0.0) {
         const double step = std::min(remaining, max_step);
-        const double scale = step / g.h;
-        launch_transport_freeze(g.st(), view());
-        launch_transport_pass(g.st(), view(), 1, scale);
-        swap_state();
-        launch_transport_pass(g.st(), view(), 0, scale);
-        swap_state();
+        substep(nullptr, step / g.h);
         remaining -= step;
         ++substeps;
     }
@@ -3900,7 +3909,7 @@ fs_status fs_grid_estimate_bytes(int width, int height, int n_liquid, int n_gas,
         const size_t coarse = std::max<size_t>(w * h, 2) - 1;
         b += coarse * coarse * 12 + (64 << 10);
         if (features & FS_FEATURE_TRANSPORT)   // advect_reference buffers
-            b += 8 * (N + 2 * (nl + ng) * N + 3 * NU + 3 * NV + 2 * std::max(NU, NV) + N) + N + 8;
+            b += 8 * (N + 2 * (nl + ng) * N + 3 * NU + 3 * NV + std::max(NU, NV) + N) + N + 8;
         if (features & FS_FEATURE_VISCOSITY) {   // ViscositySolver + blended material
             size_t vw = W, vh = H;
             for (;;) {

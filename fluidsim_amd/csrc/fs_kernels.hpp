@@ -318,18 +318,19 @@ struct TransportDev {
     const double* nu_in; double* nu_out;   // transported velocities (W+1)*H
     const double* nv_in; double* nv_out;   // W*(H+1)
     double* mom_u; double* mom_v;          // momenta
-    double* lt; double* mt;                // liquid volume and total mass transfer of the pass's faces
+    double* mt;                            // total mass transfer of the pass's faces
     double* lcw; double* gcw; double* mcw; // frozen correction weights (nl*N, ng*N, N)
     unsigned char* split;                  // frozen phase selection (fraction > 0.5)
     double* partials;                      // >= one double per 64 x 16 cell tile
-    double* out;                           // one device double: max outflow
+    double* out;                           // one device double: the first substep's scale (< 0: refused)
+    const double* scale;                   // the first substep: out, read by its passes; else null
 };
-// Density, momenta and transported velocities from u/v (rebuildMomentum), then the largest cell
-// outflow into *out (FluidGridCPU.cpp:1425-1476, 366-386).
-void launch_transport_begin(hipStream_t st, const TransportDev& t);
-// freezeComponentCorrections (FluidGridCPU.cpp:1307-1349).
-void launch_transport_freeze(hipStream_t st, const TransportDev& t);
-// One X (horizontal != 0) or Y pass of one substep: interfaces + liquid and component transfers,
+// Density, momenta and transported velocities from u/v, then the largest cell outflow into *host (pinned) and the
+// scale of the first substep of a transport over dt into *out (FluidGridCPU.cpp:1399-1476, 366-389).
+void launch_transport_begin(hipStream_t st, const TransportDev& t, double h, double dt, double max_substeps,
+    double* host);
+// One X (horizontal != 0; it comes first and freezes freezeComponentCorrections' weights, FluidGridCPU.cpp:1307-1349)
+// or Y pass of one substep: interfaces + liquid and component transfers,
 // component/fraction update with density, momentum transfer and velocity recovery
 // (FluidGridCPU.cpp:401-456).
 void launch_transport_pass(hipStream_t st, const TransportDev& t, int horizontal, double scale);
