@@ -300,11 +300,12 @@ __global__ __launch_bounds__(kFactorThreads) void k_coarse_factor(int w, int h, 
 
 // ---------------------------------------------------------------------------------------------
 // Inverse of the pinned coarse matrix for the per-cycle coarse solve (the hot path).  Goodnight's
-// sweep operator, in place, one pivot per step: the matrix lives in registers, column j in lane j
-// and rows split over sixteen wavefronts (4 per wavefront, so that a step's row updates are a short
-// chain).  A step broadcasts the pivot row through LDS (double-buffered, one barrier) and the pivot
-// column inside each wavefront by lane reads, so the 63 steps cost 63 barriers and no LDS matrix
-// traffic.  Pivots are the Schur complement diagonals (the squared Cholesky pivots); a non-positive or
+// sweep operator, in place: the matrix lives in registers, column j in lane j and rows split over sixteen wavefronts
+// (4 per wavefront, so that a step's row updates are a short chain).  A wavefront sweeps its four pivots on its own rows
+// and broadcasts the four scaled pivot rows through LDS (double-buffered, one barrier); the others then apply
+// them in the same order, the pivot column read inside each wavefront by lane.  Bound by the serial chain: 63 pivots
+// are 16 barriers and 63 divisions, 28 us on 8 x 8 cells (37 with a barrier and every thread's checks per pivot and
+// the entries assembled by one dependent load each).  Pivots are the Schur complement diagonals (the squared Cholesky pivots); a non-positive or
 // non-finite one marks the hierarchy failed exactly where the Cholesky factorisation would.
 // ---------------------------------------------------------------------------------------------
 constexpr int kSweepRows = 4;     // rows per wavefront
@@ -319,74 +320,93 @@ __device__ __forceinline__ double lane_value(double v, int k)
     return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
 }
 
-__device__ void coarse_inverse(int w, int h, const double* right, const double* down, float* ginv, int n,
+__device__ __forceinline__ void coarse_inverse(int w, int h, const double* right, const double* down, float* ginv, int n,
     PcgScalars* S, int pin)
 {
-    __shared__ double rowbuf[2][64];
-    __shared__ double pivot[2];
+    __shared__ double rowbuf[2][kSweepRows][64];
+    __shared__ int verdict[2];         // of a wavefront's pivots: bit r pinned, bit 8 + r failed
     __shared__ double assembled[64];   // diagonal before elimination (pinning bound)
     const int s = w + 2;
     const int lane = threadIdx.x & 63;
-    const int wv = threadIdx.x >> 6;
+    const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     // pinned matrix entry (i, j) of unknowns i, j (cells i + 1, j + 1)
     double a[kSweepRows];
+    // every entry of column j is one of its cell's four conductances: one round of loads
     const int cj = lane + 1;
-    const int xj = cj % w, yj = cj / w;
+    const int yj = cj / w, xj = cj - yj * w;
+    const int pj = (min(yj, h - 1) + 1) * s + xj + 1;
+    const double cl = right[pj - 1], cr = right[pj], cu = down[pj - s], cd = down[pj];
 #pragma unroll
     for (int r = 0; r < kSweepRows; ++r) {
         const int ci = wv * kSweepRows + r + 1;
+        const int yi = ci / w, xi = ci - yi * w;
         double v = 0.0;
-        if (ci <= n && cj <= n) {
-            const int xi = ci % w, yi = ci / w;
-            const int pi = (yi + 1) * s + xi + 1;
-            if (ci == cj) {
-                v = right[pi - 1] + right[pi] + down[pi - s] + down[pi];
-                assembled[lane] = v;
-            } else if (yi == yj && (xi - xj == 1 || xj - xi == 1)) {
-                v = -right[(yi + 1) * s + min(xi, xj) + 1];
-            } else if (xi == xj && (yi - yj == 1 || yj - yi == 1)) {
-                v = -down[(min(yi, yj) + 1) * s + xi + 1];
-            }
-        }
-        a[r] = v;
+        if (ci == cj)
+            v = cl + cr + cu + cd;
+        else if (yi == yj && (xi - xj == 1 || xj - xi == 1))
+            v = -(xi > xj ? cr : cl);
+        else if (xi == xj && (yi - yj == 1 || yj - yi == 1))
+            v = -(yi > yj ? cd : cu);
+        a[r] = ci <= n && cj <= n ? v : 0.0;
+        if (ci == cj && ci <= n)
+            assembled[lane] = v;
     }
     bool failed = false;
     // Solid masks: an unknown whose Schur pivot vanishes is pinned -- never swept, and its row and
     // column of the inverse are zero (the swept block is then the inverse of the other unknowns' matrix)
     unsigned long long pinned = 0ull;   // the same in every thread
-    for (int kb = 0; kb < kSweepWaves && !failed; ++kb) {
+    if (pin)
+        __syncthreads();   // assembled[]
+    // a[] of one wavefront after the sweep of pivot k, whose scaled row is t; b, the pivot column, lies in lane k
+    auto update = [&](int k, double t, int own) {
+        const bool mine = lane == k;
 #pragma unroll
-        for (int r0 = 0; r0 < kSweepRows; ++r0) {
-            const int k = kb * kSweepRows + r0;
-            if (k >= n || failed)
-                break;
-            double* row = rowbuf[k & 1];
-            if (wv == kb) {
-                // the row's wavefront alone divides and publishes the scaled row; lane k's own entry becomes 1 / d
+        for (int r = 0; r < kSweepRows; ++r) {
+            const double b = lane_value(a[r], k);
+            const double base = mine ? 0.0 : a[r];
+            a[r] = r == own ? t : base - b * t;
+        }
+    };
+    for (int kb = 0; kb * kSweepRows < n && !failed; ++kb) {
+        const int buf = kb & 1, k0 = kb * kSweepRows;
+        if (wv == kb) {
+            int code = 0;
+#pragma unroll
+            for (int r0 = 0; r0 < kSweepRows; ++r0) {
+                const int k = k0 + r0;
+                if (k >= n || code >> 8)
+                    break;
                 const double d = lane_value(a[r0], k);
+                if (pin && isfinite(d) && fabs(d) <= kPinRatio * assembled[k]) {
+                    code |= 1 << r0;
+                    continue;
+                }
+                if (!(d > 0.0) || !isfinite(d)) {
+                    code |= 256 << r0;
+                    break;
+                }
+                // lane k's own entry of a scaled row becomes 1 / d
                 const double inv_d = 1.0 / d;
-                row[lane] = lane == k ? inv_d : a[r0] * inv_d;
-                if (lane == k)
-                    pivot[k & 1] = d;
+                const double t = lane == k ? inv_d : a[r0] * inv_d;
+                rowbuf[buf][r0][lane] = t;
+                update(k, t, r0);
             }
-            __syncthreads();   // also orders the assembled[] writes before the first read
-            const double t = row[lane];
-            const double d = pivot[k & 1];
-            if (pin && isfinite(d) && fabs(d) <= kPinRatio * assembled[k]) {
-                pinned |= 1ull << k;
-                continue;
-            }
-            if (!(d > 0.0) || !isfinite(d)) {
-                failed = true;   // d is the same in every thread: the whole block leaves together
-                break;
-            }
+            if (lane == 0)
+                verdict[buf] = code;
+        }
+        __syncthreads();
+        double t[kSweepRows];
 #pragma unroll
-            for (int r = 0; r < kSweepRows; ++r) {
-                const int i = wv * kSweepRows + r;
-                const double b = lane_value(a[r], k);
-                const double base = lane == k ? 0.0 : a[r];
-                a[r] = i == k ? t : base - b * t;
-            }
+        for (int r0 = 0; r0 < kSweepRows; ++r0)
+            t[r0] = rowbuf[buf][r0][lane];
+        const int code = __builtin_amdgcn_readfirstlane(verdict[buf]);
+        failed = code >> 8 != 0;   // the same in every thread: the whole block leaves together
+        pinned |= (unsigned long long)(code & 255) << k0;
+        if (wv != kb && !failed) {
+#pragma unroll
+            for (int r0 = 0; r0 < kSweepRows; ++r0)
+                if (k0 + r0 < n && !(code >> r0 & 1))
+                    update(k0 + r0, t[r0], -1);
         }
     }
     if (failed) {
