@@ -2914,6 +2914,7 @@ fs_status fs_viscosity_solve_noalloc(fs_context* ctx, int width, int height, dou
             "null pointer");
         need(width > 0 && height > 0 && cell_size > 0.0, FS_E_INVALID_ARGUMENT, "invalid grid shape");
         need(std::isfinite(tolerance) && tolerance >= 0.0, FS_E_INVALID_ARGUMENT, "invalid tolerance");
+        static_assert(sizeof(PcgScalars) >= kViscosityLandingBytes, "the context's pinned slot holds the scalars");
         need((long long)width * height <= (1LL << 26) && viscosity_scratch_bytes(width, height) <= kViscosityScratchBytes,
             FS_E_INVALID_ARGUMENT, "grid too large for the allocation-free viscosity solve's 64 MiB scratch");
         set_device(ctx);
@@ -2921,7 +2922,7 @@ fs_status fs_viscosity_solve_noalloc(fs_context* ctx, int width, int height, dou
         double rel = 0.0;
         const int budget = max_iterations < 0 ? kViscosityBudget : max_iterations;
         const int status = viscosity_solve_scratch(ctx->device, ctx->stream, width, height, u, v, material, dt,
-            cell_size, tolerance, budget, &it, &rel);
+            cell_size, tolerance, budget, ctx->pinned, ctx->value_ready, &it, &rel);
         if (iterations)
             *iterations = it;
         if (relative_residual)

@@ -351,13 +351,15 @@ ViscositySolver* viscosity_create(int width, int height);
 // kViscosityScratchBytes per device.  viscosity_scratch_setup (with `device` current) resolves that
 // device's copy once; viscosity_scratch_bytes is the workspace a W x H solve needs;
 // viscosity_solve_scratch runs viscosity_solve's algorithm in it on device u, v and material, one call
-// at a time per device, and returns after the stream has drained.
+// at a time per device, and returns after the stream has drained; `landing` is pinned memory of
+// kViscosityLandingBytes and `landed` an event, both the caller's.
 constexpr size_t kViscosityScratchBytes = (size_t)64 << 20;
+constexpr size_t kViscosityLandingBytes = 128;
 void* viscosity_scratch_setup(int device);
 size_t viscosity_scratch_bytes(int width, int height);
 int viscosity_solve_scratch(int device, hipStream_t st, int width, int height, double* u, double* v,
-    const double* material, double dt, double spacing, double tol, int maximum, int* iterations,
-    double* relative_residual);
+    const double* material, double dt, double spacing, double tol, int maximum, void* landing, hipEvent_t landed,
+    int* iterations, double* relative_residual);
 void viscosity_destroy(ViscositySolver* s);
 size_t viscosity_bytes(const ViscositySolver* s);
 int viscosity_levels(const ViscositySolver* s);

@@ -894,7 +894,8 @@ struct ViscositySolver {
     VBuf<double> material, partials;
     VBuf<VisScalars> S;
     VisScalars* pinned = nullptr;
-    VisScalars landing{};           // read-back slot of a solver placed in an arena (no pinned memory)
+    VisScalars* landing = nullptr;  // a solver placed in an arena: the caller's pinned read-back slot ...
+    hipEvent_t landed = nullptr;    // ... and the event recorded behind the copy into it
     ScratchArena* arena = nullptr;  // non-null: every device buffer is a piece of the arena
     size_t bytes = 0;
 
@@ -957,11 +958,18 @@ struct ViscositySolver {
         return VLev{L.w, L.h, L.coef.p, L.mat.p, L.b.p, L.x.p, L.xn.p, L.r.p};
     }
 
-    VisScalars read(hipStream_t st)
+    // The scalar block; `ahead` queues work behind the copy for the device to do while the host waits and decides.
+    template <class Ahead> VisScalars read(hipStream_t st, Ahead ahead)
     {
-        VisScalars* slot = pinned ? pinned : &landing;
+        VisScalars* slot = pinned ? pinned : landing;
         vhip(hipMemcpyAsync(slot, S.p, sizeof(VisScalars), hipMemcpyDeviceToHost, st), "hipMemcpyAsync");
-        vhip(hipStreamSynchronize(st), "hipStreamSynchronize");
+        if (landed) {
+            vhip(hipEventRecord(landed, st), "hipEventRecord");
+            ahead();
+            vhip(hipEventSynchronize(landed), "hipEventSynchronize");
+        } else {
+            vhip(hipStreamSynchronize(st), "hipStreamSynchronize");
+        }
         return *slot;
     }
 
@@ -1151,11 +1159,6 @@ struct ViscositySolver {
 
     void run_batch(hipStream_t st)
     {
-        if (arena) {   // instantiating a graph allocates: the same four iterations, launched one by one
-            for (int i = 0; i < 4; ++i)
-                iteration(st, i);
-            return;
-        }
         if (!batch_exec || batch_stream != st) {
             drop_batch_graph();
             std::lock_guard<std::mutex> lock(device_setup_mutex());
@@ -1261,18 +1264,22 @@ struct ViscositySolver {
         // solve's end costs its launches, a missing one a read-back), then one at a time.  Every decision
         // is taken on the device, so the iterations and values are those of reading back after each batch.
         int rounds = last_rounds > 0 ? std::max(1, last_rounds - 1) : 0;
-        int queued = 0;
+        // A solver in an arena knows no previous solve and launches its iterations one by one: it queues the first one of
+        // the next batch behind each read-back (12 launches that exit at once where the solve has ended, against
+        // an idle device for as long as the host takes to see the scalars).
+        int queued = 0, started = 0;   // iterations of queued batches, and of the next one
         VisScalars s{};
         for (;;) {
             const int queued_before = queued;
             for (int k = 0; k < rounds && (maximum < 0 || queued < maximum); ++k) {
                 const int batch = maximum < 0 ? 4 : std::min(4, maximum - queued);
-                if (batch == 4) {
+                if (batch == 4 && !arena) {
                     run_batch(st);
                 } else {
-                    for (int i = 0; i < batch; ++i)
+                    for (int i = started; i < batch; ++i)
                         iteration(st, i);
                 }
+                started = 0;
                 queued += batch;
                 // the residual buffer that does not hold the recurrence's receives the recomputed one
                 VisApply io{};
@@ -1285,7 +1292,12 @@ struct ViscositySolver {
                     (const float2*)direction(batch), residual(0), (const float2*)residual(batch + 1), u, v,
                     (const VisScalars*)S.p);
             }
-            s = read(st);
+            s = read(st, [&] {
+                if (maximum < 0 || queued < maximum) {
+                    iteration(st, 0);
+                    started = 1;
+                }
+            });
             // (k_vis_finish ends the solve once the budget is spent: nothing left to queue means done)
             if (s.done != 0 || maximum == 0 || (rounds > 0 && queued == queued_before))
                 break;
@@ -1353,9 +1365,10 @@ size_t viscosity_scratch_bytes(int width, int height)
 }
 
 int viscosity_solve_scratch(int device, hipStream_t st, int width, int height, double* u, double* v,
-    const double* material, double dt, double spacing, double tol, int maximum, int* iterations,
-    double* relative_residual)
+    const double* material, double dt, double spacing, double tol, int maximum, void* landing, hipEvent_t landed,
+    int* iterations, double* relative_residual)
 {
+    static_assert(sizeof(VisScalars) <= kViscosityLandingBytes, "the caller's slot holds the scalar block");
     void* base = viscosity_scratch_setup(device);
     const size_t need = viscosity_scratch_bytes(width, height);
     if (need > kViscosityScratchBytes)
@@ -1370,6 +1383,8 @@ int viscosity_solve_scratch(int device, hipStream_t st, int width, int height, d
     arena.base = (unsigned char*)base;
     arena.capacity = kViscosityScratchBytes;
     ViscositySolver solver(width, height, &arena);
+    solver.landing = (VisScalars*)landing;
+    solver.landed = landed;
     const int status = solver.solve(st, u, v, material, dt, spacing, tol, maximum, iterations, relative_residual);
     // the last kernels (velocity unpack) read the scratch: done before another call may reuse it
     vhip(hipStreamSynchronize(st), "hipStreamSynchronize");
