@@ -43,19 +43,23 @@ struct Tile4 {
     bool in[4];
 };
 
-__device__ __forceinline__ Tile4 tile4(const GridDev& g, int column, int row)
+__device__ __forceinline__ Tile4 tile4(const GridDev& g, int column, int row, int thread)
 {
     Tile4 t;
-    t.x = column * kTX + (threadIdx.x & 63);
+    t.x = column * kTX + (thread & 63);
     t.xc = min(t.x, g.W - 1);
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
-        t.y[k] = row * kTY + (threadIdx.x >> 6) + 4 * k;
+        t.y[k] = row * kTY + (thread >> 6) + 4 * k;
         t.yc[k] = min(t.y[k], g.H - 1);
         t.in[k] = t.x < g.W && t.y[k] < g.H;
         t.P[k] = pidx(t.xc, t.yc[k], g.s);
     }
     return t;
+}
+__device__ __forceinline__ Tile4 tile4(const GridDev& g, int column, int row)
+{
+    return tile4(g, column, row, threadIdx.x);
 }
 
 // ------------------------------------------------------------------------------------------
@@ -586,6 +590,30 @@ __device__ __forceinline__ Recurrence recurrence(const PcgScalars* S, const doub
     return c;
 }
 
+// r = b - A (p + x) of a thread's cells in FP64, and its sum and max-norm.
+__device__ __forceinline__ void true_residual(const GridDev& g, const Tile4& T, double& sum, double& m)
+{
+    const int s = g.s;
+    double r[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        const int i = T.P[k];
+        auto at = [&](int j) { return g.p[j] + (double)g.x[j]; };
+        const double c = at(i);
+        const double product = (g.right64[i - 1] * (c - at(i - 1)) + g.right64[i] * (c - at(i + 1))) +
+                               (g.down64[i - s] * (c - at(i - s)) + g.down64[i] * (c - at(i + s)));
+        r[k] = g.b[i] - product;
+    }
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        if (T.in[k]) {
+            g.r[T.P[k]] = (float)r[k];
+            sum += r[k];
+            m = fmax(m, fabs(r[k]));
+        }
+    }
+}
+
 // The check: every workgroup reduces the update's partials itself and, where they call for it, forms the FP64
 // true residual b - A (p + x) as the new working residual.  p and x stay as they are (the neighbours read them):
 // the next direction folds x into p.  The scalar block is written by the finish launch alone.
@@ -598,30 +626,10 @@ struct Check {
         Partials<kNT, 2, 1>().all(g.fold_up, g.fold_up_n, t, lds);
         if (st != kRunning || !recurrence(g.S, t).verify)
             return;
-        const int s = g.s;
         double sum = 0.0, m = 0.0;
 #pragma unroll 1
-        for (int group = 0; group < G; ++group) {
-            const Tile4 T = tile4(g, B.x, B.y * G + group);
-            double r[4];
-#pragma unroll
-            for (int k = 0; k < 4; ++k) {
-                const int i = T.P[k];
-                auto at = [&](int j) { return g.p[j] + (double)g.x[j]; };
-                const double c = at(i);
-                const double product = (g.right64[i - 1] * (c - at(i - 1)) + g.right64[i] * (c - at(i + 1))) +
-                                       (g.down64[i - s] * (c - at(i - s)) + g.down64[i] * (c - at(i + s)));
-                r[k] = g.b[i] - product;
-            }
-#pragma unroll
-            for (int k = 0; k < 4; ++k) {
-                if (T.in[k]) {
-                    g.r[T.P[k]] = (float)r[k];
-                    sum += r[k];
-                    m = fmax(m, fabs(r[k]));
-                }
-            }
-        }
+        for (int group = 0; group < G; ++group)
+            true_residual(g, tile4(g, B.x, B.y * G + group), sum, m);
         const double bs = block_sum<kNT>(sum, lds);
         const double bm = block_max<kNT>(m, lds);
         if (threadIdx.x == 0) {
@@ -873,6 +881,84 @@ struct FinishSetup {
     }
 };
 
+// The decision after an update: t its residual (sum, max-norm), e the true one's where it was formed.
+__device__ __forceinline__ void decide(const GridDev& g, const Recurrence& c, const double (&t)[2], const double (&e)[2])
+{
+    PcgScalars* S = g.S;
+    const double n = (double)g.W * g.H;
+    S->iterations += 1;
+    S->rmax = c.rmax;
+    S->r_sum = t[0];
+    S->r_mean = t[0] / n;
+    if (c.verify) {
+        const double maximum = isfinite(e[0]) ? e[1] : INFINITY;
+        S->true_rmax = maximum;
+        S->r_sum = e[0];
+        S->flush = 1;
+        if (maximum <= S->tol) {
+            S->status = kConverged;
+        } else {
+            S->r_mean = e[0] / n;
+            if (!c.replace || maximum > kDriftRatio * c.rmax) {
+                S->restart = 1;
+                S->restarts += 1;
+            }
+            S->rmax = maximum;
+            S->window_rmax = maximum;
+        }
+    }
+    // out of budget: the next direction would never be used
+    if (S->status == kRunning && S->iterations >= S->max_iterations)
+        S->status = kStopped;
+}
+
+// Check and decision of a small grid in one launch, a launch less of the six beside its V-cycle: one workgroup, a
+// 256-thread group per tile, the sums in the order of the two launches.  61 x 47 (3 tiles) 6% per solve; with 16 tiles in
+// four rounds a check on one compute unit costs what the launch saves (128 x 128: 4341 us against 4323), so only where
+// one round takes them all.
+constexpr int kSmallTiles = 4;
+__global__ __launch_bounds__(kSmallTiles * kNT) void k_check_small(GridDev g, int columns, int tiles)
+{
+    __shared__ double lds[2][kSmallTiles * kNT / 64];
+    const int lane = threadIdx.x & 63;
+    const bool mine = lane < tiles;
+    const int st = g.S->status;
+    double t[2] = {mine ? load_partial(g.fold_up, 2 * lane) : 0.0, mine ? load_partial(g.fold_up, 2 * lane + 1) : 0.0};
+    if (st != kRunning)
+        return;
+    t[0] = wave_sum(t[0]);
+    t[1] = wave_max(t[1]);
+    const Recurrence c = recurrence(g.S, t);
+    double e[2] = {0.0, 0.0};
+    if (c.verify) {   // the same in every thread
+        const int thread = threadIdx.x & (kNT - 1), tile = threadIdx.x / kNT;
+        double sum = 0.0, m = 0.0;
+        if (tile < tiles)
+            true_residual(g, tile4(g, tile % columns, tile / columns, thread), sum, m);
+        sum = wave_sum(sum);
+        m = wave_max(m);
+        if (lane == 0) {
+            lds[0][threadIdx.x >> 6] = sum;
+            lds[1][threadIdx.x >> 6] = m;
+        }
+        __syncthreads();
+        // lane k of the first wavefront collects tile k's sums
+        if (threadIdx.x < kSmallTiles) {
+#pragma unroll
+            for (int i = 0; i < kNT / 64; ++i) {
+                e[0] += lds[0][lane * (kNT / 64) + i];
+                e[1] = fmax(e[1], lds[1][lane * (kNT / 64) + i]);
+            }
+        }
+        if (threadIdx.x < 64) {
+            e[0] = wave_sum(e[0]);
+            e[1] = wave_max(e[1]);
+        }
+    }
+    if (threadIdx.x == 0)
+        decide(g, c, t, e);
+}
+
 // The update's residual norm; where it called for a check, the true residual's verdict as well.
 struct FinishCheck {
     __device__ __forceinline__ void run(const GridDev& g, int nb, double* lds) const
@@ -883,37 +969,12 @@ struct FinishCheck {
         Partials<kNT, 2, 1>().all(g.fold_up, g.fold_up_n, t, lds);
         if (st != kRunning)
             return;
-        const double n = (double)g.W * g.H;
         const Recurrence c = recurrence(S, t);
         double e[2] = {0.0, 0.0};
         if (c.verify)
             Partials<kNT, 2, 1>().all(g.partials_tr, nb, e, lds);
-        if (threadIdx.x != 0)
-            return;
-        S->iterations += 1;
-        S->rmax = c.rmax;
-        S->r_sum = t[0];
-        S->r_mean = t[0] / n;
-        if (c.verify) {
-            const double maximum = isfinite(e[0]) ? e[1] : INFINITY;
-            S->true_rmax = maximum;
-            S->r_sum = e[0];
-            S->flush = 1;
-            if (maximum <= S->tol) {
-                S->status = kConverged;
-            } else {
-                S->r_mean = e[0] / n;
-                if (!c.replace || maximum > kDriftRatio * c.rmax) {
-                    S->restart = 1;
-                    S->restarts += 1;
-                }
-                S->rmax = maximum;
-                S->window_rmax = maximum;
-            }
-        }
-        // out of budget: the next direction would never be used
-        if (S->status == kRunning && S->iterations >= S->max_iterations)
-            S->status = kStopped;
+        if (threadIdx.x == 0)
+            decide(g, c, t, e);
     }
 };
 
@@ -1109,6 +1170,11 @@ void launch_pcg_update(hipStream_t st, const GridDev& g)
 
 void launch_pcg_check(hipStream_t st, const GridDev& g)
 {
+    const int columns = (g.W + kTX - 1) / kTX, tiles = columns * ((g.H + kTY - 1) / kTY);
+    if (tiles <= kSmallTiles) {
+        hipLaunchKernelGGL(k_check_small, dim3(1), dim3(kSmallTiles * kNT), 0, st, g, columns, tiles);
+        return;
+    }
     launch_cells<Check>(st, g);
     launch_finish<FinishCheck>(st, g);
 }
