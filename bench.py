@@ -49,7 +49,7 @@ POST_TILES = [(64, 8, 8), (64, 16, 4), (32, 8, 4), (32, 16, 2), (32, 4, 4), (32,
 HBM_PEAK_GBS = 8000.0
 PROFILES = os.path.join(HERE, "profiles")
 TRACE_PROFILE = os.path.join(HERE, "profiles", "bench_1024_kernel_trace.md")
-SQ_PROFILE = os.path.join(HERE, "profiles", "k_rb_multi_sq_counters.md")
+SQ_PROFILE = os.path.join(HERE, "profiles", "smoother_sq_counters.md")
 TAIL_KERNEL = 6   # fs_time_kernel id of the single-workgroup coarse tail
 # Algorithmic bytes per fine cell of one whole projection, by the per-iteration model: 15 FP32 CG vector
 # passes (operator + dot 4, update + max 6, dot + direction 5; s = 4 B) plus the V(nu,nu) cycle's
@@ -916,17 +916,16 @@ def main():
                                       "bytes (rocprofv3 FETCH_SIZE + WRITE_SIZE)")
         try:
             with open(SQ_PROFILE) as f:
-                covered = f"`<{fine_kernel.split('<', 1)[1].split(',float')[0]}>`" in f.read().replace(" ", "")
+                covered = f"`<{fine_kernel.split('<', 1)[1]}`" in f.read().replace(" ", "")
         except OSError:
             covered = False
         if covered:
-            out["roofline"]["limiter"] += ("; SQ counters show instruction issue and latency: VALU the busiest pipe, "
-                                           "waves waiting a third or more of their time")
+            out["roofline"]["limiter"] += "; SQ counters show instruction issue and latency, VALU the busiest pipe"
             out["roofline"]["limiter_source"] = os.path.relpath(SQ_PROFILE, HERE)
     top = traced_kernels()
     if top:
         dom = {"kernel": top[0][0], "share_of_kernel_time": top[0][1], "source": os.path.relpath(TRACE_PROFILE, HERE)}
-        if top[0][0].startswith("k_mg_tail"):
+        if top[0][0].startswith(("k_mg_tail", "k_tail")):
             # the single-workgroup tail: levels from the first untiled one down, V(4,4) at the multigrid
             # model's (10 nu + 5.5) c = 182 B per level cell, plus the FP32 coarse inverse
             shapes = [grid.multigridShape(l) for l in range(grid.multigridLevels())]
@@ -937,8 +936,7 @@ def main():
             dom.update({"avg_launch_us": tail_us, "algorithmic_bytes_per_launch": tail_bytes,
                         "achieved_gbs": tail_bytes / (tail_us * 1e-6) / 1e9,
                         "frac": tail_bytes / (tail_us * 1e-6) / 1e9 / HBM_PEAK_GBS,
-                        "limiter": "latency: one 1024-thread workgroup on one compute unit, about 60 "
-                                   "barrier-separated phases per launch"})
+                        "limiter": "latency: one workgroup on one compute unit, a chain of LDS exchanges and barriers"})
         out["roofline"]["dominant_kernel_in_trace"] = dom
     if rank == 0 and not args.no_cpu:
         gpu_state = grid.download()   # the last timed projection

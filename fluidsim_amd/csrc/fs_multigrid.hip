@@ -305,8 +305,8 @@ __global__ __launch_bounds__(kFactorThreads) void k_coarse_factor(int w, int h, 
 // and broadcasts the four scaled pivot rows through LDS (double-buffered, one barrier); the others then apply
 // them in the same order, the pivot column read inside each wavefront by lane.  Bound by the serial chain: 63 pivots
 // are 16 barriers and 63 divisions, 28 us on 8 x 8 cells (37 with a barrier and every thread's checks per pivot and
-// the entries assembled by one dependent load each).  Pivots are the Schur complement diagonals (the squared Cholesky pivots); a non-positive or
-// non-finite one marks the hierarchy failed exactly where the Cholesky factorisation would.
+// the entries assembled by one dependent load each).  Pivots are the Schur complement diagonals (the squared Cholesky
+// pivots); a non-positive or non-finite one marks the hierarchy failed exactly where the Cholesky factorisation would.
 // ---------------------------------------------------------------------------------------------
 constexpr int kSweepRows = 4;     // rows per wavefront
 constexpr int kSweepWaves = 16;   // kSweepWaves x kSweepRows >= kMaxCoarse

@@ -89,34 +89,29 @@ __device__ __forceinline__ bool stopped(const VisScalars* S)
     return S->bad != 0 || S->rnorm <= S->target || S->done != 0;
 }
 
-// Index of slot (x, y) in an array: the global slot field clamped like the reference's accessors, or an
-// LDS tile that holds the clamped values (see k_vis_smooth).  The stencils below are written once over
-// it, so the fused and the per-sweep kernels evaluate the same expressions.
-struct GlobalSlots {
-    int w, h;
-    __device__ __forceinline__ int operator()(int x, int y) const { return sidx(w, h, x, y); }
-};
+// The operator on slots in memory, every read clamped to the slot field like the reference's accessors (the batched
+// solve; fs_viscosity_rows.hpp evaluates the same expressions on slots in registers).
 
 // shear and stressProduct (ViscosityKernels.h:26-44)
-template <class I> __device__ __forceinline__ float shear_at(const float4* c, const float2* s, I at, int x, int y)
+__device__ __forceinline__ float shear(const float4* c, const float2* s, int w, int h, int x, int y)
 {
+    auto at = [=](int i, int j) { return sidx(w, h, i, j); };
     const float2 p = s[at(x, y)];
     return c[at(x, y)].y * ((p.x - s[at(x, y - 1)].x) + (p.y - s[at(x - 1, y)].y));
 }
 
 // product (ViscosityKernels.h:53-57): M s + dt K s on valid faces.
-template <class I>
-__device__ __forceinline__ float2 product_at(const float4* c, const float2* s, I at, int w, int h, int x, int y,
-    float dt)
+__device__ __forceinline__ float2 product(const float4* c, const float2* s, int w, int h, int x, int y, float dt)
 {
+    auto at = [=](int i, int j) { return sidx(w, h, i, j); };
     const int p = at(x, y);
     const float2 cv = s[p];
     const float4 a = c[p];
-    const float t = shear_at(c, s, at, x, y);
+    const float t = shear(c, s, w, h, x, y);
     const float nu = 2.0f * (c[at(x - 1, y)].x * (cv.x - s[at(x - 1, y)].x) + a.x * (cv.x - s[at(x + 1, y)].x));
     const float nv = 2.0f * (c[at(x, y - 1)].x * (cv.y - s[at(x, y - 1)].y) + a.x * (cv.y - s[at(x, y + 1)].y));
-    const float ku = nu + (t - shear_at(c, s, at, x, y + 1));
-    const float kv = nv + (t - shear_at(c, s, at, x + 1, y));
+    const float ku = nu + (t - shear(c, s, w, h, x, y + 1));
+    const float kv = nv + (t - shear(c, s, w, h, x + 1, y));
     float2 out;
     out.x = valid_u(w, h, x, y) ? a.z * cv.x + dt * ku : 0.0f;
     out.y = valid_v(w, h, x, y) ? a.w * cv.y + dt * kv : 0.0f;
@@ -124,23 +119,14 @@ __device__ __forceinline__ float2 product_at(const float4* c, const float2* s, I
 }
 
 // diagonal (ViscosityKernels.h:17-24)
-template <class I> __device__ __forceinline__ float2 diagonal_at(const float4* c, I at, int x, int y, float dt)
+__device__ __forceinline__ float2 diagonal(const float4* c, int w, int h, int x, int y, float dt)
 {
+    auto at = [=](int i, int j) { return sidx(w, h, i, j); };
     const float4 a = c[at(x, y)];
     float2 d;
     d.x = a.z + dt * (2.0f * (a.x + c[at(x - 1, y)].x) + a.y + c[at(x, y + 1)].y);
     d.y = a.w + dt * (2.0f * (a.x + c[at(x, y - 1)].x) + a.y + c[at(x + 1, y)].y);
     return d;
-}
-
-__device__ float2 product(const float4* c, const float2* s, int w, int h, int x, int y, float dt)
-{
-    return product_at(c, s, GlobalSlots{w, h}, w, h, x, y, dt);
-}
-
-__device__ __forceinline__ float2 diagonal(const float4* c, int w, int h, int x, int y, float dt)
-{
-    return diagonal_at(c, GlobalSlots{w, h}, x, y, dt);
 }
 
 #define VIS_SLOT(L)                                            \

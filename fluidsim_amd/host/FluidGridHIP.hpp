@@ -207,7 +207,7 @@ public:
     HipContext(const HipContext&) = delete;
     HipContext& operator=(const HipContext&) = delete;
     fs_context* get() const { return ctx_; }
-    // fs_context_set_batch_split: batched solves send grids above `solo_cells` cells through their
+    // fs_context_set_batch_split: batched viscosity steps send grids above `solo_cells` cells through their
     // single-grid solve beside the persistent launch (0: batch every grid).
     void setBatchSplit(long long solo_cells) { check(fs_context_set_batch_split(ctx_, solo_cells)); }
 
