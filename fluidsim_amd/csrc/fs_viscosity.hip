@@ -907,7 +907,9 @@ struct ViscositySolver {
             place(L->b, ns);
             place(L->x, ns);
             place(L->xn, ns);
-            if (!arena || levels.count == 1)   // residuals of the batched solve; the finest level's is a direction buffer
+            // residuals of the batched solve; the finest level's is a direction buffer (counted on every level when an
+            // arena is only measured: the size limit of the allocation-free solve, which needs no more)
+            if (!arena || !arena->base || levels.count == 1)
                 place(L->r, ns);
             if (w * h <= 64)
                 break;
@@ -925,8 +927,9 @@ struct ViscositySolver {
             place(material, 2 * (size_t)W * H);
         // four components a tile of k_vis_apply, three a tile of k_vis_up (60 x 12 slots or 52 x 20 at the least) or,
         // with one level, a block of k_vis_rz
-        place(partials, std::max(4 * (size_t)apply_tiles_x() * apply_tiles_y(),
-            3 * (levels.count > 1 ? (size_t)tiles(W, 52) * tiles(H, 12) : (size_t)slot_blocks(W, H))));
+        const size_t sums = std::max(4 * (size_t)apply_tiles_x() * apply_tiles_y(),
+            3 * (levels.count > 1 ? (size_t)tiles(W, 52) * tiles(H, 12) : (size_t)slot_blocks(W, H)));
+        place(partials, arena && !arena->base ? 4 * (size_t)slot_blocks(W, H) : sums);
         place(S, 1);
         if (!arena)
             pinned = (VisScalars*)pinned_alloc(sizeof(VisScalars));
