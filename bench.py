@@ -128,7 +128,7 @@ def cpu_baseline(wl, tau, budget_s, smoother=None):
     the oracle's projected state with `smoother` = (kind, sweeps, coarse sweeps), the GPU's choice, or
     None)."""
     sys.path.insert(0, os.path.join(HERE, "oracle"))
-    import oracle as O  # noqa: E402  (checker / baseline only)
+    import oracle as O  # noqa: E402  (the oracle: reference results and CPU baseline only)
 
     g = O.OracleGrid(wl.width, wl.height, wl.cell_size)
     g.configure(wl.liquid_density, wl.gas_density)
@@ -486,7 +486,7 @@ def precision_leg(size=2048, seed=3, steps=3, kernel_reps=50, stall_budget=400, 
     out = {"workload": f"obstacle_tank {size}x{size}: 40 circles/boxes over {mask.mean():.3f} of the cells, "
                        f"liquid in the bottom 70% (1000:1), vortex velocity, seed {seed}; one projection per "
                        "solve to 1e-6 of the initial max divergence", "modes": {}}
-    # the FP64 oracle's projection of the same input (checker only)
+    # the FP64 oracle's projection of the same input (reference only)
     sys.path.insert(0, os.path.join(HERE, "oracle"))
     import oracle as O  # noqa: E402
 
