@@ -858,9 +858,9 @@ struct FinishSetup {
         double t[2], e[2];
         Partials<kNT, 2, 1>().all(g.fold_up, g.fold_up_n, t, lds);
         Partials<kNT, 2, 1>().all(g.partials_tr, nb, e, lds);
-        const Outset o = outset(g, t);
         if (threadIdx.x != 0)
             return;
+        const Outset o = outset(g, t);
         S->bmax = t[1];
         S->tol = o.tol;
         if (o.zero) {
@@ -929,6 +929,7 @@ __global__ __launch_bounds__(kSmallTiles * kNT) void k_check_small(GridDev g, in
     t[0] = wave_sum(t[0]);
     t[1] = wave_max(t[1]);
     const Recurrence c = recurrence(g.S, t);
+    __syncthreads();   // every wavefront has read the scalar block before decide() changes it
     double e[2] = {0.0, 0.0};
     if (c.verify) {   // the same in every thread
         const int thread = threadIdx.x & (kNT - 1), tile = threadIdx.x / kNT;
@@ -970,6 +971,7 @@ struct FinishCheck {
         if (st != kRunning)
             return;
         const Recurrence c = recurrence(S, t);
+        __syncthreads();   // every wavefront has read the scalar block before decide() changes it
         double e[2] = {0.0, 0.0};
         if (c.verify)
             Partials<kNT, 2, 1>().all(g.partials_tr, nb, e, lds);

@@ -5,7 +5,7 @@ same state bit for bit (the same kernels' arithmetic, the reductions per grid in
 import numpy as np
 import pytest
 
-from fluidsim_amd import FS_PRECOND_DIAGONAL, FS_SMOOTHER_RED_BLACK, FluidGridHIP, batch_project
+from fluidsim_amd import FS_PRECOND_DIAGONAL, FS_PRECOND_MULTIGRID, FS_SMOOTHER_RED_BLACK, FluidGridHIP, batch_project
 from fluidsim_amd import workloads as WL
 
 pytestmark = pytest.mark.gpu
@@ -68,5 +68,41 @@ def test_batched_projections_are_the_single_ones(budget):
             assert r.max_divergence == ref.max_divergence and r.final_residual == ref.final_residual, key
             for a, b in zip(state(g), fields):
                 assert np.array_equal(a, b), key
+    for g in many:
+        g.destroy()
+
+
+@pytest.mark.parametrize("precond", [FS_PRECOND_DIAGONAL, FS_PRECOND_MULTIGRID])
+def test_small_checks_across_refreshed_residuals(precond):
+    """Grids of one to four tiles, whose check and decision share a launch of up to sixteen wavefronts, through solves that
+    refresh the residual every 32 iterations many times over: the batch's separate launches give the same bits,
+    time after time."""
+    many, dt = [], 1.0 / 120.0
+    for W, H in [(61, 47), (64, 64), (128, 32), (130, 10), (256, 16), (33, 16), (64, 17)]:
+        wl = WL.sloped_pool(W, H, 4.0)
+        g = FluidGridHIP(W, H, 4.0)
+        WL.load_into(g, wl)
+        g.setPressurePreconditioner(precond)
+        g.snapshotSave()
+        many.append(g)
+    expected = None
+    for _ in range(4):
+        got = []
+        for g in many:
+            g.snapshotRestore()
+            r = g.project(dt, 3000, 1e-9)
+            got.append((r.iterations, r.restarts, r.final_residual, r.max_divergence) + state(g))
+        for g in many:
+            g.snapshotRestore()
+        for g, r in zip(many, batch_project(many, dt, 3000, 1e-9)):
+            got.append((r.iterations, r.restarts, r.final_residual, r.max_divergence) + state(g))
+        n = len(many)
+        if precond == FS_PRECOND_DIAGONAL:
+            assert max(x[0] for x in got[:n]) > 100
+        for a, b in zip(got[:n], got[n:]):
+            assert all(np.array_equal(x, y) for x, y in zip(a, b))
+        expected = expected or got
+        for a, b in zip(got, expected):
+            assert all(np.array_equal(x, y) for x, y in zip(a, b))
     for g in many:
         g.destroy()
