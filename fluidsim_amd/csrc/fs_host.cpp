@@ -382,6 +382,8 @@ struct fs_context {
     PcgScalars* pinned = nullptr;   // host-pinned mirror of a grid's scalar block
     double* pinned_value = nullptr; // host-pinned landing slot of single device reductions
     hipEvent_t value_ready = nullptr; // recorded behind the kernel that writes it
+    void* vis_landing = nullptr;      // the allocation-free viscosity solve's read-back slot and event: its own, since
+    hipEvent_t vis_landed = nullptr;  // such a call may run beside another thread's work on this context's grids
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     DevBuf<BatchItem> batch_desc;           // descriptors of the last batched projection
     DevBuf<int> batch_maps;                 // its workgroup maps and lists
@@ -1835,6 +1837,8 @@ fs_status fs_context_create_ex(int device, int flags, fs_context** out)
         HIPC(hipHostMalloc((void**)&ctx->pinned, sizeof(PcgScalars), hipHostMallocDefault));
         HIPC(hipHostMalloc((void**)&ctx->pinned_value, sizeof(double), hipHostMallocDefault));
         HIPC(hipEventCreateWithFlags(&ctx->value_ready, hipEventDisableTiming));
+        HIPC(hipHostMalloc(&ctx->vis_landing, kViscosityLandingBytes, hipHostMallocDefault));
+        HIPC(hipEventCreateWithFlags(&ctx->vis_landed, hipEventDisableTiming));
         viscosity_scratch_setup(device);   // this device's copy of the allocation-free solve's scratch
         HIPC(hipEventCreate(&ctx->ev0));
         HIPC(hipEventCreate(&ctx->ev1));
@@ -1862,6 +1866,10 @@ fs_status fs_context_destroy(fs_context* ctx)
                 (void)hipHostFree(ctx->pinned_value);
             if (ctx->value_ready)
                 (void)hipEventDestroy(ctx->value_ready);
+            if (ctx->vis_landing)
+                (void)hipHostFree(ctx->vis_landing);
+            if (ctx->vis_landed)
+                (void)hipEventDestroy(ctx->vis_landed);
             if (ctx->batch_pinned)
                 (void)hipHostFree(ctx->batch_pinned);
             if (ctx->staging)
@@ -2914,7 +2922,6 @@ fs_status fs_viscosity_solve_noalloc(fs_context* ctx, int width, int height, dou
             "null pointer");
         need(width > 0 && height > 0 && cell_size > 0.0, FS_E_INVALID_ARGUMENT, "invalid grid shape");
         need(std::isfinite(tolerance) && tolerance >= 0.0, FS_E_INVALID_ARGUMENT, "invalid tolerance");
-        static_assert(sizeof(PcgScalars) >= kViscosityLandingBytes, "the context's pinned slot holds the scalars");
         need((long long)width * height <= (1LL << 26) && viscosity_scratch_bytes(width, height) <= kViscosityScratchBytes,
             FS_E_INVALID_ARGUMENT, "grid too large for the allocation-free viscosity solve's 64 MiB scratch");
         set_device(ctx);
@@ -2922,7 +2929,7 @@ fs_status fs_viscosity_solve_noalloc(fs_context* ctx, int width, int height, dou
         double rel = 0.0;
         const int budget = max_iterations < 0 ? kViscosityBudget : max_iterations;
         const int status = viscosity_solve_scratch(ctx->device, ctx->stream, width, height, u, v, material, dt,
-            cell_size, tolerance, budget, ctx->pinned, ctx->value_ready, &it, &rel);
+            cell_size, tolerance, budget, ctx->vis_landing, ctx->vis_landed, &it, &rel);
         if (iterations)
             *iterations = it;
         if (relative_residual)
