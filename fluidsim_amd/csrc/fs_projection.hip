@@ -185,7 +185,13 @@ __device__ __forceinline__ void coarsen_tile(const ChainLevel& L, int column, in
     }
 }
 
-__global__ __launch_bounds__(kCoarsenThreads) void k_coarsen(ChainLevel L) { coarsen_tile(L, blockIdx.x, blockIdx.y); }
+// One-dimensional: the tiles of a tall level are more than a launch has rows (65536).
+__global__ __launch_bounds__(kCoarsenThreads) void k_coarsen(ChainLevel L)
+{
+    const int columns = (L.cw + kTX - 1) / kTX;
+    const int row = (int)blockIdx.x / columns;
+    coarsen_tile(L, (int)blockIdx.x - row * columns, row);
+}
 
 // ------------------------------------------------------------------------------------------
 // Projection set-up (FluidGridCPU.cpp:1050-1090, :1728-1756), FP64.
@@ -1126,8 +1132,7 @@ void launch_coefficients(hipStream_t st, const GridDev& g) { launch_cells<Coeffi
 
 void launch_coarsen(hipStream_t st, const ChainLevel& level)
 {
-    hipLaunchKernelGGL(k_coarsen, dim3((level.cw + kTX - 1) / kTX, (level.ch + kCoarsenY - 1) / kCoarsenY),
-        dim3(kCoarsenThreads), 0, st, level);
+    hipLaunchKernelGGL(k_coarsen, dim3(batch_coarsen_blocks(level)), dim3(kCoarsenThreads), 0, st, level);
 }
 
 void launch_project_setup(hipStream_t st, const GridDev& g)

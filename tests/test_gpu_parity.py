@@ -54,7 +54,7 @@ def test_dam_break_projection_matches_oracle(oracle):
 
 
 @pytest.mark.parametrize("w,h", [(128, 128), (65, 37), (1, 129), (131, 1), (13, 9), (300, 200), (2, 67), (1, 1),
-                                 (4000, 3), (2, 3000), (1000, 700)])
+                                 (4000, 3), (2, 3000), (1000, 700), (2, 530000)])
 def test_hierarchy_is_bit_exact(oracle, w, h):
     wl = WL.sloped_pool(w, h, 4.0)
     o = oracle_grid(oracle, wl)
