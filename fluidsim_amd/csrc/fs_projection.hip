@@ -1102,9 +1102,11 @@ template <class Op> void launch_finish(hipStream_t st, const GridDev& g)
     hipLaunchKernelGGL(k_finish<Op>, dim3(1), dim3(kNT), 0, st, g, pcg_blocks(g.W, g.H));
 }
 
-template <int NC, int NSUM> void fold(hipStream_t st, const GridDev& g, const double* partials, double* out, int out_n)
+// Where the partials are reduced in place of every consumer: elsewhere `out` is the producer's own (a grid of one tile
+// has a single partial as well).
+template <int NC, int NSUM> void fold(hipStream_t st, const GridDev& g, const double* partials, double* out)
 {
-    if (out_n == 1)
+    if (out != partials)
         hipLaunchKernelGGL((k_fold_partials<NC, NSUM>), dim3(1), dim3(kNT), 0, st, partials, pcg_blocks(g.W, g.H), out);
 }
 
@@ -1138,9 +1140,9 @@ void launch_coarsen(hipStream_t st, const ChainLevel& level)
 void launch_project_setup(hipStream_t st, const GridDev& g)
 {
     launch_cells<Rhs>(st, g);
-    fold<1, 1>(st, g, g.partials_ad, g.fold_ad, g.fold_ad_n);
+    fold<1, 1>(st, g, g.partials_ad, g.fold_ad);
     launch_cells<Predict>(st, g);
-    fold<2, 1>(st, g, g.partials_up, g.fold_up, g.fold_up_n);
+    fold<2, 1>(st, g, g.partials_up, g.fold_up);
     launch_cells<InitialResidual>(st, g);
     launch_finish<FinishSetup>(st, g);
 }
@@ -1148,7 +1150,7 @@ void launch_project_setup(hipStream_t st, const GridDev& g)
 void launch_project_end(hipStream_t st, const GridDev& g)
 {
     launch_cells<FinalSum>(st, g);
-    fold<1, 1>(st, g, g.partials_ad, g.fold_ad, g.fold_ad_n);
+    fold<1, 1>(st, g, g.partials_ad, g.fold_ad);
     launch_cells<CorrectVelocity>(st, g);
     launch_cells<MaxDivergence<true>>(st, g);
     launch_finish<FinishDivergence<true>>(st, g);
@@ -1166,13 +1168,13 @@ void launch_pcg_direction_ad(hipStream_t st, const GridDev& g, int flexible)
         launch_cells<DirectionAd<true>>(st, g);
     else
         launch_cells<DirectionAd<false>>(st, g);
-    fold<1, 1>(st, g, g.partials_ad, g.fold_ad, g.fold_ad_n);
+    fold<1, 1>(st, g, g.partials_ad, g.fold_ad);
 }
 
 void launch_pcg_update(hipStream_t st, const GridDev& g)
 {
     launch_cells<Update>(st, g);
-    fold<2, 1>(st, g, g.partials_up, g.fold_up, g.fold_up_n);
+    fold<2, 1>(st, g, g.partials_up, g.fold_up);
 }
 
 void launch_pcg_check(hipStream_t st, const GridDev& g)
@@ -1190,10 +1192,10 @@ void launch_pcg_rz(hipStream_t st, const GridDev& g, int flexible)
 {
     if (flexible) {
         launch_cells<Rz<true>>(st, g);
-        fold<5, 5>(st, g, g.partials, g.fold_rz, g.fold_rz_n);
+        fold<5, 5>(st, g, g.partials, g.fold_rz);
     } else {
         launch_cells<Rz<false>>(st, g);
-        fold<3, 3>(st, g, g.partials, g.fold_rz, g.fold_rz_n);
+        fold<3, 3>(st, g, g.partials, g.fold_rz);
     }
 }
 

@@ -72,3 +72,18 @@ def test_a_spent_budget_stops_the_solve(budget):
     res = g.project(wl.dt, budget, 1e-14)
     assert not res.converged and res.iterations == budget
     g.destroy()
+
+
+def test_a_single_tile_reduces_no_partials_apart():
+    """The update of a grid of one 64 x 16 tile is one launch, as on a grid of two (a second one, reducing the single
+    partial into itself, would double it)."""
+    def fastest(H):
+        wl = box(64, H, 5)
+        g = FluidGridHIP(64, H, wl.cell_size)
+        WL.load_into(g, wl)
+        g.project(wl.dt, 3, TOL)
+        ms = min(g.timeKernel(2, 500) for _ in range(8))
+        g.destroy()
+        return ms
+    one, two = fastest(16), fastest(17)
+    assert one < 1.4 * two, (one, two)
