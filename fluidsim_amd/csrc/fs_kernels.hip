@@ -80,7 +80,25 @@ __global__ __launch_bounds__(kNT) void k_add_vortex(GridDev g, double ox, double
 
 // ---- semi-Lagrangian transport mode (build-defined; samples as FluidGridCPU::sampleVelocity) ----
 // Bound by FP64 issue (six divisions and 15 interpolations a face): std::lerp and std::clamp are written for what holds
-// here, and a 2-D launch needs no division for the cell.  1024^2 faces 47 -> 37 us, cells 31 -> 25.
+// here, and an element's row comes from a multiplication instead of divisions.  A call on 1024^2 cells 103 -> 71 us,
+// 2 x 100000 51 -> 33.  (Workgroups of 64 x 4 elements need no row at all, but leave lanes idle on narrow grids: 76
+// and 320 us.)
+
+// n / d of 0 <= n < 2^31 as one multiplication: with 2^(s-1) < d <= 2^s, magic = ceil(2^(31+s) / d) is too large by
+// less than 2^s / d parts in 2^(31+s), which is less than 1 / d after the multiplication by n.
+struct Divisor {
+    unsigned magic;
+    int shift;
+    explicit Divisor(unsigned d)
+    {
+        int s = 0;
+        while ((1u << s) < d)
+            ++s;
+        shift = 31 + s;
+        magic = (unsigned)((((unsigned long long)1 << shift) + d - 1) / d);
+    }
+    __device__ __forceinline__ int of(unsigned n) const { return (int)(((unsigned long long)n * magic) >> shift); }
+};
 
 // std::lerp for 0 <= t < 1 (its exact ends beyond that cannot occur).
 __device__ __forceinline__ double lerp_std(double a, double b, double t)
@@ -124,53 +142,51 @@ __device__ __forceinline__ void backtrace(const GridDev& g, double ox, double oy
     *sy = py - dt * vy;
 }
 
-__global__ __launch_bounds__(kNT) void k_sl_faces(GridDev g, double ox, double oy, double dt, double* nu,
-    double* nv)
+__global__ __launch_bounds__(kNT) void k_sl_faces(GridDev g, double ox, double oy, double dt, Divisor u_row,
+    Divisor v_row, double* nu, double* nv)
 {
     const int W = g.W, H = g.H;
-    const int x = blockIdx.x * 64 + (threadIdx.x & 63);
-    for (int y = blockIdx.y * (kNT / 64) + (threadIdx.x >> 6); y <= H; y += gridDim.y * (kNT / 64)) {
-        double value = 0.0, sx, sy;
-        if (blockIdx.z == 0) {
-            if (x > W || y >= H)
-                return;
-            if (x >= 1 && x < W) {
-                backtrace(g, ox, oy, ox + x * g.h, oy + (y + 0.5) * g.h, dt, &sx, &sy);
-                value = sample_scalar(g.u, W + 1, H, (sx - ox) / g.h, (sy - oy) / g.h - 0.5);
-            }
-            nu[(size_t)y * (W + 1) + x] = value;
-        } else {
-            if (x >= W)
-                return;
-            if (y >= 1 && y < H) {
-                backtrace(g, ox, oy, ox + (x + 0.5) * g.h, oy + y * g.h, dt, &sx, &sy);
-                value = sample_scalar(g.v, W, H + 1, (sx - ox) / g.h - 0.5, (sy - oy) / g.h);
-            }
-            nv[(size_t)y * W + x] = value;
+    const int t = blockIdx.x * kNT + threadIdx.x;
+    double value = 0.0, sx, sy;
+    if (blockIdx.y == 0) {
+        const int y = u_row.of(t), x = t - y * (W + 1);
+        if (y >= H)
+            return;
+        if (x >= 1 && x < W) {
+            backtrace(g, ox, oy, ox + x * g.h, oy + (y + 0.5) * g.h, dt, &sx, &sy);
+            value = sample_scalar(g.u, W + 1, H, (sx - ox) / g.h, (sy - oy) / g.h - 0.5);
         }
+        nu[t] = value;
+    } else {
+        const int y = v_row.of(t), x = t - y * W;
+        if (y > H)
+            return;
+        if (y >= 1 && y < H) {
+            backtrace(g, ox, oy, ox + (x + 0.5) * g.h, oy + y * g.h, dt, &sx, &sy);
+            value = sample_scalar(g.v, W, H + 1, (sx - ox) / g.h - 0.5, (sy - oy) / g.h);
+        }
+        nv[t] = value;
     }
 }
 
 // Cell-centred scalars (fraction, every component mass) share one backtrace per cell.
-__global__ __launch_bounds__(kNT) void k_sl_cells(GridDev g, double ox, double oy, double dt, double* fraction,
-    double* lmass, double* gmass)
+__global__ __launch_bounds__(kNT) void k_sl_cells(GridDev g, double ox, double oy, double dt, Divisor row,
+    double* fraction, double* lmass, double* gmass)
 {
     const int W = g.W, H = g.H;
     const size_t N = (size_t)W * H;
-    const int x = blockIdx.x * 64 + (threadIdx.x & 63);
-    if (x >= W)
+    const int i = blockIdx.x * kNT + threadIdx.x;
+    const int y = row.of(i), x = i - y * W;
+    if (y >= H)
         return;
-    for (int y = blockIdx.y * (kNT / 64) + (threadIdx.x >> 6); y < H; y += gridDim.y * (kNT / 64)) {
-        const size_t i = (size_t)y * W + x;
-        double sx, sy;
-        backtrace(g, ox, oy, ox + (x + 0.5) * g.h, oy + (y + 0.5) * g.h, dt, &sx, &sy);
-        const double fx = (sx - ox) / g.h - 0.5, fy = (sy - oy) / g.h - 0.5;
-        fraction[i] = sample_scalar(g.fraction, W, H, fx, fy);
-        for (int k = 0; k < g.nl; ++k)
-            lmass[(size_t)k * N + i] = sample_scalar(g.lmass + (size_t)k * N, W, H, fx, fy);
-        for (int k = 0; k < g.ng; ++k)
-            gmass[(size_t)k * N + i] = sample_scalar(g.gmass + (size_t)k * N, W, H, fx, fy);
-    }
+    double sx, sy;
+    backtrace(g, ox, oy, ox + (x + 0.5) * g.h, oy + (y + 0.5) * g.h, dt, &sx, &sy);
+    const double fx = (sx - ox) / g.h - 0.5, fy = (sy - oy) / g.h - 0.5;
+    fraction[i] = sample_scalar(g.fraction, W, H, fx, fy);
+    for (int k = 0; k < g.nl; ++k)
+        lmass[(size_t)k * N + i] = sample_scalar(g.lmass + (size_t)k * N, W, H, fx, fy);
+    for (int k = 0; k < g.ng; ++k)
+        gmass[(size_t)k * N + i] = sample_scalar(g.gmass + (size_t)k * N, W, H, fx, fy);
 }
 
 __global__ __launch_bounds__(kNT) void k_pad_copy(const double* src, double* dst, int W, int H, int to_padded)
@@ -285,11 +301,12 @@ void launch_add_vortex(hipStream_t st, const GridDev& g, double ox, double oy, d
 void launch_semi_lagrangian(hipStream_t st, const GridDev& g, double ox, double oy, double dt, double* new_u,
     double* new_v, double* new_fraction, double* new_lmass, double* new_gmass)
 {
-    constexpr int rows = kNT / 64;
-    const unsigned gy = (unsigned)std::min((g.H + 1 + rows - 1) / rows, 65535);   // rows beyond that in further turns
-    hipLaunchKernelGGL(k_sl_faces, dim3((g.W + 1 + 63) / 64, gy, 2), dim3(kNT), 0, st, g, ox, oy, dt, new_u, new_v);
-    hipLaunchKernelGGL(k_sl_cells, dim3((g.W + 63) / 64, gy), dim3(kNT), 0, st, g, ox, oy, dt, new_fraction, new_lmass,
-        new_gmass);
+    const auto blocks = [](size_t n) { return (unsigned)((n + kNT - 1) / kNT); };
+    const size_t nu = (size_t)(g.W + 1) * g.H, nv = (size_t)g.W * (g.H + 1);
+    hipLaunchKernelGGL(k_sl_faces, dim3(blocks(std::max(nu, nv)), 2), dim3(kNT), 0, st, g, ox, oy, dt,
+        Divisor((unsigned)g.W + 1), Divisor((unsigned)g.W), new_u, new_v);
+    hipLaunchKernelGGL(k_sl_cells, dim3(blocks((size_t)g.W * g.H)), dim3(kNT), 0, st, g, ox, oy, dt,
+        Divisor((unsigned)g.W), new_fraction, new_lmass, new_gmass);
 }
 
 void launch_pad_copy(hipStream_t st, const double* src, double* dst, int W, int H, int to_padded)
