@@ -1114,7 +1114,13 @@ template <int NC, int NSUM> void fold(hipStream_t st, const GridDev& g, const do
 
 // Tiles per workgroup: a consumer workgroup reads every producer workgroup's partial, blocks^2 loads in all, which shows
 // past about a thousand workgroups; four tiles each keep a 2048 x 2048 grid at 1024.  k_fold_partials takes over beyond.
-int pcg_groups(int W, int H) { return (size_t)((W + kTX - 1) / kTX) * ((H + kTY - 1) / kTY) > 1024 ? 4 : 1; }
+// A single row of tiles leaves three of four empty: 100000 x 16 projects in 3190 us with four and 2970 with one, 60000 x 32
+// (two rows) in 5190 and 5340.
+int pcg_groups(int W, int H)
+{
+    const int rows = (H + kTY - 1) / kTY;
+    return rows > 1 && (size_t)((W + kTX - 1) / kTX) * rows > 1024 ? 4 : 1;
+}
 int pcg_blocks(int W, int H)
 {
     return ((W + kTX - 1) / kTX) * (((H + kTY - 1) / kTY + pcg_groups(W, H) - 1) / pcg_groups(W, H));
@@ -1156,10 +1162,13 @@ void launch_project_end(hipStream_t st, const GridDev& g)
     launch_finish<FinishDivergence<true>>(st, g);
 }
 
+// A tile per workgroup on every grid: only the finish reads the partials (1100 x 1050 cells 19.8 us, 20.4 with the
+// solve's four).
 void launch_max_divergence(hipStream_t st, const GridDev& g)
 {
-    launch_cells<MaxDivergence<false>>(st, g);
-    launch_finish<FinishDivergence<false>>(st, g);
+    const dim3 tiles((g.W + kTX - 1) / kTX, (g.H + kTY - 1) / kTY);
+    hipLaunchKernelGGL((k_cells<MaxDivergence<false>, 1>), tiles, dim3(kNT), 0, st, g);
+    hipLaunchKernelGGL(k_finish<FinishDivergence<false>>, dim3(1), dim3(kNT), 0, st, g, (int)(tiles.x * tiles.y));
 }
 
 void launch_pcg_direction_ad(hipStream_t st, const GridDev& g, int flexible)

@@ -1,5 +1,6 @@
 """Projections at the edges of the PCG kernels' tiles: 64 x 16 cells per tile, one or four tiles per workgroup
-(more than 1024 tiles), pre-reduced partials (more than 1024 workgroups), grids of one row or column.
+(more than 1024 tiles in more than one row), pre-reduced partials (more than 1024 workgroups), grids of one row or
+column.
 
 One constant density, so the Neumann problem is diagonal in cosines and the exact velocity is known in 64 bits.
 A solve that stops at max|b - A p| <= tol max|b| leaves, with L the unit-weight Laplacian (L = G^T G, G the face
@@ -47,7 +48,7 @@ def exact(wl):
 
 @pytest.mark.parametrize("smoother", [(FS_SMOOTHER_RED_BLACK, 4, 4), (FS_SMOOTHER_CHEBYSHEV, 3, 2)])
 @pytest.mark.parametrize("W,H", [(2, 1), (1, 130), (64, 16), (65, 17), (63, 145), (300, 111), (1025, 1030),
-                                 (2112, 2050)])
+                                 (2112, 2050), (66000, 3), (35000, 20), (22000, 40)])
 def test_projection_matches_the_exact_one(W, H, smoother):
     wl = box(W, H, 7 * W + H)
     eu, ev, bound = exact(wl)
@@ -87,3 +88,18 @@ def test_a_single_tile_reduces_no_partials_apart():
         return ms
     one, two = fastest(16), fastest(17)
     assert one < 1.4 * two, (one, two)
+
+
+def test_flat_grids_visit_no_empty_tiles():
+    """r.z of a grid of one row of 1563 tiles is a launch over them and one that reduces their partials: less than twice
+    what a square grid of about as many cells takes for the first alone."""
+    def fastest(W, H):
+        wl = box(W, H, 5)
+        g = FluidGridHIP(W, H, wl.cell_size)
+        WL.load_into(g, wl)
+        g.project(wl.dt, 3, TOL)
+        ms = min(g.timeKernel(9, 300) for _ in range(8))
+        g.destroy()
+        return ms
+    flat, square = fastest(100000, 16), fastest(1265, 1265)
+    assert flat < 2.0 * square, (flat, square)
