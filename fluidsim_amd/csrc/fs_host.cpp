@@ -960,6 +960,11 @@ struct fs_grid {
         ChainDesc chain{};
         for (size_t l = from; l < levels.size(); ++l)
             chain.lev[chain.levels++] = chain_level(l);
+        const Level& last = levels.back();
+        chain.w = last.w;
+        chain.h = last.h;
+        chain.right = last.right64.p;
+        chain.down = last.down64.p;
         return chain;
     }
 
@@ -1472,7 +1477,7 @@ struct fs_grid {
     // Whether this grid's projection can be part of a batched one: decided by its shape and settings alone.
     bool batchable() const
     {
-        return batch_cell_blocks(W, H) <= kBatchTiles && tail_start <= kMaxBatchLevels && levels.size() >= 2 &&
+        return batch_cell_blocks(W, H) <= kBatchTiles && tail_start <= kMaxBatchLevels &&
                (int)chain_from() <= kMaxBatchLevels + 2 && !flexible();
     }
 

@@ -137,8 +137,10 @@ struct ChainLevel {
     float *right32, *down32, *invd32;           // and their FP32 copies and 1/diagonal (written)
 };
 struct ChainDesc {
-    int levels;
+    int levels;                                 // none on a grid of one level
     ChainLevel lev[kMaxTailLevels];
+    int w, h;                                   // the coarsest level and its FP64 conductances
+    const double *right, *down;
 };
 // One level coarsened from its finer one, with its FP32 copies and 1/diagonal.
 void launch_coarsen(hipStream_t st, const ChainLevel& level);

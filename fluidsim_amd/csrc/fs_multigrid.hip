@@ -456,10 +456,8 @@ __device__ __forceinline__ void coarse_chain(const ChainDesc& C, float* ginv, in
         }
         __syncthreads();
     }
-    if (n > 0) {
-        const ChainLevel& L = C.lev[C.levels - 1];
-        coarse_inverse(L.cw, L.ch, L.cright, L.cdown, ginv, n, S, pin);
-    }
+    if (n > 0)
+        coarse_inverse(C.w, C.h, C.right, C.down, ginv, n, S, pin);
 }
 
 __global__ __launch_bounds__(64 * kSweepWaves) void k_coarse_chain(const ChainDesc C, float* ginv, int n,

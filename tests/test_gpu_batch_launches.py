@@ -2,6 +2,8 @@
 that only the LDS tail takes, more tiles than are batched (solved on their own), with masks, both preconditioners,
 several sweep counts, absolute and relative tolerances and spent budgets.  Every grid's result is fs_project's on the
 same state bit for bit (the same kernels' arithmetic, the reductions per grid in the same order)."""
+import time
+
 import numpy as np
 import pytest
 
@@ -106,3 +108,23 @@ def test_small_checks_across_refreshed_residuals(precond):
             assert all(np.array_equal(x, y) for x, y in zip(a, b))
     for g in many:
         g.destroy()
+
+
+def test_grids_of_one_level_share_launches():
+    """Sixteen 8 x 8 grids in a batch take little longer than two (one after another they would take eight times as long)."""
+    def fastest(n):
+        many = []
+        for _ in range(n):
+            wl = WL.sloped_pool(8, 8, 4.0)
+            g = FluidGridHIP(8, 8, 4.0)
+            WL.load_into(g, wl)
+            many.append(g)
+        times = []
+        for _ in range(8):
+            t = time.perf_counter()
+            batch_project(many, 1.0 / 120.0, 20, 1e-5)
+            times.append(time.perf_counter() - t)
+        for g in many:
+            g.destroy()
+        return min(times)
+    assert fastest(16) < 4.0 * fastest(2)
