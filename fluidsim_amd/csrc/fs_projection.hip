@@ -98,7 +98,7 @@ __global__ void k_merge_failure(const PcgScalars* from, PcgScalars* S)
 // three: the tile's densities and those around it are summed once into LDS, and the faces left of and above a cell
 // are formed again instead of read back.
 // ------------------------------------------------------------------------------------------
-struct Coefficients {
+template <bool SUM> struct Coefficients {
     template <int G> __device__ __forceinline__ void run(const GridDev& g, Block B) const
     {
         constexpr int LX = kTX + 2, LY = kTY + 2, LOADS = (LX * LY + kNT - 1) / kNT;
@@ -110,19 +110,40 @@ struct Coefficients {
             const int row = B.y * G + group;
             if (group)
                 __syncthreads();
+            size_t at[LOADS];
+            double rho[LOADS] = {};
 #pragma unroll
             for (int it = 0; it < LOADS; ++it) {
                 const int e = min((int)threadIdx.x + it * kNT, LX * LY - 1);
                 const int ly = e / LX, lx = e - ly * LX;
                 const int x = min(max(B.x * kTX - 1 + lx, 0), W - 1), y = min(max(row * kTY - 1 + ly, 0), H - 1);
-                const size_t i = (size_t)y * W + x;
-                double total = 0.0;
-                for (int k = 0; k < g.nl; ++k)
-                    total += g.lmass[(size_t)k * N + i];
-                for (int k = 0; k < g.ng; ++k)
-                    total += g.gmass[(size_t)k * N + i];
-                s_rho[e] = total * inverse_cell_volume;
+                at[it] = (size_t)y * W + x;
             }
+            // component by component, the loads of two together: a cell's components one after another left a thread
+            // one load in flight (8 + 8 components at 1920 x 1080 cells: 298 us for a capillary force, 205 so; 300 x 200 61 and 44)
+            auto add = [&](const double* mass, int n) {
+                for (int k = 0; k < n; k += 2) {
+                    double m[2][LOADS];
+#pragma unroll
+                    for (int j = 0; j < 2; ++j)
+#pragma unroll
+                        for (int it = 0; it < LOADS; ++it)
+                            m[j][it] = mass[(size_t)min(k + j, n - 1) * N + at[it]];
+#pragma unroll
+                    for (int j = 0; j < 2; ++j)
+#pragma unroll
+                        for (int it = 0; it < LOADS; ++it)
+                            rho[it] += k + j < n ? m[j][it] : 0.0;
+                }
+            };
+            if constexpr (SUM) {
+                add(g.lmass, g.nl);
+                add(g.gmass, g.ng);
+            }
+#pragma unroll
+            for (int it = 0; it < LOADS; ++it)
+                s_rho[min((int)threadIdx.x + it * kNT, LX * LY - 1)] =
+                    SUM ? rho[it] * inverse_cell_volume : g.density[at[it]];
             __syncthreads();
             const Tile4 T = tile4(g, B.x, row);
 #pragma unroll
@@ -143,7 +164,8 @@ struct Coefficients {
                     const double rl = wl ? 2.0 / (s_rho[e - 1] + c) : 0.0, rr = wr ? 2.0 / (c + s_rho[e + 1]) : 0.0;
                     const double du = wu ? 2.0 / (s_rho[e - LX] + c) : 0.0, dd = wd ? 2.0 / (c + s_rho[e + LX]) : 0.0;
                     const int P = T.P[k];
-                    g.density[(size_t)y * W + x] = c;
+                    if (SUM)
+                        g.density[(size_t)y * W + x] = c;
                     g.right64[P] = rr;
                     g.down64[P] = dd;
                     level_diag_values(rl, rr, du, dd, g.invd32[P], g.right32[P], g.down32[P]);
@@ -1136,7 +1158,19 @@ void launch_merge_failure(hipStream_t st, const PcgScalars* from, PcgScalars* S)
     hipLaunchKernelGGL(k_merge_failure, dim3(1), dim3(64), 0, st, from, S);
 }
 
-void launch_coefficients(hipStream_t st, const GridDev& g) { launch_cells<Coefficients>(st, g); }
+// A tile's halo is a sixth of its cells, and their components are read again: past twelve components on a large grid the
+// densities take a launch of their own (a capillary force with 20 + 20 components: 1920 x 1080 279 us against 305 in one
+// launch, 8 + 8 199 against 205, 1024^2 161 against 166; a small grid's launch costs more than it saves, 300 x 200 53
+// against 49).
+void launch_coefficients(hipStream_t st, const GridDev& g)
+{
+    if (g.nl + g.ng > 12 && batch_cell_blocks(g.W, g.H) >= 1024) {
+        launch_density(st, g);
+        launch_cells<Coefficients<false>>(st, g);
+    } else {
+        launch_cells<Coefficients<true>>(st, g);
+    }
+}
 
 void launch_coarsen(hipStream_t st, const ChainLevel& level)
 {
@@ -1224,7 +1258,7 @@ void launch_batch_init(hipStream_t st, const BatchItem* items, const int* list, 
 
 void launch_batch_coefficients(hipStream_t st, const BatchItem* items, const BatchPart& part)
 {
-    launch_cells_batch<Coefficients>(st, items, part);
+    launch_cells_batch<Coefficients<true>>(st, items, part);
 }
 
 void launch_batch_coarsen(hipStream_t st, const BatchItem* items, const BatchPart& part, int level)
