@@ -205,6 +205,26 @@ __device__ __forceinline__ double wave_max(double v)
     return wave_combine(v, [](double a, double b) { return fmax(a, b); });
 }
 
+// Lane l receives the value of lane l - 1 / l + 1 (zero at the wavefront's end).
+__device__ __forceinline__ float from_left(float v)
+{
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x138, 0xf, 0xf, true));
+}
+__device__ __forceinline__ float from_right(float v)
+{
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x130, 0xf, 0xf, true));
+}
+__device__ __forceinline__ double from_left(double v)
+{
+    return __hiloint2double(__builtin_amdgcn_update_dpp(0, __double2hiint(v), 0x138, 0xf, 0xf, true),
+        __builtin_amdgcn_update_dpp(0, __double2loint(v), 0x138, 0xf, 0xf, true));
+}
+__device__ __forceinline__ double from_right(double v)
+{
+    return __hiloint2double(__builtin_amdgcn_update_dpp(0, __double2hiint(v), 0x130, 0xf, 0xf, true),
+        __builtin_amdgcn_update_dpp(0, __double2loint(v), 0x130, 0xf, 0xf, true));
+}
+
 // Block-wide sum in a fixed order; result valid in thread 0.  `lds` holds blockDim/64 doubles.
 template <int NT> __device__ __forceinline__ double block_sum(double v, double* lds)
 {
@@ -243,44 +263,8 @@ template <int NT> __device__ __forceinline__ double block_max(double v, double* 
 // Reads a partial written by another block of the previous launch.
 __device__ __forceinline__ double load_partial(const double* p, int i) { return p[i]; }
 
-// Sum of `n` partials with stride `k` starting at `offset`, in a fixed order; every thread returns it.
-// Loads run eight (then four) strides ahead of the additions (independent loads in flight instead of one memory
-// latency per partial); the additions keep the one-stride-at-a-time order, so the sum is unchanged.
-template <int NT>
-__device__ __forceinline__ double finish_sum(const double* partials, int n, int k, int offset, double* lds)
-{
-    double v = 0.0;
-    int i = threadIdx.x;
-    for (; i + 7 * NT < n; i += 8 * NT) {
-        double t[8];
-#pragma unroll
-        for (int u = 0; u < 8; ++u)
-            t[u] = load_partial(partials, (i + u * NT) * k + offset);
-#pragma unroll
-        for (int u = 0; u < 8; ++u)
-            v += t[u];
-    }
-    for (; i + 3 * NT < n; i += 4 * NT) {
-        double t[4];
-#pragma unroll
-        for (int u = 0; u < 4; ++u)
-            t[u] = load_partial(partials, (i + u * NT) * k + offset);
-#pragma unroll
-        for (int u = 0; u < 4; ++u)
-            v += t[u];
-    }
-    for (; i < n; i += NT)
-        v += load_partial(partials, i * k + offset);
-    double r = block_sum<NT>(v, lds);
-    __shared__ double out;
-    if (threadIdx.x == 0)
-        out = r;
-    __syncthreads();
-    r = out;
-    __syncthreads();
-    return r;
-}
-
+// Maximum of `n` partials with stride `k` starting at `offset`; every thread returns it.
+// Loads run eight (then four) strides ahead (independent loads in flight instead of one memory latency per partial).
 template <int NT>
 __device__ __forceinline__ double finish_max(const double* partials, int n, int k, int offset, double* lds)
 {
@@ -340,8 +324,8 @@ template <int NT, int NC> __device__ __forceinline__ void block_sums(double (&v)
     }
 }
 
-// The NC interleaved components of `n` partials reduced by every workgroup for itself, in finish_sum's order
-// (component c < NSUM summed, the others their maximum).  load() only issues the loads of up to kAhead strides,
+// The NC interleaved components of `n` partials reduced by every workgroup for itself, a thread's in steps of NT and then
+// the threads' in block_sum's order (component c < NSUM summed, the others their maximum).  load() only issues the loads of up to kAhead strides,
 // through clamped indices, so that a kernel's other loads travel with them; finish() adds them up with two barriers
 // for all components, and every thread returns the values.
 template <int NT, int NC, int NSUM = NC> struct Partials {

@@ -532,7 +532,6 @@ struct fs_grid {
     std::vector<Level> levels;
     int tail_start = 0;
     TailDesc tail{};
-    DevBuf<TailDesc> tail_dev;
     DevBuf<unsigned> tail_tables;
     DevBuf<float4> tail_pairs;
 
@@ -932,8 +931,6 @@ struct fs_grid {
             limit = 65536 - 4096;  // the device refused a larger dynamic LDS request
         }
         build_pair_tables();
-        bytes += tail_dev.alloc(1);
-        device_upload(tail_dev.p, &tail, sizeof(TailDesc));
     }
 
     // ---------------------------------------------------------------------------------------
@@ -1027,8 +1024,6 @@ struct fs_grid {
         if (coarse != coarse_sweeps) {
             coarse_sweeps = coarse;
             tail.sweeps = coarse;
-            if (tail_dev.p)
-                device_upload(tail_dev.p, &tail, sizeof(TailDesc));
         }
         drop_graph();
         if (kind == FS_SMOOTHER_CHEBYSHEV && !levels.empty() && !jacobi_tuned)

@@ -26,7 +26,7 @@ struct GridDev {
     float* invd32;            // padded 1/diagonal (FP32), level 0 and the diagonal preconditioner
     float* x;                 // padded FP32 correction accumulated since the last flush
     float* r;                 // padded FP32 residual
-    float* d;                 // padded FP32 direction (of the even iterations; the batched solve's only one)
+    float* d;                 // padded FP32 direction of the even iterations
     float* d2;                // padded FP32 direction of the odd iterations
     float* q;                 // padded FP32 A d
     float* zdiag;             // padded FP32 diagonal-preconditioned residual

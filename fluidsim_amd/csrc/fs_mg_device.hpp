@@ -25,6 +25,11 @@ template <> __device__ __forceinline__ bf16 stv<bf16>(float f)
     return bf16{(unsigned short)((u + 0x7fffu + ((u >> 16) & 1u)) >> 16)};
 }
 
+// Two neighbouring values, element-aligned (one load where the hardware allows it).
+template <class T> struct __attribute__((packed, aligned(alignof(T)))) Pair {
+    T a, b;
+};
+
 // XCD-aware tile order.  Workgroups of a launch are dealt to the 8 XCDs round-robin (workgroup b runs
 // on XCD b % 8), each XCD with its own L2.  Mapping the workgroups an XCD receives onto a contiguous
 // run of row-major tiles keeps neighbouring tiles, whose 8-cell halos overlap, on the same L2.  The

@@ -22,27 +22,11 @@
 #include "fs_kernels.hpp"
 #include "fs_mg_device.hpp"
 
-#include <algorithm>
 #include <type_traits>
 
 namespace fsim {
 
 namespace {
-
-// lane l receives the value of lane l - 1 / l + 1 (zero at the wavefront's end)
-__device__ __forceinline__ float from_left(float v)
-{
-    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x138, 0xf, 0xf, true));
-}
-__device__ __forceinline__ float from_right(float v)
-{
-    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x130, 0xf, 0xf, true));
-}
-
-// Two neighbouring values, element-aligned (one load where the hardware allows it).
-template <class T> struct __attribute__((packed, aligned(alignof(T)))) Pair {
-    T a, b;
-};
 
 enum RowsMode : int { kRowsPre = 0, kRowsPost = 1, kRowsPreRestrict = 2 };
 
@@ -84,7 +68,8 @@ __device__ __forceinline__ void rows_tile(const LevelViewT<C, V>& L, int cur, co
     // one, zeros all four; rows outside the grid read the first pair of the upper halo row.
     const int e = min(max(xa, -2), w) + 1;
     // (a whole wavefront per row keeps the row's part scalar and 64 bits wide; the others add it per lane in 32 bits,
-    // which reaches levels of less than kRowsWide elements)
+    // which reaches every level of a grid of 2^28 cells, the most that fs_grid_create takes: padded, thin ones have the
+    // most elements, 3 * 2^28)
     struct Index {
         size_t row;
         unsigned at;
@@ -426,9 +411,6 @@ void k_rows_batch(const BatchItem* __restrict__ items, const int* __restrict__ i
         local - row * columns, row);
 }
 
-// Elements of a level from which byte offsets of FP32 fields pass 32 bits.
-constexpr size_t kRowsWide = (size_t)1 << 30;
-
 template <int JACOBI, int MODE, class C, class V, class VC>
 void launch_rows_mode(hipStream_t st, const LevelViewT<C, V>& L, int cur, const V* rhs, const double* shift,
     const SmoothWeights& wt, int nu, const CoarseLinkT<VC>& link, const LevelViewT<C, VC>& Cl, AxisRestrict rx,
@@ -442,10 +424,8 @@ void launch_rows_mode(hipStream_t st, const LevelViewT<C, V>& L, int cur, const 
 #define FS_ROWS(G, NW, M)                                                                                        \
     hipLaunchKernelGGL((k_rows<JACOBI, MODE, G, NW, M, C, V, VC>), dim3(tiles(2 * G, NW * 64 / G * M)), dim3(64 * NW), 0, \
         st, L, cur, rhs, shift, wt, nu, link, Cl, rx, ry, status)
-    // levels too large for 32-bit byte offsets take the tiles with a wavefront per row
-    const bool wide = (size_t)L.s * (L.h + 2) >= kRowsWide;
     if constexpr (MODE == kRowsPreRestrict) {
-        switch (wide ? std::min(tile, 1) : tile) {
+        switch (tile) {
         case 0: FS_ROWS(64, 16, 8); break;
         case 1: FS_ROWS(64, 16, 4); break;
         case 2: FS_ROWS(32, 8, 4); break;
@@ -454,7 +434,7 @@ void launch_rows_mode(hipStream_t st, const LevelViewT<C, V>& L, int cur, const 
         default: FS_ROWS(16, 4, 2); break;
         }
     } else {
-        switch (wide ? tile & 1 : tile) {
+        switch (tile) {
         case 0: FS_ROWS(64, 8, 8); break;
         case 1: FS_ROWS(64, 16, 4); break;
         case 2: FS_ROWS(32, 8, 4); break;

@@ -17,19 +17,6 @@ namespace fsim {
 
 namespace {
 
-__device__ __forceinline__ float from_left(float v)
-{
-    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x138, 0xf, 0xf, true));
-}
-__device__ __forceinline__ float from_right(float v)
-{
-    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x130, 0xf, 0xf, true));
-}
-
-template <class T> struct __attribute__((packed, aligned(alignof(T)))) Pair {
-    T a, b;
-};
-
 // One level in registers.
 template <int M> struct Held {
     float x[M][2], wr[M][2], wd[M][2], wu[2], wl[M], inv[M][2], cb[M][2];

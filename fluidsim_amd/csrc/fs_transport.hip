@@ -129,18 +129,6 @@ __device__ __forceinline__ double pass_scale(const TransportDev& t, double scale
 // rebuildDensity and rebuildMomentum (FluidGridCPU.cpp:1399-1476) and the largest cell outflow (:366-386), one partial
 // per 64 x 16 tile: each cell with its left and top face, and the far walls.
 // ------------------------------------------------------------------------------------------
-// v of the next lower / higher lane.
-__device__ __forceinline__ double from_left(double v)
-{
-    return __hiloint2double(__builtin_amdgcn_update_dpp(0, __double2hiint(v), 0x138, 0xf, 0xf, true),
-        __builtin_amdgcn_update_dpp(0, __double2loint(v), 0x138, 0xf, 0xf, true));
-}
-__device__ __forceinline__ double from_right(double v)
-{
-    return __hiloint2double(__builtin_amdgcn_update_dpp(0, __double2hiint(v), 0x130, 0xf, 0xf, true),
-        __builtin_amdgcn_update_dpp(0, __double2loint(v), 0x130, 0xf, 0xf, true));
-}
-
 __global__ __launch_bounds__(kNT) void k_tr_begin(TransportDev t)
 {
     constexpr int R = 4;   // rows per wavefront: a cell's density is summed once, for the row below and the next lane too

@@ -231,8 +231,6 @@ __global__ __launch_bounds__(kVT) void k_vis_coarser(VLev F, VLev L, float spaci
         L.mat[y * L.w + x] = coarse_material(F, x, y);
 }
 
-// ---- set-up of the correction system ----
-
 // ---- transfers of the batched solve ----
 
 // Face-location bilinear transfer (ViscosityKernels.h:286-316).

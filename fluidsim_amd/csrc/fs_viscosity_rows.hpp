@@ -19,16 +19,6 @@ namespace fsim {
 
 namespace {
 
-// lane l receives the value of lane l - 1 / l + 1 (zero at the wavefront's end)
-__device__ __forceinline__ float from_left(float v)
-{
-    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x138, 0xf, 0xf, true));
-}
-__device__ __forceinline__ float from_right(float v)
-{
-    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x130, 0xf, 0xf, true));
-}
-
 // Element (row y, column x) of a slot field, clamped: the row's part is uniform in a wavefront.
 template <class T> __device__ __forceinline__ T* slot_row(T* p, int w, int h, int y)
 {
