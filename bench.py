@@ -571,8 +571,8 @@ def batch_leg(count, seed=4, splits=(0,)):
     fs_batch_project over all of them (each phase one launch over all their tiles).  Each instance's
     implicit viscosity solve (nu log-uniform 1e-3..1) is timed the same two ways: fs_apply_viscosity one
     grid after another, then fs_batch_apply_viscosity over all of them.  `splits` are the
-    fs_context_set_batch_split values timed (viscous instances above the split run the multi-kernel solve beside
-    the persistent launch; the projections have no split); the first one is the headline batched number."""
+    fs_context_set_batch_split values timed for the viscosity (instances above the split run the multi-kernel solve
+    beside the persistent launch; the projections have no split); the first one is its headline batched number."""
     from fluidsim_amd import (FluidGridHIP, FluidMixture, MixtureComponent, batch_apply_viscosity, batch_project,
                               tune_batch_smoother, FS_TRANSPORT_NONE)
     from fluidsim_amd import workloads as WL
@@ -621,21 +621,14 @@ def batch_leg(count, seed=4, splits=(0,)):
     serial_s = time.perf_counter() - t0
     note(f"serial {serial_s * 1e3:.1f} ms")
     ctx = grids[0].context
-    by_split = {}
-    for split in splits:
-        ctx.set_batch_split(split)
-        restore()
-        batch_project(grids, dt, 2000, taus)
-        restore()
-        t0 = time.perf_counter()
-        res = batch_project(grids, dt, 2000, taus)
-        by_split[split] = (time.perf_counter() - t0, res)
-        note(f"batched (split {split} cells) {by_split[split][0] * 1e3:.1f} ms")
-    batch_s, batched = by_split[splits[0]]
-    ok = all(r.converged for r in serial) and all(all(r.converged for r in v[1]) for v in by_split.values())
-    # the same projections with the red-black sweep counts fs_tune_batch_smoother picks for this batch (at
-    # the headline split), batched and one by one with that choice
-    ctx.set_batch_split(splits[0])
+    restore()
+    t0 = time.perf_counter()
+    batched = batch_project(grids, dt, 2000, taus)
+    batch_s = time.perf_counter() - t0
+    note(f"batched {batch_s * 1e3:.1f} ms")
+    ok = all(r.converged for r in serial) and all(r.converged for r in batched)
+    # the same projections with the red-black sweep counts fs_tune_batch_smoother picks for this batch, batched and
+    # one by one with that choice
     restore()
     t0 = time.perf_counter()
     tuned_choice = tune_batch_smoother(grids, dt, 2000, taus)
@@ -646,7 +639,6 @@ def batch_leg(count, seed=4, splits=(0,)):
     tuned = batch_project(grids, dt, 2000, taus)
     tuned_s = time.perf_counter() - t0
     note(f"batched with the tuned sweeps {tuned_s * 1e3:.1f} ms")
-    ctx.set_batch_split(0)
     restore()
     for g, tau in zip(grids, taus):
         g.project(dt, 2000, tau)
@@ -693,8 +685,6 @@ def batch_leg(count, seed=4, splits=(0,)):
         "batched_solves_per_s": count / batch_s,
         "speedup": serial_s / batch_s,
         "batched_ms": batch_s * 1e3,
-        "batch_split_cells": int(splits[0]),
-        "batched_ms_by_split": {str(k): v[0] * 1e3 for k, v in by_split.items()},
         "converged_all": bool(ok),
         "pcg_iterations": {"serial_mean": float(np.mean([r.iterations for r in serial])),
                            "batched_mean": float(np.mean([r.iterations for r in batched]))},
@@ -706,6 +696,7 @@ def batch_leg(count, seed=4, splits=(0,)):
         "viscosity_solves_per_s_serial": count / visc_s,
         "viscosity_solves_per_s_batched": count / visc_batch_s,
         "viscosity_speedup": visc_s / visc_batch_s,
+        "viscosity_batch_split_cells": int(splits[0]),
         "viscosity_batched_ms_by_split": {str(k): v[0] * 1e3 for k, v in visc_by_split.items()},
         "viscosity_iterations": {"serial_mean": float(np.mean(vits)), "batched_mean": float(np.mean(bvits))},
         "projection_plus_viscosity_speedup": (serial_s + visc_s) / (batch_s + visc_batch_s),

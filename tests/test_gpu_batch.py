@@ -1,16 +1,16 @@
-"""Batched projection on the GPU (fs_batch_project): one persistent launch runs the PCG iterations of
-many grids of different sizes, one workgroup per grid.
+"""Batched projection on the GPU (fs_batch_project): every phase of the projections of many grids of different sizes is
+one launch over all their tiles.
 
 Each grid's result must follow fs_project's contract and agree with the single-grid projection and with
-the FP64 oracle to the step tolerance (only the FP64 reduction order differs, so not bit for bit); a
-grid's result must be the same alone and in any batch, bit for bit (every workgroup reads only its own
-grid); diagonal and multigrid grids mix; malformed batches are rejected.
+the FP64 oracle to the step tolerance (bit for bit with the former in test_gpu_batch_launches.py); a
+grid's result must be the same alone and in any batch, bit for bit; diagonal and multigrid grids mix; malformed
+batches are rejected.  Batched viscosity (fs_batch_apply_viscosity): one persistent launch, one workgroup per grid.
 """
 import numpy as np
 import pytest
 
 from fluidsim_amd import (FS_PRECOND_DIAGONAL, FS_TRANSPORT_NONE, Context, FluidGridHIP, FluidGridState,
-                          FluidMixture, MixtureComponent, batch_project)
+                          FluidMixture, MixtureComponent, batch_apply_viscosity, batch_project)
 from fluidsim_amd import workloads as WL
 
 pytestmark = pytest.mark.gpu
@@ -95,41 +95,41 @@ def test_alone_equals_in_any_batch():
         g.destroy()
 
 
-def test_split_batch_runs_large_grids_through_the_single_grid_solve():
-    """fs_context_set_batch_split: grids above the split get fs_project's own result bit for bit (the
-    multi-kernel solve, run beside the persistent launch), the others the persistent launch's result
-    bit for bit -- each grid's route depends only on its size."""
+def test_split_leaves_batched_projections_as_they_are():
+    """fs_context_set_batch_split concerns batched viscosity only: with a split or without, every grid's batched
+    projection is fs_project's on the same state, bit for bit."""
     ctx = Context(0)
     split = 10000
     grids = [pool_grid(W, H, 300 + k, context=ctx)[0] for k, (W, H) in enumerate(SHAPES)]
     taus = [tau_of(g) for g in grids]
-    large = [W * H > split for W, H in SHAPES]
-    assert 0 < sum(large) < len(SHAPES)
+    assert 0 < sum(W * H > split for W, H in SHAPES) < len(SHAPES)
     ctx.set_batch_split(split)
     res = batch_project(grids, 0.002, 2000, taus)
     ctx.set_batch_split(0)
-    for k, ((W, H), g, r, tau) in enumerate(zip(SHAPES, grids, res, taus)):
+    unsplit = [pool_grid(W, H, 300 + k, context=ctx)[0] for k, (W, H) in enumerate(SHAPES)]
+    res0 = batch_project(unsplit, 0.002, 2000, taus)
+    for k, ((W, H), g, g0, r, r0, tau) in enumerate(zip(SHAPES, grids, unsplit, res, res0, taus)):
         ref_grid, _ = pool_grid(W, H, 300 + k, context=ctx)
-        if large[k]:
-            rr = ref_grid.project(0.002, 2000, tau)
-        else:
-            rr = batch_project([ref_grid], 0.002, 2000, tau)[0]
+        rr = ref_grid.project(0.002, 2000, tau)
         assert r.converged and r.max_divergence <= tau, (W, H, r)
-        assert (r.iterations, r.max_divergence) == (rr.iterations, rr.max_divergence), (W, H, r, rr)
-        s, sr = g.download(), ref_grid.download()
-        for name in ("u", "v", "pressure"):
-            assert np.array_equal(getattr(s, name), getattr(sr, name)), (W, H, name)
+        sr = ref_grid.download()
+        for grid, result in ((g, r), (g0, r0)):
+            assert (result.iterations, result.max_divergence) == (rr.iterations, rr.max_divergence), (W, H, result, rr)
+            s = grid.download()
+            for name in ("u", "v", "pressure"):
+                assert np.array_equal(getattr(s, name), getattr(sr, name)), (W, H, name)
         ref_grid.destroy()
     with pytest.raises(ValueError):
         ctx.set_batch_split(-1)
-    for g in grids:
+    for g in grids + unsplit:
         g.destroy()
     ctx.close()
 
 
-def test_single_stream_context_batches_every_grid():
-    """A context without the helper stream (FS_CONTEXT_SINGLE_STREAM) ignores the batch split: a grid above
-    it gets the persistent launch's result, bit for bit the one it gets alone in an unsplit batch."""
+def test_single_stream_context_projects_batches_alike():
+    """A grid's projection in a batch on a context without the helper stream (FS_CONTEXT_SINGLE_STREAM) is the one it gets
+    alone, bit for bit; and its viscosity in a batch ignores the split, so a grid above it gets the persistent
+    launch's result."""
     ctx = Context(0, single_stream=True)
     W, H = SHAPES[6]                                  # 200 x 150 = 30000 cells, above the split below
     a, _ = pool_grid(W, H, 500, context=ctx)
@@ -142,6 +142,15 @@ def test_single_stream_context_batches_every_grid():
     assert r.converged and (r.iterations, r.max_divergence) == (rb.iterations, rb.max_divergence)
     assert np.array_equal(a.download().pressure, b.download().pressure)
     for g in small + [a, b]:
+        g.destroy()
+    va, vb, vs = (viscous_grid(w, h, 70, 0.05, context=ctx) for w, h in ((W, H), (W, H), (40, 30)))
+    ctx.set_batch_split(10000)
+    n = batch_apply_viscosity([vs, va], 0.01)[1]
+    ctx.set_batch_split(0)
+    assert n > 0 and batch_apply_viscosity([vb], 0.01) == [n]
+    x, y = va.download(), vb.download()
+    assert np.array_equal(x.u, y.u) and np.array_equal(x.v, y.v)
+    for g in (va, vb, vs):
         g.destroy()
     ctx.close()
 
@@ -290,8 +299,6 @@ def test_batched_viscosity_matches_single_solves():
     the same stopping rule as fs_apply_viscosity on the same grid (iteration counts within 2, velocities
     within the 1e-4 solve tolerance), grids without viscosity are untouched, and a grid's result is the
     same alone and in the batch, bit for bit."""
-    from fluidsim_amd import batch_apply_viscosity
-
     dt = 0.01
     grids = [viscous_grid(W, H, 60 + k, nu) for k, (W, H, nu) in enumerate(VISC_SHAPES)]
     singles = [viscous_grid(W, H, 60 + k, nu) for k, (W, H, nu) in enumerate(VISC_SHAPES)]
@@ -320,8 +327,6 @@ def test_split_batched_viscosity_runs_large_grids_through_the_single_grid_solve(
     """With fs_context_set_batch_split, grids above the split get fs_apply_viscosity's result bit for bit
     (their own solve, beside the persistent launch) and the others the persistent launch's result bit
     for bit."""
-    from fluidsim_amd import batch_apply_viscosity
-
     dt = 0.01
     ctx = Context(0)
     split = 10000
@@ -348,8 +353,6 @@ def test_batched_viscosity_of_c4_instances_matches_the_oracle(oracle):
     step agrees with the FP64 oracle's FluidGridGPU::applyViscosity restatement on the same state within
     3e-4 of the velocity scale (the solve stops at a 1e-4 relative residual in the mass norm; the GPU
     iterates in FP32), the bar of the single-grid viscosity tests."""
-    from fluidsim_amd import batch_apply_viscosity
-
     wls = [wl for wl in WL.batch_instances(4, 40) if wl.width * wl.height <= 120_000][:12]
     assert len(wls) == 12 and max(wl.width * wl.height for wl in wls) > 60_000
     dt = wls[0].dt

@@ -1,7 +1,7 @@
 """Batched timesteps on the GPU (fs_batch_step) and the serving loop's batched route.
 
 fs_batch_step is fs_step on many grids at once, each with its own dt, budget and tolerance; its viscosity
-solves and projections run in the batched persistent launches.  Checked here:
+solves run in one persistent launch and its projections in launches shared by all grids.  Checked here:
   - each grid's step agrees with fs_step on a copy: the fractions bit for bit after the first step
     (transport runs first, from the same state), velocities to the batched solves' rounding, iteration
     counts within a few, and every projection converges;
