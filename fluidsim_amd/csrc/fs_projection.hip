@@ -940,7 +940,7 @@ __device__ __forceinline__ void decide(const GridDev& g, const Recurrence& c, co
         S->status = kStopped;
 }
 
-// Check and decision of a small grid in one launch, a launch less of the six beside its V-cycle: one workgroup, a
+// Check and decision of a small grid in one launch, four launches beside its V-cycle instead of five: one workgroup, a
 // 256-thread group per tile, the sums in the order of the two launches.  61 x 47 (3 tiles) 6% per solve; with 16 tiles in
 // four rounds a check on one compute unit costs what the launch saves (128 x 128: 4341 us against 4323), so only where
 // one round takes them all.

@@ -17,8 +17,9 @@
 // What bounds it: VALU issue and latency on tiles that fit the chip once, HBM beyond.  Measured against the same
 // smoothers on LDS tiles (per launch): red-black V(4) post-smoothing 2048^2 65.3 -> 25.7 us, 1920x1080 34.2 -> 15.5,
 // 1024^2 18.1 -> 9.5, 256^2 5.9 -> 5.1; pre-smoothing + residual + restriction 2048^2 54.5 -> 27.9, 1920x1080
-// 29.7 -> 15.9, 257x129 9.3 -> 5.8; Chebyshev with 8 sweeps post 2048^2 65.7 -> 39.4, pre + restriction
-// 71.1 -> 43.1, 257x129 9.7 -> 7.4 (about 2.3 us of each is the launch).
+// 29.7 -> 15.9, 257x129 9.3 -> 5.8; Chebyshev with 8 sweeps post 2048^2 65.7 -> 37.2 (on a tile chosen for it; 42 to 48
+// on those the tuner may keep from 3 sweeps), pre + restriction 71.1 -> 43.1, 257x129 9.7 -> 7.4 (about 2.3 us of
+// each is the launch).
 #include "fs_kernels.hpp"
 #include "fs_mg_device.hpp"
 

@@ -14,8 +14,9 @@
  *     "requires uniform WebGPU" throws, FS_E_DEVICE / FS_E_RUNTIME to std::runtime_error;
  *   - numerical non-convergence is NOT an error: it is reported in fs_projection_result;
  *   - fs_last_error() returns the message of the last failing call on this thread;
- *   - a grid is owned by one thread (FluidGridBase.h:37-39); distinct grids may be used from
- *     distinct threads.
+ *   - a grid is owned by one thread (FluidGridBase.h:37-39); grids of distinct contexts may be used from
+ *     distinct threads at once.  The grids of one context share its stream and read-back slots: one thread at a
+ *     time (fs_viscosity_solve_noalloc alone may run beside them, it has a slot of its own).
  *
  * Layouts are the reference's (FluidGridCPU.h:128-130, FluidGridTypes.h:10-20): cells W*H
  * row-major with y growing downward, u (W+1)*H, v W*(H+1), component masses component-major
@@ -415,7 +416,7 @@ fs_status fs_context_set_batch_split(fs_context* ctx, long long solo_cells);
  * split, and fs_batch_project's shared launches; grids with 16-bit multigrid levels project one by one).  results[i]
  * follows fs_step's contract: a grid stops after its first substep whose projection does not converge, and
  * dts[i] <= 0 leaves it untouched with physical_steps = 0.  Values agree with fs_step to rounding (the batched
- * solves reduce in another order), and a grid's result does not depend on the other grids of the batch.  A
+ * viscosity solves reduce in another order), and a grid's result does not depend on the other grids of the batch.  A
  * grid whose step fails (transport, viscosity or solver error) stops there; statuses[i] (may be NULL)
  * receives FS_OK or FS_E_RUNTIME per grid, and the call returns FS_E_RUNTIME with the lowest failing index's
  * message after every other grid has been stepped. */
