@@ -742,7 +742,8 @@ def main():
     ap.add_argument("--batch-instances", type=int, default=256, help="size of the C4 batched-solve leg (0: skip)")
     ap.add_argument("--batch-only", action="store_true")
     ap.add_argument("--batch-splits", type=str, default="131072,0",
-                    help="fs_context_set_batch_split values to time (cells; the first is reported as batched)")
+                    help="fs_context_set_batch_split values to time for the batched viscosity (cells; the first is "
+                         "reported)")
     ap.add_argument("--precision-size", type=int, default=2048, help="side of the C3 mixed-precision leg (0: skip)")
     ap.add_argument("--precision-steps", type=int, default=3)
     ap.add_argument("--precision-only", action="store_true")
